@@ -24,10 +24,10 @@
  * two workgroups per CU to cover them).
  *
  * Any M and N (rows are clamped on load, stores are bounded); K must be a multiple
- * of 8 with 16-byte aligned rows, otherwise the scalar kernel below takes over (the
- * only such caller is the 3-channel input convolution of the VAE encoder).
+ * of 8 with 16-byte aligned rows, otherwise the scalar kernel below takes over.
  *
- * Convolution with a multiple of 64 input channels (every layer of the VAE but its first) is an
+ * Convolution with a handful of input or output channels (the VAE's first and last layers) has kernels of its own
+ * (conv_gfx950.hip). With a multiple of 64 input channels it is an
  * implicit GEMM: the image is converted to bf16 once and k_gemm_dma fetches the pixels under each
  * tap itself, so the k x k patches are never written out. Other shapes gather the patches as bf16
  * rows into scratch (what the reference does for all of them, iris_cuda.cu:959-985) and run the
@@ -985,6 +985,8 @@ int iris_hip_conv2d(void *stream, uint16_t *scratch, size_t scratch_bytes, float
     const int ow = (width + pad_before + pad_after - k) / stride + 1;
     if (oh <= 0 || ow <= 0) return 0;
     const int ohw = oh * ow, row_len = k * k * cin;
+    const int direct = iris_hip_conv2d_direct(stream, out, in, w, bias, h, width, cin, cout, k, stride, pad_before, oh, ow);
+    if (direct != -2) return direct;
 
     /* Implicit GEMM: the image once as bf16 (the rows a chunk of output rows needs), then k_gemm_dma in its
      * convolution mode straight on it; no patch matrix. Needs cin % 64 == 0 (a k tile inside one tap). */

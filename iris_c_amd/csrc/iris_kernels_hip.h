@@ -154,6 +154,11 @@ int iris_hip_conv2d(void *stream, uint16_t *scratch, size_t scratch_bytes, float
                     const uint16_t *w, const float *bias, int h, int width, int cin, int cout, int k,
                     int stride, int pad_before, int pad_after);
 
+/* Convolution of the shapes that need neither scratch nor a patch matrix (conv_gfx950.hip); -2 = not one of them, nothing
+ * enqueued. oh, ow: output size. */
+int iris_hip_conv2d_direct(void *stream, float *out, const float *in, const uint16_t *w, const float *bias, int h, int width,
+                           int cin, int cout, int k, int stride, int pad_before, int oh, int ow);
+
 /* Linear layer through hipBLASLt (linear_hipblaslt.cpp; the library is opened with dlopen at the
  * first call). Returns 0 when the product was enqueued, 1 when the caller must use its own
  * kernel: library absent, or no algorithm for this problem. Operands contiguous as above. */

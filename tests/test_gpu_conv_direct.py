@@ -1,0 +1,45 @@
+"""The convolutions that work straight on the f32 image (conv_gfx950.hip), at the sizes where their tiles and remainders
+begin and end, against the CPU oracle (bf16-rounded operands, f32 sums: the bar is the rounding of the sum's order)."""
+import numpy as np
+import pytest
+
+import oracle as O
+from gpu_harness import Dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    return Dev()
+
+
+def conv_case(dev, orc, h, w, cin, cout, k, stride, pb, pa, bias=True):
+    rng = np.random.default_rng(h * 1000 + w + cout)
+    img = rng.standard_normal((h * w, cin)).astype(np.float32)
+    wt = O.f32_to_bf16((rng.standard_normal((cout, k * k * cin)) * 0.1).astype(np.float32))
+    b = rng.standard_normal(cout).astype(np.float32) if bias else np.zeros(cout, np.float32)
+    want = orc.dev_conv2d(img, wt, b, h, w, k, stride, pb, pa)
+    guard = 64                                               # floats behind the output that must stay as they are
+    out = dev.put(np.full(want.size + guard, 7.0, np.float32))
+    dev.lib.iris_dev_conv2d(out, dev.put(img), dev.put(wt), dev.put(b) if bias else None, h, w, cin, cout, k, stride, pb, pa)
+    dev.check()
+    got = dev.get(out, (want.size + guard,), np.float32)
+    dev.free_all()
+    assert (got[want.size:] == 7.0).all()
+    np.testing.assert_allclose(got[:want.size].reshape(want.shape), want, atol=2e-5 * np.sqrt(k * k * cin))
+
+
+@pytest.mark.parametrize("h,w,cin,cout,k,stride,pb,pa,bias", [
+    (1, 1, 3, 128, 3, 1, 1, 1, True), (37, 29, 3, 128, 3, 1, 1, 1, True), (16, 5, 3, 130, 3, 1, 1, 1, False),
+    (20, 21, 3, 260, 3, 2, 0, 1, True), (9, 9, 8, 64, 2, 1, 0, 0, True), (17, 3, 1, 12, 5, 1, 2, 2, True)])
+def test_few_input_channels(dev, orc, h, w, cin, cout, k, stride, pb, pa, bias):
+    conv_case(dev, orc, h, w, cin, cout, k, stride, pb, pa, bias)
+
+
+@pytest.mark.parametrize("h,w,cin,cout,k,stride,pb,pa,bias", [
+    (1, 1, 128, 3, 3, 1, 1, 1, True), (16, 32, 128, 3, 3, 1, 1, 1, True), (17, 33, 128, 3, 3, 1, 1, 1, False),
+    (40, 70, 32, 3, 3, 1, 1, 1, True), (15, 31, 64, 2, 3, 1, 0, 0, True), (33, 20, 64, 28, 1, 1, 0, 0, True),
+    (21, 34, 128, 7, 2, 1, 0, 1, True)])
+def test_few_output_channels(dev, orc, h, w, cin, cout, k, stride, pb, pa, bias):
+    conv_case(dev, orc, h, w, cin, cout, k, stride, pb, pa, bias)
