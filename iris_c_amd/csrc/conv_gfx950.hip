@@ -4,12 +4,14 @@
  *
  * k_conv_few_in: k * k * cin <= 32, the 3-channel input of the VAE encoder.
  * k_conv_few_out: k * k * cout <= 28, the 3-channel output of the VAE decoder.
+ * k_conv_3x3: 3 x 3, stride 1, cin a multiple of 64: every other layer of the VAE but the 1 x 1 and the halving ones.
  *
- * Both are bound by memory: one side of the product is so thin that the image on the other side is all there is to
- * move. The image is rounded to bf16 on the way into the matrix core, products are summed in f32.
+ * The first two are bound by memory: one side of the product is so thin that the image on the other side is all there
+ * is to move. The image is rounded to bf16 on the way into the matrix core, products are summed in f32.
  */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 #include "iris_kernels_hip.h"
 
@@ -204,6 +206,211 @@ k_conv_few_out(float *__restrict__ out, const float *__restrict__ in, const uint
     }
 }
 
+/* ---- 3 x 3 ----
+ *
+ * A workgroup makes 16 x 16 output pixels of 128 channels. For 64 input channels at a time, the 18 x 18 pixels under the
+ * tile are read ONCE as f32, rounded and kept in the LDS; the nine taps are nine shifted views of them, so the image
+ * passes from the L2 to the CU 1.27 times instead of nine, and no bf16 copy of it is made first. The weights of a (tap,
+ * 64 channels) step, 128 rows of 128 B, go straight from memory into one of three LDS stages.
+ *
+ * Eight waves, 4 (rows of four pixels) x 2 (64 channels), two per SIMD: a wave owns 64 pixels x 64 channels = 4 x 4
+ * accumulator blocks, and a step is 32 products per wave: 16 of the first half of the step's channels, the barrier, 16 of
+ * the second half. The operands of a half are requested from the LDS one half ahead, across the barrier too.
+ *  - In front of the barrier of step s the wave waits until its own share of the weights of step s + 1 has landed and its
+ *    last operands of step s have been read; so behind it stage s % 3 is free, and the weights of step s + 3 are
+ *    requested into it: they have two steps to land.
+ *  - The pixels of the next 64 channels (2592 pieces of 8 channels, six per thread) are fetched into registers in steps
+ *    0 - 5 and written to the other image buffer three steps later: the wait of the step before covers them, since loads
+ *    complete in order and the weights that it waits for were requested behind them.
+ * A pixel takes 160 B of LDS (64 channels + 32 B): the 16 lanes that a 128-bit read serves together are eight pixels with
+ * one chunk and the eight between them with the next, and with a stride of ten 16 B units, whichever pixel the
+ * tap starts at, they fall into distinct bank windows; a tap's shift is an immediate offset. Weight rows are swizzled as
+ * in gemm_conv_gfx950.hip.
+ *
+ * Measured against a bf16 copy of the image + implicit product that fetches every tap from the L2 (copy + product):
+ * 512 x 512 pixels, 128 -> 128 30 + 118 -> 91 us, 256 -> 128 76 + 214 -> 141 us (1100 TFLOP/s), 256 -> 256 88 + 290 ->
+ * 271 us (1140). A step takes 0.68 us (1500 cycles, 1024 of them products); a workgroup's first pixels and its stores
+ * take 11 us that nothing overlaps. */
+constexpr int C3_T = 16, C3_H = C3_T + 2, C3_PIXELS = C3_H * C3_H, C3_ROW = 80, C3_IMG = C3_PIXELS * C3_ROW;   /* elements */
+constexpr int C3_N = 128, C3_STAGE = C3_N * 64, C3_UNITS = 6;
+constexpr int C3_LDS = (2 * C3_IMG + 3 * C3_STAGE) * 2;
+
+__device__ __forceinline__ uint32_t lds_address(const uint16_t *p) {
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
+}
+
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"                /* M0 in a clobber list */
+__global__ void __launch_bounds__(512, 2)
+k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t *__restrict__ W, const float *__restrict__ bias,
+           ConvShape s, int tiles_x, int tiles_n, int total, int per_xcd) {
+    extern __shared__ __align__(16) uint16_t lds[];            /* image, image, weights, weights, weights */
+    /* an XCD takes a contiguous range of the tiles, the channel tiles of a pixel tile next to each other: they share the
+     * image in its L2 */
+    const int work = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if (work >= total) return;
+    const int tile = work / tiles_n, n0 = (work - tile * tiles_n) * C3_N;
+    const int ty0 = tile / tiles_x * C3_T, tx0 = tile % tiles_x * C3_T;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lg = lane >> 4, wm = wave & 3, wn = wave >> 2;
+
+    /* image staging: unit u of this thread is channels 8 (tid % 8) .. + 7 of pixel tid / 8 + 64 u of the rimmed tile; a
+     * pixel outside the image reads the first one and is zeroed */
+    uint32_t uoff[C3_UNITS];                                   /* bytes from the channel group's first value */
+    bool inside[C3_UNITS];
+#pragma unroll
+    for (int u = 0; u < C3_UNITS; u++) {
+        const int px = (tid >> 3) + 64 * u, py = px / C3_H, y = ty0 + py - s.pad, x = tx0 + (px - py * C3_H) - s.pad;
+        inside[u] = px < C3_PIXELS && y >= 0 && y < s.h && x >= 0 && x < s.w;
+        uoff[u] = ((inside[u] ? (uint32_t)(y * s.w + x) * (uint32_t)s.cin : 0u) + 8u * (tid & 7)) * 4u;
+    }
+    const int st_off = (tid >> 3) * C3_ROW + 8 * (tid & 7);
+    auto put = [&](int img, int u, f32x4 lo, f32x4 hi) {
+        u32x4 v = {pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3])};
+        if (!inside[u]) v = u32x4{0, 0, 0, 0};
+        if (u + 1 < C3_UNITS || tid < 8 * (C3_PIXELS - 64 * (C3_UNITS - 1)))
+            *reinterpret_cast<u32x4 *>(&lds[img + st_off + u * 64 * C3_ROW]) = v;
+    };
+
+    /* weights: rows 16 wave .. + 15 of a stage in two pieces of eight rows; rows past the last channel repeat it (their
+     * results are never stored) */
+    const int row_len = 9 * s.cin;
+    uint32_t woff[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int r = 16 * wave + 8 * j + (lane >> 3), n = n0 + r < s.cout ? n0 + r : s.cout - 1;
+        woff[j] = ((uint32_t)n * (uint32_t)row_len + 8u * ((lane & 7) ^ ((r >> 1) & 7))) * 2u;
+    }
+    uint16_t *w_lds = lds + 2 * C3_IMG;
+    auto request = [&](int tap, int c0, int stage) {
+        const uint16_t *src = W + (size_t)tap * s.cin + c0;
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                         ::"s"(lds_address(w_lds + stage * C3_STAGE + (16 * wave + 8 * j) * 64)), "v"(woff[j]), "s"(src) : "memory", "m0");
+    };
+
+    f32x4 acc[4][4];                                           /* [16 channels][row of 16 pixels] */
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+#pragma unroll
+        for (int b = 0; b < 4; b++) acc[a][b] = f32x4{0, 0, 0, 0};
+    u32x4 av[2][4], bv[2][4];
+    int a_rd[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) a_rd[ks] = 2 * C3_IMG + (64 * wn + li) * 64 + 8 * ((4 * ks + lg) ^ (li >> 1));
+    const int b_rd = (4 * wm * C3_H + li) * C3_ROW + 8 * lg;
+    auto operands = [&](int img, int tap, int ks) {            /* stage of a tap: tap % 3, nine steps per channel group */
+#pragma unroll
+        for (int a = 0; a < 4; a++) av[ks][a] = *reinterpret_cast<const u32x4 *>(&lds[a_rd[ks] + (tap % 3) * C3_STAGE + 16 * a * 64]);
+#pragma unroll
+        for (int b = 0; b < 4; b++)
+            bv[ks][b] = *reinterpret_cast<const u32x4 *>(&lds[img + b_rd + ((b + tap / 3) * C3_H + tap % 3) * C3_ROW + 32 * ks]);
+    };
+    auto products = [&](int ks) {
+#pragma unroll
+        for (int a = 0; a < 4; a++)
+#pragma unroll
+            for (int b = 0; b < 4; b++) acc[a][b] = mfma(av[ks][a], bv[ks][b], acc[a][b]);
+    };
+
+    const int groups = s.cin / 64;
+    f32x4 xr[3][2];                                            /* three image units on their way */
+    /* One group of 64 channels: nine steps. `img` holds it, the next one goes to `other`. */
+    auto channel_group = [&](auto last_group, int g, int img, int other) {
+        constexpr bool LAST = decltype(last_group)::value;
+        const float *next = in + 64 * (g + 1);
+#pragma unroll
+        for (int t = 0; t < 9; t++) {
+            operands(img, t, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            if (!LAST && t >= 3) put(other, t - 3, xr[t % 3][0], xr[t % 3][1]);
+            if (!LAST && t < C3_UNITS) {
+                asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(xr[t % 3][0]) : "v"(uoff[t]), "s"(next) : "memory");
+                asm volatile("global_load_dwordx4 %0, %1, %2 offset:16" : "=v"(xr[t % 3][1]) : "v"(uoff[t]), "s"(next) : "memory");
+            }
+            products(0);
+            __builtin_amdgcn_sched_barrier(0);
+            /* newer than the weights of step t + 1: the image loads of steps t - 1 and t, the weights of step t + 2 */
+            constexpr int IMAGE = LAST ? 0 : 2;
+            const int newer = (t >= 1 && t - 1 < C3_UNITS ? IMAGE : 0) + (t < C3_UNITS ? IMAGE : 0) + (LAST && t > 6 ? 0 : 2);
+            if (newer == 6) asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            else if (newer == 4) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            else if (newer == 2) asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if (!LAST && t >= 2 && t - 2 < C3_UNITS) asm volatile("" : "+v"(xr[(t - 2) % 3][0]), "+v"(xr[(t - 2) % 3][1]));
+            if (!LAST || t < 8) operands(t < 8 ? img : other, t < 8 ? t + 1 : 0, 0);
+            if (!LAST || t < 6) request(t < 6 ? t + 3 : t - 6, 64 * (t < 6 ? g : g + 1), t % 3);
+            __builtin_amdgcn_sched_barrier(0);
+            products(1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    request(0, 0, 0);
+    request(1, 0, 1);
+    request(2, 0, 2);
+    {
+        f32x4 first[C3_UNITS][2];
+#pragma unroll
+        for (int u = 0; u < C3_UNITS; u++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                first[u][i] = *reinterpret_cast<const f32x4 *>(reinterpret_cast<const char *>(in) + uoff[u] + 16 * i);
+#pragma unroll
+        for (int u = 0; u < C3_UNITS; u++) put(0, u, first[u][0], first[u][1]);
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    operands(0, 0, 0);
+    int img = 0;
+    for (int g = 0; g + 1 < groups; g++) {
+        channel_group(std::false_type{}, g, img, C3_IMG - img);
+        img = C3_IMG - img;
+    }
+    channel_group(std::true_type{}, groups - 1, img, C3_IMG - img);
+
+    /* acc[a][b][r]: channel n0 + 64 wn + 16 a + 4 lg + r of pixel (4 wm + b, li) of the tile. Through the LDS (every wave has
+     * passed the last step's barrier, behind which nothing is read from it; 16 KB per wave), so that a store instruction
+     * covers four pixels x 256 B. */
+    float *buf = reinterpret_cast<float *>(lds) + wave * 4096;
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+#pragma unroll
+        for (int a = 0; a < 4; a++) *reinterpret_cast<f32x4 *>(&buf[(16 * b + li) * 64 + 4 * ((4 * a + lg) ^ li)]) = acc[a][b];
+    const int c = lane & 15, n = n0 + 64 * wn + 4 * c;
+    const bool whole = s.cout % 4 == 0 && ((uintptr_t)out & 15) == 0;
+    f32x4 bias4 = {0, 0, 0, 0};
+    for (int e = 0; e < 4; e++)
+        if (bias && n + e < s.cout) bias4[e] = bias[n + e];
+#pragma unroll
+    for (int it = 0; it < 16; it++) {
+        const int row = 4 * it + (lane >> 4), y = ty0 + 4 * wm + (row >> 4), x = tx0 + (row & 15);
+        const f32x4 v = *reinterpret_cast<const f32x4 *>(&buf[row * 64 + 4 * (c ^ (row & 15))]) + bias4;
+        if (y >= s.oh || x >= s.ow) continue;
+        float *dst = out + ((size_t)y * s.ow + x) * s.cout + n;
+        if (whole) {
+            if (n < s.cout) *reinterpret_cast<f32x4 *>(dst) = v;
+        } else {
+            for (int e = 0; e < 4; e++)
+                if (n + e < s.cout) dst[e] = v[e];
+        }
+    }
+}
+#pragma clang diagnostic pop
+
+int launch_3x3(hipStream_t st, float *out, const float *in, const uint16_t *W, const float *bias, const ConvShape &s) {
+    static bool configured = false;
+    if (!configured) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_conv_3x3), hipFuncAttributeMaxDynamicSharedMemorySize, C3_LDS);
+        if (e != hipSuccess) return (int)e;
+        configured = true;
+    }
+    const int tiles_x = (s.ow + C3_T - 1) / C3_T, tiles_n = (s.cout + C3_N - 1) / C3_N;
+    const int total = tiles_x * ((s.oh + C3_T - 1) / C3_T) * tiles_n, per_xcd = (total + 7) / 8;
+    hipLaunchKernelGGL(k_conv_3x3, dim3((unsigned)per_xcd * 8), dim3(512), C3_LDS, st, out, in, W, bias, s, tiles_x, tiles_n, total, per_xcd);
+    return (int)hipGetLastError();
+}
+
 template <int STEPS>
 int launch_few_out(hipStream_t st, float *out, const float *in, const uint16_t *W, const float *bias, const ConvShape &s) {
     static bool configured = false;
@@ -240,6 +447,10 @@ int iris_hip_conv2d_direct(void *stream, float *out, const float *in, const uint
     if (k <= FO_MAX_K && k * k * cout <= FO_ROWS && stride == 1 && (cin == 32 || cin == 64 || cin == 128) && al16(in) && al16(w))
         return cin == 32 ? launch_few_out<1>(st, out, in, w, bias, s) : cin == 64 ? launch_few_out<2>(st, out, in, w, bias, s)
                                                                                : launch_few_out<4>(st, out, in, w, bias, s);
+    /* a thread's byte offsets into image and weights are 32-bit */
+    if (k == 3 && stride == 1 && cin % 64 == 0 && al16(in) && al16(w) && (size_t)h * width * cin * 4 < ((size_t)1 << 32) &&
+        (size_t)cout * 9 * cin * 2 < ((size_t)1 << 32))
+        return launch_3x3(st, out, in, w, bias, s);
     return -2;
 }
 

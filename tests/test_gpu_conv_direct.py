@@ -43,3 +43,11 @@ def test_few_input_channels(dev, orc, h, w, cin, cout, k, stride, pb, pa, bias):
     (21, 34, 128, 7, 2, 1, 0, 1, True)])
 def test_few_output_channels(dev, orc, h, w, cin, cout, k, stride, pb, pa, bias):
     conv_case(dev, orc, h, w, cin, cout, k, stride, pb, pa, bias)
+
+
+@pytest.mark.parametrize("h,w,cin,cout,pb,pa,bias", [
+    (1, 1, 64, 128, 1, 1, True), (16, 16, 64, 128, 1, 1, True), (17, 15, 128, 128, 1, 1, False), (33, 47, 192, 256, 1, 1, True),
+    (18, 19, 64, 130, 0, 0, True), (3, 34, 320, 37, 2, 1, True), (20, 5, 512, 512, 1, 1, True), (16, 33, 256, 3, 0, 1, False)])
+def test_three_by_three(dev, orc, h, w, cin, cout, pb, pa, bias):
+    """Tile edges (16 x 16 pixels, 128 channels), one to eight groups of 64 input channels, padding of other widths."""
+    conv_case(dev, orc, h, w, cin, cout, 3, 1, pb, pa, bias)
