@@ -19,7 +19,7 @@ HOSTDEFS = -D__HIP_PLATFORM_AMD__=1
 CFLAGS   = -O2 -fPIC -Wall -Wextra -std=c11 $(HOSTDEFS) -I$(CSRC) -Iinclude -I$(ROCM_HOME)/include
 
 HIP_SRCS = $(CSRC)/qknorm_rope.hip $(CSRC)/fa_fwd_gfx950.hip $(CSRC)/fa_fwd_hd512_gfx950.hip $(CSRC)/attn_generic.hip \
-           $(CSRC)/ew_norm_ops.hip $(CSRC)/gemm_conv_gfx950.hip $(CSRC)/conv_gfx950.hip $(CSRC)/rope_tables.hip
+           $(CSRC)/ew_norm_ops.hip $(CSRC)/gemm_conv_gfx950.hip $(CSRC)/gemm_tiles_gfx950.hip $(CSRC)/conv_gfx950.hip $(CSRC)/rope_tables.hip
 HIP_OBJS = $(HIP_SRCS:.hip=.o)
 HOST_HDRS = include/iris_dev.h include/iris_rope.h $(CSRC)/iris_kernels_hip.h $(CSRC)/iris_rope_internal.h
 

@@ -197,7 +197,8 @@ void iris_dev_attention_qnorm(uint16_t *out, int ldo,
  * (iris_transformer_flux.c:3795-3800 and 3833-3837, iris_transformer_flux3.c:692-694,
  * iris_transformer_zimage.c:1947-1949, iris_qwen3.c:1589-1593), which all issue exactly these three calls. The
  * library's own GEMM can normalise each 256 x 256 output tile while it still sits in the LDS, which saves the
- * pass that reads and rewrites the Q and K rows: that one-launch kernel runs unless the vendor GEMM is selected
+ * pass that reads and rewrites the Q and K rows (rows too few to fill the chip with such tiles: smaller tiles and the
+ * norm kernel): that kernel runs unless the vendor GEMM is selected
  * (iris_dev_linear_backend(2)) and present, for head_dim 128, rows >= 256, out >= 256 and
  * a multiple of 128, in a multiple of 64 and 16-byte aligned operands; its bits are those of the two calls
  * above on the own GEMM. Otherwise the entry issues the two calls itself (the vendor GEMM followed by the norm

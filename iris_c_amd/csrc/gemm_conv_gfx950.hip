@@ -11,8 +11,9 @@
  * the 16x16 accumulator a lane then holds four consecutive n of one output row m,
  * a single 16-byte (f32) or 8-byte (bf16) store.
  *
- * Three kernels. M, N >= 256 with K a multiple of 128 (every linear layer of the models at their
- * sequence lengths) take k_gemm_w4: tiles of 256 rows x 256, 224 or 192 columns on four waves, one per
+ * Products with too few 256-row tiles to fill the chip (short sequences) take k_gemm_tiles (gemm_tiles_gfx950.hip). For
+ * the rest, three kernels. M, N >= 256 with K a multiple of 128 (every linear layer of the models at their
+ * larger sequence lengths) take k_gemm_w4: tiles of 256 rows x 256, 224 or 192 columns on four waves, one per
  * SIMD, staged through registers. Other shapes with M, N >= 256 and K a multiple of 64, and the convolutions, take
  * k_gemm_dma: the same tiles on 8 waves, loaded straight into LDS. Both are described where they are
  * defined and give the same bits. Everything else with K a multiple of 8 takes k_gemm_bf16:
@@ -854,24 +855,43 @@ static int four_wave_width(int M, int N) {
     return best;
 }
 
-/* Which kernel a linear layer takes, host arithmetic only: 3 = k_gemm_w4 with tiles of 32 na columns, 2 = k_gemm_dma,
- * 1 = k_gemm_bf16, 0 = k_gemm_scalar. */
-struct GemmPlan { int kernel, na; };
-static GemmPlan plan_gemm(int M, int N, int K, int out_size, bool operands_aligned16, bool out_aligned16) {
+/* Which kernel a linear layer takes, host arithmetic only: 4 = k_gemm_tiles (gemm_tiles_gfx950.hip) with its tile `na` and
+ * `splits` ranges of K, 3 = k_gemm_w4 with tiles of 32 na columns, 2 = k_gemm_dma, 1 = k_gemm_bf16, 0 = k_gemm_scalar.
+ *
+ * Between 4 and 3 the estimated times decide: a k tile costs a four-wave workgroup 0.175 us per 32 columns (0.155 in a
+ * grid that leaves most CUs idle), its ends 4 us a round. Where 4 is chosen it measured, weights from HBM (four-wave or
+ * 128 x 128 kernel before): 512 x 9728 -> 2560 146 -> 38 us, 320 x 12288 -> 3072 179 -> 36, 512 x 3072 -> 9216 52 -> 37,
+ * 118 x 2560 -> 6144 41 -> 17, 80 x 12288 -> 3072 183 -> 23, 1000 x 12288 -> 3072 182 -> 75, 2115 x 3072 -> 9216 111 -> 98,
+ * 2115 x 9216 -> 3072 136 -> 103. Long grids of full rows stay: 4608 x 3072 -> 9216 would take 5 rounds of 160 x 256. */
+struct GemmPlan { int kernel, na, splits; };
+static GemmPlan plan_gemm(int M, int N, int K, int out_size, bool operands_aligned16, bool out_aligned16, size_t part_bytes) {
+    int shape = 0, splits = 1;
+    const float tiles_us = operands_aligned16 && out_aligned16 ? iris_hip_gemm_tiles_plan(M, N, K, out_size, part_bytes, &shape, &splits) : -1.0f;
     if (K > 0 && K % TK == 0 && operands_aligned16 && M >= DT && N >= DT && (size_t)K * 2 * 8 < ((size_t)1 << 31)) {
-        if (four_wave_shape(M, N, K, (size_t)out_size) && out_aligned16) return {3, four_wave_width(M, N)};
-        return {2, 8};
+        if (four_wave_shape(M, N, K, (size_t)out_size) && out_aligned16) {
+            const int na = four_wave_width(M, N);
+            const long wgs = (long)((M + DT - 1) / DT) * ((N + 32 * na - 1) / (32 * na)), rounds = (wgs + 255) / 256;
+            const float us = 4.0f + (float)rounds * ((float)(K / TK) * (wgs <= 128 ? 0.155f : 0.175f) * (float)na + 4.0f);
+            if (tiles_us < 0.0f || tiles_us >= us) return {3, na, 1};
+            return {4, shape, splits};
+        }
+        if (tiles_us < 0.0f) return {2, 8, 1};
     }
-    if (K > 0 && K % 8 == 0 && operands_aligned16) return {1, 0};
-    return {0, 0};
+    if (tiles_us >= 0.0f) return {4, shape, splits};
+    if (K > 0 && K % 8 == 0 && operands_aligned16) return {1, 0, 1};
+    return {0, 0, 1};
 }
 
+/* part: workspace for partial sums, part_bytes long (0: no ranges of K) */
 template <typename OUT>
-int gemm(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K) {
+int gemm(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, float *part, size_t part_bytes) {
     if (M <= 0 || N <= 0) return 0;
     const bool aligned16 = ((uintptr_t)x & 15) == 0 && ((uintptr_t)W & 15) == 0;
-    const GemmPlan plan = plan_gemm(M, N, K, (int)sizeof(OUT), aligned16, ((uintptr_t)y & 15) == 0);
-    if (plan.kernel == 3 || plan.kernel == 2) {
+    const GemmPlan plan = plan_gemm(M, N, K, (int)sizeof(OUT), aligned16, ((uintptr_t)y & 15) == 0, part_bytes);
+    if (plan.kernel == 4) {
+        const int e = iris_hip_gemm_tiles(st, y, (int)sizeof(OUT), x, W, M, N, K, plan.na, plan.splits, part);
+        if (e) return e;
+    } else if (plan.kernel == 3 || plan.kernel == 2) {
         const ConvGeom none = {};
         int e;
         if (plan.kernel == 3) {
@@ -933,26 +953,26 @@ k_add_bias_rows(float *__restrict__ y, const float *__restrict__ bias, int cols,
 
 extern "C" {
 
-/* The kernel a linear layer of these sizes takes (aligned operands): plan[0] = 3 four waves, 2 eight waves with
- * direct loads, 1 the 128 x 128 kernel, 0 scalar; plan[1] = columns of a tile of the four-wave kernel. No GPU needed. */
+/* The kernel a linear layer of these sizes takes (aligned operands): plan[0] = 4 the tiles of gemm_tiles_gfx950.hip, 3 four
+ * waves, 2 eight waves with direct loads, 1 the 128 x 128 kernel, 0 scalar; plan[1] = columns of a tile of the four-wave
+ * kernel, or the ranges of K of the first. No GPU needed. */
 void iris_hip_linear_plan(int rows, int in, int out, int out_bytes, int *plan) {
-    const GemmPlan p = plan_gemm(rows, out, in, out_bytes, true, true);
-    plan[0] = p.kernel; plan[1] = p.kernel == 3 ? 32 * p.na : 0;
+    const GemmPlan p = plan_gemm(rows, out, in, out_bytes, true, true, IRIS_LINEAR_PART_BYTES);
+    plan[0] = p.kernel; plan[1] = p.kernel == 3 ? 32 * p.na : p.kernel == 4 ? p.splits : 0;
 }
 
-int iris_hip_linear_f32(void *stream, float *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out) {
-    return gemm<float>((hipStream_t)stream, y, x, W, rows, out, in);
+int iris_hip_linear_f32(void *stream, float *part, float *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out) {
+    return gemm<float>((hipStream_t)stream, y, x, W, rows, out, in, part, IRIS_LINEAR_PART_BYTES);
 }
-int iris_hip_linear_bf16(void *stream, uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out) {
-    return gemm<uint16_t>((hipStream_t)stream, y, x, W, rows, out, in);
+int iris_hip_linear_bf16(void *stream, float *part, uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out) {
+    return gemm<uint16_t>((hipStream_t)stream, y, x, W, rows, out, in, part, IRIS_LINEAR_PART_BYTES);
 }
 
-/* Zeroes the first IRIS_CONV_ZERO_BYTES of a freshly allocated convolution scratch buffer: the page that taps
- * outside the image read. iris_hip_conv2d never writes there. */
 /* y = x W^T as bf16 with the per-head RMSNorm + rotary embedding (head_dim 128) of columns [0, q_cols) (weights
- * wq) and [q_cols, q_cols + k_cols) (weights wk) applied in the GEMM's epilogue. Returns -2, with nothing
- * enqueued, for a shape the tiled kernel does not take: the caller then runs the two steps one after the other. */
-int iris_hip_linear_bf16_qknorm(void *stream, uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out,
+ * wq) and [q_cols, q_cols + k_cols) (weights wk): applied in the GEMM's epilogue, or, where the plain layer takes the tiles
+ * of gemm_tiles_gfx950.hip, by the norm kernel behind it. Returns -2, with nothing
+ * enqueued, for a shape the tiled kernels do not take: the caller then runs the two steps one after the other. */
+int iris_hip_linear_bf16_qknorm(void *stream, float *part, uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out,
                                 int q_cols, int k_cols, const float *wq, const float *wk, const float *rope_cos,
                                 const float *rope_sin, float eps, int split_half) {
     const int M = rows, N = out, K = in;
@@ -962,6 +982,14 @@ int iris_hip_linear_bf16_qknorm(void *stream, uint16_t *y, const uint16_t *x, co
     if (!tiled || N % 128 || q_cols < 0 || k_cols < 0 || q_cols % 128 || k_cols % 128 || q_cols + k_cols > N ||
         q_cols + k_cols == 0)
         return -2;
+    if (plan_gemm(M, N, K, 2, true, true, IRIS_LINEAR_PART_BYTES).kernel == 4) {
+        const int qh = q_cols / 128, kh = k_cols / 128;
+        if ((long long)M * (qh + kh) >= (1 << 24) || qh + kh >= 256) return -2;
+        const int e = gemm<uint16_t>((hipStream_t)stream, y, x, W, M, N, K, part, IRIS_LINEAR_PART_BYTES);
+        if (e) return e;
+        return qh ? iris_hip_norm_rope_hd128(stream, y, kh ? y + q_cols : nullptr, N, wq, wk, rope_cos, rope_sin, M, qh, kh, eps, split_half)
+                  : iris_hip_norm_rope_hd128(stream, y, nullptr, N, wk, nullptr, rope_cos, rope_sin, M, kh, 0, eps, split_half);
+    }
     const ConvGeom none = {};
     const QkNorm qn = {wq, k_cols ? wk : wq, rope_cos, rope_sin, q_cols, q_cols + k_cols, eps, split_half};
     if (M % DT == 0 && N % 256 == 0 && four_wave_shape(M, N, K, 2))   /* whole tiles: a tile holds two whole heads */
@@ -969,6 +997,8 @@ int iris_hip_linear_bf16_qknorm(void *stream, uint16_t *y, const uint16_t *x, co
     return launch_gemm_dma<uint16_t, 256, false, true>((hipStream_t)stream, y, x, W, M, N, K, none, qn);
 }
 
+/* Zeroes the first IRIS_CONV_ZERO_BYTES of a freshly allocated convolution scratch buffer: the page that taps
+ * outside the image read. iris_hip_conv2d never writes there. */
 int iris_hip_conv2d_prepare_scratch(void *stream, uint16_t *scratch) {
     hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, (hipStream_t)stream, reinterpret_cast<uint32_t *>(scratch),
                        IRIS_CONV_ZERO_BYTES / 4);
@@ -1033,7 +1063,7 @@ int iris_hip_conv2d(void *stream, uint16_t *scratch, size_t scratch_bytes, float
         const size_t n = (size_t)np * row_len / (vec ? 8 : 1);
         if (vec) hipLaunchKernelGGL(k_im2col<8>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, scratch, in, h, width, cin, k, stride, pad_before, ow, p0, n);
         else hipLaunchKernelGGL(k_im2col<1>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, scratch, in, h, width, cin, k, stride, pad_before, ow, p0, n);
-        int e = gemm<float>(st, out + (size_t)p0 * cout, scratch, w, np, cout, row_len);
+        int e = gemm<float>(st, out + (size_t)p0 * cout, scratch, w, np, cout, row_len, nullptr, 0);
         if (e) return e;
     }
     if (bias) {

@@ -131,19 +131,24 @@ int iris_hip_group_norm_static_setup(void);
 int iris_hip_group_norm_static(void *stream, float *out, const float *in, const float *gamma,
                                const float *beta, int hw, int c, int groups, float eps, int do_silu);
 
-/* ---- linear layers and convolution (gemm_conv_gfx950.hip) ---- */
+/* ---- linear layers and convolution (gemm_conv_gfx950.hip, gemm_tiles_gfx950.hip) ---- */
 /* y[rows, out] = x[rows, in] @ W[out, in]^T, contiguous; MFMA kernel when in % 8 == 0 and
- * x, W are 16-byte aligned, scalar kernel otherwise */
-int iris_hip_linear_f32(void *stream, float *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out);
-int iris_hip_linear_bf16(void *stream, uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out);
-/* -2 = shape not taken, nothing enqueued */
-/* Which kernel a linear layer of these sizes takes with aligned operands, host arithmetic only: plan[0] = 3 the
- * four-wave 256-row tiles, 2 the eight-wave ones, 1 the 128 x 128 kernel, 0 the scalar kernel; plan[1] = the tile width
- * of the four-wave kernel (256, 224 or 192 columns). */
+ * x, W are 16-byte aligned, scalar kernel otherwise. part: IRIS_LINEAR_PART_BYTES of private workspace, 16-byte aligned,
+ * for the partial sums of products whose K is cut into ranges. */
+#define IRIS_LINEAR_PART_BYTES ((size_t)64 << 20)
+int iris_hip_linear_f32(void *stream, float *part, float *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out);
+int iris_hip_linear_bf16(void *stream, float *part, uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out);
+/* Which kernel a linear layer of these sizes takes with aligned operands, host arithmetic only: plan[0] = 4 the tiles for
+ * short sequences, 3 the four-wave 256-row tiles, 2 the eight-wave ones, 1 the 128 x 128 kernel, 0 the scalar kernel;
+ * plan[1] = the tile width of the four-wave kernel (256, 224 or 192 columns), the number of K ranges of the first. */
 void iris_hip_linear_plan(int rows, int in, int out, int out_bytes, int *plan);
+float iris_hip_gemm_tiles_plan(int M, int N, int K, int out_size, size_t part_bytes, int *shape, int *splits);
+int iris_hip_gemm_tiles(void *stream, void *y, int out_size, const uint16_t *x, const uint16_t *W, int M, int N, int K,
+                        int shape, int splits, float *part);
 
-int iris_hip_linear_bf16_qknorm(void *stream, uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out,
-                                int q_cols, int k_cols, const float *wq, const float *wk, const float *rope_cos,
+/* -2 = shape not taken, nothing enqueued */
+int iris_hip_linear_bf16_qknorm(void *stream, float *part, uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in,
+                                int out, int q_cols, int k_cols, const float *wq, const float *wk, const float *rope_cos,
                                 const float *rope_sin, float eps, int split_half);
 /* Convolution. `scratch` is a private device buffer, 16-byte aligned, whose first IRIS_CONV_ZERO_BYTES are zeroed
  * once by iris_hip_conv2d_prepare_scratch and never written again (the page that taps outside the image read);

@@ -32,6 +32,9 @@ static const char *g_last_kernel = "none";
 #ifndef IRIS_DEV_PATH_ONLY
 #define CONV_SCRATCH_BYTES ((size_t)256 << 20)
 static uint16_t *g_conv_scratch = NULL;
+/* partial sums of linear layers whose K is cut into ranges; allocated at initialisation, so that a linear layer never
+ * allocates and can be captured into a graph at its first call */
+static float *g_linear_part = NULL;
 static float *g_gn_scratch = NULL;
 static size_t g_gn_scratch_floats = 0;
 #endif
@@ -83,6 +86,11 @@ int iris_dev_init(void) {
     /* some hosts report an empty marketing name */
     snprintf(g_name, sizeof(g_name), "%s (%s, %d CUs, %d MHz)", prop.name[0] ? prop.name : "AMD Instinct",
              prop.gcnArchName, prop.multiProcessorCount, prop.clockRate / 1000);
+    if (!g_linear_part && hipMalloc((void **)&g_linear_part, IRIS_LINEAR_PART_BYTES) != hipSuccess) {
+        (void)hipGetLastError();
+        g_linear_part = NULL;
+        return 0;
+    }
     if (hipStreamCreate(&g_stream) != hipSuccess) return 0;
     /* address of the in-library scratch of iris_dev_group_norm_noalloc on this device; if the lookup
      * fails here the entry point tries again at its first call and reports it there */
@@ -112,6 +120,8 @@ void iris_dev_cleanup(void) {
     if (!g_ready) return;
     check(hipStreamSynchronize(g_stream), "sync");
     if (g_conv_scratch) check(hipFree(g_conv_scratch), "free");
+    if (g_linear_part) check(hipFree(g_linear_part), "free");
+    g_linear_part = NULL;
     if (g_gn_scratch) check(hipFree(g_gn_scratch), "free");
     if (g_rope_stage) check(hipFree(g_rope_stage), "free");
     if (g_q_scratch) check(hipFree(g_q_scratch), "free");
@@ -464,7 +474,7 @@ void iris_dev_linear_f32(float *y, const uint16_t *x, const uint16_t *W, int row
     if (!need_ready("linear")) return;
     if (linear_by_library(y, 0, x, W, rows, in, out)) return;
     g_last_kernel = "linear_mfma";
-    LAUNCH("linear", iris_hip_linear_f32(g_stream, y, x, W, rows, in, out));
+    LAUNCH("linear", iris_hip_linear_f32(g_stream, g_linear_part, y, x, W, rows, in, out));
 }
 
 void iris_dev_linear_bf16(uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out) {
@@ -473,7 +483,7 @@ void iris_dev_linear_bf16(uint16_t *y, const uint16_t *x, const uint16_t *W, int
     if (!need_ready("linear")) return;
     if (linear_by_library(y, 1, x, W, rows, in, out)) return;
     g_last_kernel = "linear_mfma";
-    LAUNCH("linear", iris_hip_linear_bf16(g_stream, y, x, W, rows, in, out));
+    LAUNCH("linear", iris_hip_linear_bf16(g_stream, g_linear_part, y, x, W, rows, in, out));
 }
 
 void iris_dev_linear_bf16_qknorm(uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out,
@@ -490,7 +500,7 @@ void iris_dev_linear_bf16_qknorm(uint16_t *y, const uint16_t *x, const uint16_t 
     int one_launch = head_dim == 128 && q_heads + k_heads > 0 &&
                      (g_linear_backend != 2 || !iris_lt_available() || in % 8 != 0);
     if (one_launch) {
-        int err = iris_hip_linear_bf16_qknorm(g_stream, y, x, W, rows, in, out, q_heads * 128, k_heads * 128, wq, wk,
+        int err = iris_hip_linear_bf16_qknorm(g_stream, g_linear_part, y, x, W, rows, in, out, q_heads * 128, k_heads * 128, wq, wk,
                                               rope_cos, rope_sin, eps, split_half != 0);
         if (err == 0) { g_last_kernel = "linear_mfma_qknorm"; return; }
         if (err != -2) { check((hipError_t)err, "linear_qknorm launch"); return; }

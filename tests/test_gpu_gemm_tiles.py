@@ -1,0 +1,92 @@
+"""k_gemm_tiles (gemm_tiles_gfx950.hip): every tile and K ranges at their edges, against a float64 product of the same bf16
+operands. The bar is that of the other linear kernels: f32 accumulation noise for f32 outputs, half a bf16 ulp more for bf16."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle as O
+from gpu_harness import Dev
+
+pytestmark = pytest.mark.gpu
+TILES = [(128, 128), (128, 192), (128, 256), (64, 256), (160, 192), (160, 256)]
+
+
+@pytest.fixture(scope="module")
+def dev():
+    return Dev()
+
+
+def operands(rows, k, out):
+    rng = np.random.default_rng(rows * 7 + k + out)
+    x = O.f32_to_bf16(rng.standard_normal((rows, k)).astype(np.float32))
+    W = O.f32_to_bf16((rng.standard_normal((out, k)) * 0.05).astype(np.float32))
+    return x, W, O.bf16_to_f32(x).astype(np.float64) @ O.bf16_to_f32(W).astype(np.float64).T
+
+
+def check(got, want, k, bf16):
+    scale = np.sqrt(k) * 0.05
+    if bf16:
+        assert np.all(np.abs(O.bf16_to_f32(got) - want) <= np.abs(want) * 2.0 ** -8 * 1.01 + scale * 2e-5)
+    else:
+        assert np.abs(got - want).max() <= scale * 2e-5
+
+
+# rows and columns beyond whole tiles (the last tile holds 1 .. all but one row), k tiles: fewer than, as many as and one more
+# than the ring holds, odd and even numbers of them, ranges of unequal length
+@pytest.mark.parametrize("shape", range(len(TILES)))
+@pytest.mark.parametrize("more_rows,more_cols,k,splits", [(0, 0, 64, 1), (1, 8, 128, 1), (-1, -8, 192, 1), (0, 72, 256, 1), (33, 0, 320, 1),
+                                                          (-63, 8, 704, 3), (0, 0, 640, 2), (1, 8, 832, 6)])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_every_tile(dev, shape, more_rows, more_cols, k, splits, bf16):
+    rows, out = TILES[shape][0] + more_rows, TILES[shape][1] + more_cols
+    x, W, want = operands(rows, k, out)
+    lib = dev.lib
+    lib.iris_hip_gemm_tiles.restype = C.c_int
+    lib.iris_hip_gemm_tiles.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p] + [C.c_int] * 5 + [C.c_void_p]
+    guard = 512
+    fill = np.full(rows * out + guard, 7, np.uint16 if bf16 else np.float32)
+    dy, part = dev.put(fill), dev.alloc(splits * rows * out * 4)
+    assert lib.iris_hip_gemm_tiles(lib.iris_dev_stream(), dy, 2 if bf16 else 4, dev.put(x), dev.put(W), rows, out, k, shape, splits, part) == 0
+    dev.check()
+    got = dev.get(dy, fill.shape, fill.dtype)
+    dev.free_all()
+    assert (got[rows * out:] == 7).all()
+    check(got[:rows * out].reshape(rows, out), want, k, bf16)
+
+
+@pytest.mark.parametrize("rows,k,out", [(1, 512, 128), (77, 2048, 1544), (130, 1536, 136), (300, 4096, 640), (500, 1024, 3072)])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_linear_layers_that_take_it(dev, rows, k, out, bf16):
+    plan = (C.c_int * 2)()
+    dev.lib.iris_hip_linear_plan(rows, k, out, 2 if bf16 else 4, plan)
+    assert plan[0] == 4
+    x, W, want = operands(rows, k, out)
+    dy = dev.alloc(rows * out * (2 if bf16 else 4))
+    fn = dev.lib.iris_dev_linear_bf16 if bf16 else dev.lib.iris_dev_linear_f32
+    for _ in range(2):                                       # the second call finds the first one's partial sums in the workspace
+        fn(dy, dev.put(x), dev.put(W), rows, k, out)
+    dev.check()
+    got = dev.get(dy, (rows, out), np.uint16 if bf16 else np.float32)
+    dev.free_all()
+    check(got, want, k, bf16)
+
+
+def test_projection_with_norm_takes_the_same_kernel(dev):
+    """The projection that normalises its own columns, at a size whose plain layer takes these tiles: the bits of the two calls."""
+    rows, k, heads = 320, 1024, 6
+    out = 3 * heads * 128
+    rng = np.random.default_rng(3)
+    x, W, _ = operands(rows, k, out)
+    w = [dev.put((1 + 0.05 * rng.standard_normal(128)).astype(np.float32)) for _ in range(2)]
+    ang = rng.uniform(-3, 3, (rows, 64)).astype(np.float32)
+    cos, sin, dx, dW = dev.put(np.cos(ang)), dev.put(np.sin(ang)), dev.put(x), dev.put(W)
+    one, two = dev.alloc(rows * out * 2), dev.alloc(rows * out * 2)
+    dev.lib.iris_dev_linear_bf16_qknorm(one, dx, dW, rows, k, out, heads, heads, 128, w[0], w[1], cos, sin, 1e-6, 0)
+    assert dev.dev.last_kernel() == "linear_mfma_qknorm"
+    dev.lib.iris_dev_linear_bf16(two, dx, dW, rows, k, out)
+    dev.lib.iris_dev_head_norm_rope_qk(two, C.c_void_p(two + 2 * heads * 128), out, w[0], w[1], cos, sin, rows, heads, heads, 128, 1e-6, 0)
+    dev.check()
+    a, b = dev.get(one, (rows, out), np.uint16), dev.get(two, (rows, out), np.uint16)
+    dev.free_all()
+    assert np.array_equal(a, b)
