@@ -11,7 +11,6 @@
  */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
-#include <type_traits>
 
 #include "iris_kernels_hip.h"
 
@@ -227,13 +226,20 @@ k_conv_few_out(float *__restrict__ out, const float *__restrict__ in, const uint
  * tap starts at, they fall into distinct bank windows; a tap's shift is an immediate offset. Weight rows are swizzled as
  * in gemm_conv_gfx950.hip.
  *
+ * A workgroup takes 152 KB of LDS, so a CU runs one, and it is persistent: while it multiplies the last channel group of a
+ * tile it fetches the first of the next, and the next steps run while its stores are on their way (they count in the
+ * waits, see channel_group). One tile per workgroup, 11 us of the 23 us of a tile of 128 input channels were its first
+ * pixels' and its stores' latency: 91 -> 82 us for 128 -> 128 channels.
+ *
  * Measured against a bf16 copy of the image + implicit product that fetches every tap from the L2 (copy + product):
- * 512 x 512 pixels, 128 -> 128 30 + 118 -> 91 us, 256 -> 128 76 + 214 -> 141 us (1100 TFLOP/s), 256 -> 256 88 + 290 ->
- * 271 us (1140). A step takes 0.68 us (1500 cycles, 1024 of them products); a workgroup's first pixels and its stores
- * take 11 us that nothing overlaps. */
+ * 512 x 512 pixels, 128 -> 128 30 + 118 -> 82 us (the image and the result alone take 50 us to move), 256 -> 128 76 + 214
+ * -> 135 us (1150 TFLOP/s), 256 -> 256 88 + 290 -> 263 us (1180). A step takes 0.7 us: 256 of them at a time are 1500
+ * TFLOP/s, what a large plain product reaches on this card. */
 constexpr int C3_T = 16, C3_H = C3_T + 2, C3_PIXELS = C3_H * C3_H, C3_ROW = 80, C3_IMG = C3_PIXELS * C3_ROW;   /* elements */
 constexpr int C3_N = 128, C3_STAGE = C3_N * 64, C3_UNITS = 6;
-constexpr int C3_LDS = (2 * C3_IMG + 3 * C3_STAGE) * 2;
+constexpr int C3_BIAS = 2 * C3_IMG + 3 * C3_STAGE;             /* the bias of all output channels, f32 */
+constexpr int C3_MAX_COUT = (160 * 1024 - 2 * C3_BIAS) / 4 / C3_N * C3_N;
+constexpr int C3_STORES = 16;                                  /* store instructions of a wave in the epilogue of a whole tile */
 
 __device__ __forceinline__ uint32_t lds_address(const uint16_t *p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
@@ -244,26 +250,36 @@ __device__ __forceinline__ uint32_t lds_address(const uint16_t *p) {
 __global__ void __launch_bounds__(512, 2)
 k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t *__restrict__ W, const float *__restrict__ bias,
            ConvShape s, int tiles_x, int tiles_n, int total, int per_xcd) {
-    extern __shared__ __align__(16) uint16_t lds[];            /* image, image, weights, weights, weights */
-    /* an XCD takes a contiguous range of the tiles, the channel tiles of a pixel tile next to each other: they share the
-     * image in its L2 */
-    const int work = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-    if (work >= total) return;
-    const int tile = work / tiles_n, n0 = (work - tile * tiles_n) * C3_N;
-    const int ty0 = tile / tiles_x * C3_T, tx0 = tile % tiles_x * C3_T;
+    extern __shared__ __align__(16) uint16_t lds[];            /* image, image, weights, weights, weights, bias */
+    /* an XCD takes a contiguous range of the tiles, the channel tiles of a pixel tile next to each other (they share the
+     * image in its L2), dealt out to its workgroups in turn */
+    const int xcd_end = min((int)(blockIdx.x % 8 + 1) * per_xcd, total), stride = gridDim.x / 8;
+    int work = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if (work >= xcd_end) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4, wm = wave & 3, wn = wave >> 2;
+    float *bias_lds = reinterpret_cast<float *>(lds + C3_BIAS);
+    for (int i = tid; i < tiles_n * C3_N; i += 512) bias_lds[i] = bias && i < s.cout ? bias[i] : 0.0f;
 
+    int ty0, tx0, n0;                                          /* of the tile `work` */
+    auto place = [&](int w, int &ty, int &tx, int &n) {
+        const int tile = w / tiles_n;
+        n = (w - tile * tiles_n) * C3_N;
+        ty = tile / tiles_x * C3_T;
+        tx = tile % tiles_x * C3_T;
+    };
     /* image staging: unit u of this thread is channels 8 (tid % 8) .. + 7 of pixel tid / 8 + 64 u of the rimmed tile; a
      * pixel outside the image reads the first one and is zeroed */
     uint32_t uoff[C3_UNITS];                                   /* bytes from the channel group's first value */
     bool inside[C3_UNITS];
+    auto aim_image = [&](int ty, int tx) {
 #pragma unroll
-    for (int u = 0; u < C3_UNITS; u++) {
-        const int px = (tid >> 3) + 64 * u, py = px / C3_H, y = ty0 + py - s.pad, x = tx0 + (px - py * C3_H) - s.pad;
-        inside[u] = px < C3_PIXELS && y >= 0 && y < s.h && x >= 0 && x < s.w;
-        uoff[u] = ((inside[u] ? (uint32_t)(y * s.w + x) * (uint32_t)s.cin : 0u) + 8u * (tid & 7)) * 4u;
-    }
+        for (int u = 0; u < C3_UNITS; u++) {
+            const int px = (tid >> 3) + 64 * u, py = px / C3_H, y = ty + py - s.pad, x = tx + (px - py * C3_H) - s.pad;
+            inside[u] = px < C3_PIXELS && y >= 0 && y < s.h && x >= 0 && x < s.w;
+            uoff[u] = ((inside[u] ? (uint32_t)(y * s.w + x) * (uint32_t)s.cin : 0u) + 8u * (tid & 7)) * 4u;
+        }
+    };
     const int st_off = (tid >> 3) * C3_ROW + 8 * (tid & 7);
     auto put = [&](int img, int u, f32x4 lo, f32x4 hi) {
         u32x4 v = {pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3])};
@@ -275,26 +291,30 @@ k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t
     /* weights: rows 16 wave .. + 15 of a stage in two pieces of eight rows; rows past the last channel repeat it (their
      * results are never stored) */
     const int row_len = 9 * s.cin;
-    uint32_t woff[2];
+    uint32_t woff[2], woff_next[2];
+    auto aim_weights = [&](int n, uint32_t *off) {
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int r = 16 * wave + 8 * j + (lane >> 3), n = n0 + r < s.cout ? n0 + r : s.cout - 1;
-        woff[j] = ((uint32_t)n * (uint32_t)row_len + 8u * ((lane & 7) ^ ((r >> 1) & 7))) * 2u;
-    }
+        for (int j = 0; j < 2; j++) {
+            const int r = 16 * wave + 8 * j + (lane >> 3), row = n + r < s.cout ? n + r : s.cout - 1;
+            off[j] = ((uint32_t)row * (uint32_t)row_len + 8u * ((lane & 7) ^ ((r >> 1) & 7))) * 2u;
+        }
+    };
     uint16_t *w_lds = lds + 2 * C3_IMG;
-    auto request = [&](int tap, int c0, int stage) {
+    auto request = [&](const uint32_t *off, int tap, int c0, int stage) {
         const uint16_t *src = W + (size_t)tap * s.cin + c0;
 #pragma unroll
         for (int j = 0; j < 2; j++)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                         ::"s"(lds_address(w_lds + stage * C3_STAGE + (16 * wave + 8 * j) * 64)), "v"(woff[j]), "s"(src) : "memory", "m0");
+                         ::"s"(lds_address(w_lds + stage * C3_STAGE + (16 * wave + 8 * j) * 64)), "v"(off[j]), "s"(src) : "memory", "m0");
     };
 
     f32x4 acc[4][4];                                           /* [16 channels][row of 16 pixels] */
+    auto clear = [&]() {
 #pragma unroll
-    for (int a = 0; a < 4; a++)
+        for (int a = 0; a < 4; a++)
 #pragma unroll
-        for (int b = 0; b < 4; b++) acc[a][b] = f32x4{0, 0, 0, 0};
+            for (int b = 0; b < 4; b++) acc[a][b] = f32x4{0, 0, 0, 0};
+    };
     u32x4 av[2][4], bv[2][4];
     int a_rd[2];
 #pragma unroll
@@ -314,42 +334,81 @@ k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t
             for (int b = 0; b < 4; b++) acc[a][b] = mfma(av[ks][a], bv[ks][b], acc[a][b]);
     };
 
-    const int groups = s.cin / 64;
     f32x4 xr[3][2];                                            /* three image units on their way */
-    /* One group of 64 channels: nine steps. `img` holds it, the next one goes to `other`. */
-    auto channel_group = [&](auto last_group, int g, int img, int other) {
-        constexpr bool LAST = decltype(last_group)::value;
-        const float *next = in + 64 * (g + 1);
+    /* One group of 64 channels: nine steps. `img` holds it; what comes next, the image from `next` on and the weights
+     * from channel c_next on, goes to `other` and to the stages as they fall free. first: of a tile, behind the epilogue
+     * of the one before. */
+    auto channel_group = [&](bool first, int c0, int img, int other, const float *next, int c_next) {
 #pragma unroll
         for (int t = 0; t < 9; t++) {
             operands(img, t, 1);
             __builtin_amdgcn_sched_barrier(0);
-            if (!LAST && t >= 3) put(other, t - 3, xr[t % 3][0], xr[t % 3][1]);
-            if (!LAST && t < C3_UNITS) {
+            if (t >= 3) put(other, t - 3, xr[t % 3][0], xr[t % 3][1]);
+            if (t < C3_UNITS) {
                 asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(xr[t % 3][0]) : "v"(uoff[t]), "s"(next) : "memory");
                 asm volatile("global_load_dwordx4 %0, %1, %2 offset:16" : "=v"(xr[t % 3][1]) : "v"(uoff[t]), "s"(next) : "memory");
             }
             products(0);
             __builtin_amdgcn_sched_barrier(0);
-            /* newer than the weights of step t + 1: the image loads of steps t - 1 and t, the weights of step t + 2 */
-            constexpr int IMAGE = LAST ? 0 : 2;
-            const int newer = (t >= 1 && t - 1 < C3_UNITS ? IMAGE : 0) + (t < C3_UNITS ? IMAGE : 0) + (LAST && t > 6 ? 0 : 2);
-            if (newer == 6) asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            else if (newer == 4) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            else if (newer == 2) asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            if (!LAST && t >= 2 && t - 2 < C3_UNITS) asm volatile("" : "+v"(xr[(t - 2) % 3][0]), "+v"(xr[(t - 2) % 3][1]));
-            if (!LAST || t < 8) operands(t < 8 ? img : other, t < 8 ? t + 1 : 0, 0);
-            if (!LAST || t < 6) request(t < 6 ? t + 3 : t - 6, 64 * (t < 6 ? g : g + 1), t % 3);
+            /* newer than the weights of step t + 1: the image loads of steps t - 1 and t, the weights of step t + 2, and the
+             * stores of the epilogue in front of step 0 (where they were not counted on, everything before them has landed) */
+            const int newer = (t >= 1 && t - 1 < C3_UNITS ? 2 : 0) + (t < C3_UNITS ? 2 : 0) + 2;
+            if (t < 2 && first) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(newer + C3_STORES) : "memory");
+            else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(newer) : "memory");
+            if (t >= 2 && t - 2 < C3_UNITS) asm volatile("" : "+v"(xr[(t - 2) % 3][0]), "+v"(xr[(t - 2) % 3][1]));
+            operands(t < 8 ? img : other, t < 8 ? t + 1 : 0, 0);
+            if (t < 6) request(woff, t + 3, c0, t % 3);
+            else request(woff_next, t - 6, c_next, t % 3);
             __builtin_amdgcn_sched_barrier(0);
             products(1);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
 
-    request(0, 0, 0);
-    request(1, 0, 1);
-    request(2, 0, 2);
+    /* acc[a][b][r]: channel n0 + 64 wn + 16 a + 4 lg + r of pixel (4 wm + b, li) of the tile. Through the image buffer that the
+     * last group has been read from (every wave has passed the barrier behind its last reads; 4 KB per wave, a row of 16
+     * pixels at a time), so that a store instruction covers four pixels x 256 B. */
+    const int c = lane & 15;
+    const bool chunks = s.cout % 4 == 0 && ((uintptr_t)out & 15) == 0;
+    auto epilogue = [&](int img, bool more) {
+        float *buf = reinterpret_cast<float *>(lds + img) + wave * 1024;
+        const int n = n0 + 64 * wn + 4 * c;
+        const f32x4 bias4 = *reinterpret_cast<const f32x4 *>(bias_lds + n);
+        const bool whole = chunks && ty0 + C3_T <= s.oh && tx0 + C3_T <= s.ow && n0 + C3_N <= s.cout;
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+#pragma unroll
+            for (int a = 0; a < 4; a++) *reinterpret_cast<f32x4 *>(&buf[li * 64 + 4 * ((4 * a + lg) ^ li)]) = acc[a][b];
+            const int y = ty0 + 4 * wm + b;
+            f32x4 v[4];
+#pragma unroll
+            for (int it = 0; it < 4; it++) {
+                const int row = 4 * it + (lane >> 4);
+                v[it] = *reinterpret_cast<const f32x4 *>(&buf[row * 64 + 4 * (c ^ row)]) + bias4;
+            }
+            float *dst = out + ((size_t)y * s.ow + tx0 + (lane >> 4)) * s.cout + n;
+            if (whole) {
+#pragma unroll
+                for (int it = 0; it < 4; it++) *reinterpret_cast<f32x4 *>(dst + (size_t)(4 * it) * s.cout) = v[it];
+            } else if (y < s.oh) {
+#pragma unroll
+                for (int it = 0; it < 4; it++) {
+                    if (tx0 + 4 * it + (lane >> 4) >= s.ow) continue;
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (n + e < s.cout) dst[(size_t)(4 * it) * s.cout + e] = v[it][e];
+                }
+            }
+        }
+        /* the next steps count on C3_STORES stores in flight, or on none of what came before them */
+        if (more && !whole) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    };
+
+    const int groups = s.cin / 64;
+    place(work, ty0, tx0, n0);
+    aim_weights(n0, woff);
+    for (int t = 0; t < 3; t++) request(woff, t, 0, t);
+    aim_image(ty0, tx0);
     {
         f32x4 first[C3_UNITS][2];
 #pragma unroll
@@ -362,52 +421,50 @@ k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t
     }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     operands(0, 0, 0);
-    int img = 0;
-    for (int g = 0; g + 1 < groups; g++) {
-        channel_group(std::false_type{}, g, img, C3_IMG - img);
+    clear();
+    woff_next[0] = woff[0];
+    woff_next[1] = woff[1];
+    int ty = ty0, tx = tx0, n = n0;                            /* where the next group's image and weights come from */
+    for (int img = 0, g = 0;;) {
+        const bool last = g + 1 == groups, more = work + stride < xcd_end;
+        if (last && more) {
+            place(work + stride, ty, tx, n);
+            aim_image(ty, tx);
+            aim_weights(n, woff_next);
+        } else if (last) {
+            /* nothing comes next: the same loads, of a few cached bytes that nobody uses */
+#pragma unroll
+            for (int u = 0; u < C3_UNITS; u++) { inside[u] = false; uoff[u] = 32u * (tid & 7); }
+        }
+        channel_group(g == 0, 64 * g, img, C3_IMG - img, last ? in : in + 64 * (g + 1), last ? 0 : 64 * (g + 1));
+        if (last) {
+            epilogue(img, more);
+            if (!more) break;
+            clear();
+            work += stride;
+            ty0 = ty; tx0 = tx; n0 = n;
+            woff[0] = woff_next[0];
+            woff[1] = woff_next[1];
+        }
+        g = last ? 0 : g + 1;
         img = C3_IMG - img;
     }
-    channel_group(std::true_type{}, groups - 1, img, C3_IMG - img);
-
-    /* acc[a][b][r]: channel n0 + 64 wn + 16 a + 4 lg + r of pixel (4 wm + b, li) of the tile. Through the LDS (every wave has
-     * passed the last step's barrier, behind which nothing is read from it; 16 KB per wave), so that a store instruction
-     * covers four pixels x 256 B. */
-    float *buf = reinterpret_cast<float *>(lds) + wave * 4096;
-#pragma unroll
-    for (int b = 0; b < 4; b++)
-#pragma unroll
-        for (int a = 0; a < 4; a++) *reinterpret_cast<f32x4 *>(&buf[(16 * b + li) * 64 + 4 * ((4 * a + lg) ^ li)]) = acc[a][b];
-    const int c = lane & 15, n = n0 + 64 * wn + 4 * c;
-    const bool whole = s.cout % 4 == 0 && ((uintptr_t)out & 15) == 0;
-    f32x4 bias4 = {0, 0, 0, 0};
-    for (int e = 0; e < 4; e++)
-        if (bias && n + e < s.cout) bias4[e] = bias[n + e];
-#pragma unroll
-    for (int it = 0; it < 16; it++) {
-        const int row = 4 * it + (lane >> 4), y = ty0 + 4 * wm + (row >> 4), x = tx0 + (row & 15);
-        const f32x4 v = *reinterpret_cast<const f32x4 *>(&buf[row * 64 + 4 * (c ^ (row & 15))]) + bias4;
-        if (y >= s.oh || x >= s.ow) continue;
-        float *dst = out + ((size_t)y * s.ow + x) * s.cout + n;
-        if (whole) {
-            if (n < s.cout) *reinterpret_cast<f32x4 *>(dst) = v;
-        } else {
-            for (int e = 0; e < 4; e++)
-                if (n + e < s.cout) dst[e] = v[e];
-        }
-    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           /* no load into the LDS is left when it is given up */
 }
 #pragma clang diagnostic pop
 
 int launch_3x3(hipStream_t st, float *out, const float *in, const uint16_t *W, const float *bias, const ConvShape &s) {
     static bool configured = false;
     if (!configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_conv_3x3), hipFuncAttributeMaxDynamicSharedMemorySize, C3_LDS);
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_conv_3x3), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (e != hipSuccess) return (int)e;
         configured = true;
     }
     const int tiles_x = (s.ow + C3_T - 1) / C3_T, tiles_n = (s.cout + C3_N - 1) / C3_N;
     const int total = tiles_x * ((s.oh + C3_T - 1) / C3_T) * tiles_n, per_xcd = (total + 7) / 8;
-    hipLaunchKernelGGL(k_conv_3x3, dim3((unsigned)per_xcd * 8), dim3(512), C3_LDS, st, out, in, W, bias, s, tiles_x, tiles_n, total, per_xcd);
+    const unsigned lds = 2 * C3_BIAS + 4 * C3_N * (unsigned)tiles_n;
+    /* one workgroup per CU (its LDS): 32 per XCD, each walking the XCD's tiles */
+    hipLaunchKernelGGL(k_conv_3x3, dim3((unsigned)(per_xcd < 32 ? per_xcd : 32) * 8), dim3(512), lds, st, out, in, W, bias, s, tiles_x, tiles_n, total, per_xcd);
     return (int)hipGetLastError();
 }
 
@@ -448,7 +505,7 @@ int iris_hip_conv2d_direct(void *stream, float *out, const float *in, const uint
         return cin == 32 ? launch_few_out<1>(st, out, in, w, bias, s) : cin == 64 ? launch_few_out<2>(st, out, in, w, bias, s)
                                                                                : launch_few_out<4>(st, out, in, w, bias, s);
     /* a thread's byte offsets into image and weights are 32-bit */
-    if (k == 3 && stride == 1 && cin % 64 == 0 && al16(in) && al16(w) && (size_t)h * width * cin * 4 < ((size_t)1 << 32) &&
+    if (k == 3 && stride == 1 && cin % 64 == 0 && cout <= C3_MAX_COUT && al16(in) && al16(w) && (size_t)h * width * cin * 4 < ((size_t)1 << 32) &&
         (size_t)cout * 9 * cin * 2 < ((size_t)1 << 32))
         return launch_3x3(st, out, in, w, bias, s);
     return -2;
