@@ -13,10 +13,10 @@
  *
  * Products with too few 256-row tiles to fill the chip (short sequences) take k_gemm_tiles (gemm_tiles_gfx950.hip). For
  * the rest, three kernels. M, N >= 256 with K a multiple of 128 (every linear layer of the models at their
- * larger sequence lengths) take k_gemm_w4: tiles of 256 rows x 256, 224 or 192 columns on four waves, one per
- * SIMD, staged through registers. Other shapes with M, N >= 256 and K a multiple of 64, and the convolutions, take
- * k_gemm_dma: the same tiles on 8 waves, loaded straight into LDS. Both are described where they are
- * defined and give the same bits. Everything else with K a multiple of 8 takes k_gemm_bf16:
+ * larger sequence lengths) take k_gemm_wide: tiles of 256 rows x 256, 224 or 192 columns on eight waves, every memory
+ * instruction in a gap between two products. Other shapes with M, N >= 256 and K a multiple of 64, and the convolutions
+ * that have no kernel of their own, take k_gemm_dma: the same tiles with the loads and reads in groups. Both give the same
+ * bits. Everything else with K a multiple of 8 takes k_gemm_bf16:
  * Workgroup = WM x WN waves (2 x 2 in use), tile 128 (m) x 128 (n), K in steps of 64; a wave owns
  * 64 x 64 = 4 x 4 accumulator blocks and reads 8 operands from LDS per 16 MFMAs. One
  * LDS stage of [W tile | x tile], rows padded to 160 B so that the 16 lanes the LDS
@@ -193,24 +193,14 @@ __device__ __forceinline__ uint32_t lds_address(const uint16_t *p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
 }
 
-/* The per-head RMSNorm + rotary embedding of the leading columns of a projection, applied by the GEMM to its
- * own output tile (head_dim 128): columns [0, q_cols) are heads normalised with wq, [q_cols, qk_cols) with wk,
- * the rest is stored as it is. */
-struct QkNorm {
-    const float *wq, *wk, *rope_cos, *rope_sin;  /* [128], [128], [M, 64], [M, 64] */
-    int q_cols, qk_cols;
-    float eps;
-    int split_half;
-};
-
 /* M0 (the LDS address of a direct load) is named as clobbered by the asm statements below; the
  * compiler reserves that register for its own short-lived uses and remarks on it. */
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-template <typename OUT, int TN, bool CONV, bool QKN = false>
+template <typename OUT, int TN, bool CONV>
 __global__ void __launch_bounds__(512, 2)
 k_gemm_dma(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *__restrict__ W,
-           int M, int N, int K, int tiles_m, int total, int per_xcd, ConvGeom geo, QkNorm qn) {
+           int M, int N, int K, int tiles_m, int total, int per_xcd, ConvGeom geo) {
     constexpr int WAVES_N = TN / 64, WAVES_M = 8 / WAVES_N;    /* wave grid */
     constexpr int NB = DT / WAVES_M / 16;                      /* x blocks (16 rows) per wave: 8 or 4 */
     constexpr int HALVES = NB / 4;
@@ -376,60 +366,6 @@ k_gemm_dma(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *
      * LDS serves a wave's instructions in order, so the reads see the writes without a barrier. */
     constexpr int PER16 = 16 / (int)sizeof(OUT);               /* outputs per 16 B */
     const int mw = m0 + 16 * NB * wm, nw = n0 + 64 * wn;
-    if constexpr (QKN) {
-        /* A head (128 columns) spans the blocks of two waves, so a tile with head columns in it is staged as a
-         * whole: 256 rows x 512 B fill the 128 KB exactly. 16 B chunk c of row r sits in slot
-         * (c & 16) | ((c ^ r) & 15): the 16 rows of a write and the 16 chunks of a head vector both spread over
-         * all banks. Then a 16-lane row per (token, head) vector, 32 vectors a pass, through the same function
-         * as the stand-alone kernel: the stored bits are those of the plain projection followed by that kernel. */
-        static_assert(sizeof(OUT) == 2 && TN == 256 && !CONV, "bf16 projection tiles of 256 x 256 only");
-        if (n0 < qn.qk_cols) {                                  /* the same for the whole workgroup */
-#pragma unroll
-            for (int b = 0; b < NB; b++)
-#pragma unroll
-                for (int a = 0; a < 4; a++) {
-                    const int row = 16 * NB * wm + 16 * b + li, chunk = 8 * wn + 2 * a + (lg >> 1);
-                    const int slot = (chunk & 16) | ((chunk ^ li) & 15);
-                    *reinterpret_cast<uint2 *>(&dlds[row * 256 + 8 * slot + 4 * (lg & 1)]) =
-                        make_uint2(pack_bf16(acc[a][b][0], acc[a][b][1]), pack_bf16(acc[a][b][2], acc[a][b][3]));
-                }
-            __syncthreads();
-            const int sub = tid & 15, head = (tid >> 4) & 1, row_in = tid >> 5;
-            const int n_head = n0 + 128 * head, n = n_head + 8 * sub;
-            const bool normed = n_head < qn.qk_cols;
-            float w8[8] = {};
-            if (normed) {
-                const float *wsel = (n_head < qn.q_cols ? qn.wq : qn.wk) + 8 * sub;
-                const float4 w0 = *reinterpret_cast<const float4 *>(wsel), w1 = *reinterpret_cast<const float4 *>(wsel + 4);
-                w8[0] = w0.x; w8[1] = w0.y; w8[2] = w0.z; w8[3] = w0.w; w8[4] = w1.x; w8[5] = w1.y; w8[6] = w1.z; w8[7] = w1.w;
-            }
-            const int tcol = qn.split_half ? 8 * (sub & 7) : 4 * sub;
-            const int chunk = 16 * head + sub;
-#pragma unroll 4
-            for (int pass = 0; pass < DT / 16; pass++) {
-                const int row = 16 * pass + row_in, m = m0 + row;
-                if (m >= M || n_head >= N) continue;            /* the same for the 16 lanes of a vector */
-                u32x4 v = *reinterpret_cast<const u32x4 *>(&dlds[row * 256 + 8 * ((chunk & 16) | ((chunk ^ row) & 15))]);
-                if (normed) {
-                    const float *cr = qn.rope_cos + (size_t)m * 64 + tcol, *sr = qn.rope_sin + (size_t)m * 64 + tcol;
-                    float cv[8] = {}, sv[8] = {};
-                    const float4 c0 = *reinterpret_cast<const float4 *>(cr), s0 = *reinterpret_cast<const float4 *>(sr);
-                    cv[0] = c0.x; cv[1] = c0.y; cv[2] = c0.z; cv[3] = c0.w;
-                    sv[0] = s0.x; sv[1] = s0.y; sv[2] = s0.z; sv[3] = s0.w;
-                    if (qn.split_half) {
-                        const float4 c1 = *reinterpret_cast<const float4 *>(cr + 4), s1 = *reinterpret_cast<const float4 *>(sr + 4);
-                        cv[4] = c1.x; cv[5] = c1.y; cv[6] = c1.z; cv[7] = c1.w;
-                        sv[4] = s1.x; sv[5] = s1.y; sv[6] = s1.z; sv[7] = s1.w;
-                        v = nr_vector_hd128<true>(v, w8, cv, sv, qn.eps, sub);
-                    } else {
-                        v = nr_vector_hd128<false>(v, w8, cv, sv, qn.eps, sub);
-                    }
-                }
-                *reinterpret_cast<u32x4 *>(reinterpret_cast<uint16_t *>(y) + (size_t)m * N + n) = v;
-            }
-            return;
-        }
-    }
     const float *bias = CONV ? geo.bias : nullptr;
     const bool staged = N % PER16 == 0 && ((uintptr_t)y & 15) == 0;
     if (staged) {
@@ -489,185 +425,177 @@ k_gemm_dma(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *
         }
     }
 }
-/* ---- tiles of 256 rows x 256, 224 or 192 columns x 64 on FOUR waves, one per SIMD with the whole register file ----
+/* ---- tiles of 256 rows x 256, 224 or 192 columns ----
  *
- * For M, N >= 256 and K a multiple of 128. Each wave owns 128 rows x 16 NA columns = NA x 8 accumulator
- * blocks, up to 256 registers that live in AGPRs (the products are asm statements, so that they stay there),
- * so an operand read from the LDS feeds NA or eight products: with NA = 8, 32 reads per 128 MFMAs and k tile, two
- * thirds of the LDS traffic of the 8-wave kernel. A wave that is alone on its SIMD has nobody to hide its other instructions behind:
- * it issues in order, and what stands between two products must fit into the 12 cycles the matrix core still
- * works on the first. Hence
- *  - the tiles are staged through registers (a direct HBM -> LDS load blocks the issuing wave for about 100
- *    cycles): NA + 8 loads of 16 B per thread and k tile, two tiles ahead (two register sets), each written to
- *    the LDS as two 8-byte halves (a 16-byte LDS write takes longer to issue than the gap: 1265 -> 1302 TFLOP/s);
- *  - every gap between two products holds at most one memory instruction: odd gaps of steps 0 - 2 the copies
- *    registers -> LDS of tile kt + 1 and the loads of tile kt + 3, even gaps the operand reads of the next step
- *    (all of them bunched at the step boundaries: 1160 TFLOP/s; two and a load per fourth gap: 1230; one per gap:
- *    1253);
- *  - one barrier per k tile, behind the products of step 2.
- * Same LDS layout as above (128 B rows, chunk c of row r in slot c ^ ((r >> 1) & 7)), two stages. Same bits as the
- * 8-wave kernel (same products in the same order per accumulator). Timing-only ablations at 4608 x 3072 -> 27648,
- * 1270 TFLOP/s as it stood then: without the barrier 1262 -> 1305 (+3.5 %), without the global loads 1451, without
- * loads and LDS writes 1711 (what 128 MFMAs and 32 operand reads per k tile run at), with loads that always hit
- * the same cached tile 1396. */
+ * For M, N >= 256, K a multiple of 128: every linear layer of the models at their larger sequence lengths. Eight waves, two
+ * per SIMD, 4 (rows of 64) x 2: a wave owns 64 rows x 16 NA columns = NA x 4 accumulator blocks (NA = 8, 7, 6, so that the
+ * launcher can pick the width whose grid fills the last round of the 256 CUs best). A k tile of 64 is four steps: k-step
+ * 0 with the first and the second half of the columns, then k-step 1; the operands of a step are requested from the LDS
+ * during the step before. What the kernel lives on:
+ *  - every memory instruction stands in a gap of its own between two products. All waves of the CU leave a barrier
+ *    together, so what is bunched behind it is not hidden by the other wave of the SIMD but added to the products;
+ *  - no branches: a request past the end of K asks for the last tile again, into a stage that nobody reads. With a
+ *    uniform branch around each request a k tile of 256 x 256 took 2550 cycles, without them 2230, of which the products
+ *    are 2048;
+ *  - the LDS holds two stages of x and three of W (160 KB at 256 columns). The stage of x that a barrier sets free is
+ *    requested at once (first gaps of step 3), W one step at a time in steps 0 - 2: rows from the L2 or HBM take as long
+ *    as a whole k tile. x spread over two steps instead: 4608 x 12288 -> 3072 284 us, as it is 244.
+ * Tiles are dealt out as in k_gemm_dma, in bands of four tile rows (2 and 8 within 1 %).
+ *
+ * Against the kernel it replaces (four waves of 128 x 128, one per SIMD, staged through registers), weights from HBM, us:
+ * 4608 x 3072 -> 9216 203 -> 188 (1390 TFLOP/s), -> 18432 408 -> 378, -> 27648 593 -> 566, 12288 -> 3072 257 -> 244, 9216 -> 3072
+ * 195 -> 186. With everything in the L2 4096 x 8192 -> 4096 runs at 1530 TFLOP/s, 2060 on zeros: the rest is the chip's
+ * power. Tried on it: k tiles of 32 in five stages (a direct load of sixteen 64 B rows takes longer than one of eight
+ * 128 B rows: 1170 TFLOP/s), a second barrier that frees the stages earlier (2 - 4 % slower). */
+/* The per-head RMSNorm + rotary embedding of the leading columns of a projection, applied by the GEMM to its
+ * own output tile (head_dim 128): columns [0, q_cols) are heads normalised with wq, [q_cols, qk_cols) with wk,
+ * the rest is stored as it is. */
+struct QkNorm {
+    const float *wq, *wk, *rope_cos, *rope_sin;  /* [128], [128], [M, 64], [M, 64] */
+    int q_cols, qk_cols;
+    float eps;
+    int split_half;
+};
+
+template <int NA>
+struct Wide {
+    static constexpr int TM = DT, TN = 32 * NA, XS = TM * TK, WS = TN * TK;          /* elements of an x and of a W stage */
+    static constexpr int WP = (TN / 8 + 7) / 8;                                      /* 8-row pieces of W per wave and k tile */
+    static constexpr int LDS = 2 * (2 * XS + 3 * WS) > 128 * 1024 ? 2 * (2 * XS + 3 * WS) : 128 * 1024;   /* the epilogue takes 128 KB */
+};
+
 template <typename OUT, int NA, bool QKN>
-__global__ void __launch_bounds__(256, 1)
-k_gemm_w4(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *__restrict__ W,
-          int M, int N, int K, int tiles_m, int total, int per_xcd, QkNorm qn, int streaming_out) {
-    /* NA blocks of 16 output columns per wave: tiles of 256 rows x TN = 32 NA columns (256, 224 or 192), so that the
-     * launcher can pick the width whose grid fills the last round of the 256 CUs best. */
-    constexpr int TN = 32 * NA;
-    constexpr int STAGE = (TN + DT) * TK;                      /* elements: W tile then x tile */
-    constexpr int NCW = NA, NCX = 8, NCH = NCW + NCX;          /* 16 B chunks of W and of x per thread and k tile: rows srow + 32 c */
-    extern __shared__ __align__(16) uint16_t dlds[];          /* two stages (and room for the epilogue) */
+__global__ void __launch_bounds__(512, 2)
+k_gemm_wide(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *__restrict__ W, int M, int N, int K,
+            int tiles_m, int total, int per_xcd, QkNorm qn, int streaming_out) {
+    using T = Wide<NA>;
+    constexpr int TM = T::TM, TN = T::TN, XS = T::XS, WS = T::WS, WP = T::WP, H0 = (NA + 1) / 2, H1 = NA / 2;
+    static_assert(WP <= 4 && H1 >= 3, "");
+    extern __shared__ __align__(16) uint16_t dlds[];           /* x, x, W, W, W */
     const int work = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
     if (work >= total) return;
-    constexpr int BAND = 4;                                    /* tile rows per band; 2, 6, 9, 18 measure the same or worse */
+    constexpr int BAND = 4;
     const int tiles_n = total / tiles_m;
     const int band = work / (BAND * tiles_n), in_band = work - band * (BAND * tiles_n);
     const int band_rows = min(tiles_m - band * BAND, BAND);
-    const int bm = band * BAND + in_band % band_rows, bn = in_band / band_rows;
-    /* The last tile of a row or column of tiles is moved back so that it ends with the matrix: it overlaps its
-     * neighbour, and both write the same bits there (an output's products are summed in the same order whatever
-     * tile it is in). So no row is ever clamped and no store bounded. */
-    const int m0 = min(bm * DT, M - DT), n0 = min(bn * TN, N - TN);
+    const int m0 = (band * BAND + in_band % band_rows) * TM, n0 = in_band / band_rows * TN;
+    const int last_tile = K / TK - 1;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int li = lane & 15, lg = lane >> 4;
-    const int wm = wave & 1, wn = wave >> 1;
+    const int li = lane & 15, lg = lane >> 4, wm = wave & 3, wn = wave >> 2;
 
-    /* staging: chunk tid % 8 of rows tid / 8 + 32 c; (row >> 1) & 7 is the same for all c, and the loads of a
-     * thread differ by uniform offsets */
-    const int srow = tid >> 3, schunk = tid & 7;
-    const int st_off = srow * TK + 8 * (schunk ^ ((srow >> 1) & 7));
-    const char *wt = reinterpret_cast<const char *>(W + (size_t)n0 * K), *xt = reinterpret_cast<const char *>(x + (size_t)m0 * K);   /* uniform tile bases */
-    const uint32_t lane_b = (uint32_t)(srow * K + 8 * schunk) * 2u;            /* this thread's bytes into a tile row block: never changes */
-    uint32_t tile_b = 0;                                                        /* uniform: bytes of the k tile to fetch next */
-    const uint32_t cstride = 64u * (uint32_t)K;                                 /* 32 rows, in bytes */
-    const int nk = K / TK, nk_tiles = nk;
-    u32x4 wreg[2][NCW], xreg[2][NCX];                          /* two tiles on their way at any time */
-    int fetched = 0;                                           /* tiles requested so far; tile_b stays on the last tile at the end */
-    auto fetch_one = [&](int set, int c) {                     /* c < NCW: chunk c of W, else chunk c - NCW of x */
-        if (c < NCW) wreg[set][c] = *reinterpret_cast<const u32x4 *>(wt + (size_t)(tile_b + c * cstride) + lane_b);
-        else xreg[set][c - NCW] = *reinterpret_cast<const u32x4 *>(xt + (size_t)(tile_b + (c - NCW) * cstride) + lane_b);
+    /* the 8-row pieces this wave fetches of every stage; rows past the end of a matrix repeat its last row (their outputs
+     * are never stored), pieces past the end of a stage its last piece; chunk c of row r sits in slot c ^ ((r >> 1) & 7) */
+    uint32_t xoff[4], woff[WP];
+    int wpiece[WP];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int r = 8 * (4 * wave + j) + (lane >> 3);
+        xoff[j] = ((uint32_t)min(m0 + r, M - 1) * (uint32_t)K + 8u * ((lane & 7) ^ ((r >> 1) & 7))) * 2u;
+    }
+#pragma unroll
+    for (int j = 0; j < WP; j++) {
+        wpiece[j] = min(WP * wave + j, TN / 8 - 1);
+        const int r = 8 * wpiece[j] + (lane >> 3);
+        woff[j] = ((uint32_t)min(n0 + r, N - 1) * (uint32_t)K + 8u * ((lane & 7) ^ ((r >> 1) & 7))) * 2u;
+    }
+    const uint32_t lds0 = lds_address(dlds);
+    auto request_x = [&](int j, int kt, uint32_t stage) {      /* stage: bytes into the LDS */
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                     ::"s"(lds0 + stage + (4 * wave + j) * 1024), "v"(xoff[j]), "s"(x + (size_t)kt * TK) : "memory", "m0");
     };
-    auto fetched_tile = [&]() { fetched++; tile_b += fetched < nk_tiles ? 2u * TK : 0u; };
-    auto store_half = [&](int set, int stage, int c, int hi) {  /* 8 of the 16 bytes of chunk c */
-        uint16_t *w_dst = dlds + stage * STAGE + st_off + 4 * hi;
-        const u32x4 v = c < NCW ? wreg[set][c] : xreg[set][c - NCW];
-        uint16_t *dst = c < NCW ? w_dst + 32 * c * TK : w_dst + TN * TK + 32 * (c - NCW) * TK;
-        *reinterpret_cast<uint2 *>(dst) = hi ? make_uint2(v[2], v[3]) : make_uint2(v[0], v[1]);
+    auto request_w = [&](int j, int kt, uint32_t stage) {
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                     ::"s"(lds0 + stage + wpiece[j] * 1024), "v"(woff[j]), "s"(W + (size_t)kt * TK) : "memory", "m0");
     };
-    auto store_one = [&](int set, int stage, int c) { store_half(set, stage, c, 0); store_half(set, stage, c, 1); };
 
-    f32x4 acc[NA][8];                                          /* [a: 16 columns][b: 16 rows] */
+    f32x4 acc[NA][4];                                          /* [16 columns][16 rows] */
 #pragma unroll
     for (int a = 0; a < NA; a++)
 #pragma unroll
-        for (int b = 0; b < 8; b++) acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
-    int a_rd[2], b_rd[2];
+        for (int b = 0; b < 4; b++) acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    u32x4 av[NA], bv[2][4];                                    /* W operands of a k-step, x operands of both */
+    int a_rd[2], b_rd[2];                                      /* bytes into a stage */
 #pragma unroll
     for (int ks = 0; ks < 2; ks++) {
-        const int slot = 8 * ((4 * ks + lg) ^ (li >> 1));
-        a_rd[ks] = (16 * NA * wn + li) * TK + slot;
-        b_rd[ks] = TN * TK + (128 * wm + li) * TK + slot;
+        const int slot = 16 * ((4 * ks + lg) ^ (li >> 1));
+        a_rd[ks] = (16 * NA * wn + li) * 128 + slot;
+        b_rd[ks] = (64 * wm + li) * 128 + slot;
     }
-
-    /* Four steps of 4 NA MFMAs per k tile: k-step ks = step / 2, x blocks 4 (step % 2) .. + 3. The operands of a
-     * step are requested from the LDS during the step before it, across the tile boundary too. One barrier per
-     * tile, behind the products of step 2: by then every wave has written its share of tile kt + 1 and has read
-     * the last operands of tile kt, so after it the stage of tile kt + 1 is complete and the stage of tile kt is
-     * free for tile kt + 2. The products are asm statements with the accumulators in AGPRs. */
-    u32x4 av[2][NA], bv[2][4];
-    auto read_a_one = [&](const uint16_t *stage, int ks, int a) {
-        av[ks][a] = *reinterpret_cast<const u32x4 *>(&stage[a_rd[ks] + 16 * a * TK]);
+    const char *lds_b = reinterpret_cast<const char *>(dlds);
+    auto read_a = [&](uint32_t stage, int ks, int a) { av[a] = *reinterpret_cast<const u32x4 *>(lds_b + stage + a_rd[ks] + 2048 * a); };
+    auto read_b = [&](uint32_t stage, int ks, int b) { bv[ks][b] = *reinterpret_cast<const u32x4 *>(lds_b + stage + b_rd[ks] + 2048 * b); };
+    /* operand i of the first half of a k-step, in the order its products use them */
+    auto read_first = [&](uint32_t xs, uint32_t ws, int ks, int i) {
+        if (i == 0) read_a(ws, ks, 0);
+        else if (i < 5) read_b(xs, ks, i - 1);
+        else if (i < 4 + H0) read_a(ws, ks, i - 4);
     };
-    auto read_b_one = [&](const uint16_t *stage, int step, int b) {
-        bv[step & 1][b] = *reinterpret_cast<const u32x4 *>(&stage[b_rd[step >> 1] + 16 * (4 * (step & 1) + b) * TK]);
-    };
-    auto products = [&](int step, auto &&between) {
-        const int ks = step >> 1, half = step & 1;
+    auto products = [&](int ks, int a0, int a1, auto &&gap) {
 #pragma unroll
-        for (int b = 0; b < 4; b++)
-#pragma unroll
-            for (int a = 0; a < NA; a++) {
-                asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[a][4 * half + b]) : "v"(av[ks][a]), "v"(bv[step & 1][b]));
-                between(NA * b + a);
-            }
+        for (int g = 0; g < 4 * (a1 - a0); g++) {
+            const int a = a0 + g / 4, b = g % 4;
+            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av[a]), __builtin_bit_cast(bf16x8, bv[ks][b]), acc[a][b], 0, 0, 0);
+            gap(g);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     };
 
+    /* stages: x of this tile and of the next, W of this tile, the next and the one after */
+    uint32_t x_cur = 0, x_nxt = 2 * XS, w_cur = 4 * XS, w_nxt = 4 * XS + 2 * WS, w_far = 4 * XS + 4 * WS;
+    const int second = min(1, last_tile);
 #pragma unroll
-    for (int c = 0; c < NCH; c++) fetch_one(0, c);             /* tile 0 */
-    fetched_tile();
+    for (int j = 0; j < WP; j++) request_w(j, 0, w_cur);
 #pragma unroll
-    for (int c = 0; c < NCH; c++) store_one(0, 0, c);
+    for (int j = 0; j < 4; j++) request_x(j, 0, x_cur);
 #pragma unroll
-    for (int c = 0; c < NCH; c++) fetch_one(1, c);             /* tiles 1 and 2 (or the last tile again) wait in the registers */
-    fetched_tile();
+    for (int j = 0; j < WP; j++) request_w(j, second, w_nxt);
 #pragma unroll
-    for (int c = 0; c < NCH; c++) fetch_one(0, c);
-    fetched_tile();
-    lds_barrier();
+    for (int j = 0; j < 4; j++) request_x(j, second, x_nxt);
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(WP + 4) : "memory");
 #pragma unroll
-    for (int a = 0; a < NA; a++) read_a_one(dlds, 0, a);
-#pragma unroll
-    for (int b = 0; b < 4; b++) read_b_one(dlds, 0, b);
+    for (int i = 0; i < 4 + H0; i++) read_first(x_cur, w_cur, 0, i);
 
-    /* One k tile: `set` holds tile kt + 1 on entry and tile kt + 3 on exit. */
-    auto k_tile = [&](int kt, int set) {
-        const uint16_t *cur = dlds + (kt & 1) * STAGE, *nxt = dlds + ((kt + 1) & 1) * STAGE;
-        const int nstage = (kt + 1) & 1;
-        /* At most one memory instruction behind a product: the wave issues in order, and what it issues between
-         * two products has to fit into the 12 cycles the matrix core still works on the first. Even gaps: the
-         * operands of the next step in the order its products use them (4 x-blocks, and for an odd step the NA
-         * W-blocks of its k-step). Odd gaps of steps 0 - 2, 6 NA of them: the 3 NCH staging jobs in order, chunk by
-         * chunk two 8-byte copies registers -> LDS of tile kt + 1 and then the load of the same chunk of tile
-         * kt + 3 into the registers just freed; the few that do not fit (NA = 7: 45 jobs, 42 odd gaps) take the
-         * even gaps of step 2 behind its four reads. */
-        constexpr int ODD = 2 * NA;                             /* odd gaps per step */
-        auto staging_job = [&](int j) {
-            if (j >= 3 * NCH) return;
-            const int c = j / 3, part = j - 3 * c;
-            if (part < 2) store_half(set, nstage, c, part);
-            else fetch_one(set, c);
-        };
-        auto slot = [&](int step, int i) {
-            const int r = i >> 1;
-            if (i & 1) {
-                if (step < 3) staging_job(ODD * step + r);
-            } else {
-                if (step == 0 && r < 4) read_b_one(cur, 1, r);
-                if (step == 1) { if (r < 4) read_b_one(cur, 2, r); else if (r < 4 + NA) read_a_one(cur, 1, r - 4); }
-                if (step == 2) { if (r < 4) read_b_one(cur, 3, r); else staging_job(3 * ODD + r - 4); }
-                if (step == 3) { if (r < 4) read_b_one(nxt, 0, r); else if (r < 4 + NA) read_a_one(nxt, 0, r - 4); }
-            }
-        };
-        products(0, [&](int i) { slot(0, i); });
-        products(1, [&](int i) { slot(1, i); });
-        products(2, [&](int i) { slot(2, i); });
-        fetched_tile();
-        lds_barrier();
-        products(3, [&](int i) { slot(3, i); });
-    };
-    for (int kt = 0; kt < nk; kt += 2) {                       /* nk is even */
-        k_tile(kt, 1);
-        k_tile(kt + 1, 0);
+    for (int t = 0; t <= last_tile; t++) {
+        const int after_next = min(t + 2, last_tile);
+        products(0, 0, H0, [&](int g) {
+            if (g < H1) read_a(w_cur, 0, H0 + g);
+            if (g == 6) request_w(0, after_next, w_far);
+            if (g == 10 && WP > 3) request_w(WP - 1, after_next, w_far);
+        });
+        products(0, H0, NA, [&](int g) { read_first(x_cur, w_cur, 1, g); });
+        products(1, 0, H0, [&](int g) {
+            if (g < H1) read_a(w_cur, 1, H0 + g);
+            if (g == 6) request_w(1, after_next, w_far);
+            if (g == 9) request_w(2, after_next, w_far);
+        });
+        /* This wave has read its last operands of the tile, and its share of the next one has landed: newer than that are
+         * only the W pieces requested in this tile. Behind the barrier the tile's stages are free. */
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(WP) : "memory");
+        products(1, H0, NA, [&](int g) {                       /* x at gaps 0, 2, 4, 6, the reads in the others */
+            if (g < 8 && g % 2 == 0) request_x(g / 2, after_next, x_cur);
+            else read_first(x_nxt, w_nxt, 0, g < 8 ? g / 2 : g - 4);
+        });
+        const uint32_t x_free = x_cur, w_free = w_cur;
+        x_cur = x_nxt; x_nxt = x_free;
+        w_cur = w_nxt; w_nxt = w_far; w_far = w_free;
     }
-    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");                /* the last products have left the matrix core before the accumulators are read */
-    lds_barrier();                                              /* the LDS is reused by the epilogue */
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");         /* the LDS is reused by the epilogue */
 
-    /* acc[a][b][r] = y[m0 + 128 wm + 16 b + li][n0 + 16 NA wn + 16 a + 4 lg + r] */
-    constexpr int PER16 = 16 / (int)sizeof(OUT);
-    const int mw = m0 + 128 * wm, nw = n0 + 16 * NA * wn;
+    /* acc[a][b][r] = y[m0 + 64 wm + 16 b + li][n0 + 16 NA wn + 16 a + 4 lg + r] */
+    constexpr int PER16 = 16 / (int)sizeof(OUT);               /* outputs per 16 B; the launcher has N a multiple of it */
+    const int mw = m0 + 64 * wm, nw = n0 + 16 * NA * wn;
     if constexpr (QKN) {
-        /* the whole 256 x 256 bf16 tile in the LDS (128 KB), then a 16-lane row per (token, head) vector: see k_gemm_dma */
+        /* A tile with head columns in it is staged as a whole: 256 rows x 512 B fill 128 KB. 16 B chunk c of row r sits in
+         * slot (c & 16) | ((c ^ r) & 15): the 16 rows of a write and the 16 chunks of a head vector both spread over all
+         * banks. Then a 16-lane row per (token, head) vector, 32 vectors a pass, through the same function as the
+         * stand-alone kernel: the stored bits are those of the plain projection followed by that kernel. */
         static_assert(sizeof(OUT) == 2 && NA == 8, "bf16 projection, tiles of two whole heads");
-        if (n0 < qn.qk_cols) {
+        if (n0 < qn.qk_cols) {                                  /* the same for the whole workgroup */
 #pragma unroll
-            for (int b = 0; b < 8; b++)
+            for (int b = 0; b < 4; b++)
 #pragma unroll
                 for (int a = 0; a < 8; a++) {
-                    const int row = 128 * wm + 16 * b + li, chunk = 16 * wn + 2 * a + (lg >> 1);
+                    const int row = 64 * wm + 16 * b + li, chunk = 16 * wn + 2 * a + (lg >> 1);
                     const int slot = (chunk & 16) | ((chunk ^ li) & 15);
                     *reinterpret_cast<uint2 *>(&dlds[row * 256 + 8 * slot + 4 * (lg & 1)]) =
                         make_uint2(pack_bf16(acc[a][b][0], acc[a][b][1]), pack_bf16(acc[a][b][2], acc[a][b][3]));
@@ -684,12 +612,10 @@ k_gemm_w4(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *_
             }
             const int tcol = qn.split_half ? 8 * (sub & 7) : 4 * sub;
             const int chunk = 16 * head + sub;
-            /* whole tiles: no row or head of the tile lies outside y, so the passes are straight-line code and the
-             * table loads of eight of them are in flight together (the wave has its SIMD to itself: nothing else
-             * hides their latency) */
-#pragma unroll 8
-            for (int pass = 0; pass < DT / 8; pass++) {
-                const int row = 8 * pass + row_in, m = m0 + row;
+#pragma unroll 4
+            for (int pass = 0; pass < DT / 16; pass++) {
+                const int row = 16 * pass + row_in, m = m0 + row;
+                if (m >= M || n_head >= N) continue;            /* the same for the 16 lanes of a vector */
                 u32x4 v = *reinterpret_cast<const u32x4 *>(&dlds[row * 256 + 8 * ((chunk & 16) | ((chunk ^ row) & 15))]);
                 if (normed) {
                     const float *cr = qn.rope_cos + (size_t)m * 64 + tcol, *sr = qn.rope_sin + (size_t)m * 64 + tcol;
@@ -711,68 +637,48 @@ k_gemm_w4(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *_
             return;
         }
     }
-    const bool staged = N % PER16 == 0 && ((uintptr_t)y & 15) == 0;
-    if (staged) {
-        /* through the LDS (free after the loop's last barrier; 32 KB per wave, its own region, no workgroup barrier), so
-         * that the stores leave as 16 B per lane along the rows. LDS serves a wave's instructions in order. */
-        uint16_t *mine = dlds + wave * 16384;
-        if constexpr (sizeof(OUT) == 4) {
-            float *buf = reinterpret_cast<float *>(mine);       /* 64 rows x 128 f32 at a time, chunk c of row r in slot (c & 16) | ((c ^ r) & 15) */
+    uint16_t *mine = dlds + wave * 8192;                       /* 16 KB, a wave's own region: no barrier */
+    if constexpr (sizeof(OUT) == 4) {
+        float *buf = reinterpret_cast<float *>(mine);          /* 32 rows x 128 f32 at a time, chunk c of row r in slot (c & 16) | ((c ^ r) & 15) */
 #pragma unroll
-            for (int half = 0; half < 2; half++) {
+        for (int half = 0; half < 2; half++) {
 #pragma unroll
-                for (int bb = 0; bb < 4; bb++)
-#pragma unroll
-                    for (int a = 0; a < NA; a++) {
-                        const int chunk = 4 * a + lg;
-                        *reinterpret_cast<f32x4 *>(&buf[(16 * bb + li) * 128 + 4 * ((chunk & 16) | ((chunk ^ li) & 15))]) = acc[a][4 * half + bb];
-                    }
-#pragma unroll
-                for (int it = 0; it < 32; it++) {
-                    const int row = 2 * it + (lane >> 5), c = lane & 31;
-                    f32x4 v = *reinterpret_cast<const f32x4 *>(&buf[row * 128 + 4 * ((c & 16) | ((c ^ row) & 15))]);
-                    const int m = mw + 64 * half + row, n = nw + 4 * c;
-                    if (c < 4 * NA) {
-                        f32x4 *dst = reinterpret_cast<f32x4 *>(reinterpret_cast<float *>(y) + (size_t)m * N + n);
-                        if (streaming_out) __builtin_nontemporal_store(v, dst);
-                        else *dst = v;
-                    }
-                }
-            }
-        } else {
-            uint16_t *buf = mine;                               /* 128 rows x 128 bf16, chunk c of row r in slot c ^ (r % 16) */
-#pragma unroll
-            for (int b = 0; b < 8; b++)
+            for (int b = 0; b < 2; b++)
 #pragma unroll
                 for (int a = 0; a < NA; a++) {
-                    const int chunk = 2 * a + (lg >> 1);
-                    *reinterpret_cast<uint2 *>(&buf[(16 * b + li) * 128 + 8 * (chunk ^ li) + 4 * (lg & 1)]) =
-                        make_uint2(pack_bf16(acc[a][b][0], acc[a][b][1]), pack_bf16(acc[a][b][2], acc[a][b][3]));
+                    const int chunk = 4 * a + lg;
+                    *reinterpret_cast<f32x4 *>(&buf[(16 * b + li) * 128 + 4 * ((chunk & 16) | ((chunk ^ li) & 15))]) = acc[a][2 * half + b];
                 }
 #pragma unroll
-            for (int it = 0; it < 32; it++) {
-                const int row = 4 * it + (lane >> 4), c = lane & 15;
-                const u32x4 v = *reinterpret_cast<const u32x4 *>(&buf[row * 128 + 8 * (c ^ (row & 15))]);
-                const int m = mw + row, n = nw + 8 * c;
-                if (c < 2 * NA) {
-                    u32x4 *dst = reinterpret_cast<u32x4 *>(reinterpret_cast<uint16_t *>(y) + (size_t)m * N + n);
+            for (int it = 0; it < 16; it++) {
+                const int row = 2 * it + (lane >> 5), c = lane & 31, m = mw + 32 * half + row, n = nw + PER16 * c;
+                const f32x4 v = *reinterpret_cast<const f32x4 *>(&buf[row * 128 + 4 * ((c & 16) | ((c ^ row) & 15))]);
+                if (c < 4 * NA && m < M && n < N) {
+                    f32x4 *dst = reinterpret_cast<f32x4 *>(reinterpret_cast<float *>(y) + (size_t)m * N + n);
                     if (streaming_out) __builtin_nontemporal_store(v, dst);
                     else *dst = v;
                 }
             }
         }
-        return;
-    }
+    } else {
+        uint16_t *buf = mine;                                  /* 64 rows x 128 bf16, chunk c of row r in slot c ^ (r % 16) */
 #pragma unroll
-    for (int b = 0; b < 8; b++) {
-        const int m = mw + 16 * b + li;
-        if (m >= M) continue;
+        for (int b = 0; b < 4; b++)
 #pragma unroll
-        for (int a = 0; a < NA; a++) {
-            const int n = nw + 16 * a + 4 * lg;
-            if (n >= N) continue;
-            f32x4 v = acc[a][b];
-            store4(y + (size_t)m * N + n, v, N - n);
+            for (int a = 0; a < NA; a++) {
+                const int chunk = 2 * a + (lg >> 1);
+                *reinterpret_cast<uint2 *>(&buf[(16 * b + li) * 128 + 8 * (chunk ^ li) + 4 * (lg & 1)]) =
+                    make_uint2(pack_bf16(acc[a][b][0], acc[a][b][1]), pack_bf16(acc[a][b][2], acc[a][b][3]));
+            }
+#pragma unroll
+        for (int it = 0; it < 16; it++) {
+            const int row = 4 * it + (lane >> 4), c = lane & 15, m = mw + row, n = nw + PER16 * c;
+            const u32x4 v = *reinterpret_cast<const u32x4 *>(&buf[row * 128 + 8 * (c ^ (row & 15))]);
+            if (c < 2 * NA && m < M && n < N) {
+                u32x4 *dst = reinterpret_cast<u32x4 *>(reinterpret_cast<uint16_t *>(y) + (size_t)m * N + n);
+                if (streaming_out) __builtin_nontemporal_store(v, dst);
+                else *dst = v;
+            }
         }
     }
 }
@@ -781,20 +687,19 @@ k_gemm_w4(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *_
 
 constexpr int DMA_LDS_BYTES = 128 * 1024;        /* two stages of (256 + 256) x 128 B; also the 8 x 16 KB of the epilogue */
 
-template <typename OUT, int TN, bool CONV, bool QKN = false>
-int launch_gemm_dma(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, const ConvGeom &geo,
-                    const QkNorm &qn = QkNorm{}) {
+template <typename OUT, int TN, bool CONV>
+int launch_gemm_dma(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, const ConvGeom &geo) {
     static bool configured = false;
     if (!configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_gemm_dma<OUT, TN, CONV, QKN>),
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_gemm_dma<OUT, TN, CONV>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, DMA_LDS_BYTES);
         if (e != hipSuccess) return (int)e;
         configured = true;
     }
     const int tiles_m = (M + DT - 1) / DT, tiles_n = (N + TN - 1) / TN, total = tiles_m * tiles_n;
     const int per_xcd = (total + 7) / 8;
-    hipLaunchKernelGGL((k_gemm_dma<OUT, TN, CONV, QKN>), dim3((unsigned)per_xcd * 8), dim3(512), DMA_LDS_BYTES, st, y, x, W, M, N, K,
-                       tiles_m, total, per_xcd, geo, qn);
+    hipLaunchKernelGGL((k_gemm_dma<OUT, TN, CONV>), dim3((unsigned)per_xcd * 8), dim3(512), DMA_LDS_BYTES, st, y, x, W, M, N, K,
+                       tiles_m, total, per_xcd, geo);
     return (int)hipGetLastError();
 }
 
@@ -813,11 +718,11 @@ k_gemm_scalar(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_
 }
 
 template <typename OUT, int NA, bool QKN = false>
-int launch_gemm_w4(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, const QkNorm &qn = QkNorm{}) {
+int launch_gemm_wide(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, const QkNorm &qn = QkNorm{}) {
     static bool configured = false;
     if (!configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_gemm_w4<OUT, NA, QKN>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, DMA_LDS_BYTES);
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_gemm_wide<OUT, NA, QKN>),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, Wide<NA>::LDS);
         if (e != hipSuccess) return (int)e;
         configured = true;
     }
@@ -825,25 +730,23 @@ int launch_gemm_w4(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W,
     const int per_xcd = (total + 7) / 8;
     /* An output of 192 MB or more cannot stay in the 256 MB Infinity Cache next to the operands: stored with the
      * streaming hint it does not push the weights out on its way (4608 x 3072 -> 27648: f32 output 671 -> 626 us, bf16
-     * 594 -> 585; smaller outputs are within 1 % either way and keep the plain stores, which leave them cached for the
-     * operator that reads them next). */
+     * 594 -> 585 when it was introduced; smaller outputs are within 1 % either way and keep the plain stores, which leave
+     * them cached for the operator that reads them next). */
     const int streaming_out = (size_t)M * N * sizeof(OUT) >= ((size_t)192 << 20);
-    hipLaunchKernelGGL((k_gemm_w4<OUT, NA, QKN>), dim3((unsigned)per_xcd * 8), dim3(256), DMA_LDS_BYTES, st, y, x, W, M, N, K,
+    hipLaunchKernelGGL((k_gemm_wide<OUT, NA, QKN>), dim3((unsigned)per_xcd * 8), dim3(512), Wide<NA>::LDS, st, y, x, W, M, N, K,
                        tiles_m, total, per_xcd, qn, streaming_out);
     return (int)hipGetLastError();
 }
 
-/* What the four-wave kernel takes: at least one tile each way (its last tiles are moved back to end with the
- * matrix, so the sizes need not be multiples of the tile), an even number of k tiles, 16-byte stores, and tiles
- * of less than 4 GB. */
-static bool four_wave_shape(int M, int N, int K, size_t out_size) {
-    return M >= DT && N >= 256 && K % (2 * TK) == 0 && N % (16 / (int)out_size) == 0 &&
-           (size_t)K * 2 * (DT + 32) < ((size_t)1 << 32);             /* a thread's byte offsets into a tile are 32-bit */
+/* What that kernel takes: 16-byte stores, and 32-bit byte offsets into the operands. */
+static bool wide_shape(int M, int N, int K, size_t out_size) {
+    return M >= DT && N >= 256 && K % (2 * TK) == 0 && N % (16 / (int)out_size) == 0 && ((size_t)M * K * 2) >> 32 == 0 &&
+           ((size_t)N * K * 2) >> 32 == 0;
 }
 
 /* The tile width (32 NA columns) whose grid wastes least of its last round of 256 workgroups: time goes with
  * rounds x width. 4608 x 9216 outputs: 648 tiles of 256 columns are 2.53 rounds, 756 of 224 are 2.95. */
-static int four_wave_width(int M, int N) {
+static int wide_width(int M, int N) {
     const long tiles_m = (M + DT - 1) / DT;
     int best = 8;
     long best_cost = 0;
@@ -856,22 +759,22 @@ static int four_wave_width(int M, int N) {
 }
 
 /* Which kernel a linear layer takes, host arithmetic only: 4 = k_gemm_tiles (gemm_tiles_gfx950.hip) with its tile `na` and
- * `splits` ranges of K, 3 = k_gemm_w4 with tiles of 32 na columns, 2 = k_gemm_dma, 1 = k_gemm_bf16, 0 = k_gemm_scalar.
+ * `splits` ranges of K, 3 = k_gemm_wide with tiles of 32 na columns, 2 = k_gemm_dma, 1 = k_gemm_bf16, 0 = k_gemm_scalar.
  *
- * Between 4 and 3 the estimated times decide: a k tile costs a four-wave workgroup 0.175 us per 32 columns (0.155 in a
- * grid that leaves most CUs idle), its ends 4 us a round. Where 4 is chosen it measured, weights from HBM (four-wave or
- * 128 x 128 kernel before): 512 x 9728 -> 2560 146 -> 38 us, 320 x 12288 -> 3072 179 -> 36, 512 x 3072 -> 9216 52 -> 37,
- * 118 x 2560 -> 6144 41 -> 17, 80 x 12288 -> 3072 183 -> 23, 1000 x 12288 -> 3072 182 -> 75, 2115 x 3072 -> 9216 111 -> 98,
- * 2115 x 9216 -> 3072 136 -> 103. Long grids of full rows stay: 4608 x 3072 -> 9216 would take 5 rounds of 160 x 256. */
+ * Between 4 and 3 the estimated times decide: a k tile costs a workgroup of k_gemm_wide 0.175 us per 32 columns (0.145 in a
+ * grid that leaves most CUs idle), its ends 4 us a round. Measured, weights from HBM, us of 4 against 3 at its best width:
+ * 512 x 9728 -> 2560 38 against 138, 512 x 3072 -> 9216 38 / 50, 1000 x 12288 -> 3072 76 / 175, 2115 x 9216 -> 3072 104 / 122,
+ * 2115 x 3072 -> 9216 100 / 104; and where 3 is taken 512 x 3072 -> 18432 79 / 58, 1000 x 3072 -> 27648 156 / 136,
+ * 2115 x 3072 -> 18432 209 / 194, 2912 x 12288 -> 4096 265 / 224. */
 struct GemmPlan { int kernel, na, splits; };
 static GemmPlan plan_gemm(int M, int N, int K, int out_size, bool operands_aligned16, bool out_aligned16, size_t part_bytes) {
     int shape = 0, splits = 1;
     const float tiles_us = operands_aligned16 && out_aligned16 ? iris_hip_gemm_tiles_plan(M, N, K, out_size, part_bytes, &shape, &splits) : -1.0f;
     if (K > 0 && K % TK == 0 && operands_aligned16 && M >= DT && N >= DT && (size_t)K * 2 * 8 < ((size_t)1 << 31)) {
-        if (four_wave_shape(M, N, K, (size_t)out_size) && out_aligned16) {
-            const int na = four_wave_width(M, N);
+        if (wide_shape(M, N, K, (size_t)out_size) && out_aligned16) {
+            const int na = wide_width(M, N);
             const long wgs = (long)((M + DT - 1) / DT) * ((N + 32 * na - 1) / (32 * na)), rounds = (wgs + 255) / 256;
-            const float us = 4.0f + (float)rounds * ((float)(K / TK) * (wgs <= 128 ? 0.155f : 0.175f) * (float)na + 4.0f);
+            const float us = 4.0f + (float)rounds * ((float)(K / TK) * (wgs <= 128 ? 0.145f : 0.175f) * (float)na + 4.0f);
             if (tiles_us < 0.0f || tiles_us >= us) return {3, na, 1};
             return {4, shape, splits};
         }
@@ -895,8 +798,8 @@ int gemm(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, in
         const ConvGeom none = {};
         int e;
         if (plan.kernel == 3) {
-            e = plan.na == 8 ? launch_gemm_w4<OUT, 8>(st, y, x, W, M, N, K)
-              : plan.na == 7 ? launch_gemm_w4<OUT, 7>(st, y, x, W, M, N, K) : launch_gemm_w4<OUT, 6>(st, y, x, W, M, N, K);
+            e = plan.na == 8 ? launch_gemm_wide<OUT, 8>(st, y, x, W, M, N, K)
+              : plan.na == 7 ? launch_gemm_wide<OUT, 7>(st, y, x, W, M, N, K) : launch_gemm_wide<OUT, 6>(st, y, x, W, M, N, K);
         } else {
             e = launch_gemm_dma<OUT, 256, false>(st, y, x, W, M, N, K, none);
         }
@@ -953,9 +856,9 @@ k_add_bias_rows(float *__restrict__ y, const float *__restrict__ bias, int cols,
 
 extern "C" {
 
-/* The kernel a linear layer of these sizes takes (aligned operands): plan[0] = 4 the tiles of gemm_tiles_gfx950.hip, 3 four
- * waves, 2 eight waves with direct loads, 1 the 128 x 128 kernel, 0 scalar; plan[1] = columns of a tile of the four-wave
- * kernel, or the ranges of K of the first. No GPU needed. */
+/* The kernel a linear layer of these sizes takes (aligned operands): plan[0] = 4 the tiles of gemm_tiles_gfx950.hip, 3
+ * k_gemm_wide, 2 k_gemm_dma, 1 the 128 x 128 kernel, 0 scalar; plan[1] = columns of a tile of k_gemm_wide, or the ranges of
+ * K of the first. No GPU needed. */
 void iris_hip_linear_plan(int rows, int in, int out, int out_bytes, int *plan) {
     const GemmPlan p = plan_gemm(rows, out, in, out_bytes, true, true, IRIS_LINEAR_PART_BYTES);
     plan[0] = p.kernel; plan[1] = p.kernel == 3 ? 32 * p.na : p.kernel == 4 ? p.splits : 0;
@@ -969,9 +872,9 @@ int iris_hip_linear_bf16(void *stream, float *part, uint16_t *y, const uint16_t 
 }
 
 /* y = x W^T as bf16 with the per-head RMSNorm + rotary embedding (head_dim 128) of columns [0, q_cols) (weights
- * wq) and [q_cols, q_cols + k_cols) (weights wk): applied in the GEMM's epilogue, or, where the plain layer takes the tiles
- * of gemm_tiles_gfx950.hip, by the norm kernel behind it. Returns -2, with nothing
- * enqueued, for a shape the tiled kernels do not take: the caller then runs the two steps one after the other. */
+ * wq) and [q_cols, q_cols + k_cols) (weights wk): applied in the GEMM's epilogue where the plain layer takes 256-column
+ * tiles of k_gemm_wide (a tile then holds two whole heads), by the norm kernel behind it elsewhere. Returns -2, with
+ * nothing enqueued, for a shape it does not take: the caller then runs the two steps one after the other. */
 int iris_hip_linear_bf16_qknorm(void *stream, float *part, uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out,
                                 int q_cols, int k_cols, const float *wq, const float *wk, const float *rope_cos,
                                 const float *rope_sin, float eps, int split_half) {
@@ -979,22 +882,19 @@ int iris_hip_linear_bf16_qknorm(void *stream, float *part, uint16_t *y, const ui
     const uintptr_t all = (uintptr_t)x | (uintptr_t)W | (uintptr_t)y | (uintptr_t)wq | (uintptr_t)wk | (uintptr_t)rope_cos |
                           (uintptr_t)rope_sin;
     const bool tiled = K > 0 && K % TK == 0 && (all & 15) == 0 && M >= DT && N >= DT && (size_t)K * 2 * 8 < ((size_t)1 << 31);
+    const int qh = q_cols / 128, kh = k_cols / 128;
     if (!tiled || N % 128 || q_cols < 0 || k_cols < 0 || q_cols % 128 || k_cols % 128 || q_cols + k_cols > N ||
-        q_cols + k_cols == 0)
+        q_cols + k_cols == 0 || (long long)M * (qh + kh) >= (1 << 24) || qh + kh >= 256)
         return -2;
-    if (plan_gemm(M, N, K, 2, true, true, IRIS_LINEAR_PART_BYTES).kernel == 4) {
-        const int qh = q_cols / 128, kh = k_cols / 128;
-        if ((long long)M * (qh + kh) >= (1 << 24) || qh + kh >= 256) return -2;
-        const int e = gemm<uint16_t>((hipStream_t)stream, y, x, W, M, N, K, part, IRIS_LINEAR_PART_BYTES);
-        if (e) return e;
-        return qh ? iris_hip_norm_rope_hd128(stream, y, kh ? y + q_cols : nullptr, N, wq, wk, rope_cos, rope_sin, M, qh, kh, eps, split_half)
-                  : iris_hip_norm_rope_hd128(stream, y, nullptr, N, wk, nullptr, rope_cos, rope_sin, M, kh, 0, eps, split_half);
+    const GemmPlan plan = plan_gemm(M, N, K, 2, true, true, IRIS_LINEAR_PART_BYTES);
+    if (plan.kernel == 3 && plan.na == 8) {
+        const QkNorm qn = {wq, k_cols ? wk : wq, rope_cos, rope_sin, q_cols, q_cols + k_cols, eps, split_half};
+        return launch_gemm_wide<uint16_t, 8, true>((hipStream_t)stream, y, x, W, M, N, K, qn);
     }
-    const ConvGeom none = {};
-    const QkNorm qn = {wq, k_cols ? wk : wq, rope_cos, rope_sin, q_cols, q_cols + k_cols, eps, split_half};
-    if (M % DT == 0 && N % 256 == 0 && four_wave_shape(M, N, K, 2))   /* whole tiles: a tile holds two whole heads */
-        return launch_gemm_w4<uint16_t, 8, true>((hipStream_t)stream, y, x, W, M, N, K, qn);
-    return launch_gemm_dma<uint16_t, 256, false, true>((hipStream_t)stream, y, x, W, M, N, K, none, qn);
+    const int e = gemm<uint16_t>((hipStream_t)stream, y, x, W, M, N, K, part, IRIS_LINEAR_PART_BYTES);
+    if (e) return e;
+    return qh ? iris_hip_norm_rope_hd128(stream, y, kh ? y + q_cols : nullptr, N, wq, wk, rope_cos, rope_sin, M, qh, kh, eps, split_half)
+              : iris_hip_norm_rope_hd128(stream, y, nullptr, N, wk, nullptr, rope_cos, rope_sin, M, kh, 0, eps, split_half);
 }
 
 /* Zeroes the first IRIS_CONV_ZERO_BYTES of a freshly allocated convolution scratch buffer: the page that taps
