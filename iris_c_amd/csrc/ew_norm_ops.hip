@@ -306,7 +306,8 @@ __device__ __forceinline__ Moments from_shifted(float n, float k, float s, float
 
 /* part[(g * nblocks + b)] = moments of group g over the pixels of block b. Coalesced form: needs
  * c % 4 == 0, cg % 4 == 0 and (c / 4) dividing 256; a thread keeps one quad of channels (inside
- * one group), the workgroup walks 256 / (c / 4) pixels per step with 16-byte loads. */
+ * one group), the workgroup walks 256 / (c / 4) pixels per step with 16-byte loads, eight of them in flight per thread:
+ * 512 x 512 x 256 63 -> 49 us, 1024 x 1024 x 128 115 -> 101 (5.3 TB/s). */
 __global__ void __launch_bounds__(ROW_THREADS)
 k_gn_moments_quads(Moments *__restrict__ part, const float *__restrict__ in, int hw, int c, int cg, int per_block) {
     __shared__ Moments sh[ROW_THREADS];
@@ -316,13 +317,22 @@ k_gn_moments_quads(Moments *__restrict__ part, const float *__restrict__ in, int
     float n = 0.0f, k = 0.0f, s = 0.0f, ss = 0.0f;
     int p = start + sub;
     if (p < end) k = in[(size_t)p * c + 4 * q];
-    for (; p < end; p += ppi) {
-        const float4 v = *reinterpret_cast<const float4 *>(in + (size_t)p * c + 4 * q);
+    auto take = [&](const float4 v) {
         const float a0 = v.x - k, a1 = v.y - k, a2 = v.z - k, a3 = v.w - k;
         s += (a0 + a1) + (a2 + a3);
         ss += (a0 * a0 + a1 * a1) + (a2 * a2 + a3 * a3);
         n += 4.0f;
+    };
+    const size_t step = (size_t)ppi * c;
+    const float *src = in + (size_t)p * c + 4 * q;
+    for (; p + 7 * ppi < end; p += 8 * ppi, src += 8 * step) {
+        float4 v[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = *reinterpret_cast<const float4 *>(src + i * step);
+#pragma unroll
+        for (int i = 0; i < 8; i++) take(v[i]);
     }
+    for (; p < end; p += ppi, src += step) take(*reinterpret_cast<const float4 *>(src));
     sh[threadIdx.x] = from_shifted(n, k, s, ss);
     __syncthreads();
     const int groups = c / cg, qpg = cg >> 2;
