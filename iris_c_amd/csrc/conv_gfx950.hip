@@ -4,7 +4,8 @@
  *
  * k_conv_few_in: k * k * cin <= 32, the 3-channel input of the VAE encoder.
  * k_conv_few_out: k * k * cout <= 28, the 3-channel output of the VAE decoder.
- * k_conv_3x3: 3 x 3, stride 1, cin a multiple of 64: every other layer of the VAE but the 1 x 1 and the halving ones.
+ * k_conv_1x1: cin a multiple of 128, at most 512, cout at most 256: the VAE's skip connections.
+ * k_conv_3x3: 3 x 3, stride 1, cin a multiple of 64: every other layer of the VAE but the halving ones.
  *
  * The first two are bound by memory: one side of the product is so thin that the image on the other side is all there
  * is to move. The image is rounded to bf16 on the way into the matrix core, products are summed in f32.
@@ -203,6 +204,124 @@ k_conv_few_out(float *__restrict__ out, const float *__restrict__ in, const uint
             for (int kx = 0; kx < s.k; kx++) v += zp[(ky * hx + kx) * FO_ROWS + (ky * s.k + kx) * s.cout + co];
         out[((size_t)oy * s.ow + ox) * s.cout + co] = v + (bias ? bias[co] : 0.0f);
     }
+}
+
+/* ---- 1 x 1 ----
+ *
+ * A product of the image with a small matrix. A workgroup keeps the weights of 128 output channels in the LDS for as long as
+ * it lives, as A operands in the order the waves read them, and its eight waves walk blocks of 32 pixels: a wave fetches
+ * its pixels straight into registers as f32 (two 16-byte loads per k-step, so that a load covers 64 B of a pixel), rounds
+ * them there and multiplies them with all 128 channels, half an LDS read per product. While a group of 128 input channels
+ * is multiplied the next one, or the next block's first, is on its way. Nothing is shared between waves but the weights:
+ * no barrier.
+ * What bounds it is the image and the result: 512 x 512 pixels, 256 -> 128 channels 76 + 65 us as a bf16 copy and an implicit
+ * product, 91 here (402 MB; eight waves of 32 pixels 93). With more than two tiles of channels the image is read once for
+ * each (512 -> 1536 over 16384 pixels: 84 us against 61), so those stay with the copy and a plain product. */
+constexpr int C1_N = 128, C1_MAX_CIN = 512, C1_WAVES = 16, C1_OUT = 512;   /* output channels of a workgroup; f32 of LDS per wave for its stores */
+
+__global__ void __launch_bounds__(64 * C1_WAVES, 4)
+k_conv_1x1(float *__restrict__ out, const float *__restrict__ in, const uint16_t *__restrict__ W, const float *__restrict__ bias,
+           int pixels, int cin, int cout, int tiles_n, int total, int per_xcd) {
+    extern __shared__ __align__(16) float lds1[];              /* C1_WAVES x C1_OUT, then the weights: [k-step][8][64 lanes] x 16 B */
+    u32x4 *wf = reinterpret_cast<u32x4 *>(lds1 + C1_WAVES * C1_OUT);
+    /* the channel tiles of a pixel range next to each other on an XCD: they share the image in its L2 */
+    const int work = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if (work >= total) return;
+    const int n0 = work % tiles_n * C1_N, slot = work / tiles_n, slots = total / tiles_n;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, lg = lane >> 4;
+
+    for (int i = threadIdx.x; i < cin / 32 * 512; i += 64 * C1_WAVES) {
+        const int ks = i >> 9, n = n0 + 16 * ((i >> 6) & 7) + (i & 15), g = (i >> 4) & 3;
+        u32x4 v = {0, 0, 0, 0};
+        if (n < cout) {                                        /* a lane's eight channels are 4 g .. + 3 and 16 + 4 g .. + 3 */
+            const uint16_t *src = W + (size_t)n * cin + 32 * ks + 4 * g;
+            const uint2 lo = *reinterpret_cast<const uint2 *>(src), hi = *reinterpret_cast<const uint2 *>(src + 16);
+            v = u32x4{lo.x, lo.y, hi.x, hi.y};
+        }
+        wf[i] = v;
+    }
+    __syncthreads();
+
+    const int blocks = (pixels + 15) / 16, groups = cin / 128, stride = slots * C1_WAVES;
+    float *buf = lds1 + wave * C1_OUT;
+    const int c = lane & 7;
+    f32x4 bias4[4];
+#pragma unroll
+    for (int h = 0; h < 4; h++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int n = n0 + 32 * h + 4 * c + e;
+            bias4[h][e] = bias && n < cout ? bias[n] : 0.0f;
+        }
+    const bool chunks = cout % 4 == 0 && ((uintptr_t)out & 15) == 0;
+
+    f32x4 raw[8];                                              /* [k-step, half] of a group of 128 channels */
+    auto fetch = [&](int block, int group) {
+        const int p = min(16 * block + li, pixels - 1);
+        const float *src = in + (size_t)p * cin + 128 * group + 4 * lg;
+#pragma unroll
+        for (int i = 0; i < 8; i++) raw[i] = *reinterpret_cast<const f32x4 *>(src + 16 * i);
+    };
+    int block = slot * C1_WAVES + wave;
+    if (block < blocks) fetch(block, 0);
+    for (; block < blocks; block += stride) {
+        f32x4 acc[8];
+#pragma unroll
+        for (int a = 0; a < 8; a++) acc[a] = f32x4{0, 0, 0, 0};
+        for (int group = 0; group < groups; group++) {
+            u32x4 bv[4];
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) {
+                const f32x4 lo = raw[2 * ks], hi = raw[2 * ks + 1];
+                bv[ks] = u32x4{pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3])};
+            }
+            const bool last = group + 1 == groups;
+            if (!last || block + stride < blocks) fetch(last ? block + stride : block, last ? 0 : group + 1);
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++)
+#pragma unroll
+                for (int a = 0; a < 8; a++) acc[a] = mfma(wf[((4 * group + ks) * 8 + a) * 64 + lane], bv[ks], acc[a]);
+        }
+        /* acc[a][r]: channel n0 + 16 a + 4 lg + r of pixel 16 block + li. Through the LDS (a wave's own region), 16
+         * pixels x 32 channels at a time, so that a store instruction covers eight pixels x 128 B. */
+#pragma unroll
+        for (int h = 0; h < 4; h++) {
+#pragma unroll
+            for (int a = 0; a < 2; a++) *reinterpret_cast<f32x4 *>(&buf[li * 32 + 4 * ((4 * a + lg) ^ (li & 7))]) = acc[2 * h + a];
+#pragma unroll
+            for (int it = 0; it < 2; it++) {
+                const int row = 8 * it + (lane >> 3), p = 16 * block + row, n = n0 + 32 * h + 4 * c;
+                const f32x4 v = *reinterpret_cast<const f32x4 *>(&buf[row * 32 + 4 * (c ^ (row & 7))]) + bias4[h];
+                if (p >= pixels) continue;
+                float *dst = out + (size_t)p * cout + n;
+                if (chunks) {
+                    if (n < cout) *reinterpret_cast<f32x4 *>(dst) = v;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (n + e < cout) dst[e] = v[e];
+                }
+            }
+        }
+    }
+}
+
+int launch_1x1(hipStream_t st, float *out, const float *in, const uint16_t *W, const float *bias, int pixels, int cin, int cout) {
+    static bool configured = false;
+    if (!configured) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_conv_1x1), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (e != hipSuccess) return (int)e;
+        configured = true;
+    }
+    /* about one workgroup per CU, but no more than there are blocks of 16 x 16 pixels for */
+    const int tiles_n = (cout + C1_N - 1) / C1_N, most = (pixels + 16 * C1_WAVES - 1) / (16 * C1_WAVES);
+    int slots = 256 / tiles_n;
+    if (slots > most) slots = most;
+    if (slots < 1) slots = 1;
+    const int total = slots * tiles_n, per_xcd = (total + 7) / 8;
+    hipLaunchKernelGGL(k_conv_1x1, dim3((unsigned)per_xcd * 8), dim3(64 * C1_WAVES), C1_WAVES * C1_OUT * 4 + cin * 256, st, out, in, W, bias, pixels,
+                       cin, cout, tiles_n, total, per_xcd);
+    return (int)hipGetLastError();
 }
 
 /* ---- 3 x 3 ----
@@ -504,6 +623,8 @@ int iris_hip_conv2d_direct(void *stream, float *out, const float *in, const uint
     if (k <= FO_MAX_K && k * k * cout <= FO_ROWS && stride == 1 && (cin == 32 || cin == 64 || cin == 128) && al16(in) && al16(w))
         return cin == 32 ? launch_few_out<1>(st, out, in, w, bias, s) : cin == 64 ? launch_few_out<2>(st, out, in, w, bias, s)
                                                                                : launch_few_out<4>(st, out, in, w, bias, s);
+    if (k == 1 && stride == 1 && oh == h && ow == width && cin % 128 == 0 && cin <= C1_MAX_CIN && cout <= 2 * C1_N && al16(in) && ((uintptr_t)w & 7) == 0)
+        return launch_1x1(st, out, in, w, bias, h * width, cin, cout);
     /* a thread's byte offsets into image and weights are 32-bit */
     if (k == 3 && stride == 1 && cin % 64 == 0 && cout <= C3_MAX_COUT && al16(in) && al16(w) && (size_t)h * width * cin * 4 < ((size_t)1 << 32) &&
         (size_t)cout * 9 * cin * 2 < ((size_t)1 << 32))

@@ -467,7 +467,7 @@ struct Wide {
 template <typename OUT, int NA, bool QKN>
 __global__ void __launch_bounds__(512, 2)
 k_gemm_wide(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *__restrict__ W, int M, int N, int K,
-            int tiles_m, int total, int per_xcd, QkNorm qn, int streaming_out) {
+            int tiles_m, int total, int per_xcd, QkNorm qn, const float *__restrict__ bias, int streaming_out) {
     using T = Wide<NA>;
     constexpr int TM = T::TM, TN = T::TN, XS = T::XS, WS = T::WS, WP = T::WP, H0 = (NA + 1) / 2, H1 = NA / 2;
     static_assert(WP <= 4 && H1 >= 3, "");
@@ -652,8 +652,9 @@ k_gemm_wide(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t 
 #pragma unroll
             for (int it = 0; it < 16; it++) {
                 const int row = 2 * it + (lane >> 5), c = lane & 31, m = mw + 32 * half + row, n = nw + PER16 * c;
-                const f32x4 v = *reinterpret_cast<const f32x4 *>(&buf[row * 128 + 4 * ((c & 16) | ((c ^ row) & 15))]);
+                f32x4 v = *reinterpret_cast<const f32x4 *>(&buf[row * 128 + 4 * ((c & 16) | ((c ^ row) & 15))]);
                 if (c < 4 * NA && m < M && n < N) {
+                    if (bias) v += *reinterpret_cast<const f32x4 *>(bias + n);
                     f32x4 *dst = reinterpret_cast<f32x4 *>(reinterpret_cast<float *>(y) + (size_t)m * N + n);
                     if (streaming_out) __builtin_nontemporal_store(v, dst);
                     else *dst = v;
@@ -718,7 +719,7 @@ k_gemm_scalar(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_
 }
 
 template <typename OUT, int NA, bool QKN = false>
-int launch_gemm_wide(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, const QkNorm &qn = QkNorm{}) {
+int launch_gemm_wide(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, const float *bias, const QkNorm &qn = QkNorm{}) {
     static bool configured = false;
     if (!configured) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_gemm_wide<OUT, NA, QKN>),
@@ -734,7 +735,7 @@ int launch_gemm_wide(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *
      * them cached for the operator that reads them next). */
     const int streaming_out = (size_t)M * N * sizeof(OUT) >= ((size_t)192 << 20);
     hipLaunchKernelGGL((k_gemm_wide<OUT, NA, QKN>), dim3((unsigned)per_xcd * 8), dim3(512), Wide<NA>::LDS, st, y, x, W, M, N, K,
-                       tiles_m, total, per_xcd, qn, streaming_out);
+                       tiles_m, total, per_xcd, qn, bias, streaming_out);
     return (int)hipGetLastError();
 }
 
@@ -785,25 +786,36 @@ static GemmPlan plan_gemm(int M, int N, int K, int out_size, bool operands_align
     return {0, 0, 1};
 }
 
-/* part: workspace for partial sums, part_bytes long (0: no ranges of K) */
+__global__ void __launch_bounds__(256)
+k_add_bias_rows(float *__restrict__ y, const float *__restrict__ bias, int cols, size_t n) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) y[i] += bias[i % cols];
+}
+
+int add_bias_rows(hipStream_t st, float *y, const float *bias, int rows, int cols) {
+    const size_t n = (size_t)rows * cols;
+    hipLaunchKernelGGL(k_add_bias_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, y, bias, cols, n);
+    return (int)hipGetLastError();
+}
+
+/* part: workspace for partial sums, part_bytes long (0: no ranges of K). bias [N], f32 outputs only: added in the epilogue
+ * where the kernel can, in a pass of its own elsewhere. */
 template <typename OUT>
-int gemm(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, float *part, size_t part_bytes) {
+int gemm(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, float *part, size_t part_bytes,
+         const float *bias = nullptr) {
     if (M <= 0 || N <= 0) return 0;
     const bool aligned16 = ((uintptr_t)x & 15) == 0 && ((uintptr_t)W & 15) == 0;
     const GemmPlan plan = plan_gemm(M, N, K, (int)sizeof(OUT), aligned16, ((uintptr_t)y & 15) == 0, part_bytes);
+    const float *fused = (plan.kernel == 3 || (plan.kernel == 4 && plan.splits == 1)) && ((uintptr_t)bias & 15) == 0 ? bias : nullptr;
+    int e = 0;
     if (plan.kernel == 4) {
-        const int e = iris_hip_gemm_tiles(st, y, (int)sizeof(OUT), x, W, M, N, K, plan.na, plan.splits, part);
-        if (e) return e;
-    } else if (plan.kernel == 3 || plan.kernel == 2) {
+        e = iris_hip_gemm_tiles(st, y, (int)sizeof(OUT), x, W, M, N, K, fused, plan.na, plan.splits, part);
+    } else if (plan.kernel == 3) {
+        e = plan.na == 8 ? launch_gemm_wide<OUT, 8>(st, y, x, W, M, N, K, fused)
+          : plan.na == 7 ? launch_gemm_wide<OUT, 7>(st, y, x, W, M, N, K, fused) : launch_gemm_wide<OUT, 6>(st, y, x, W, M, N, K, fused);
+    } else if (plan.kernel == 2) {
         const ConvGeom none = {};
-        int e;
-        if (plan.kernel == 3) {
-            e = plan.na == 8 ? launch_gemm_wide<OUT, 8>(st, y, x, W, M, N, K)
-              : plan.na == 7 ? launch_gemm_wide<OUT, 7>(st, y, x, W, M, N, K) : launch_gemm_wide<OUT, 6>(st, y, x, W, M, N, K);
-        } else {
-            e = launch_gemm_dma<OUT, 256, false>(st, y, x, W, M, N, K, none);
-        }
-        if (e) return e;
+        e = launch_gemm_dma<OUT, 256, false>(st, y, x, W, M, N, K, none);
     } else if (plan.kernel == 1) {
         /* 2 x 2 waves (128 x 128 tiles) measured best on the transformer shapes: 4 x 2 and 2 x 4 are
          * 5-8 % slower on the wide projections, 4 x 1 and 2 x 1 15-30 % slower. */
@@ -813,6 +825,10 @@ int gemm(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, in
     } else {
         const size_t n = (size_t)M * N;
         hipLaunchKernelGGL(k_gemm_scalar<OUT>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, y, x, W, M, N, K);
+    }
+    if (e) return e;
+    if constexpr (sizeof(OUT) == 4) {
+        if (bias && !fused) return add_bias_rows(st, y, bias, M, N);
     }
     return (int)hipGetLastError();
 }
@@ -844,12 +860,6 @@ k_im2col(uint16_t *__restrict__ cols, const float *__restrict__ in, int h, int w
 __global__ void __launch_bounds__(64)
 k_zero_words(uint32_t *__restrict__ p, int n) {
     for (int i = threadIdx.x; i < n; i += 64) p[i] = 0u;
-}
-
-__global__ void __launch_bounds__(256)
-k_add_bias_rows(float *__restrict__ y, const float *__restrict__ bias, int cols, size_t n) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) y[i] += bias[i % cols];
 }
 
 }  // namespace
@@ -889,7 +899,7 @@ int iris_hip_linear_bf16_qknorm(void *stream, float *part, uint16_t *y, const ui
     const GemmPlan plan = plan_gemm(M, N, K, 2, true, true, IRIS_LINEAR_PART_BYTES);
     if (plan.kernel == 3 && plan.na == 8) {
         const QkNorm qn = {wq, k_cols ? wk : wq, rope_cos, rope_sin, q_cols, q_cols + k_cols, eps, split_half};
-        return launch_gemm_wide<uint16_t, 8, true>((hipStream_t)stream, y, x, W, M, N, K, qn);
+        return launch_gemm_wide<uint16_t, 8, true>((hipStream_t)stream, y, x, W, M, N, K, nullptr, qn);
     }
     const int e = gemm<uint16_t>((hipStream_t)stream, y, x, W, M, N, K, part, IRIS_LINEAR_PART_BYTES);
     if (e) return e;
@@ -918,12 +928,26 @@ int iris_hip_conv2d(void *stream, uint16_t *scratch, size_t scratch_bytes, float
     const int direct = iris_hip_conv2d_direct(stream, out, in, w, bias, h, width, cin, cout, k, stride, pad_before, oh, ow);
     if (direct != -2) return direct;
 
-    /* Implicit GEMM: the image once as bf16 (the rows a chunk of output rows needs), then k_gemm_dma in its
-     * convolution mode straight on it; no patch matrix. Needs cin % 64 == 0 (a k tile inside one tap). */
     if (scratch_bytes <= IRIS_CONV_ZERO_BYTES) return (int)hipErrorInvalidValue;
     const uint16_t *zeros = scratch;
     scratch += IRIS_CONV_ZERO_BYTES / sizeof(uint16_t);
     scratch_bytes -= IRIS_CONV_ZERO_BYTES;
+
+    /* 1 x 1 without padding or stride (and more output channels than conv_gfx950.hip keeps at hand): the image as bf16
+     * rows, in chunks that fit the scratch, and a plain product. 16384 x 512 -> 1536: 61 us as an implicit product, 55 so. */
+    if (k == 1 && stride == 1 && oh == h && ow == width && cin % TK == 0 && scratch_bytes >= (size_t)cin * sizeof(uint16_t)) {
+        const long rows = (long)(scratch_bytes / ((size_t)cin * sizeof(uint16_t)));
+        for (long p0 = 0; p0 < ohw; p0 += rows) {
+            const int np = (int)(ohw - p0 < rows ? ohw - p0 : rows);
+            int e = iris_hip_f32_to_bf16(stream, scratch, in + (size_t)p0 * cin, (size_t)np * cin);
+            if (!e) e = gemm<float>(st, out + (size_t)p0 * cout, scratch, w, np, cout, cin, nullptr, 0, bias);
+            if (e) return e;
+        }
+        return 0;
+    }
+
+    /* Implicit GEMM: the image once as bf16 (the rows a chunk of output rows needs), then k_gemm_dma in its
+     * convolution mode straight on it; no patch matrix. Needs cin % 64 == 0 (a k tile inside one tap). */
     const size_t in_row_bytes = (size_t)width * cin * sizeof(uint16_t);
     if (cin % TK == 0 && cout >= 128 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)in & 15) == 0 && ((uintptr_t)scratch & 15) == 0 &&
         scratch_bytes / in_row_bytes >= (size_t)k) {
@@ -947,10 +971,7 @@ int iris_hip_conv2d(void *stream, uint16_t *scratch, size_t scratch_bytes, float
                                       : launch_gemm_dma<float, 128, true>(st, dst, virtual_image, w, m, cout, row_len, geo);
             if (e) return e;
         }
-        if (bias && !bias_fused) {
-            const size_t n = (size_t)ohw * cout;
-            hipLaunchKernelGGL(k_add_bias_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, out, bias, cout, n);
-        }
+        if (bias && !bias_fused) return add_bias_rows(st, out, bias, ohw, cout);
         return (int)hipGetLastError();
     }
 
@@ -963,12 +984,8 @@ int iris_hip_conv2d(void *stream, uint16_t *scratch, size_t scratch_bytes, float
         const size_t n = (size_t)np * row_len / (vec ? 8 : 1);
         if (vec) hipLaunchKernelGGL(k_im2col<8>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, scratch, in, h, width, cin, k, stride, pad_before, ow, p0, n);
         else hipLaunchKernelGGL(k_im2col<1>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, scratch, in, h, width, cin, k, stride, pad_before, ow, p0, n);
-        int e = gemm<float>(st, out + (size_t)p0 * cout, scratch, w, np, cout, row_len, nullptr, 0);
+        int e = gemm<float>(st, out + (size_t)p0 * cout, scratch, w, np, cout, row_len, nullptr, 0, bias);
         if (e) return e;
-    }
-    if (bias) {
-        const size_t n = (size_t)ohw * cout;
-        hipLaunchKernelGGL(k_add_bias_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, out, bias, cout, n);
     }
     return (int)hipGetLastError();
 }

@@ -59,7 +59,7 @@ struct Tile {
 template <typename OUT, int NB, int WM, int NA, int WN, int KG, int STAGES>
 __global__ void __launch_bounds__(64 * WM * WN * KG, 2)
 k_gemm_tiles(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *__restrict__ W, int M, int N, int K,
-             int tiles_m, int tiles_n, int splits, int total, int per_xcd) {
+             const float *__restrict__ bias, int tiles_m, int tiles_n, int splits, int total, int per_xcd) {
     using T = Tile<NB, WM, NA, WN, KG, STAGES>;
     constexpr int TM = T::TM, TN = T::TN, STAGE = T::STAGE, PIECES = T::PIECES;
     static_assert(T::LDS <= 160 * 1024 && NA <= 4 && (KG == 1 || (KG == 2 && NB % 2 == 0)), "");
@@ -228,8 +228,11 @@ k_gemm_tiles(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t
 #pragma unroll
         for (int it = 0; it < 4 * NBS; it++) {
             const int row = 4 * it + (lane >> 4), c = lane & 15, m = mw + row, n = nw + 4 * c;
-            const f32x4 v = *reinterpret_cast<const f32x4 *>(&buf[row * 64 + 4 * (c ^ (row & 15))]);
-            if (c < 4 * NA && m < M && n < N) *reinterpret_cast<f32x4 *>(dst + (size_t)m * N + n) = v;
+            f32x4 v = *reinterpret_cast<const f32x4 *>(&buf[row * 64 + 4 * (c ^ (row & 15))]);
+            if (c < 4 * NA && m < M && n < N) {
+                if (bias) v += *reinterpret_cast<const f32x4 *>(bias + n);
+                *reinterpret_cast<f32x4 *>(dst + (size_t)m * N + n) = v;
+            }
         }
     } else {
         uint16_t *buf = mine;                                  /* chunk c of row r in slot c ^ (r % 8) */
@@ -272,7 +275,7 @@ k_gemm_sum(OUT *__restrict__ y, const float *__restrict__ part, size_t n, int sp
 }
 
 template <typename OUT, int NB, int WM, int NA, int WN, int KG, int STAGES>
-int launch_tiles(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, int splits) {
+int launch_tiles(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, const float *bias, int splits) {
     using T = Tile<NB, WM, NA, WN, KG, STAGES>;
     static bool configured = false;
     if (!configured) {
@@ -283,7 +286,7 @@ int launch_tiles(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, i
     }
     const int tiles_m = (M + T::TM - 1) / T::TM, tiles_n = (N + T::TN - 1) / T::TN, total = tiles_m * tiles_n * splits, per_xcd = (total + 7) / 8;
     hipLaunchKernelGGL((k_gemm_tiles<OUT, NB, WM, NA, WN, KG, STAGES>), dim3((unsigned)per_xcd * 8), dim3(T::THREADS), T::LDS, st, y, x, W, M, N, K,
-                       tiles_m, tiles_n, splits, total, per_xcd);
+                       bias, tiles_m, tiles_n, splits, total, per_xcd);
     return (int)hipGetLastError();
 }
 
@@ -296,14 +299,14 @@ constexpr Shape SHAPES[] = {{128, 128, 0.50f, 0.55f}, {128, 192, 0.62f, 0.65f}, 
 constexpr int NSHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
 
 template <typename OUT>
-int launch_shape(hipStream_t st, int shape, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, int splits) {
+int launch_shape(hipStream_t st, int shape, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, const float *bias, int splits) {
     switch (shape) {
-    case 0: return launch_tiles<OUT, 4, 2, 4, 2, 2, 4>(st, y, x, W, M, N, K, splits);
-    case 1: return launch_tiles<OUT, 4, 2, 3, 4, 1, 4>(st, y, x, W, M, N, K, splits);
-    case 2: return launch_tiles<OUT, 4, 2, 4, 4, 1, 3>(st, y, x, W, M, N, K, splits);
-    case 3: return launch_tiles<OUT, 4, 1, 4, 4, 2, 4>(st, y, x, W, M, N, K, splits);
-    case 4: return launch_tiles<OUT, 5, 2, 3, 4, 1, 3>(st, y, x, W, M, N, K, splits);
-    case 5: return launch_tiles<OUT, 5, 2, 4, 4, 1, 3>(st, y, x, W, M, N, K, splits);
+    case 0: return launch_tiles<OUT, 4, 2, 4, 2, 2, 4>(st, y, x, W, M, N, K, bias, splits);
+    case 1: return launch_tiles<OUT, 4, 2, 3, 4, 1, 4>(st, y, x, W, M, N, K, bias, splits);
+    case 2: return launch_tiles<OUT, 4, 2, 4, 4, 1, 3>(st, y, x, W, M, N, K, bias, splits);
+    case 3: return launch_tiles<OUT, 4, 1, 4, 4, 2, 4>(st, y, x, W, M, N, K, bias, splits);
+    case 4: return launch_tiles<OUT, 5, 2, 3, 4, 1, 3>(st, y, x, W, M, N, K, bias, splits);
+    case 5: return launch_tiles<OUT, 5, 2, 4, 4, 1, 3>(st, y, x, W, M, N, K, bias, splits);
     default: return (int)hipErrorInvalidValue;
     }
 }
@@ -334,12 +337,15 @@ float iris_hip_gemm_tiles_plan(int M, int N, int K, int out_size, size_t part_by
     return best;
 }
 
-/* part: splits * M * N floats, 16-byte aligned, when splits > 1. x, W, y 16-byte aligned. */
-int iris_hip_gemm_tiles(void *stream, void *y, int out_size, const uint16_t *x, const uint16_t *W, int M, int N, int K, int shape, int splits, float *part) {
+/* part: splits * M * N floats, 16-byte aligned, when splits > 1. x, W, y, bias 16-byte aligned; bias (or null) [N], with f32
+ * outputs and one range only. */
+int iris_hip_gemm_tiles(void *stream, void *y, int out_size, const uint16_t *x, const uint16_t *W, int M, int N, int K, const float *bias, int shape,
+                        int splits, float *part) {
     hipStream_t st = (hipStream_t)stream;
     if (splits == 1)
-        return out_size == 2 ? launch_shape<uint16_t>(st, shape, (uint16_t *)y, x, W, M, N, K, 1) : launch_shape<float>(st, shape, (float *)y, x, W, M, N, K, 1);
-    int e = launch_shape<float>(st, shape, part, x, W, M, N, K, splits);
+        return out_size == 2 ? launch_shape<uint16_t>(st, shape, (uint16_t *)y, x, W, M, N, K, nullptr, 1)
+                             : launch_shape<float>(st, shape, (float *)y, x, W, M, N, K, bias, 1);
+    int e = launch_shape<float>(st, shape, part, x, W, M, N, K, nullptr, splits);
     if (e) return e;
     const size_t n = (size_t)M * N;
     const dim3 grid((unsigned)((n / 8 + 255) / 256));

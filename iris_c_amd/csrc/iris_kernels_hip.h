@@ -144,7 +144,7 @@ int iris_hip_linear_bf16(void *stream, float *part, uint16_t *y, const uint16_t 
 void iris_hip_linear_plan(int rows, int in, int out, int out_bytes, int *plan);
 float iris_hip_gemm_tiles_plan(int M, int N, int K, int out_size, size_t part_bytes, int *shape, int *splits);
 int iris_hip_gemm_tiles(void *stream, void *y, int out_size, const uint16_t *x, const uint16_t *W, int M, int N, int K,
-                        int shape, int splits, float *part);
+                        const float *bias, int shape, int splits, float *part);
 
 /* -2 = shape not taken, nothing enqueued */
 int iris_hip_linear_bf16_qknorm(void *stream, float *part, uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in,

@@ -51,3 +51,11 @@ def test_few_output_channels(dev, orc, h, w, cin, cout, k, stride, pb, pa, bias)
 def test_three_by_three(dev, orc, h, w, cin, cout, pb, pa, bias):
     """Tile edges (16 x 16 pixels, 128 channels), one to eight groups of 64 input channels, padding of other widths."""
     conv_case(dev, orc, h, w, cin, cout, 3, 1, pb, pa, bias)
+
+
+@pytest.mark.parametrize("h,w,cin,cout,bias", [(1, 1, 128, 128, True), (8, 4, 128, 128, True), (257, 1, 256, 130, False), (33, 31, 512, 64, True),
+                                               (300, 1, 512, 1536, True), (2000, 1, 512, 1536, True), (90, 91, 384, 256, True), (17, 16, 64, 320, True), (9, 9, 128, 258, True), (128, 128, 128, 3, False)])
+def test_one_by_one(dev, orc, h, w, cin, cout, bias):
+    """One block of 16 pixels and less, more blocks than waves, one and two tiles of 128 channels, a ragged one; and what goes
+    through the bf16 copy and a plain product with the bias in its epilogue or behind it."""
+    conv_case(dev, orc, h, w, cin, cout, 1, 1, 0, 0, bias)

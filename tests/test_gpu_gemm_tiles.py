@@ -43,11 +43,11 @@ def test_every_tile(dev, shape, more_rows, more_cols, k, splits, bf16):
     x, W, want = operands(rows, k, out)
     lib = dev.lib
     lib.iris_hip_gemm_tiles.restype = C.c_int
-    lib.iris_hip_gemm_tiles.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p] + [C.c_int] * 5 + [C.c_void_p]
+    lib.iris_hip_gemm_tiles.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p] + [C.c_int] * 3 + [C.c_void_p] + [C.c_int] * 2 + [C.c_void_p]
     guard = 512
     fill = np.full(rows * out + guard, 7, np.uint16 if bf16 else np.float32)
     dy, part = dev.put(fill), dev.alloc(splits * rows * out * 4)
-    assert lib.iris_hip_gemm_tiles(lib.iris_dev_stream(), dy, 2 if bf16 else 4, dev.put(x), dev.put(W), rows, out, k, shape, splits, part) == 0
+    assert lib.iris_hip_gemm_tiles(lib.iris_dev_stream(), dy, 2 if bf16 else 4, dev.put(x), dev.put(W), rows, out, k, None, shape, splits, part) == 0
     dev.check()
     got = dev.get(dy, fill.shape, fill.dtype)
     dev.free_all()
