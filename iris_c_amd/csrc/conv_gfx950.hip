@@ -331,34 +331,32 @@ int launch_1x1(hipStream_t st, float *out, const float *in, const uint16_t *W, c
  * passes from the L2 to the CU 1.27 times instead of nine, and no bf16 copy of it is made first. The weights of a (tap,
  * 64 channels) step, 128 rows of 128 B, go straight from memory into one of three LDS stages.
  *
- * Eight waves, 4 (rows of four pixels) x 2 (64 channels), two per SIMD: a wave owns 64 pixels x 64 channels = 4 x 4
- * accumulator blocks, and a step is 32 products per wave: 16 of the first half of the step's channels, the barrier, 16 of
- * the second half. The operands of a half are requested from the LDS one half ahead, across the barrier too.
- *  - In front of the barrier of step s the wave waits until its own share of the weights of step s + 1 has landed and its
- *    last operands of step s have been read; so behind it stage s % 3 is free, and the weights of step s + 3 are
- *    requested into it: they have two steps to land.
- *  - The pixels of the next 64 channels (2592 pieces of 8 channels, six per thread) are fetched into registers in steps
- *    0 - 5 and written to the other image buffer three steps later: the wait of the step before covers them, since loads
- *    complete in order and the weights that it waits for were requested behind them.
+ * Twelve waves, three per SIMD, with roles of their own, so that nobody's loads stand in the way of anybody else's:
+ *  - Waves 0 - 7 multiply: 4 (rows of four pixels) x 2 (64 channels), a wave owns 64 pixels x 64 channels = 4 x 4
+ *    accumulator blocks, and a step is 32 products: 16 of the first half of the step's channels, the barrier, 16 of the
+ *    second half. The operands of a half are read from the LDS in the gaps between the products of the half before, one to
+ *    a gap, across the barrier too. They issue no load and wait for none, so a tile's stores drain under the next tile.
+ *  - Waves 8 - 11 bring everything in. The image: 2592 units of 8 channels x pixel per group of 64 channels, 11 a thread,
+ *    all of them in registers on their way while the group before is multiplied. One or two a step are rounded and written
+ *    to the image buffer that the last group has left (the epilogue borrows it until the barrier of step 0), and
+ *    requested again for the group after the next, of the next tile if there is one. The weights: those of step s + 2
+ *    into the stage that the barrier of step s - 1 has set free; they have landed in front of the barrier of step s + 1.
  * A pixel takes 160 B of LDS (64 channels + 32 B): the 16 lanes that a 128-bit read serves together are eight pixels with
  * one chunk and the eight between them with the next, and with a stride of ten 16 B units, whichever pixel the
  * tap starts at, they fall into distinct bank windows; a tap's shift is an immediate offset. Weight rows are swizzled as
- * in gemm_conv_gfx950.hip.
+ * in gemm_conv_gfx950.hip. A workgroup takes 152 KB of LDS, so a CU runs one, and it is persistent.
  *
- * A workgroup takes 152 KB of LDS, so a CU runs one, and it is persistent: while it multiplies the last channel group of a
- * tile it fetches the first of the next, and the next steps run while its stores are on their way (they count in the
- * waits, see channel_group). One tile per workgroup, 11 us of the 23 us of a tile of 128 input channels were its first
- * pixels' and its stores' latency: 91 -> 82 us for 128 -> 128 channels.
- *
- * Measured against a bf16 copy of the image + implicit product that fetches every tap from the L2 (copy + product):
- * 512 x 512 pixels, 128 -> 128 30 + 118 -> 82 us (the image and the result alone take 50 us to move), 256 -> 128 76 + 214
- * -> 135 us (1150 TFLOP/s), 256 -> 256 88 + 290 -> 263 us (1180). A step takes 0.7 us: 256 of them at a time are 1500
- * TFLOP/s, what a large plain product reaches on this card. */
+@@MEASURED@@ */
 constexpr int C3_T = 16, C3_H = C3_T + 2, C3_PIXELS = C3_H * C3_H, C3_ROW = 80, C3_IMG = C3_PIXELS * C3_ROW;   /* elements */
-constexpr int C3_N = 128, C3_STAGE = C3_N * 64, C3_UNITS = 6;
+constexpr int C3_N = 128, C3_STAGE = C3_N * 64;
+constexpr int C3_MUL = 8, C3_BRING = 4, C3_THREADS = 64 * (C3_MUL + C3_BRING);           /* waves that multiply, that bring pixels and weights */
+constexpr int C3_UNITS = (C3_PIXELS * 8 + 64 * C3_BRING - 1) / (64 * C3_BRING), C3_PIECES = C3_N / 8 / C3_BRING;
 constexpr int C3_BIAS = 2 * C3_IMG + 3 * C3_STAGE;             /* the bias of all output channels, f32 */
 constexpr int C3_MAX_COUT = (160 * 1024 - 2 * C3_BIAS) / 4 / C3_N * C3_N;
-constexpr int C3_STORES = 16;                                  /* store instructions of a wave in the epilogue of a whole tile */
+/* units written and requested again in a step of a channel group */
+__device__ constexpr int c3_first(int t) { return t < 1 ? 0 : t < 4 ? 2 * (t - 1) : t + 2; }
+__device__ constexpr int c3_units(int t) { return c3_first(t + 1) - c3_first(t); }
+static_assert(c3_first(9) == C3_UNITS && c3_units(0) == 0, "");
 
 __device__ __forceinline__ uint32_t lds_address(const uint16_t *p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
@@ -366,7 +364,7 @@ __device__ __forceinline__ uint32_t lds_address(const uint16_t *p) {
 
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"                /* M0 in a clobber list */
-__global__ void __launch_bounds__(512, 2)
+__global__ void __launch_bounds__(C3_THREADS, 3)
 k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t *__restrict__ W, const float *__restrict__ bias,
            ConvShape s, int tiles_x, int tiles_n, int total, int per_xcd) {
     extern __shared__ __align__(16) uint16_t lds[];            /* image, image, weights, weights, weights, bias */
@@ -376,122 +374,176 @@ k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t
     int work = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
     if (work >= xcd_end) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int li = lane & 15, lg = lane >> 4, wm = wave & 3, wn = wave >> 2;
+    const int groups = s.cin / 64;
     float *bias_lds = reinterpret_cast<float *>(lds + C3_BIAS);
-    for (int i = tid; i < tiles_n * C3_N; i += 512) bias_lds[i] = bias && i < s.cout ? bias[i] : 0.0f;
+    for (int i = tid; i < tiles_n * C3_N; i += C3_THREADS) bias_lds[i] = bias && i < s.cout ? bias[i] : 0.0f;
 
-    int ty0, tx0, n0;                                          /* of the tile `work` */
-    auto place = [&](int w, int &ty, int &tx, int &n) {
-        const int tile = w / tiles_n;
-        n = (w - tile * tiles_n) * C3_N;
-        ty = tile / tiles_x * C3_T;
-        tx = tile % tiles_x * C3_T;
-    };
-    /* image staging: unit u of this thread is channels 8 (tid % 8) .. + 7 of pixel tid / 8 + 64 u of the rimmed tile; a
-     * pixel outside the image reads the first one and is zeroed */
-    uint32_t uoff[C3_UNITS];                                   /* bytes from the channel group's first value */
-    bool inside[C3_UNITS];
-    auto aim_image = [&](int ty, int tx) {
+    /* Every wave passes one barrier here in front and nine per channel group, in every role. */
+    if (wave >= C3_MUL) {
+        __builtin_amdgcn_s_setprio(3);
+        const int bt = tid - 64 * C3_MUL, bw = wave - C3_MUL, px0 = bt >> 3;
+        /* weights: rows 8 (C3_PIECES bw + j) .. + 7 of a stage; rows past the last channel repeat it (their results are never
+         * stored). When nothing comes next the last requests are of weights that nobody uses. */
+        const int row_len = 9 * s.cin;
+        uint32_t woff[C3_PIECES];
+        auto aim_weights = [&](int w) {
+            const int n = w % tiles_n * C3_N;
+#pragma unroll
+            for (int j = 0; j < C3_PIECES; j++) {
+                const int r = 8 * (C3_PIECES * bw + j) + (lane >> 3), row = n + r < s.cout ? n + r : s.cout - 1;
+                woff[j] = ((uint32_t)row * (uint32_t)row_len + 8u * ((lane & 7) ^ ((r >> 1) & 7))) * 2u;
+            }
+        };
+        const uint32_t stages = lds_address(lds + 2 * C3_IMG + C3_PIECES * bw * 8 * 64);
+        auto request = [&](int tap, int c0) {                  /* the stage of a tap: tap % 3 */
+            const uint16_t *src = W + (size_t)tap * s.cin + c0;
+#pragma unroll
+            for (int j = 0; j < C3_PIECES; j++)
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                             ::"s"(stages + 2 * (tap % 3 * C3_STAGE + 8 * j * 64)), "v"(woff[j]), "s"(src) : "memory", "m0");
+        };
+        /* pixels: unit u of this thread is channels 8 (bt % 8) .. + 7 of pixel bt / 8 + 32 u of the rimmed tile; a pixel
+         * outside the image reads the first one and is zeroed */
+        uint32_t off[C3_UNITS], inside = 0, held = 0;          /* bytes from the channel group's first value; bit u: in the image */
+        int w = work, g = 0;                                   /* where the next loads come from */
+        const float *src = in;
+        auto aim = [&]() {
+            const int tile = w / tiles_n, ty = tile / tiles_x * C3_T - s.pad, tx = tile % tiles_x * C3_T - s.pad;
+            int first = px0;
+            asm volatile("" : "+v"(first));                    /* worked out here for every tile: kept over the loop it all spills */
+            inside = 0;
+#pragma unroll
+            for (int u = 0; u < C3_UNITS; u++) {
+                const int px = first + 8 * C3_BRING * u, py = px / C3_H, y = ty + py, x = tx + (px - py * C3_H);
+                const bool ok = px < C3_PIXELS && y >= 0 && y < s.h && x >= 0 && x < s.w;
+                if (ok) inside |= 1u << u;
+                off[u] = ((ok ? (uint32_t)(y * s.w + x) * (uint32_t)s.cin : 0u) + 8u * (bt & 7)) * 4u;
+            }
+        };
+        auto advance = [&]() {
+            if (g + 1 < groups) {
+                g++;
+                src += 64;
+            } else {
+                src = in;
+                g = 0;
+                w += stride;
+                if (w < xcd_end) {
+                    aim();
+                } else {                                       /* nothing comes next: the same loads, of a few cached bytes that nobody uses */
+                    inside = 0;
+#pragma unroll
+                    for (int u = 0; u < C3_UNITS; u++) off[u] = 32u * (bt & 7);
+                }
+            }
+        };
+        f32x4 xr[C3_UNITS][2];
+        auto load = [&](int u) {
+            const char *p = reinterpret_cast<const char *>(src) + off[u];
+            xr[u][0] = *reinterpret_cast<const f32x4 *>(p);
+            xr[u][1] = *reinterpret_cast<const f32x4 *>(p + 16);
+        };
+        auto put = [&](int img, int u) {
+            const f32x4 lo = xr[u][0], hi = xr[u][1];
+            u32x4 v = {pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3])};
+            if (!(held >> u & 1)) v = u32x4{0, 0, 0, 0};
+            if (u + 1 < C3_UNITS || px0 < C3_PIXELS - 8 * C3_BRING * (C3_UNITS - 1))
+                *reinterpret_cast<u32x4 *>(&lds[img + (px0 + 8 * C3_BRING * u) * C3_ROW + 8 * (bt & 7)]) = v;
+        };
+        aim_weights(work);
+        request(0, 0);
+        request(1, 0);
+        aim();
+#pragma unroll
+        for (int u = 0; u < C3_UNITS; u++) load(u);
+        held = inside;
+        advance();
 #pragma unroll
         for (int u = 0; u < C3_UNITS; u++) {
-            const int px = (tid >> 3) + 64 * u, py = px / C3_H, y = ty + py - s.pad, x = tx + (px - py * C3_H) - s.pad;
-            inside[u] = px < C3_PIXELS && y >= 0 && y < s.h && x >= 0 && x < s.w;
-            uoff[u] = ((inside[u] ? (uint32_t)(y * s.w + x) * (uint32_t)s.cin : 0u) + 8u * (tid & 7)) * 4u;
+            put(0, u);
+            load(u);
+            __builtin_amdgcn_sched_barrier(0);
         }
-    };
-    const int st_off = (tid >> 3) * C3_ROW + 8 * (tid & 7);
-    auto put = [&](int img, int u, f32x4 lo, f32x4 hi) {
-        u32x4 v = {pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3])};
-        if (!inside[u]) v = u32x4{0, 0, 0, 0};
-        if (u + 1 < C3_UNITS || tid < 8 * (C3_PIXELS - 64 * (C3_UNITS - 1)))
-            *reinterpret_cast<u32x4 *>(&lds[img + st_off + u * 64 * C3_ROW]) = v;
-    };
-
-    /* weights: rows 16 wave .. + 15 of a stage in two pieces of eight rows; rows past the last channel repeat it (their
-     * results are never stored) */
-    const int row_len = 9 * s.cin;
-    uint32_t woff[2], woff_next[2];
-    auto aim_weights = [&](int n, uint32_t *off) {
+        /* everything older than the loads just issued is there */
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * C3_UNITS) : "memory");
+        for (int img = 0, gg = 0; work < xcd_end; img = C3_IMG - img) {
+            const bool last = gg + 1 == groups;
+            held = inside;
+            advance();
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int r = 16 * wave + 8 * j + (lane >> 3), row = n + r < s.cout ? n + r : s.cout - 1;
-            off[j] = ((uint32_t)row * (uint32_t)row_len + 8u * ((lane & 7) ^ ((r >> 1) & 7))) * 2u;
+            for (int t = 0; t < 9; t++) {
+                if (t == 7 && last && work + stride < xcd_end) aim_weights(work + stride);
+                if (t < 7) request(t + 2, 64 * gg);
+                else request(t - 7, last ? 0 : 64 * (gg + 1));
+#pragma unroll
+                for (int u = c3_first(t); u < c3_first(t + 1); u++) {
+                    put(C3_IMG - img, u);
+                    load(u);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                /* newer than the weights of step t + 1: two loads a unit in the step that requested them and in this
+                 * one, and the weights of step t + 2 */
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier"
+                             ::"n"(2 * (c3_units(t > 0 ? t - 1 : 8) + c3_units(t)) + C3_PIECES) : "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            gg = last ? 0 : gg + 1;
+            if (last) work += stride;
         }
-    };
-    uint16_t *w_lds = lds + 2 * C3_IMG;
-    auto request = [&](const uint32_t *off, int tap, int c0, int stage) {
-        const uint16_t *src = W + (size_t)tap * s.cin + c0;
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                         ::"s"(lds_address(w_lds + stage * C3_STAGE + (16 * wave + 8 * j) * 64)), "v"(off[j]), "s"(src) : "memory", "m0");
-    };
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       /* no load into the LDS is left when it is given up */
+        return;
+    }
 
-    f32x4 acc[4][4];                                           /* [16 channels][row of 16 pixels] */
+    const int li = lane & 15, lg = lane >> 4, wm = wave & 3, wn = wave >> 2;
+    /* [16 channels][row of 16 pixels]. The products are asm statements: left to itself the compiler gives a product's result
+     * other registers than its summand, and 168 are not enough for that. It does not know then when a result is there
+     * and when a summand must be: `settle` stands between the products and any other use of acc. */
+    f32x4 acc[4][4];
+    auto settle = [&]() {
+        asm volatile("s_nop 15" : "+v"(acc[0][0]), "+v"(acc[0][1]), "+v"(acc[0][2]), "+v"(acc[0][3]), "+v"(acc[1][0]), "+v"(acc[1][1]),
+                                  "+v"(acc[1][2]), "+v"(acc[1][3]), "+v"(acc[2][0]), "+v"(acc[2][1]), "+v"(acc[2][2]), "+v"(acc[2][3]),
+                                  "+v"(acc[3][0]), "+v"(acc[3][1]), "+v"(acc[3][2]), "+v"(acc[3][3]));
+    };
     auto clear = [&]() {
 #pragma unroll
         for (int a = 0; a < 4; a++)
 #pragma unroll
             for (int b = 0; b < 4; b++) acc[a][b] = f32x4{0, 0, 0, 0};
+        settle();
     };
     u32x4 av[2][4], bv[2][4];
     int a_rd[2];
 #pragma unroll
     for (int ks = 0; ks < 2; ks++) a_rd[ks] = 2 * C3_IMG + (64 * wn + li) * 64 + 8 * ((4 * ks + lg) ^ (li >> 1));
     const int b_rd = (4 * wm * C3_H + li) * C3_ROW + 8 * lg;
-    auto operands = [&](int img, int tap, int ks) {            /* stage of a tap: tap % 3, nine steps per channel group */
-#pragma unroll
-        for (int a = 0; a < 4; a++) av[ks][a] = *reinterpret_cast<const u32x4 *>(&lds[a_rd[ks] + (tap % 3) * C3_STAGE + 16 * a * 64]);
-#pragma unroll
-        for (int b = 0; b < 4; b++)
-            bv[ks][b] = *reinterpret_cast<const u32x4 *>(&lds[img + b_rd + ((b + tap / 3) * C3_H + tap % 3) * C3_ROW + 32 * ks]);
+    /* operand i of a half step, in the order its products use them; stage of a tap: tap % 3, nine steps per channel group */
+    auto operand = [&](int img, int tap, int ks, int i) {
+        if (i == 0 || i > 4) {
+            const int a = i == 0 ? 0 : i - 4;
+            av[ks][a] = *reinterpret_cast<const u32x4 *>(&lds[a_rd[ks] + (tap % 3) * C3_STAGE + 16 * a * 64]);
+        } else {
+            bv[ks][i - 1] = *reinterpret_cast<const u32x4 *>(&lds[img + b_rd + ((i - 1 + tap / 3) * C3_H + tap % 3) * C3_ROW + 32 * ks]);
+        }
     };
-    auto products = [&](int ks) {
+    auto products = [&](int ks, int img, int tap) {            /* img, tap: of the operands read on the way */
 #pragma unroll
-        for (int a = 0; a < 4; a++)
-#pragma unroll
-            for (int b = 0; b < 4; b++) acc[a][b] = mfma(av[ks][a], bv[ks][b], acc[a][b]);
-    };
-
-    f32x4 xr[3][2];                                            /* three image units on their way */
-    /* One group of 64 channels: nine steps. `img` holds it; what comes next, the image from `next` on and the weights
-     * from channel c_next on, goes to `other` and to the stages as they fall free. first: of a tile, behind the epilogue
-     * of the one before. */
-    auto channel_group = [&](bool first, int c0, int img, int other, const float *next, int c_next) {
-#pragma unroll
-        for (int t = 0; t < 9; t++) {
-            operands(img, t, 1);
-            __builtin_amdgcn_sched_barrier(0);
-            if (t >= 3) put(other, t - 3, xr[t % 3][0], xr[t % 3][1]);
-            if (t < C3_UNITS) {
-                asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(xr[t % 3][0]) : "v"(uoff[t]), "s"(next) : "memory");
-                asm volatile("global_load_dwordx4 %0, %1, %2 offset:16" : "=v"(xr[t % 3][1]) : "v"(uoff[t]), "s"(next) : "memory");
-            }
-            products(0);
-            __builtin_amdgcn_sched_barrier(0);
-            /* newer than the weights of step t + 1: the image loads of steps t - 1 and t, the weights of step t + 2, and the
-             * stores of the epilogue in front of step 0 (where they were not counted on, everything before them has landed) */
-            const int newer = (t >= 1 && t - 1 < C3_UNITS ? 2 : 0) + (t < C3_UNITS ? 2 : 0) + 2;
-            if (t < 2 && first) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(newer + C3_STORES) : "memory");
-            else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(newer) : "memory");
-            if (t >= 2 && t - 2 < C3_UNITS) asm volatile("" : "+v"(xr[(t - 2) % 3][0]), "+v"(xr[(t - 2) % 3][1]));
-            operands(t < 8 ? img : other, t < 8 ? t + 1 : 0, 0);
-            if (t < 6) request(woff, t + 3, c0, t % 3);
-            else request(woff_next, t - 6, c_next, t % 3);
-            __builtin_amdgcn_sched_barrier(0);
-            products(1);
+        for (int i = 0; i < 16; i++) {
+            asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc[i / 4][i % 4]) : "v"(av[ks][i / 4]), "v"(bv[ks][i % 4]));
+            if (i < 8) operand(img, tap, ks ^ 1, i);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-
     /* acc[a][b][r]: channel n0 + 64 wn + 16 a + 4 lg + r of pixel (4 wm + b, li) of the tile. Through the image buffer that the
-     * last group has been read from (every wave has passed the barrier behind its last reads; 4 KB per wave, a row of 16
-     * pixels at a time), so that a store instruction covers four pixels x 256 B. */
-    const int c = lane & 15;
+     * last group has been read from (every wave has passed the barrier behind its last reads, and the next pixels go into
+     * it behind the next barrier; 4 KB per wave, a row of 16 pixels at a time), so that a store instruction covers four
+     * pixels x 256 B. */
     const bool chunks = s.cout % 4 == 0 && ((uintptr_t)out & 15) == 0;
-    auto epilogue = [&](int img, bool more) {
+    auto epilogue = [&](int img) {
+        const int tile = work / tiles_n, n0 = (work - tile * tiles_n) * C3_N, ty0 = tile / tiles_x * C3_T, tx0 = tile % tiles_x * C3_T;
         float *buf = reinterpret_cast<float *>(lds + img) + wave * 1024;
-        const int n = n0 + 64 * wn + 4 * c;
+        int li = lane & 15, lg = lane >> 4;
+        asm volatile("" : "+v"(li), "+v"(lg));                 /* the addresses are worked out here: kept over the loop they spill */
+        const int c = li, n = n0 + 64 * wn + 4 * c;
         const f32x4 bias4 = *reinterpret_cast<const f32x4 *>(bias_lds + n);
         const bool whole = chunks && ty0 + C3_T <= s.oh && tx0 + C3_T <= s.ow && n0 + C3_N <= s.cout;
 #pragma unroll
@@ -502,73 +554,45 @@ k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t
             f32x4 v[4];
 #pragma unroll
             for (int it = 0; it < 4; it++) {
-                const int row = 4 * it + (lane >> 4);
+                const int row = 4 * it + lg;
                 v[it] = *reinterpret_cast<const f32x4 *>(&buf[row * 64 + 4 * (c ^ row)]) + bias4;
             }
-            float *dst = out + ((size_t)y * s.ow + tx0 + (lane >> 4)) * s.cout + n;
+            float *dst = out + ((size_t)y * s.ow + tx0 + lg) * s.cout + n;
             if (whole) {
 #pragma unroll
                 for (int it = 0; it < 4; it++) *reinterpret_cast<f32x4 *>(dst + (size_t)(4 * it) * s.cout) = v[it];
             } else if (y < s.oh) {
 #pragma unroll
                 for (int it = 0; it < 4; it++) {
-                    if (tx0 + 4 * it + (lane >> 4) >= s.ow) continue;
+                    if (tx0 + 4 * it + lg >= s.ow) continue;
 #pragma unroll
                     for (int e = 0; e < 4; e++)
                         if (n + e < s.cout) dst[(size_t)(4 * it) * s.cout + e] = v[it][e];
                 }
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        /* the next steps count on C3_STORES stores in flight, or on none of what came before them */
-        if (more && !whole) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     };
 
-    const int groups = s.cin / 64;
-    place(work, ty0, tx0, n0);
-    aim_weights(n0, woff);
-    for (int t = 0; t < 3; t++) request(woff, t, 0, t);
-    aim_image(ty0, tx0);
-    {
-        f32x4 first[C3_UNITS][2];
-#pragma unroll
-        for (int u = 0; u < C3_UNITS; u++)
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-                first[u][i] = *reinterpret_cast<const f32x4 *>(reinterpret_cast<const char *>(in) + uoff[u] + 16 * i);
-#pragma unroll
-        for (int u = 0; u < C3_UNITS; u++) put(0, u, first[u][0], first[u][1]);
-    }
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    operands(0, 0, 0);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     clear();
-    woff_next[0] = woff[0];
-    woff_next[1] = woff[1];
-    int ty = ty0, tx = tx0, n = n0;                            /* where the next group's image and weights come from */
-    for (int img = 0, g = 0;;) {
-        const bool last = g + 1 == groups, more = work + stride < xcd_end;
-        if (last && more) {
-            place(work + stride, ty, tx, n);
-            aim_image(ty, tx);
-            aim_weights(n, woff_next);
-        } else if (last) {
-            /* nothing comes next: the same loads, of a few cached bytes that nobody uses */
 #pragma unroll
-            for (int u = 0; u < C3_UNITS; u++) { inside[u] = false; uoff[u] = 32u * (tid & 7); }
+    for (int i = 0; i < 8; i++) operand(0, 0, 0, i);
+    for (int img = 0, g = 0; work < xcd_end; img = C3_IMG - img) {
+#pragma unroll
+        for (int t = 0; t < 9; t++) {
+            products(0, img, t);
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            products(1, t < 8 ? img : C3_IMG - img, t < 8 ? t + 1 : 0);
         }
-        channel_group(g == 0, 64 * g, img, C3_IMG - img, last ? in : in + 64 * (g + 1), last ? 0 : 64 * (g + 1));
-        if (last) {
-            epilogue(img, more);
-            if (!more) break;
+        if (++g == groups) {
+            settle();
+            epilogue(img);
             clear();
+            g = 0;
             work += stride;
-            ty0 = ty; tx0 = tx; n0 = n;
-            woff[0] = woff_next[0];
-            woff[1] = woff_next[1];
         }
-        g = last ? 0 : g + 1;
-        img = C3_IMG - img;
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           /* no load into the LDS is left when it is given up */
 }
 #pragma clang diagnostic pop
 
@@ -583,7 +607,7 @@ int launch_3x3(hipStream_t st, float *out, const float *in, const uint16_t *W, c
     const int total = tiles_x * ((s.oh + C3_T - 1) / C3_T) * tiles_n, per_xcd = (total + 7) / 8;
     const unsigned lds = 2 * C3_BIAS + 4 * C3_N * (unsigned)tiles_n;
     /* one workgroup per CU (its LDS): 32 per XCD, each walking the XCD's tiles */
-    hipLaunchKernelGGL(k_conv_3x3, dim3((unsigned)(per_xcd < 32 ? per_xcd : 32) * 8), dim3(512), lds, st, out, in, W, bias, s, tiles_x, tiles_n, total, per_xcd);
+    hipLaunchKernelGGL(k_conv_3x3, dim3((unsigned)(per_xcd < 32 ? per_xcd : 32) * 8), dim3(C3_THREADS), lds, st, out, in, W, bias, s, tiles_x, tiles_n, total, per_xcd);
     return (int)hipGetLastError();
 }
 
