@@ -6,12 +6,14 @@
  * k_conv_few_out: k * k * cout <= 28, the 3-channel output of the VAE decoder.
  * k_conv_1x1: cin a multiple of 128, at most 512, cout at most 256: the VAE's skip connections.
  * k_conv_3x3: 3 x 3, stride 1, cin a multiple of 64: every other layer of the VAE but the halving ones.
+ * k_conv_3x3_half: 3 x 3, stride 2, cin a multiple of 32, cout at least 128: those.
  *
  * The first two are bound by memory: one side of the product is so thin that the image on the other side is all there
  * is to move. The image is rounded to bf16 on the way into the matrix core, products are summed in f32.
  */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 #include "iris_kernels_hip.h"
 
@@ -346,7 +348,12 @@ int launch_1x1(hipStream_t st, float *out, const float *in, const uint16_t *W, c
  * tap starts at, they fall into distinct bank windows; a tap's shift is an immediate offset. Weight rows are swizzled as
  * in gemm_conv_gfx950.hip. A workgroup takes 152 KB of LDS, so a CU runs one, and it is persistent.
  *
-@@MEASURED@@ */
+ * Measured against a bf16 copy of the image + implicit product that fetches every tap from the L2 (copy + product), against
+ * eight waves that did everything (and stood still while a tile's stores landed), and now: 512 x 512 pixels, 128 -> 128
+ * 30 + 118, 79, 73 us (the image and the result alone take 50 us to move), 256 -> 128 76 + 214, 129, 123, 256 -> 256 88 + 290,
+ * 253, 235 us (1320 TFLOP/s). With nothing to bring in, the products and stores of the last take 192 us; the image costs 42 of
+ * the rest, the weights 25, all at a clock that the chip's power has brought down to 2.0 GHz. Pixels and weights on waves of
+ * their own (three and one) 1 % slower. */
 constexpr int C3_T = 16, C3_H = C3_T + 2, C3_PIXELS = C3_H * C3_H, C3_ROW = 80, C3_IMG = C3_PIXELS * C3_ROW;   /* elements */
 constexpr int C3_N = 128, C3_STAGE = C3_N * 64;
 constexpr int C3_MUL = 8, C3_BRING = 4, C3_THREADS = 64 * (C3_MUL + C3_BRING);           /* waves that multiply, that bring pixels and weights */
@@ -611,6 +618,278 @@ int launch_3x3(hipStream_t st, float *out, const float *in, const uint16_t *W, c
     return (int)hipGetLastError();
 }
 
+/* ---- 3 x 3 with stride 2 ----
+ *
+ * The halving layers of the VAE encoder, in the manner of k_conv_3x3: 8 x 16 output pixels of 128 channels, the 17 x 33 pixels
+ * under them read once as f32 and kept in the LDS as bf16, 32 channels at a time in two buffers. A step is a row of three
+ * taps: eight waves, 4 (two rows of pixels) x 2 (64 channels), take 24 products each, the operands of a tap read in the gaps
+ * between the products of the one before; the barrier stands in front of the last tap's products. Behind the barrier of
+ * step s its weights' stage (two of 24 KB) is free and wave 11 requests those of step s + 2. Waves 8 - 10 keep the pixels of
+ * the next group but one on their way, four units of 8 channels x pixel a step.
+ * A pixel takes 80 B: neighbouring outputs' pixels are 160 B apart, as in k_conv_3x3. 16 B chunk c of weight row r sits
+ * in slot c ^ {0, 2, 3, 1}[r / 4 % 4] of its 64 B: the 16 lanes that a 128-bit read serves together, rows 0 - 3 and
+ * 12 - 15 with one chunk and 4 - 11 with its neighbour, then hit distinct bank windows.
+ * Bound by the image where there are few channels (512 x 512 x 128 in, 167 MB with the result: 30 us at the rate of a copy), by
+ * the products otherwise. Against a bf16 copy of the image + implicit product: 512 x 512, 128 -> 128 63 -> 42 us, 1024 x 1024
+ * 304 -> 164, 128 x 128 30 -> 12, 256 x 256, 256 -> 256 77 -> 28, 128 x 128, 512 -> 512 119 -> 42, 256 x 256 143 -> 113. Pixels
+ * straight into registers under every tap instead of a shared tile (nine reads of 2.25 outputs' pixels each): 55 us for the
+ * first, 92 for 256 -> 256: a CU takes in 50 - 65 KB/us of what is not in its XCD's L2. */
+constexpr int H3_TY = 8, H3_TX = 16, H3_HY = 2 * H3_TY + 1, H3_HX = 2 * H3_TX + 1, H3_PIXELS = H3_HY * H3_HX, H3_C = 32, H3_ROW = 40;
+constexpr int H3_IMG = H3_PIXELS * H3_ROW, H3_TAP = C3_N * H3_C, H3_STAGE = 3 * H3_TAP;      /* elements */
+constexpr int H3_BRING = 3, H3_THREADS = 64 * (C3_MUL + H3_BRING + 1), H3_PIECES = H3_STAGE / 512;
+constexpr int H3_UNITS = (H3_PIXELS * 4 + 64 * H3_BRING - 1) / (64 * H3_BRING);
+constexpr int H3_OUT = 2 * H3_IMG + 2 * H3_STAGE, H3_BIAS = H3_OUT + C3_MUL * 1024;          /* 2 KB per wave for its stores; bias */
+constexpr int H3_MAX_COUT = (160 * 1024 - 2 * H3_BIAS) / 4 / C3_N * C3_N;
+static_assert(H3_UNITS == 12 && H3_PIECES == 24 && H3_IMG % 8 == 0, "four units a step");
+
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"                /* M0 in a clobber list */
+__global__ void __launch_bounds__(H3_THREADS, 3)
+k_conv_3x3_half(float *__restrict__ out, const float *__restrict__ in, const uint16_t *__restrict__ W, const float *__restrict__ bias,
+                ConvShape s, int tiles_x, int tiles_n, int total, int per_xcd) {
+    extern __shared__ __align__(16) uint16_t lds[];            /* image, image, weights, weights, outputs, bias */
+    const int xcd_end = min((int)(blockIdx.x % 8 + 1) * per_xcd, total), stride = gridDim.x / 8;
+    int work = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if (work >= xcd_end) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int groups = s.cin / H3_C;
+    float *bias_lds = reinterpret_cast<float *>(lds + H3_BIAS);
+    for (int i = tid; i < tiles_n * C3_N; i += H3_THREADS) bias_lds[i] = bias && i < s.cout ? bias[i] : 0.0f;
+
+    /* Every wave passes one barrier here in front and three per channel group, in every role. */
+    if (wave >= C3_MUL + H3_BRING) {
+        /* weights: request j brings rows 16 (j % 8) .. + 15 of tap j / 8 of the row; rows past the last channel repeat it
+         * (their results are never stored). When nothing comes next the last requests are of weights that nobody uses. */
+        __builtin_amdgcn_s_setprio(3);
+        uint32_t off[8];
+        auto aim = [&](int w) {
+            const int n = w % tiles_n * C3_N;
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const int r = 16 * j + (lane >> 2), row = n + r < s.cout ? n + r : s.cout - 1, k4 = (r >> 2) & 3;
+                const int swizzle = ((k4 << 1) ^ (k4 >> 1) * 3) & 3;
+                off[j] = ((uint32_t)row * (uint32_t)(9 * s.cin) + 8u * ((lane & 3) ^ swizzle)) * 2u;
+            }
+        };
+        const uint32_t stages = lds_address(lds + 2 * H3_IMG);
+        auto request = [&](int row, int c0, int stage) {
+#pragma unroll
+            for (int j = 0; j < H3_PIECES; j++)
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                             ::"s"(stages + 2 * (stage * H3_STAGE + j * 512)), "v"(off[j % 8]), "s"(W + (size_t)(3 * row + j / 8) * s.cin + c0)
+                             : "memory", "m0");
+        };
+        aim(work);
+        request(0, 0, 0);
+        request(1, 0, 1);
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(H3_PIECES) : "memory");
+        for (int g = 0, stage = 0; work < xcd_end;) {
+            const bool last = g + 1 == groups;
+#pragma unroll
+            for (int t = 0; t < 3; t++) {
+                asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");      /* those of the next step are there */
+                if (t == 1 && last && work + stride < xcd_end) aim(work + stride);
+                if (t == 0) request(2, H3_C * g, stage);
+                else request(t - 1, last ? 0 : H3_C * (g + 1), stage);
+                stage ^= 1;
+            }
+            g = last ? 0 : g + 1;
+            if (last) work += stride;
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       /* no load into the LDS is left when it is given up */
+        return;
+    }
+    if (wave >= C3_MUL) {
+        /* pixels: unit u of this thread is channels 8 (bt % 4) .. + 7 of pixel bt / 4 + 48 u of the rimmed tile; a pixel
+         * outside the image reads the first one and is zeroed */
+        __builtin_amdgcn_s_setprio(3);
+        const int bt = tid - 64 * C3_MUL, px0 = bt >> 2;
+        uint32_t off[H3_UNITS], inside = 0, held = 0;          /* bytes from the channel group's first value; bit u: in the image */
+        int w = work, g = 0;                                   /* where the next loads come from */
+        const float *src = in;
+        auto aim = [&]() {
+            const int tile = w / tiles_n, ty = tile / tiles_x * (2 * H3_TY) - s.pad, tx = tile % tiles_x * (2 * H3_TX) - s.pad;
+            int first = px0;
+            asm volatile("" : "+v"(first));                    /* worked out here for every tile: kept over the loop it all spills */
+            inside = 0;
+#pragma unroll
+            for (int u = 0; u < H3_UNITS; u++) {
+                const int px = first + 16 * H3_BRING * u, py = px / H3_HX, y = ty + py, x = tx + (px - py * H3_HX);
+                const bool ok = px < H3_PIXELS && y >= 0 && y < s.h && x >= 0 && x < s.w;
+                if (ok) inside |= 1u << u;
+                off[u] = ((ok ? (uint32_t)(y * s.w + x) * (uint32_t)s.cin : 0u) + 8u * (bt & 3)) * 4u;
+            }
+        };
+        auto advance = [&]() {
+            if (g + 1 < groups) {
+                g++;
+                src += H3_C;
+            } else {
+                src = in;
+                g = 0;
+                w += stride;
+                if (w < xcd_end) {
+                    aim();
+                } else {                                       /* nothing comes next: the same loads, of a few cached bytes that nobody uses */
+                    inside = 0;
+#pragma unroll
+                    for (int u = 0; u < H3_UNITS; u++) off[u] = 32u * (bt & 3);
+                }
+            }
+        };
+        f32x4 xr[H3_UNITS][2];
+        auto load = [&](int u) {
+            const char *p = reinterpret_cast<const char *>(src) + off[u];
+            xr[u][0] = *reinterpret_cast<const f32x4 *>(p);
+            xr[u][1] = *reinterpret_cast<const f32x4 *>(p + 16);
+        };
+        auto put = [&](int img, int u) {
+            const f32x4 lo = xr[u][0], hi = xr[u][1];
+            u32x4 v = {pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3])};
+            if (!(held >> u & 1)) v = u32x4{0, 0, 0, 0};
+            if (u + 1 < H3_UNITS || px0 < H3_PIXELS - 16 * H3_BRING * (H3_UNITS - 1))
+                *reinterpret_cast<u32x4 *>(&lds[img + (px0 + 16 * H3_BRING * u) * H3_ROW + 8 * (bt & 3)]) = v;
+        };
+        aim();
+#pragma unroll
+        for (int u = 0; u < H3_UNITS; u++) load(u);
+        held = inside;
+        advance();
+#pragma unroll
+        for (int u = 0; u < H3_UNITS; u++) {
+            put(0, u);
+            load(u);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        for (int img = 0, gg = 0; work < xcd_end; img = H3_IMG - img) {
+            held = inside;
+            advance();
+#pragma unroll
+            for (int t = 0; t < 3; t++) {
+#pragma unroll
+                for (int u = 4 * t; u < 4 * t + 4; u++) {
+                    put(H3_IMG - img, u);
+                    load(u);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            }
+            if (++gg == groups) { gg = 0; work += stride; }
+        }
+        return;
+    }
+
+    const int li = lane & 15, lg = lane >> 4, wm = wave & 3, wn = wave >> 2;
+    f32x4 acc[4][2];                                           /* [16 channels][row of 16 pixels] */
+    auto clear = [&]() {
+#pragma unroll
+        for (int a = 0; a < 4; a++)
+#pragma unroll
+            for (int b = 0; b < 2; b++) acc[a][b] = f32x4{0, 0, 0, 0};
+    };
+    u32x4 av[2][4], bv[2][2];
+    const int k4 = li >> 2, a_rd = 2 * H3_IMG + (64 * wn + li) * H3_C + 8 * (lg ^ (((k4 << 1) ^ (k4 >> 1) * 3) & 3));
+    const int b_rd = (4 * wm * H3_HX + 2 * li) * H3_ROW + 8 * lg;
+    /* operand i of a tap, in the order its products use them */
+    auto operand = [&](int set, int img, int stage, int ky, int kx, int i) {
+        if (i == 0 || i > 2) {
+            const int a = i == 0 ? 0 : i - 2;
+            av[set][a] = *reinterpret_cast<const u32x4 *>(&lds[a_rd + stage * H3_STAGE + kx * H3_TAP + 16 * a * H3_C]);
+        } else {
+            bv[set][i - 1] = *reinterpret_cast<const u32x4 *>(&lds[img + b_rd + ((2 * (i - 1) + ky) * H3_HX + kx) * H3_ROW]);
+        }
+    };
+    auto products = [&](int set, int img, int stage, int ky, int kx) {       /* img .. kx: of the operands read on the way */
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            acc[i / 2][i % 2] = mfma(av[set][i / 2], bv[set][i % 2], acc[i / 2][i % 2]);
+            if (i < 6) operand(set ^ 1, img, stage, ky, kx, i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    /* acc[a][b][r]: channel n0 + 64 wn + 16 a + 4 lg + r of pixel (2 wm + b, li) of the tile. Through the LDS (2 KB, a wave's
+     * own region), 16 pixels x 32 channels at a time, so that a store instruction covers eight pixels x 128 B. */
+    const bool chunks = s.cout % 4 == 0 && ((uintptr_t)out & 15) == 0;
+    auto epilogue = [&]() {
+        const int tile = work / tiles_n, n0 = (work - tile * tiles_n) * C3_N, ty0 = tile / tiles_x * H3_TY, tx0 = tile % tiles_x * H3_TX;
+        float *buf = reinterpret_cast<float *>(lds + H3_OUT) + wave * 512;
+        const int c = lane & 7;
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            const int y = ty0 + 2 * wm + b;
+#pragma unroll
+            for (int half = 0; half < 2; half++) {
+#pragma unroll
+                for (int a = 0; a < 2; a++) *reinterpret_cast<f32x4 *>(&buf[li * 32 + 4 * ((4 * a + lg) ^ (li & 7))]) = acc[2 * half + a][b];
+                const int n = n0 + 64 * wn + 32 * half + 4 * c;
+                const f32x4 bias4 = *reinterpret_cast<const f32x4 *>(bias_lds + n);
+#pragma unroll
+                for (int it = 0; it < 2; it++) {
+                    const int row = 8 * it + (lane >> 3), x = tx0 + row;
+                    const f32x4 v = *reinterpret_cast<const f32x4 *>(&buf[row * 32 + 4 * (c ^ (row & 7))]) + bias4;
+                    if (y >= s.oh || x >= s.ow) continue;
+                    float *dst = out + ((size_t)y * s.ow + x) * s.cout + n;
+                    if (chunks) {
+                        if (n < s.cout) *reinterpret_cast<f32x4 *>(dst) = v;
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; e++)
+                            if (n + e < s.cout) dst[e] = v[e];
+                    }
+                }
+            }
+        }
+    };
+
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < 6; i++) operand(0, 0, 0, 0, 0, i);
+    clear();
+    /* nine taps a group, so operand sets and stages change places from one group to the next: two groups a turn */
+    int img = 0, g = 0;
+    auto channel_group = [&](auto odd) {
+        constexpr int o = decltype(odd)::value;
+#pragma unroll
+        for (int t = 0; t < 3; t++) {
+            const int stage = (t + o) & 1;
+            products((3 * t + o) & 1, img, stage, t, 1);
+            products((3 * t + 1 + o) & 1, img, stage, t, 2);
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            products((3 * t + 2 + o) & 1, t < 2 ? img : H3_IMG - img, stage ^ 1, t < 2 ? t + 1 : 0, 0);
+        }
+        img = H3_IMG - img;
+        if (++g == groups) {
+            epilogue();
+            clear();
+            g = 0;
+            work += stride;
+        }
+    };
+    while (work < xcd_end) {
+        channel_group(std::integral_constant<int, 0>{});
+        if (work >= xcd_end) break;
+        channel_group(std::integral_constant<int, 1>{});
+    }
+}
+#pragma clang diagnostic pop
+
+int launch_3x3_half(hipStream_t st, float *out, const float *in, const uint16_t *W, const float *bias, const ConvShape &s) {
+    static bool configured = false;
+    if (!configured) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_conv_3x3_half), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (e != hipSuccess) return (int)e;
+        configured = true;
+    }
+    const int tiles_x = (s.ow + H3_TX - 1) / H3_TX, tiles_n = (s.cout + C3_N - 1) / C3_N;
+    const int total = tiles_x * ((s.oh + H3_TY - 1) / H3_TY) * tiles_n, per_xcd = (total + 7) / 8;
+    const unsigned lds = 2 * H3_BIAS + 4 * C3_N * (unsigned)tiles_n;
+    hipLaunchKernelGGL(k_conv_3x3_half, dim3((unsigned)(per_xcd < 32 ? per_xcd : 32) * 8), dim3(H3_THREADS), lds, st, out, in, W, bias, s, tiles_x,
+                       tiles_n, total, per_xcd);
+    return (int)hipGetLastError();
+}
+
 template <int STEPS>
 int launch_few_out(hipStream_t st, float *out, const float *in, const uint16_t *W, const float *bias, const ConvShape &s) {
     static bool configured = false;
@@ -653,6 +932,9 @@ int iris_hip_conv2d_direct(void *stream, float *out, const float *in, const uint
     if (k == 3 && stride == 1 && cin % 64 == 0 && cout <= C3_MAX_COUT && al16(in) && al16(w) && (size_t)h * width * cin * 4 < ((size_t)1 << 32) &&
         (size_t)cout * 9 * cin * 2 < ((size_t)1 << 32))
         return launch_3x3(st, out, in, w, bias, s);
+    if (k == 3 && stride == 2 && cin % H3_C == 0 && cout >= 128 && cout <= H3_MAX_COUT && al16(in) && al16(w) &&
+        (size_t)h * width * cin * 4 < ((size_t)1 << 32) && (size_t)cout * 9 * cin * 2 < ((size_t)1 << 32))
+        return launch_3x3_half(st, out, in, w, bias, s);
     return -2;
 }
 

@@ -28,7 +28,7 @@
  * of 8 with 16-byte aligned rows, otherwise the scalar kernel below takes over.
  *
  * Convolution with a handful of input or output channels (the VAE's first and last layers) has kernels of its own
- * (conv_gfx950.hip), and so has 3 x 3 with stride 1. Otherwise, with a multiple of 64 input channels it is an
+ * (conv_gfx950.hip), and so has 3 x 3 with strides 1 and 2. Otherwise, with a multiple of 64 input channels it is an
  * implicit GEMM: the image is converted to bf16 once and k_gemm_dma fetches the pixels under each
  * tap itself, so the k x k patches are never written out. Other shapes gather the patches as bf16
  * rows into scratch (what the reference does for all of them, iris_cuda.cu:959-985) and run the

@@ -59,3 +59,13 @@ def test_one_by_one(dev, orc, h, w, cin, cout, bias):
     """One block of 16 pixels and less, more blocks than waves, one and two tiles of 128 channels, a ragged one; and what goes
     through the bf16 copy and a plain product with the bias in its epilogue or behind it."""
     conv_case(dev, orc, h, w, cin, cout, 1, 1, 0, 0, bias)
+
+
+@pytest.mark.parametrize("h,w,cin,cout,pb,pa,bias", [
+    (2, 2, 128, 128, 0, 1, True), (16, 32, 32, 128, 0, 1, True), (17, 33, 64, 128, 0, 0, False), (33, 32, 128, 130, 0, 1, True),
+    (31, 67, 96, 256, 1, 1, True), (46, 44, 256, 256, 0, 1, True), (40, 41, 160, 260, 2, 0, False), (5, 200, 512, 129, 1, 0, True),
+    (150, 340, 128, 256, 0, 1, True)])
+def test_three_by_three_stride_two(dev, orc, h, w, cin, cout, pb, pa, bias):
+    """Tile edges (8 x 16 output pixels, 128 channels), one to sixteen groups of 32 input channels (odd and even numbers of them),
+    padding of other widths, more tiles than workgroups."""
+    conv_case(dev, orc, h, w, cin, cout, 3, 2, pb, pa, bias)
