@@ -5,9 +5,9 @@
  * accesses per lane where the pointers and sizes allow it, a scalar form of
  * the same kernel otherwise.
  *
- * Row normalisations use one workgroup per row and keep the row in registers
- * between the statistics and the write (rows up to 4096 floats; longer rows
- * are read again, from cache).
+ * Row normalisations use one workgroup per row, a wave for short rows, and
+ * keep the row in registers between the statistics and the write (rows up to
+ * 4096 floats; longer rows are read again, from cache).
  * Statistics follow the reference: LayerNorm takes the mean first and the
  * variance about it. Group norm takes its statistics in ONE pass over the
  * image (coalesced per-pixel reads, per-workgroup partial moments of every
@@ -166,19 +166,23 @@ __device__ __forceinline__ float block_sum(float v, float *sh) {
 enum NormKind { LAYER_NORM_MOD, RMS_NORM_MOD, RMS_NORM_RESIDUAL };
 constexpr int ROW_VECS = 4;           /* float4 per thread kept in registers: rows up to 4096 floats */
 
-/* One workgroup of 256 threads per row. CACHE: dim % 4 == 0, dim <= 4096, 16-byte aligned rows -> the row stays in
- * registers between the statistics and the write, and everything the write needs is requested before the first sum is
- * waited for; otherwise it is read again. p0/p1 are (shift, scale) for LayerNorm, (w, scale) for RMSNorm, (w, gate) for
- * the residual form; out_bf is unused by the latter.
- * A wave per row instead leaves a short sequence with few waves of long chains, and a long one with a single generation
+/* TPR threads per row: a workgroup of 256, or a wave for many rows of up to 1024 floats. CACHE: dim % 4 == 0, dim <= 4096,
+ * 16-byte aligned rows -> the row stays in registers between the statistics and the write, and everything the write needs is
+ * requested before the first sum is waited for; otherwise it is read again. p0/p1 are (shift, scale) for LayerNorm,
+ * (w, scale) for RMSNorm, (w, gate) for the residual form; out_bf is unused by the latter.
+ * A wave per row of thousands of floats leaves a short sequence with few waves of long chains, and a long one with a single generation
  * of waves that first all read and then all write: 4608 x 3072 LayerNorm 23.1 us, now 18.8;
  * 512 x 2560 RMSNorm 7.2 us, now 5.3; 512 x 3072 LayerNorm 9.7 us, now 5.1. */
-template <int KIND, bool CACHE>
+template <int KIND, bool CACHE, int TPR>
 __global__ void __launch_bounds__(ROW_THREADS)
 k_row_norm(uint16_t *__restrict__ out_bf, float *__restrict__ xres, const float *__restrict__ src,
-           const float *__restrict__ p0, const float *__restrict__ p1, int dim, float eps) {
+           const float *__restrict__ p0, const float *__restrict__ p1, int rows, int dim, float eps, unsigned grid_x) {
     __shared__ float sh[4];
-    const size_t row_off = (size_t)blockIdx.x * dim;
+    const unsigned row = (blockIdx.y * grid_x + blockIdx.x) * (ROW_THREADS / TPR) + threadIdx.x / TPR;
+    if (row >= (unsigned)rows) return;                                  /* the same for all threads of a row */
+    const int tid = threadIdx.x % TPR;
+    auto row_sum = [&](float v) { return TPR == 64 ? wave_sum(v) : block_sum(v, sh); };
+    const size_t row_off = (size_t)row * dim;
     const float *xr = src + row_off;
     const int nvec = dim >> 2;
     float4 keep[ROW_VECS], pa[ROW_VECS], pb[ROW_VECS], res[ROW_VECS];
@@ -188,12 +192,12 @@ k_row_norm(uint16_t *__restrict__ out_bf, float *__restrict__ xres, const float 
     if (CACHE) {
 #pragma unroll
         for (int j = 0; j < ROW_VECS; j++) {
-            const int v = threadIdx.x + j * ROW_THREADS;
+            const int v = tid + j * TPR;
             keep[j] = v < nvec ? *reinterpret_cast<const float4 *>(xr + 4 * v) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         }
 #pragma unroll
         for (int j = 0; j < ROW_VECS; j++) {
-            const int v = threadIdx.x + j * ROW_THREADS;
+            const int v = tid + j * TPR;
             pa[j] = pb[j] = res[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             if (v < nvec) {
                 if (pa_src) pa[j] = *reinterpret_cast<const float4 *>(pa_src + 4 * v);
@@ -206,9 +210,9 @@ k_row_norm(uint16_t *__restrict__ out_bf, float *__restrict__ xres, const float 
             s += KIND == LAYER_NORM_MOD ? (keep[j].x + keep[j].y) + (keep[j].z + keep[j].w)
                                         : (keep[j].x * keep[j].x + keep[j].y * keep[j].y) + (keep[j].z * keep[j].z + keep[j].w * keep[j].w);
     } else {
-        for (int i = threadIdx.x; i < dim; i += ROW_THREADS) s += KIND == LAYER_NORM_MOD ? xr[i] : xr[i] * xr[i];
+        for (int i = tid; i < dim; i += TPR) s += KIND == LAYER_NORM_MOD ? xr[i] : xr[i] * xr[i];
     }
-    s = block_sum(s, sh);
+    s = row_sum(s);
     float mean = 0.0f, inv;
     if (KIND == LAYER_NORM_MOD) {
         mean = s / (float)dim;
@@ -216,14 +220,14 @@ k_row_norm(uint16_t *__restrict__ out_bf, float *__restrict__ xres, const float 
         if (CACHE) {
 #pragma unroll
             for (int j = 0; j < ROW_VECS; j++)
-                if ((int)threadIdx.x + j * ROW_THREADS < nvec) {
+                if (tid + j * TPR < nvec) {
                     const float a = keep[j].x - mean, b = keep[j].y - mean, c = keep[j].z - mean, d = keep[j].w - mean;
                     v += (a * a + b * b) + (c * c + d * d);
                 }
         } else {
-            for (int i = threadIdx.x; i < dim; i += ROW_THREADS) { const float d = xr[i] - mean; v += d * d; }
+            for (int i = tid; i < dim; i += TPR) { const float d = xr[i] - mean; v += d * d; }
         }
-        inv = 1.0f / sqrtf(block_sum(v, sh) / (float)dim + eps);
+        inv = 1.0f / sqrtf(row_sum(v) / (float)dim + eps);
     } else {
         inv = 1.0f / sqrtf(s / (float)dim + eps);
     }
@@ -231,7 +235,7 @@ k_row_norm(uint16_t *__restrict__ out_bf, float *__restrict__ xres, const float 
     if (CACHE) {
 #pragma unroll
         for (int j = 0; j < ROW_VECS; j++) {
-            const int v = threadIdx.x + j * ROW_THREADS;
+            const int v = tid + j * TPR;
             if (v >= nvec) continue;
             const float xin[4] = {keep[j].x, keep[j].y, keep[j].z, keep[j].w};
             const float av[4] = {pa[j].x, pa[j].y, pa[j].z, pa[j].w}, bv[4] = {pb[j].x, pb[j].y, pb[j].z, pb[j].w};
@@ -258,7 +262,7 @@ k_row_norm(uint16_t *__restrict__ out_bf, float *__restrict__ xres, const float 
             }
         }
     } else {
-        for (int i = threadIdx.x; i < dim; i += ROW_THREADS) {
+        for (int i = tid; i < dim; i += TPR) {
             float r;
             if (KIND == LAYER_NORM_MOD) {
                 r = (xr[i] - mean) * inv;
@@ -281,8 +285,17 @@ int launch_row_norm(hipStream_t st, uint16_t *out_bf, float *xres, const float *
     if (rows <= 0 || dim <= 0) return 0;
     const bool cache = dim % 4 == 0 && dim <= 4 * ROW_THREADS * ROW_VECS && al16(src) && al16(xres) && al16(p0) && al16(p1) &&
                        ((uintptr_t)out_bf & 7) == 0;
-    if (cache) hipLaunchKernelGGL((k_row_norm<KIND, true>), dim3(rows), dim3(ROW_THREADS), 0, st, out_bf, xres, src, p0, p1, dim, eps);
-    else hipLaunchKernelGGL((k_row_norm<KIND, false>), dim3(rows), dim3(ROW_THREADS), 0, st, out_bf, xres, src, p0, p1, dim, eps);
+    /* a wave per row where rows are short and enough of them to fill the chip: 100000 x 128 RMSNorm 69 us with a workgroup
+     * each, 23 so, 20000 x 1024 LayerNorm 26 / 19; 300 x 1024 3.8 / 4.4 */
+    const bool wave = dim <= 4 * 64 * ROW_VECS && rows >= 2048;
+    const unsigned blocks = wave ? ((unsigned)rows + ROW_THREADS / 64 - 1) / (ROW_THREADS / 64) : (unsigned)rows;
+    /* a grid dimension holds less than 2^32 threads */
+    const unsigned gx = blocks < 1u << 20 ? blocks : 1u << 20;
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(gx, (blocks + gx - 1) / gx), dim3(ROW_THREADS), 0, st, out_bf, xres, src, p0, p1, rows, dim, eps, gx);
+    };
+    if (wave) cache ? go(k_row_norm<KIND, true, 64>) : go(k_row_norm<KIND, false, 64>);
+    else cache ? go(k_row_norm<KIND, true, ROW_THREADS>) : go(k_row_norm<KIND, false, ROW_THREADS>);
     return (int)hipGetLastError();
 }
 
