@@ -933,10 +933,16 @@ int iris_hip_conv2d(void *stream, uint16_t *scratch, size_t scratch_bytes, float
     scratch += IRIS_CONV_ZERO_BYTES / sizeof(uint16_t);
     scratch_bytes -= IRIS_CONV_ZERO_BYTES;
 
-    /* 1 x 1 without padding or stride (and more output channels than conv_gfx950.hip keeps at hand): the image as bf16
-     * rows, in chunks that fit the scratch, and a plain product. 16384 x 512 -> 1536: 61 us as an implicit product, 55 so. */
-    if (k == 1 && stride == 1 && oh == h && ow == width && cin % TK == 0 && scratch_bytes >= (size_t)cin * sizeof(uint16_t)) {
-        const long rows = (long)(scratch_bytes / ((size_t)cin * sizeof(uint16_t)));
+    /* 1 x 1 without padding or stride (and more output channels than conv_gfx950.hip keeps at hand) where the plain product
+     * takes smaller tiles than the implicit one below: the image as bf16 rows, in chunks that fit the scratch, and that
+     * product. An attention block with 512 -> 1536 over 1024 pixels 82 -> 69 us, over 4096 122 -> 117. Over more pixels
+     * k_gemm_wide on the copy is 4 us faster than the implicit product by itself (16384: 59 - 63 us with the copy against 64),
+     * but the head_dim-512 attention kernel behind it then runs 20 - 30 us longer: the block 611 against 573, 14391 pixels
+     * 527 / 497, 9216 273 / 261, 7200 198 / 196. */
+    const long rows = (long)(scratch_bytes / ((size_t)cin * sizeof(uint16_t)));
+    const bool aligned_w = ((uintptr_t)w & 15) == 0 && ((uintptr_t)out & 15) == 0;
+    if (k == 1 && stride == 1 && oh == h && ow == width && rows > 0 &&
+        plan_gemm(ohw < rows ? ohw : (int)rows, cout, cin, 4, aligned_w, aligned_w, 0).kernel == 4) {
         for (long p0 = 0; p0 < ohw; p0 += rows) {
             const int np = (int)(ohw - p0 < rows ? ohw - p0 : rows);
             int e = iris_hip_f32_to_bf16(stream, scratch, in + (size_t)p0 * cin, (size_t)np * cin);
