@@ -425,10 +425,10 @@ k_gemm_dma(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *
         }
     }
 }
-/* ---- tiles of 256 rows x 256, 224 or 192 columns ----
+/* ---- tiles of 256 rows x 256, 224, 192 or 160 columns ----
  *
  * For M, N >= 256, K a multiple of 128: every linear layer of the models at their larger sequence lengths. Eight waves, two
- * per SIMD, 4 (rows of 64) x 2: a wave owns 64 rows x 16 NA columns = NA x 4 accumulator blocks (NA = 8, 7, 6, so that the
+ * per SIMD, 4 (rows of 64) x 2: a wave owns 64 rows x 16 NA columns = NA x 4 accumulator blocks (NA = 8, 7, 6, 5, so that the
  * launcher can pick the width whose grid fills the last round of the 256 CUs best). A k tile of 64 is four steps: k-step
  * 0 with the first and the second half of the columns, then k-step 1; the operands of a step are requested from the LDS
  * during the step before. What the kernel lives on:
@@ -470,7 +470,7 @@ k_gemm_wide(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t 
             int tiles_m, int total, int per_xcd, QkNorm qn, const float *__restrict__ bias, int streaming_out) {
     using T = Wide<NA>;
     constexpr int TM = T::TM, TN = T::TN, XS = T::XS, WS = T::WS, WP = T::WP, H0 = (NA + 1) / 2, H1 = NA / 2;
-    static_assert(WP <= 4 && H1 >= 3, "");
+    static_assert(WP <= 4 && H1 >= 2, "");
     extern __shared__ __align__(16) uint16_t dlds[];           /* x, x, W, W, W */
     const int work = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
     if (work >= total) return;
@@ -571,9 +571,15 @@ k_gemm_wide(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t 
         /* This wave has read its last operands of the tile, and its share of the next one has landed: newer than that are
          * only the W pieces requested in this tile. Behind the barrier the tile's stages are free. */
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(WP) : "memory");
-        products(1, H0, NA, [&](int g) {                       /* x at gaps 0, 2, 4, 6, the reads in the others */
-            if (g < 8 && g % 2 == 0) request_x(g / 2, after_next, x_cur);
-            else read_first(x_nxt, w_nxt, 0, g < 8 ? g / 2 : g - 4);
+        products(1, H0, NA, [&](int g) {                       /* x at gaps 0, 2, 4, 6, the reads in the others: two to a gap where there are no more */
+            if (g < 8 && g % 2 == 0) {
+                request_x(g / 2, after_next, x_cur);
+            } else if (H1 == 2) {
+                read_first(x_nxt, w_nxt, 0, g - 1);
+                read_first(x_nxt, w_nxt, 0, g);
+            } else {
+                read_first(x_nxt, w_nxt, 0, g < 8 ? g / 2 : g - 4);
+            }
         });
         const uint32_t x_free = x_cur, w_free = w_cur;
         x_cur = x_nxt; x_nxt = x_free;
@@ -746,14 +752,17 @@ static bool wide_shape(int M, int N, int K, size_t out_size) {
 }
 
 /* The tile width (32 NA columns) whose grid wastes least of its last round of 256 workgroups: time goes with
- * rounds x width. 4608 x 9216 outputs: 648 tiles of 256 columns are 2.53 rounds, 756 of 224 are 2.95. */
+ * rounds x width. 4608 x 9216 outputs: 648 tiles of 256 columns are 2.53 rounds, 756 of 224 are 2.95. 160 columns read half as
+ * much again from the LDS per product as 256 and are only taken where they fill one round that wider tiles leave a fifth idle,
+ * 512 rows: 2560 -> 19456 204 tiles of 192 columns 52.5 us, 244 of 160 51.3; 3072 -> 18432 57.5 / 56.0, 4096 -> 20480 78.2 / 74.9. */
 static int wide_width(int M, int N) {
     const long tiles_m = (M + DT - 1) / DT;
     int best = 8;
     long best_cost = 0;
-    for (int na = 8; na >= 6; na--) {
+    for (int na = 8; na >= 5; na--) {
         const long tiles = tiles_m * ((N + 32 * na - 1) / (32 * na));
-        const long cost = ((tiles + 255) / 256) * na * (na == 8 ? 100 : 102);      /* the narrower tiles reuse operands a little less */
+        if (na == 5 && (tiles <= 192 || tiles > 256)) continue;
+        const long cost = ((tiles + 255) / 256) * na * (na == 8 ? 100 : na > 5 ? 102 : 108);      /* the narrower tiles reuse operands a little less */
         if (na == 8 || cost < best_cost) { best = na; best_cost = cost; }
     }
     return best;
@@ -812,7 +821,8 @@ int gemm(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, in
         e = iris_hip_gemm_tiles(st, y, (int)sizeof(OUT), x, W, M, N, K, fused, plan.na, plan.splits, part);
     } else if (plan.kernel == 3) {
         e = plan.na == 8 ? launch_gemm_wide<OUT, 8>(st, y, x, W, M, N, K, fused)
-          : plan.na == 7 ? launch_gemm_wide<OUT, 7>(st, y, x, W, M, N, K, fused) : launch_gemm_wide<OUT, 6>(st, y, x, W, M, N, K, fused);
+          : plan.na == 7 ? launch_gemm_wide<OUT, 7>(st, y, x, W, M, N, K, fused)
+          : plan.na == 6 ? launch_gemm_wide<OUT, 6>(st, y, x, W, M, N, K, fused) : launch_gemm_wide<OUT, 5>(st, y, x, W, M, N, K, fused);
     } else if (plan.kernel == 2) {
         const ConvGeom none = {};
         e = launch_gemm_dma<OUT, 256, false>(st, y, x, W, M, N, K, none);

@@ -72,6 +72,25 @@ def test_linear_layers_that_take_it(dev, rows, k, out, bf16):
     check(got, want, k, bf16)
 
 
+@pytest.mark.parametrize("rows,k,out", [(512, 128, 19456), (449, 384, 18448), (257, 256, 20480)])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_wide_tiles_of_160_columns(dev, rows, k, out, bf16):
+    """k_gemm_wide's narrowest tile: two to six k tiles, a last tile of one row, of 48 and of 96 columns."""
+    plan = (C.c_int * 2)()
+    dev.lib.iris_hip_linear_plan(rows, k, out, 2 if bf16 else 4, plan)
+    assert list(plan) == [3, 160]
+    x, W, want = operands(rows, k, out)
+    guard = 512
+    fill = np.full(rows * out + guard, 7, np.uint16 if bf16 else np.float32)
+    dy = dev.put(fill)
+    (dev.lib.iris_dev_linear_bf16 if bf16 else dev.lib.iris_dev_linear_f32)(dy, dev.put(x), dev.put(W), rows, k, out)
+    dev.check()
+    got = dev.get(dy, fill.shape, fill.dtype)
+    dev.free_all()
+    assert (got[rows * out:] == 7).all()
+    check(got[:rows * out].reshape(rows, out), want, k, bf16)
+
+
 def test_projection_with_norm_takes_the_same_kernel(dev):
     """The projection that normalises its own columns, at a size whose plain layer takes these tiles: the bits of the two calls."""
     rows, k, heads = 320, 1024, 6
