@@ -13,7 +13,7 @@
  *
  * Products with too few 256-row tiles to fill the chip (short sequences) take k_gemm_tiles (gemm_tiles_gfx950.hip). For
  * the rest, three kernels. M, N >= 256 with K a multiple of 128 (every linear layer of the models at their
- * larger sequence lengths) take k_gemm_wide: tiles of 256 rows x 256, 224 or 192 columns on eight waves, every memory
+ * larger sequence lengths) take k_gemm_wide: tiles of 256 rows x 256 - 160 columns on eight waves, every memory
  * instruction in a gap between two products. Other shapes with M, N >= 256 and K a multiple of 64, and the convolutions
  * that have no kernel of their own, take k_gemm_dma: the same tiles with the loads and reads in groups. Both give the same
  * bits. Everything else with K a multiple of 8 takes k_gemm_bf16:
@@ -885,10 +885,10 @@ void iris_hip_linear_plan(int rows, int in, int out, int out_bytes, int *plan) {
 }
 
 int iris_hip_linear_f32(void *stream, float *part, float *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out) {
-    return gemm<float>((hipStream_t)stream, y, x, W, rows, out, in, part, IRIS_LINEAR_PART_BYTES);
+    return gemm<float>((hipStream_t)stream, y, x, W, rows, out, in, part, part ? IRIS_LINEAR_PART_BYTES : 0);
 }
 int iris_hip_linear_bf16(void *stream, float *part, uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out) {
-    return gemm<uint16_t>((hipStream_t)stream, y, x, W, rows, out, in, part, IRIS_LINEAR_PART_BYTES);
+    return gemm<uint16_t>((hipStream_t)stream, y, x, W, rows, out, in, part, part ? IRIS_LINEAR_PART_BYTES : 0);
 }
 
 /* y = x W^T as bf16 with the per-head RMSNorm + rotary embedding (head_dim 128) of columns [0, q_cols) (weights
@@ -906,12 +906,13 @@ int iris_hip_linear_bf16_qknorm(void *stream, float *part, uint16_t *y, const ui
     if (!tiled || N % 128 || q_cols < 0 || k_cols < 0 || q_cols % 128 || k_cols % 128 || q_cols + k_cols > N ||
         q_cols + k_cols == 0 || (long long)M * (qh + kh) >= (1 << 24) || qh + kh >= 256)
         return -2;
-    const GemmPlan plan = plan_gemm(M, N, K, 2, true, true, IRIS_LINEAR_PART_BYTES);
+    const size_t part_bytes = part ? IRIS_LINEAR_PART_BYTES : 0;
+    const GemmPlan plan = plan_gemm(M, N, K, 2, true, true, part_bytes);
     if (plan.kernel == 3 && plan.na == 8) {
         const QkNorm qn = {wq, k_cols ? wk : wq, rope_cos, rope_sin, q_cols, q_cols + k_cols, eps, split_half};
         return launch_gemm_wide<uint16_t, 8, true>((hipStream_t)stream, y, x, W, M, N, K, nullptr, qn);
     }
-    const int e = gemm<uint16_t>((hipStream_t)stream, y, x, W, M, N, K, part, IRIS_LINEAR_PART_BYTES);
+    const int e = gemm<uint16_t>((hipStream_t)stream, y, x, W, M, N, K, part, part_bytes);
     if (e) return e;
     return qh ? iris_hip_norm_rope_hd128(stream, y, kh ? y + q_cols : nullptr, N, wq, wk, rope_cos, rope_sin, M, qh, kh, eps, split_half)
               : iris_hip_norm_rope_hd128(stream, y, nullptr, N, wk, nullptr, rope_cos, rope_sin, M, kh, 0, eps, split_half);

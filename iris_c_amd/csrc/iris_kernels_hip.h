@@ -134,7 +134,7 @@ int iris_hip_group_norm_static(void *stream, float *out, const float *in, const 
 /* ---- linear layers and convolution (gemm_conv_gfx950.hip, gemm_tiles_gfx950.hip) ---- */
 /* y[rows, out] = x[rows, in] @ W[out, in]^T, contiguous; MFMA kernel when in % 8 == 0 and
  * x, W are 16-byte aligned, scalar kernel otherwise. part: IRIS_LINEAR_PART_BYTES of private workspace, 16-byte aligned,
- * for the partial sums of products whose K is cut into ranges. */
+ * for the partial sums of products whose K is cut into ranges, or NULL: K then stays whole. */
 #define IRIS_LINEAR_PART_BYTES ((size_t)64 << 20)
 int iris_hip_linear_f32(void *stream, float *part, float *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out);
 int iris_hip_linear_bf16(void *stream, float *part, uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out);

@@ -87,9 +87,8 @@ int iris_dev_init(void) {
     snprintf(g_name, sizeof(g_name), "%s (%s, %d CUs, %d MHz)", prop.name[0] ? prop.name : "AMD Instinct",
              prop.gcnArchName, prop.multiProcessorCount, prop.clockRate / 1000);
     if (!g_linear_part && hipMalloc((void **)&g_linear_part, IRIS_LINEAR_PART_BYTES) != hipSuccess) {
-        (void)hipGetLastError();
+        (void)hipGetLastError();                             /* linear layers then leave K whole */
         g_linear_part = NULL;
-        return 0;
     }
     if (hipStreamCreate(&g_stream) != hipSuccess) return 0;
     /* address of the in-library scratch of iris_dev_group_norm_noalloc on this device; if the lookup

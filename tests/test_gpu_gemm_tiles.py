@@ -72,6 +72,20 @@ def test_linear_layers_that_take_it(dev, rows, k, out, bf16):
     check(got, want, k, bf16)
 
 
+def test_without_a_workspace_k_stays_whole(dev):
+    rows, k, out = 300, 4096, 640
+    x, W, want = operands(rows, k, out)
+    lib = dev.lib
+    lib.iris_hip_linear_f32.restype = C.c_int
+    lib.iris_hip_linear_f32.argtypes = [C.c_void_p] * 5 + [C.c_int] * 3
+    dy = dev.alloc(rows * out * 4)
+    assert lib.iris_hip_linear_f32(lib.iris_dev_stream(), None, dy, dev.put(x), dev.put(W), rows, k, out) == 0
+    dev.check()
+    got = dev.get(dy, (rows, out), np.float32)
+    dev.free_all()
+    check(got, want, k, False)
+
+
 @pytest.mark.parametrize("rows,k,out", [(512, 128, 19456), (449, 384, 18448), (257, 256, 20480)])
 @pytest.mark.parametrize("bf16", [False, True])
 def test_wide_tiles_of_160_columns(dev, rows, k, out, bf16):
