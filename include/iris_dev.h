@@ -124,7 +124,9 @@ void iris_dev_fill_rows(float *out, const float *row, int rows, int dim); /* out
 /* k x k convolution of a channels-last f32 image [h * width, cin] into [oh * ow, cout] with
  * zero padding of pad_before / pad_after pixels on each axis,
  *   oh = (h + pad_before + pad_after - k) / stride + 1 (same for ow),
- * w: bf16 [cout, k * k * cin] in (ky, kx, c) order, bias may be NULL (reference iris_dev.h:111-121) */
+ * w: bf16 [cout, k * k * cin] in (ky, kx, c) order, bias may be NULL (reference iris_dev.h:111-121).
+ * out may share memory with in as long as the image as bf16 (cin a multiple of 64 and cout >= 128), or else its patches, fit
+ * the 256 MB of private scratch: such a call copies them there first, and is slower than one into other memory. */
 void iris_dev_conv2d(float *out, const float *in, const uint16_t *w, const float *bias,
                      int h, int width, int cin, int cout, int k, int stride,
                      int pad_before, int pad_after);

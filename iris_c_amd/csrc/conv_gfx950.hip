@@ -308,6 +308,12 @@ k_conv_1x1(float *__restrict__ out, const float *__restrict__ in, const uint16_t
     }
 }
 
+/* workgroups per tile of channels: about one per CU in all, but no more than there are blocks of 16 x 16 pixels for */
+int one_by_one_slots(int pixels, int cout) {
+    const int slots = 256 / ((cout + C1_N - 1) / C1_N), most = (pixels + 16 * C1_WAVES - 1) / (16 * C1_WAVES);
+    return slots < 1 ? 1 : slots < most ? slots : most;
+}
+
 int launch_1x1(hipStream_t st, float *out, const float *in, const uint16_t *W, const float *bias, int pixels, int cin, int cout) {
     static bool configured = false;
     if (!configured) {
@@ -315,11 +321,7 @@ int launch_1x1(hipStream_t st, float *out, const float *in, const uint16_t *W, c
         if (e != hipSuccess) return (int)e;
         configured = true;
     }
-    /* about one workgroup per CU, but no more than there are blocks of 16 x 16 pixels for */
-    const int tiles_n = (cout + C1_N - 1) / C1_N, most = (pixels + 16 * C1_WAVES - 1) / (16 * C1_WAVES);
-    int slots = 256 / tiles_n;
-    if (slots > most) slots = most;
-    if (slots < 1) slots = 1;
+    const int tiles_n = (cout + C1_N - 1) / C1_N, slots = one_by_one_slots(pixels, cout);
     const int total = slots * tiles_n, per_xcd = (total + 7) / 8;
     hipLaunchKernelGGL(k_conv_1x1, dim3((unsigned)per_xcd * 8), dim3(64 * C1_WAVES), C1_WAVES * C1_OUT * 4 + cin * 256, st, out, in, W, bias, pixels,
                        cin, cout, tiles_n, total, per_xcd);
@@ -904,38 +906,79 @@ int launch_few_out(hipStream_t st, float *out, const float *in, const uint16_t *
 }
 
 inline bool al16(const void *p) { return ((uintptr_t)p & 15) == 0; }
+inline bool overlap(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {
+    return (uintptr_t)a < (uintptr_t)b + b_bytes && (uintptr_t)b < (uintptr_t)a + a_bytes;
+}
+
+/* five workgroups of k_conv_few_in a CU (32 KB of LDS each); a wave fetches its weights once for all its groups */
+inline unsigned few_in_columns(int groups) { return groups < 1280 * FI_WAVES ? (unsigned)(groups + FI_WAVES - 1) / FI_WAVES : 1280u; }
+
+enum Route { OTHER, FEW_IN, FEW_OUT, ONE_BY_ONE, THREE, THREE_HALF };
+
+/* Which kernel a convolution takes, host arithmetic only. All of them store results while other workgroups still read the
+ * image around them, so an output that shares memory with the image goes elsewhere: those routes copy the image first. */
+Route route(const ConvShape &s, const void *out, const void *in, const void *w) {
+    const size_t in_bytes = (size_t)s.h * s.w * s.cin * 4, out_bytes = (size_t)s.oh * s.ow * s.cout * 4;
+    if (overlap(out, out_bytes, in, in_bytes)) return OTHER;
+    if (s.k * s.k * s.cin <= 32 && (long)s.oh * s.ow <= (1L << 30)) return FEW_IN;
+    if (s.k <= FO_MAX_K && s.k * s.k * s.cout <= FO_ROWS && s.stride == 1 && (s.cin == 32 || s.cin == 64 || s.cin == 128) && al16(in) && al16(w))
+        return FEW_OUT;
+    if (s.k == 1 && s.stride == 1 && s.oh == s.h && s.ow == s.w && s.cin % 128 == 0 && s.cin <= C1_MAX_CIN && s.cout <= 2 * C1_N && al16(in) &&
+        ((uintptr_t)w & 7) == 0)
+        return ONE_BY_ONE;
+    /* a thread's byte offsets into image and weights are 32-bit */
+    const bool offsets = in_bytes < ((size_t)1 << 32) && (size_t)s.cout * 9 * s.cin * 2 < ((size_t)1 << 32);
+    if (s.k == 3 && s.stride == 1 && s.cin % 64 == 0 && s.cout <= C3_MAX_COUT && al16(in) && al16(w) && offsets) return THREE;
+    if (s.k == 3 && s.stride == 2 && s.cin % H3_C == 0 && s.cout >= 128 && s.cout <= H3_MAX_COUT && al16(in) && al16(w) && offsets) return THREE_HALF;
+    return OTHER;
+}
 
 }  // namespace
 
 extern "C" {
+
+/* plan[0] = the kernel such a convolution takes: 1 k_conv_few_in, 2 k_conv_few_out, 3 k_conv_1x1, 4 k_conv_3x3, 5 k_conv_3x3_half,
+ * 0 none of them; plan[1] = how many pieces of work its busiest wave (1, 3) or workgroup takes one after the other.
+ * No GPU needed: the addresses are only compared. */
+void iris_hip_conv2d_plan(const void *out, const void *in, const void *w, int h, int width, int cin, int cout, int k, int stride,
+                          int pad_before, int pad_after, int *plan) {
+    const int oh = (h + pad_before + pad_after - k) / stride + 1, ow = (width + pad_before + pad_after - k) / stride + 1;
+    const ConvShape s = {h, width, cin, cout, k, stride, pad_before, oh, ow};
+    const auto turns = [](long work, long takers) { return (int)((work + takers - 1) / takers); };
+    const auto tiles = [&](int ty, int tx) { return (long)((oh + ty - 1) / ty) * ((ow + tx - 1) / tx) * ((cout + C3_N - 1) / C3_N); };
+    plan[0] = route(s, out, in, w);
+    plan[1] = 1;
+    if (plan[0] == FEW_IN) {
+        const int groups = (int)(((long)oh * ow + 15) / 16);
+        plan[1] = turns(groups, (long)few_in_columns(groups) * FI_WAVES);
+    } else if (plan[0] == ONE_BY_ONE) {
+        plan[1] = turns(((long)h * width + 15) / 16, (long)one_by_one_slots(h * width, cout) * C1_WAVES);
+    } else if (plan[0] == THREE || plan[0] == THREE_HALF) {
+        plan[1] = turns((plan[0] == THREE ? tiles(C3_T, C3_T) : tiles(H3_TY, H3_TX)), 256);
+    }
+}
 
 /* The shapes these kernels take; -2, with nothing enqueued, for any other. */
 int iris_hip_conv2d_direct(void *stream, float *out, const float *in, const uint16_t *w, const float *bias, int h, int width,
                            int cin, int cout, int k, int stride, int pad_before, int oh, int ow) {
     hipStream_t st = (hipStream_t)stream;
     const ConvShape s = {h, width, cin, cout, k, stride, pad_before, oh, ow};
-    if (k * k * cin <= 32 && (long)oh * ow <= (1L << 30)) {
+    switch (route(s, out, in, w)) {
+    case FEW_IN: {
         const int groups = (int)(((long)oh * ow + 15) / 16);
-        const bool aligned = cout % 4 == 0 && al16(out);
-        /* five workgroups a CU (32 KB of LDS each); a wave fetches its weights once for all its groups */
-        const dim3 grid((unsigned)(groups < 1280 * FI_WAVES ? (groups + FI_WAVES - 1) / FI_WAVES : 1280), (unsigned)((cout + FI_COLS - 1) / FI_COLS));
-        if (aligned) hipLaunchKernelGGL(k_conv_few_in<true>, grid, dim3(64 * FI_WAVES), 0, st, out, in, w, bias, s, groups);
+        const dim3 grid(few_in_columns(groups), (unsigned)((cout + FI_COLS - 1) / FI_COLS));
+        if (cout % 4 == 0 && al16(out)) hipLaunchKernelGGL(k_conv_few_in<true>, grid, dim3(64 * FI_WAVES), 0, st, out, in, w, bias, s, groups);
         else hipLaunchKernelGGL(k_conv_few_in<false>, grid, dim3(64 * FI_WAVES), 0, st, out, in, w, bias, s, groups);
         return (int)hipGetLastError();
     }
-    if (k <= FO_MAX_K && k * k * cout <= FO_ROWS && stride == 1 && (cin == 32 || cin == 64 || cin == 128) && al16(in) && al16(w))
+    case FEW_OUT:
         return cin == 32 ? launch_few_out<1>(st, out, in, w, bias, s) : cin == 64 ? launch_few_out<2>(st, out, in, w, bias, s)
                                                                                : launch_few_out<4>(st, out, in, w, bias, s);
-    if (k == 1 && stride == 1 && oh == h && ow == width && cin % 128 == 0 && cin <= C1_MAX_CIN && cout <= 2 * C1_N && al16(in) && ((uintptr_t)w & 7) == 0)
-        return launch_1x1(st, out, in, w, bias, h * width, cin, cout);
-    /* a thread's byte offsets into image and weights are 32-bit */
-    if (k == 3 && stride == 1 && cin % 64 == 0 && cout <= C3_MAX_COUT && al16(in) && al16(w) && (size_t)h * width * cin * 4 < ((size_t)1 << 32) &&
-        (size_t)cout * 9 * cin * 2 < ((size_t)1 << 32))
-        return launch_3x3(st, out, in, w, bias, s);
-    if (k == 3 && stride == 2 && cin % H3_C == 0 && cout >= 128 && cout <= H3_MAX_COUT && al16(in) && al16(w) &&
-        (size_t)h * width * cin * 4 < ((size_t)1 << 32) && (size_t)cout * 9 * cin * 2 < ((size_t)1 << 32))
-        return launch_3x3_half(st, out, in, w, bias, s);
-    return -2;
+    case ONE_BY_ONE: return launch_1x1(st, out, in, w, bias, h * width, cin, cout);
+    case THREE: return launch_3x3(st, out, in, w, bias, s);
+    case THREE_HALF: return launch_3x3_half(st, out, in, w, bias, s);
+    default: return -2;
+    }
 }
 
 }  // extern "C"

@@ -163,6 +163,9 @@ int iris_hip_conv2d(void *stream, uint16_t *scratch, size_t scratch_bytes, float
  * enqueued. oh, ow: output size. */
 int iris_hip_conv2d_direct(void *stream, float *out, const float *in, const uint16_t *w, const float *bias, int h, int width,
                            int cin, int cout, int k, int stride, int pad_before, int oh, int ow);
+/* which of those kernels a convolution takes (0: none), host arithmetic only */
+void iris_hip_conv2d_plan(const void *out, const void *in, const void *w, int h, int width, int cin, int cout, int k, int stride,
+                          int pad_before, int pad_after, int *plan);
 
 /* Linear layer through hipBLASLt (linear_hipblaslt.cpp; the library is opened with dlopen at the
  * first call). Returns 0 when the product was enqueued, 1 when the caller must use its own

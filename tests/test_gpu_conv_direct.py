@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from gpu_harness import Dev
+from gpu_harness import Dev, ptr_add
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +69,24 @@ def test_three_by_three_stride_two(dev, orc, h, w, cin, cout, pb, pa, bias):
     """Tile edges (8 x 16 output pixels, 128 channels), one to sixteen groups of 32 input channels (odd and even numbers of them),
     padding of other widths, more tiles than workgroups."""
     conv_case(dev, orc, h, w, cin, cout, 3, 2, pb, pa, bias)
+
+
+@pytest.mark.parametrize("h,w,cin,cout,k,stride,pb,pa,shift", [
+    (40, 50, 128, 128, 3, 1, 1, 1, 0), (40, 50, 128, 256, 3, 1, 1, 1, 4096), (33, 47, 256, 128, 1, 1, 0, 0, 0), (41, 37, 128, 256, 3, 2, 0, 1, 0),
+    (60, 70, 128, 3, 3, 1, 1, 1, 0), (70, 60, 3, 128, 3, 1, 1, 1, 64), (90, 30, 64, 64, 3, 1, 1, 1, 0)])
+def test_output_in_the_image_s_own_memory(dev, orc, h, w, cin, cout, k, stride, pb, pa, shift):
+    """The result begins `shift` floats into the image: every route that such a call can take has read the image by then."""
+    rng = np.random.default_rng(h + w + cout)
+    img = rng.standard_normal((h * w, cin)).astype(np.float32)
+    wt = O.f32_to_bf16((rng.standard_normal((cout, k * k * cin)) * 0.1).astype(np.float32))
+    b = rng.standard_normal(cout).astype(np.float32)
+    want = orc.dev_conv2d(img, wt, b, h, w, k, stride, pb, pa)
+    room = np.zeros(max(img.size, shift + want.size), np.float32)
+    room[:img.size] = img.ravel()
+    mem = dev.put(room)
+    out = ptr_add(mem, 4 * shift)
+    dev.lib.iris_dev_conv2d(out, mem, dev.put(wt), dev.put(b), h, w, cin, cout, k, stride, pb, pa)
+    dev.check()
+    got = dev.get(out, want.shape, np.float32)
+    dev.free_all()
+    np.testing.assert_allclose(got, want, atol=2e-5 * np.sqrt(k * k * cin))

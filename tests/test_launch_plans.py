@@ -85,6 +85,40 @@ def test_linear_layers_of_the_models_take_the_four_wave_kernel_in_the_width_that
     assert linear_plan(512, 256, 258, 4)[0] == 2             # f32 rows of 258 columns cannot take 16-byte stores
 
 
+# ------------------------------------------------------------------ the convolutions' kernel choice
+FEW_IN, FEW_OUT, ONE_BY_ONE, THREE, THREE_HALF = 1, 2, 3, 4, 5
+
+
+@pytest.fixture(scope="module")
+def conv_plan():
+    lib = C.CDLL(iris_c_amd.LIB_PATH)
+    lib.iris_hip_conv2d_plan.argtypes = [C.c_void_p] * 3 + [C.c_int] * 8 + [C.POINTER(C.c_int)]
+    lib.iris_hip_conv2d_plan.restype = None
+
+    def call(h, w, cin, cout, k, stride=1, pb=0, pa=0, out=1 << 44, img=1 << 40, wt=1 << 46):
+        """The addresses are only compared, never read."""
+        p = (C.c_int * 2)()
+        lib.iris_hip_conv2d_plan(out, img, wt, h, w, cin, cout, k, stride, pb, pa, p)
+        return p[0]
+    return call
+
+
+@pytest.mark.parametrize("kernel,h,w,cin,cout,k,stride,pb,pa", [
+    (FEW_IN, 512, 512, 3, 128, 3, 1, 1, 1), (FEW_OUT, 512, 512, 128, 3, 3, 1, 1, 1), (ONE_BY_ONE, 512, 512, 256, 128, 1, 1, 0, 0),
+    (THREE, 256, 256, 128, 128, 3, 1, 1, 1), (THREE_HALF, 256, 256, 128, 128, 3, 2, 0, 1)])
+def test_convolutions_whose_output_shares_memory_with_the_image_take_a_route_that_copies_it_first(conv_plan, kernel, h, w, cin, cout, k,
+                                                                                                 stride, pb, pa):
+    """The kernels that read the image directly store tiles whose surroundings other workgroups have still to read."""
+    img = 1 << 40
+    oh, ow = (h + pb + pa - k) // stride + 1, (w + pb + pa - k) // stride + 1
+    in_bytes, out_bytes = h * w * cin * 4, oh * ow * cout * 4
+    call = lambda out: conv_plan(h, w, cin, cout, k, stride, pb, pa, out=out, img=img)
+    for out in (img, img + 16, img + in_bytes - 16, img - out_bytes + 16):
+        assert call(out) == 0
+    for out in (img + in_bytes, img - out_bytes, 1 << 44):
+        assert call(out) == kernel
+
+
 def test_profile_summaries_say_which_source_they_were_taken_on():
     """Every summary under profiles/ names the commit and the hash of the kernel source it was measured on, and
     bench.py can tell from the C2 counter file whether its traffic figure belongs to the kernel source in the tree."""
