@@ -91,7 +91,9 @@ void iris_dev_attention(uint16_t *out, int ldo,
 void iris_dev_f32_to_bf16(uint16_t *dst, const float *src, size_t n);
 
 /* y[rows, out] = x[rows, in] @ W[out, in]^T: bf16 inputs, f32 accumulation, f32 or bf16
- * output; all matrices contiguous (reference iris_dev.h:48-53) */
+ * output; all matrices contiguous (reference iris_dev.h:48-53). A product of few rows may be cut into ranges of `in` whose
+ * f32 partial sums pass through private memory. Under stream capture it is not, so a captured layer may be replayed on any
+ * stream, beside any other; its f32 sums are then taken in another order than the same call's outside. */
 void iris_dev_linear_f32(float *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out);
 void iris_dev_linear_bf16(uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out);
 

@@ -33,7 +33,7 @@ static const char *g_last_kernel = "none";
 #define CONV_SCRATCH_BYTES ((size_t)256 << 20)
 static uint16_t *g_conv_scratch = NULL;
 /* partial sums of linear layers whose K is cut into ranges; allocated at initialisation, so that a linear layer never
- * allocates and can be captured into a graph at its first call */
+ * allocates */
 static float *g_linear_part = NULL;
 static float *g_gn_scratch = NULL;
 static size_t g_gn_scratch_floats = 0;
@@ -467,13 +467,22 @@ static int linear_by_library(void *y, int out_bf16, const uint16_t *x, const uin
     return 1;
 }
 
+/* The workspace of the next linear layer, or NULL: K then stays whole. The stream orders the layers that share it, but a layer
+ * that is captured may be replayed on any stream, beside others: it gets none. */
+static float *linear_part(void) {
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (g_linear_part && hipStreamIsCapturing(g_stream, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone)
+        return g_linear_part;
+    return NULL;
+}
+
 void iris_dev_linear_f32(float *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out) {
     if (rows <= 0 || out <= 0) return;
     if (in <= 0) { fail(-1, "linear", "in must be positive"); return; }
     if (!need_ready("linear")) return;
     if (linear_by_library(y, 0, x, W, rows, in, out)) return;
     g_last_kernel = "linear_mfma";
-    LAUNCH("linear", iris_hip_linear_f32(g_stream, g_linear_part, y, x, W, rows, in, out));
+    LAUNCH("linear", iris_hip_linear_f32(g_stream, linear_part(), y, x, W, rows, in, out));
 }
 
 void iris_dev_linear_bf16(uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out) {
@@ -482,7 +491,7 @@ void iris_dev_linear_bf16(uint16_t *y, const uint16_t *x, const uint16_t *W, int
     if (!need_ready("linear")) return;
     if (linear_by_library(y, 1, x, W, rows, in, out)) return;
     g_last_kernel = "linear_mfma";
-    LAUNCH("linear", iris_hip_linear_bf16(g_stream, g_linear_part, y, x, W, rows, in, out));
+    LAUNCH("linear", iris_hip_linear_bf16(g_stream, linear_part(), y, x, W, rows, in, out));
 }
 
 void iris_dev_linear_bf16_qknorm(uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out,
@@ -499,7 +508,7 @@ void iris_dev_linear_bf16_qknorm(uint16_t *y, const uint16_t *x, const uint16_t 
     int one_launch = head_dim == 128 && q_heads + k_heads > 0 &&
                      (g_linear_backend != 2 || !iris_lt_available() || in % 8 != 0);
     if (one_launch) {
-        int err = iris_hip_linear_bf16_qknorm(g_stream, g_linear_part, y, x, W, rows, in, out, q_heads * 128, k_heads * 128, wq, wk,
+        int err = iris_hip_linear_bf16_qknorm(g_stream, linear_part(), y, x, W, rows, in, out, q_heads * 128, k_heads * 128, wq, wk,
                                               rope_cos, rope_sin, eps, split_half != 0);
         if (err == 0) { g_last_kernel = "linear_mfma_qknorm"; return; }
         if (err != -2) { check((hipError_t)err, "linear_qknorm launch"); return; }

@@ -26,12 +26,19 @@ class Graphs:
         self.rt.hipGraphLaunch.argtypes = [_vp, _vp]
         self.rt.hipGraphExecDestroy.argtypes = [_vp]
         self.rt.hipGraphDestroy.argtypes = [_vp]
+        self.rt.hipGraphGetNodes.argtypes = [_vp, _vp, C.POINTER(C.c_size_t)]
+        self.rt.hipStreamCreate.argtypes = [C.POINTER(_vp)]
+        self.rt.hipStreamSynchronize.argtypes = [_vp]
+        self.rt.hipStreamDestroy.argtypes = [_vp]
 
     def capture(self, stream, fn):
         assert self.rt.hipStreamBeginCapture(stream, 0) == 0          # hipStreamCaptureModeGlobal
         fn()
         graph, run = _vp(), _vp()
         assert self.rt.hipStreamEndCapture(stream, C.byref(graph)) == 0 and graph
+        nodes = C.c_size_t()
+        assert self.rt.hipGraphGetNodes(graph, None, C.byref(nodes)) == 0
+        self.nodes = nodes.value
         assert self.rt.hipGraphInstantiate(C.byref(run), graph, None, None, 0) == 0
         self.rt.hipGraphDestroy(graph)
         return run
@@ -184,4 +191,55 @@ def test_head_dim_512_attention_with_key_ranges_replayed_from_a_graph(causal_and
         lib.iris_dev_sync()
         assert np.array_equal(dev.get(out, (seq, hd), np.uint16), want), f"replay {replay}"
     g.rt.hipGraphExecDestroy(run)
+    dev.free_all()
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+def test_captured_linear_layer_uses_no_shared_memory(bf16):
+    """300 x 4096 -> 640 is cut into ranges of K, whose partial sums share the library's workspace in stream order. Captured,
+    the layer is one kernel on its own operands, so its replays on another stream and eager layers that use the
+    workspace meanwhile both give their results. The replay sums K in another order: f32 rounding apart from the eager call."""
+    import oracle as O
+    dev, g = Dev(), Graphs()
+    lib, stream = dev.lib, _vp(dev.lib.iris_dev_stream())
+    rows, k, out = 300, 4096, 640
+    plan = (C.c_int * 2)()
+    lib.iris_hip_linear_plan(rows, k, out, 2 if bf16 else 4, plan)
+    assert plan[0] == 4 and plan[1] > 1
+    rng = np.random.default_rng(8)
+    x = O.f32_to_bf16(rng.standard_normal((rows, k)).astype(np.float32))
+    weights = [O.f32_to_bf16((rng.standard_normal((out, k)) * 0.05).astype(np.float32)) for _ in range(2)]
+    want = [O.bf16_to_f32(x).astype(np.float64) @ O.bf16_to_f32(w).astype(np.float64).T for w in weights]
+    dx, (w1, w2) = dev.put(x), [dev.put(w) for w in weights]
+    size = 2 if bf16 else 4
+    captured, eager = dev.alloc(rows * out * size), dev.alloc(rows * out * size)
+    layer = lib.iris_dev_linear_bf16 if bf16 else lib.iris_dev_linear_f32
+
+    def check(ptr, w):
+        got = dev.get(ptr, (rows, out), np.uint16 if bf16 else np.float32)
+        got = O.bf16_to_f32(got) if bf16 else got
+        # f32 sums of 4096 products of size 0.05, and the rounding to bf16
+        assert (np.abs(got - want[w]) <= 2e-5 * np.sqrt(k) * 0.05 + (np.abs(want[w]) * 2.0 ** -8 * 1.01 if bf16 else 0.0)).all()
+
+    layer(eager, dx, w2, rows, k, out)
+    run = g.capture(stream, lambda: layer(captured, dx, w1, rows, k, out))
+    assert g.nodes == 1
+    dev.check()
+    lib.iris_dev_sync()
+    other = _vp()
+    assert g.rt.hipStreamCreate(C.byref(other)) == 0
+    junk = np.full(rows * out * size // 2, 0x7fc0, np.uint16)
+    for replay in range(4):
+        for p in (captured, eager):
+            lib.iris_dev_upload(p, junk.ctypes.data_as(_vp), junk.nbytes)
+        for _ in range(8):
+            assert g.rt.hipGraphLaunch(run, other) == 0
+            layer(eager, dx, w2, rows, k, out)
+        assert g.rt.hipStreamSynchronize(other) == 0
+        lib.iris_dev_sync()
+        dev.check()
+        check(captured, 0)
+        check(eager, 1)
+    g.rt.hipGraphExecDestroy(run)
+    g.rt.hipStreamDestroy(other)
     dev.free_all()
