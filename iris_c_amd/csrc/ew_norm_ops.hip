@@ -118,31 +118,38 @@ k_swiglu(uint16_t *__restrict__ out, int ldo, const uint16_t *__restrict__ gate,
     }
 }
 
-/* nearest-neighbour 2x upsampling of a channels-last image: a thread reads VEC channels of an input pixel once and
- * stores them to the four output pixels (one thread per
- * output: 65 us for 256 x 256 x 256, so 50). */
+/* nearest-neighbour 2x upsampling of a channels-last image: a thread reads the VEC channels under an output column and
+ * stores them to both output rows, so that a wave's store is one run of memory whatever the channels, and the second read
+ * of a pixel comes from the cache. Bound by the stores. Against a thread per output value, and one per input value with
+ * four stores (runs of VEC channels: slow where they are all of a pixel), us: 512 x 512 x 4 5.0, 6.0, now 4.75; x 8 7.9, 9.3,
+ * 7.4; 256 x 256 x 12 4.35, 5.0, 4.1; 512 x 512 x 128 132, 120, 110; 1024 x 1024 x 128 516, 476, 437 (6.1 TB/s). */
 template <int VEC>
 __global__ void __launch_bounds__(EW_THREADS)
 k_upsample2x(float *__restrict__ out, const float *__restrict__ in, int w, int c, size_t n) {
-    const size_t i = (size_t)blockIdx.x * EW_THREADS + threadIdx.x;              /* which VEC channels of the input */
+    const size_t i = (size_t)blockIdx.x * EW_THREADS + threadIdx.x;              /* which VEC channels of a row pair of outputs */
     if (i >= n) return;
     const unsigned per_pixel = (unsigned)c / VEC;
-    size_t p;
-    unsigned y;
-    if (n >> 32 == 0) { p = (unsigned)i / per_pixel; y = (unsigned)p / (unsigned)w; }     /* 32-bit divisions where they do */
-    else { p = i / per_pixel; y = (unsigned)(p / (unsigned)w); }
-    const unsigned ch = (unsigned)(i - p * per_pixel) * VEC, x = (unsigned)(p - (size_t)y * w);
-    const size_t row = (size_t)2 * w * c;
-    float *dst = out + (size_t)(2 * y) * row + (size_t)(2 * x) * c + ch;
-    if (VEC == 4) {
-        const float4 v = *reinterpret_cast<const float4 *>(in + i * VEC);
-        *reinterpret_cast<float4 *>(dst) = v;
-        *reinterpret_cast<float4 *>(dst + c) = v;
-        *reinterpret_cast<float4 *>(dst + row) = v;
-        *reinterpret_cast<float4 *>(dst + row + c) = v;
+    const size_t per_row = (size_t)2 * w * per_pixel;
+    size_t y, r, x;
+    if (n >> 32 == 0) {                                        /* 32-bit divisions where they do */
+        y = (unsigned)i / (unsigned)per_row;
+        r = (unsigned)i - (unsigned)y * (unsigned)per_row;
+        x = (unsigned)r / per_pixel;
     } else {
-        const float v = in[i];
-        dst[0] = v; dst[c] = v; dst[row] = v; dst[row + c] = v;
+        y = i / per_row;
+        r = i - y * per_row;
+        x = r / per_pixel;
+    }
+    const float *src = in + (y * w + x / 2) * c + (r - x * per_pixel) * VEC;
+    float *dst = out + (2 * y * per_row + r) * VEC;
+    if (VEC == 4) {
+        const float4 v = *reinterpret_cast<const float4 *>(src);
+        *reinterpret_cast<float4 *>(dst) = v;
+        *reinterpret_cast<float4 *>(dst + per_row * VEC) = v;
+    } else {
+        const float v = *src;
+        dst[0] = v;
+        dst[per_row] = v;
     }
 }
 
@@ -516,7 +523,7 @@ int iris_hip_swiglu(void *stream, uint16_t *out, int ldo, const uint16_t *gate, 
 }
 
 int iris_hip_upsample2x(void *stream, float *out, const float *in, int h, int width, int c) {
-    const size_t n = (size_t)h * width * c;
+    const size_t n = (size_t)2 * h * width * c;                /* values of the upper output rows */
     if (!n) return 0;
     hipStream_t st = (hipStream_t)stream;
     if (al16(out) && al16(in) && c % 4 == 0)
