@@ -171,16 +171,11 @@ __device__ __forceinline__ float block_sum(float v, float *sh) {
 }
 
 enum NormKind { LAYER_NORM_MOD, RMS_NORM_MOD, RMS_NORM_RESIDUAL };
-constexpr int ROW_VECS = 4;           /* float4 per thread kept in registers: rows up to 4096 floats */
-
-/* TPR threads per row: a workgroup of 256, or a wave for many rows of up to 1024 floats. CACHE: dim % 4 == 0, dim <= 4096,
- * 16-byte aligned rows -> the row stays in registers between the statistics and the write, and everything the write needs is
- * requested before the first sum is waited for; otherwise it is read again. p0/p1 are (shift, scale) for LayerNorm,
- * (w, scale) for RMSNorm, (w, gate) for the residual form; out_bf is unused by the latter.
- * A wave per row of thousands of floats leaves a short sequence with few waves of long chains, and a long one with a single generation
- * of waves that first all read and then all write: 4608 x 3072 LayerNorm 23.1 us, now 18.8;
- * 512 x 2560 RMSNorm 7.2 us, now 5.3; 512 x 3072 LayerNorm 9.7 us, now 5.1. */
-template <int KIND, bool CACHE, int TPR>
+/* TPR threads per row: a workgroup of 256, or a wave. VECS > 0: dim % 4 == 0, dim <= 4 * TPR * VECS, 16-byte aligned rows -> the
+ * row stays in registers between the statistics and the write; EARLY: and everything the write needs is requested
+ * before the first sum is waited for. VECS = 0: the row is read again. p0/p1 are (shift, scale) for LayerNorm,
+ * (w, scale) for RMSNorm, (w, gate) for the residual form; out_bf is unused by the latter. */
+template <int KIND, int TPR, int VECS, bool EARLY>
 __global__ void __launch_bounds__(ROW_THREADS)
 k_row_norm(uint16_t *__restrict__ out_bf, float *__restrict__ xres, const float *__restrict__ src,
            const float *__restrict__ p0, const float *__restrict__ p1, int rows, int dim, float eps, unsigned grid_x) {
@@ -192,28 +187,32 @@ k_row_norm(uint16_t *__restrict__ out_bf, float *__restrict__ xres, const float 
     const size_t row_off = (size_t)row * dim;
     const float *xr = src + row_off;
     const int nvec = dim >> 2;
-    float4 keep[ROW_VECS], pa[ROW_VECS], pb[ROW_VECS], res[ROW_VECS];
+    constexpr bool CACHE = VECS > 0;
+    constexpr int N = CACHE ? VECS : 1;
+    float4 keep[N], pa[N], pb[N], res[N];
     const float *pa_src = KIND == LAYER_NORM_MOD ? p1 : p0, *pb_src = KIND == LAYER_NORM_MOD ? p0 : p1;   /* scale | w, shift | scale | gate */
 
     float s = 0.0f;
     if (CACHE) {
 #pragma unroll
-        for (int j = 0; j < ROW_VECS; j++) {
+        for (int j = 0; j < VECS; j++) {
             const int v = tid + j * TPR;
             keep[j] = v < nvec ? *reinterpret_cast<const float4 *>(xr + 4 * v) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         }
+        if (EARLY) {
 #pragma unroll
-        for (int j = 0; j < ROW_VECS; j++) {
-            const int v = tid + j * TPR;
-            pa[j] = pb[j] = res[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (v < nvec) {
-                if (pa_src) pa[j] = *reinterpret_cast<const float4 *>(pa_src + 4 * v);
-                if (pb_src) pb[j] = *reinterpret_cast<const float4 *>(pb_src + 4 * v);
-                if (KIND == RMS_NORM_RESIDUAL) res[j] = *reinterpret_cast<const float4 *>(xres + row_off + 4 * v);
+            for (int j = 0; j < VECS; j++) {
+                const int v = tid + j * TPR;
+                pa[j] = pb[j] = res[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                if (v < nvec) {
+                    if (pa_src) pa[j] = *reinterpret_cast<const float4 *>(pa_src + 4 * v);
+                    if (pb_src) pb[j] = *reinterpret_cast<const float4 *>(pb_src + 4 * v);
+                    if (KIND == RMS_NORM_RESIDUAL) res[j] = *reinterpret_cast<const float4 *>(xres + row_off + 4 * v);
+                }
             }
         }
 #pragma unroll
-        for (int j = 0; j < ROW_VECS; j++)
+        for (int j = 0; j < VECS; j++)
             s += KIND == LAYER_NORM_MOD ? (keep[j].x + keep[j].y) + (keep[j].z + keep[j].w)
                                         : (keep[j].x * keep[j].x + keep[j].y * keep[j].y) + (keep[j].z * keep[j].z + keep[j].w * keep[j].w);
     } else {
@@ -226,7 +225,7 @@ k_row_norm(uint16_t *__restrict__ out_bf, float *__restrict__ xres, const float 
         float v = 0.0f;
         if (CACHE) {
 #pragma unroll
-            for (int j = 0; j < ROW_VECS; j++)
+            for (int j = 0; j < VECS; j++)
                 if (tid + j * TPR < nvec) {
                     const float a = keep[j].x - mean, b = keep[j].y - mean, c = keep[j].z - mean, d = keep[j].w - mean;
                     v += (a * a + b * b) + (c * c + d * d);
@@ -241,9 +240,14 @@ k_row_norm(uint16_t *__restrict__ out_bf, float *__restrict__ xres, const float 
 
     if (CACHE) {
 #pragma unroll
-        for (int j = 0; j < ROW_VECS; j++) {
+        for (int j = 0; j < VECS; j++) {
             const int v = tid + j * TPR;
             if (v >= nvec) continue;
+            if (!EARLY) {                                       /* without a branch: an absent operand reads the row instead */
+                pa[j] = *reinterpret_cast<const float4 *>((pa_src ? pa_src : xr) + 4 * v);
+                pb[j] = *reinterpret_cast<const float4 *>((pb_src ? pb_src : xr) + 4 * v);
+                if (KIND == RMS_NORM_RESIDUAL) res[j] = *reinterpret_cast<const float4 *>(xres + row_off + 4 * v);
+            }
             const float xin[4] = {keep[j].x, keep[j].y, keep[j].z, keep[j].w};
             const float av[4] = {pa[j].x, pa[j].y, pa[j].z, pa[j].w}, bv[4] = {pb[j].x, pb[j].y, pb[j].z, pb[j].w};
             float r[4];
@@ -286,23 +290,42 @@ k_row_norm(uint16_t *__restrict__ out_bf, float *__restrict__ xres, const float 
     }
 }
 
+enum RowRoute { ROW_WORKGROUP, ROW_WORKGROUP_REREAD, ROW_WAVE, ROW_WAVE_2048, ROW_WAVE_4096, ROW_WAVE_REREAD };
+
+/* A workgroup per row until the chip is full of them (1280 - 1536 rows at a time), then a wave per row as long as a row is short
+ * enough for one: many rows pay for two barriers each what few rows gain from short chains. us, workgroup / wave:
+ *   LayerNorm  1000 x 1024 4.05 / 4.05, 1800 x 1024 4.97 / 4.07, 3000 x 1536 7.1 / 5.7, 3000 x 2048 7.8 / 6.9, 3000 x 2560 9.3 / 9.7;
+ *   RMSNorm    3000 x 1024 5.1 / 3.8, 12800 x 512 12.4 / 6.4, 3000 x 2048 6.2 / 5.8, 3000 x 2560 7.6 / 9.4;
+ *   residual   1500 x 512 4.7 / 4.0, 12800 x 1152 34.4 / 28.7, 3000 x 1536 12.1 / 11.7, 12800 x 2048 48.2 / 47.7, 2300 x 2048 11.2 / 13.1.
+ * Tens of thousands of longer LayerNorm rows (they come from HBM) are 5 - 10 % faster in waves again: 60000 x 4096 290 / 265. */
+RowRoute row_route(int kind, int rows, int dim, bool aligned) {
+    const bool far = kind == LAYER_NORM_MOD && rows >= 32768;
+    if (!aligned || dim % 4 || dim > 4096) return (dim <= 1024 && rows >= 2048) || far ? ROW_WAVE_REREAD : ROW_WORKGROUP_REREAD;
+    if (rows > 1280 && dim <= 1024) return ROW_WAVE;
+    if (rows > 1280 && dim <= (kind == RMS_NORM_RESIDUAL ? 1536 : 2048)) return ROW_WAVE_2048;
+    return far ? ROW_WAVE_4096 : ROW_WORKGROUP;
+}
+
 template <int KIND>
 int launch_row_norm(hipStream_t st, uint16_t *out_bf, float *xres, const float *src, const float *p0,
                     const float *p1, int rows, int dim, float eps) {
     if (rows <= 0 || dim <= 0) return 0;
-    const bool cache = dim % 4 == 0 && dim <= 4 * ROW_THREADS * ROW_VECS && al16(src) && al16(xres) && al16(p0) && al16(p1) &&
-                       ((uintptr_t)out_bf & 7) == 0;
-    /* a wave per row where rows are short and enough of them to fill the chip: 100000 x 128 RMSNorm 69 us with a workgroup
-     * each, 23 so, 20000 x 1024 LayerNorm 26 / 19; 300 x 1024 3.8 / 4.4 */
-    const bool wave = dim <= 4 * 64 * ROW_VECS && rows >= 2048;
-    const unsigned blocks = wave ? ((unsigned)rows + ROW_THREADS / 64 - 1) / (ROW_THREADS / 64) : (unsigned)rows;
+    const RowRoute route = row_route(KIND, rows, dim, al16(src) && al16(xres) && al16(p0) && al16(p1) && ((uintptr_t)out_bf & 7) == 0);
+    const unsigned blocks = route >= ROW_WAVE ? ((unsigned)rows + ROW_THREADS / 64 - 1) / (ROW_THREADS / 64) : (unsigned)rows;
     /* a grid dimension holds less than 2^32 threads */
     const unsigned gx = blocks < 1u << 20 ? blocks : 1u << 20;
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(gx, (blocks + gx - 1) / gx), dim3(ROW_THREADS), 0, st, out_bf, xres, src, p0, p1, rows, dim, eps, gx);
     };
-    if (wave) cache ? go(k_row_norm<KIND, true, 64>) : go(k_row_norm<KIND, false, 64>);
-    else cache ? go(k_row_norm<KIND, true, ROW_THREADS>) : go(k_row_norm<KIND, false, ROW_THREADS>);
+    switch (route) {
+    case ROW_WORKGROUP: go(k_row_norm<KIND, ROW_THREADS, 4, true>); break;
+    case ROW_WORKGROUP_REREAD: go(k_row_norm<KIND, ROW_THREADS, 0, false>); break;
+    case ROW_WAVE: go(k_row_norm<KIND, 64, 4, true>); break;
+    /* with the residual's rows too there are not enough registers to ask for everything early */
+    case ROW_WAVE_2048: go(k_row_norm<KIND, 64, 8, KIND != RMS_NORM_RESIDUAL>); break;
+    case ROW_WAVE_4096: go(k_row_norm<LAYER_NORM_MOD, 64, 16, false>); break;
+    case ROW_WAVE_REREAD: go(k_row_norm<KIND, 64, 0, false>); break;
+    }
     return (int)hipGetLastError();
 }
 
@@ -521,6 +544,10 @@ int iris_hip_swiglu(void *stream, uint16_t *out, int ldo, const uint16_t *gate, 
         hipLaunchKernelGGL(k_swiglu<1>, dim3(blocks_for(n, EW_THREADS)), dim3(EW_THREADS), 0, st, out, ldo, gate, up, ldi, cols, n);
     return (int)hipGetLastError();
 }
+
+/* How a row norm is dealt out, host arithmetic only: kind 0 LayerNorm, 1 RMSNorm, 2 its residual form; 0 a workgroup per row that
+ * keeps the row in registers, 1 one that reads it again, 2 - 4 a wave that keeps up to 1024, 2048, 4096 floats, 5 one that reads again. */
+int iris_hip_row_norm_plan(int kind, int rows, int dim, int aligned) { return row_route(kind, rows, dim, aligned != 0); }
 
 int iris_hip_upsample2x(void *stream, float *out, const float *in, int h, int width, int c) {
     const size_t n = (size_t)2 * h * width * c;                /* values of the upper output rows */

@@ -110,6 +110,7 @@ int iris_hip_fill_rows(void *stream, float *out, const float *row, int rows, int
 int iris_hip_residual(void *stream, float *x, const float *a, const float *gate, int rows, int dim);
 int iris_hip_swiglu(void *stream, uint16_t *out, int ldo, const uint16_t *gate, const uint16_t *up,
                     int ldi, int rows, int cols);
+int iris_hip_row_norm_plan(int kind, int rows, int dim, int aligned);
 int iris_hip_upsample2x(void *stream, float *out, const float *in, int h, int width, int c);
 int iris_hip_layer_norm_mod(void *stream, uint16_t *out, const float *x, const float *shift,
                             const float *scale, int rows, int dim, float eps);

@@ -1,5 +1,5 @@
-"""Row norms at both sides of the choice between a wave and a workgroup per row (1024 floats, 2048 rows), with and without the
-row kept in registers, against the CPU oracle (bf16 results: one unit in the last place, from the order of the f32 sums)."""
+"""Row norms at both sides of the choices between a wave and a workgroup per row, with and without the row kept in
+registers, against the CPU oracle (bf16 results: one unit in the last place, from the order of the f32 sums)."""
 import numpy as np
 import pytest
 
@@ -16,6 +16,18 @@ def dev():
 
 @pytest.mark.parametrize("rows,dim", [(2047, 64), (2048, 64), (2049, 128), (2051, 1024), (2048, 1028), (2049, 33), (2050, 1023), (3, 1024)])
 def test_both_routes(dev, orc, rows, dim):
+    compare(dev, orc, rows, dim)
+
+
+# the last rows of a workgroup's and the first of a wave's, lengths that end inside and at the end of what a wave keeps, and as many
+# long rows as LayerNorm deals out in waves again
+@pytest.mark.parametrize("rows,dim", [(1280, 1024), (1281, 1024), (1283, 64), (1281, 1028), (1285, 1536), (1282, 1540), (1283, 2048), (1281, 2052),
+                                      (32768, 2052), (32769, 1030)])
+def test_edges_of_the_routes(dev, orc, rows, dim):
+    compare(dev, orc, rows, dim)
+
+
+def compare(dev, orc, rows, dim):
     rng = np.random.default_rng(rows + dim)
     x = (2 * rng.standard_normal((rows, dim)) + 0.7).astype(np.float32)
     p = [(0.3 * rng.standard_normal(dim) + at).astype(np.float32) for at in (0.0, 0.0, 1.0)]

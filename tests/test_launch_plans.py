@@ -119,6 +119,24 @@ def test_convolutions_whose_output_shares_memory_with_the_image_take_a_route_tha
         assert call(out) == kernel
 
 
+# ------------------------------------------------------------------ row norms
+def test_row_norms_take_a_wave_per_row_where_rows_are_many_and_short_and_a_workgroup_elsewhere():
+    lib = C.CDLL(iris_c_amd.LIB_PATH)
+    layer, rms, residual = 0, 1, 2
+    workgroup, workgroup_reread, wave, wave_2048, wave_4096, wave_reread = range(6)
+    plan = lambda kind, rows, dim, aligned=1: lib.iris_hip_row_norm_plan(kind, rows, dim, aligned)
+    for kind in (layer, rms, residual):
+        assert plan(kind, 1280, 64) == plan(kind, 1, 4096) == plan(kind, 20000, 3072) == workgroup
+        assert plan(kind, 1281, 64) == plan(kind, 2047, 1024) == wave
+        assert plan(kind, 3000, 1028) == plan(kind, 12800, 1536) == wave_2048
+        assert plan(kind, 3000, 2052) == plan(kind, 4608, 3072) == workgroup
+        assert plan(kind, 2048, 1023) == plan(kind, 2048, 1024, 0) == wave_reread
+        assert plan(kind, 2047, 1023) == plan(kind, 4608, 3071) == plan(kind, 4608, 3072, 0) == plan(kind, 512, 5120) == workgroup_reread
+    assert plan(layer, 3000, 2048) == plan(rms, 3000, 2048) == wave_2048 and plan(residual, 3000, 1540) == workgroup
+    assert plan(layer, 32768, 2052) == wave_4096 and plan(rms, 32768, 2052) == plan(residual, 32768, 2052) == workgroup
+    assert plan(layer, 32768, 5120) == wave_reread and plan(rms, 32768, 5120) == workgroup_reread
+
+
 def test_profile_summaries_say_which_source_they_were_taken_on():
     """Every summary under profiles/ names the commit and the hash of the kernel source it was measured on, and
     bench.py can tell from the C2 counter file whether its traffic figure belongs to the kernel source in the tree."""
