@@ -915,15 +915,31 @@ inline unsigned few_in_columns(int groups) { return groups < 1280 * FI_WAVES ? (
 
 enum Route { OTHER, FEW_IN, FEW_OUT, ONE_BY_ONE, THREE, THREE_HALF };
 
+/* With 1 x 1 there are no taps to save, and a thread adds up and stores all the channels of its pixel: k_conv_1x1 or a copy are
+ * faster from 5 channels on (128 -> 16 over 512 x 512 41 us against 33 in k_conv_1x1; 64 -> 28 over 128 x 128 13.5 / 10.2), with 64
+ * input channels from 17 (64 -> 16 9.9 / 10.0). And where an image is not as wide as a tile, as one of width 1 that a
+ * caller makes of all its pixels, most of a tile is empty: what fits two workgroups a CU is still faster so, beyond that the
+ * estimates decide (a round of 512 tiles takes 2.7 us + 0.036 per input channel; 65536 x 1, 128 -> 3, 1 x 1 45 us / 12). */
+bool few_out_pays(const ConvShape &s, long out_pixels, float copied_us) {
+    if (s.k == 1 && s.cout > (s.cin <= 64 ? 16 : 4)) return false;
+    const long tiles = (long)((s.oh + FO_TY - 1) / FO_TY) * ((s.ow + FO_TX - 1) / FO_TX);
+    if (tiles <= 512 || tiles * FO_TX * FO_TY <= 2 * out_pixels) return true;
+    return 3.0f + (float)((tiles + 511) / 512) * (2.7f + 0.036f * (float)s.cin) < copied_us;
+}
+
 /* Which kernel a convolution takes, host arithmetic only. All of them store results while other workgroups still read the
  * image around them, so an output that shares memory with the image goes elsewhere: those routes copy the image first. */
 Route route(const ConvShape &s, const void *out, const void *in, const void *w) {
     const size_t in_bytes = (size_t)s.h * s.w * s.cin * 4, out_bytes = (size_t)s.oh * s.ow * s.cout * 4;
     if (overlap(out, out_bytes, in, in_bytes)) return OTHER;
     if (s.k * s.k * s.cin <= 32 && (long)s.oh * s.ow <= (1L << 30)) return FEW_IN;
-    if (s.k <= FO_MAX_K && s.k * s.k * s.cout <= FO_ROWS && s.stride == 1 && (s.cin == 32 || s.cin == 64 || s.cin == 128) && al16(in) && al16(w))
+    const bool plain = s.k == 1 && s.stride == 1 && s.oh == s.h && s.ow == s.w;
+    const long out_pixels = (long)s.oh * s.ow;
+    const float copied_us = iris_hip_conv2d_copied_us((long)s.h * s.w, out_pixels, s.cin, s.cout, s.k, plain);
+    if (s.k <= FO_MAX_K && s.k * s.k * s.cout <= FO_ROWS && s.stride == 1 && (s.cin == 32 || s.cin == 64 || s.cin == 128) && al16(in) && al16(w) &&
+        few_out_pays(s, out_pixels, copied_us))
         return FEW_OUT;
-    if (s.k == 1 && s.stride == 1 && s.oh == s.h && s.ow == s.w && s.cin % 128 == 0 && s.cin <= C1_MAX_CIN && s.cout <= 2 * C1_N && al16(in) &&
+    if (plain && s.cin % 128 == 0 && s.cin <= C1_MAX_CIN && s.cout <= 2 * C1_N && al16(in) &&
         ((uintptr_t)w & 7) == 0)
         return ONE_BY_ONE;
     /* a thread's byte offsets into image and weights are 32-bit */

@@ -776,7 +776,7 @@ static int wide_width(int M, int N) {
  * 512 x 9728 -> 2560 38 against 138, 512 x 3072 -> 9216 38 / 50, 1000 x 12288 -> 3072 76 / 175, 2115 x 9216 -> 3072 104 / 122,
  * 2115 x 3072 -> 9216 100 / 104; and where 3 is taken 512 x 3072 -> 18432 79 / 58, 1000 x 3072 -> 27648 156 / 136,
  * 2115 x 3072 -> 18432 209 / 194, 2912 x 12288 -> 4096 265 / 224. */
-struct GemmPlan { int kernel, na, splits; };
+struct GemmPlan { int kernel, na, splits; float us; };       /* us: estimate, where there is one */
 static GemmPlan plan_gemm(int M, int N, int K, int out_size, bool operands_aligned16, bool out_aligned16, size_t part_bytes) {
     int shape = 0, splits = 1;
     const float tiles_us = operands_aligned16 && out_aligned16 ? iris_hip_gemm_tiles_plan(M, N, K, out_size, part_bytes, &shape, &splits) : -1.0f;
@@ -785,14 +785,14 @@ static GemmPlan plan_gemm(int M, int N, int K, int out_size, bool operands_align
             const int na = wide_width(M, N);
             const long wgs = (long)((M + DT - 1) / DT) * ((N + 32 * na - 1) / (32 * na)), rounds = (wgs + 255) / 256;
             const float us = 4.0f + (float)rounds * ((float)(K / TK) * (wgs <= 128 ? 0.145f : 0.175f) * (float)na + 4.0f);
-            if (tiles_us < 0.0f || tiles_us >= us) return {3, na, 1};
-            return {4, shape, splits};
+            if (tiles_us < 0.0f || tiles_us >= us) return {3, na, 1, us};
+            return {4, shape, splits, tiles_us};
         }
-        if (tiles_us < 0.0f) return {2, 8, 1};
+        if (tiles_us < 0.0f) return {2, 8, 1, 0.0f};
     }
-    if (tiles_us >= 0.0f) return {4, shape, splits};
-    if (K > 0 && K % 8 == 0 && operands_aligned16) return {1, 0, 1};
-    return {0, 0, 1};
+    if (tiles_us >= 0.0f) return {4, shape, splits, tiles_us};
+    if (K > 0 && K % 8 == 0 && operands_aligned16) return {1, 0, 1, 0.0f};
+    return {0, 0, 1, 0.0f};
 }
 
 __global__ void __launch_bounds__(256)
@@ -916,6 +916,24 @@ int iris_hip_linear_bf16_qknorm(void *stream, float *part, uint16_t *y, const ui
     if (e) return e;
     return qh ? iris_hip_norm_rope_hd128(stream, y, kh ? y + q_cols : nullptr, N, wq, wk, rope_cos, rope_sin, M, qh, kh, eps, split_half)
               : iris_hip_norm_rope_hd128(stream, y, nullptr, N, wk, nullptr, rope_cos, rope_sin, M, kh, 0, eps, split_half);
+}
+
+/* About what a convolution takes in us through the routes of iris_hip_conv2d below that copy the image, host arithmetic only, for
+ * the choice between them and the kernels of conv_gfx950.hip. Measured, us, in brackets the estimate: 4096 pixels in a column,
+ * 512 -> 512, 3 x 3 114 (115); 20000, 128 -> 128 30 (31); 3 x 3, 1024 -> 1024, 3000 x 2 221 (219); 1 x 1, 256 -> 128, 9216 pixels
+ * 16 (15); gathered: 65536 x 1, 32 -> 3, 3 x 3 27 (25), 20000 x 1, 512 -> 64, 3 x 3 102 (123), 1 x 1, 384 -> 100, 9216 19 (17). */
+float iris_hip_conv2d_copied_us(long in_pixels, long out_pixels, int cin, int cout, int k, int plain) {
+    const float copy = 1.1e-6f * (float)in_pixels * (float)cin, nk = (float)(k * k) * (float)cin / TK;
+    if (plain && out_pixels < (1L << 31)) {
+        const GemmPlan p = plan_gemm((int)out_pixels, cout, cin, 4, true, true, 0);
+        if (p.kernel == 4) return copy + p.us;
+    }
+    if (cin % TK == 0 && cout >= 128) {
+        const int wide = cout >= 256;
+        const long tiles = ((out_pixels + 255) / 256) * ((cout + (wide ? 255 : 127)) / (wide ? 256 : 128)), rounds = (tiles + 255) / 256;
+        return 4.0f + copy + (float)rounds * (nk * (!wide ? 1.1f : tiles > 192 ? 1.6f : 1.42f) + (wide ? 8.0f : 4.0f));
+    }
+    return 8.2f + 0.7f * nk + (k == 1 ? 1.0e-6f : 0.7e-6f) * (float)out_pixels * (float)(k * k) * (float)cin;
 }
 
 /* Zeroes the first IRIS_CONV_ZERO_BYTES of a freshly allocated convolution scratch buffer: the page that taps

@@ -164,6 +164,8 @@ int iris_hip_conv2d(void *stream, uint16_t *scratch, size_t scratch_bytes, float
  * enqueued. oh, ow: output size. */
 int iris_hip_conv2d_direct(void *stream, float *out, const float *in, const uint16_t *w, const float *bias, int h, int width,
                            int cin, int cout, int k, int stride, int pad_before, int oh, int ow);
+/* an estimate of its other routes (those that copy the image first); plain: 1 x 1, no stride and no padding */
+float iris_hip_conv2d_copied_us(long in_pixels, long out_pixels, int cin, int cout, int k, int plain);
 /* which of those kernels a convolution takes (0: none), host arithmetic only */
 void iris_hip_conv2d_plan(const void *out, const void *in, const void *w, int h, int width, int cin, int cout, int k, int stride,
                           int pad_before, int pad_after, int *plan);

@@ -45,6 +45,11 @@ def test_few_output_channels(dev, orc, h, w, cin, cout, k, stride, pb, pa, bias)
     conv_case(dev, orc, h, w, cin, cout, k, stride, pb, pa, bias)
 
 
+@pytest.mark.parametrize("h,w,cin,cout,k,pad", [(30000, 1, 128, 3, 1, 0), (1, 30000, 64, 3, 1, 0), (20000, 1, 32, 3, 3, 1), (3, 9000, 128, 3, 3, 1)])
+def test_few_output_channels_of_images_thinner_than_a_tile(dev, orc, h, w, cin, cout, k, pad):
+    conv_case(dev, orc, h, w, cin, cout, k, 1, pad, pad)
+
+
 @pytest.mark.parametrize("h,w,cin,cout,pb,pa,bias", [
     (1, 1, 64, 128, 1, 1, True), (16, 16, 64, 128, 1, 1, True), (17, 15, 128, 128, 1, 1, False), (33, 47, 192, 256, 1, 1, True),
     (18, 19, 64, 130, 0, 0, True), (3, 34, 320, 37, 2, 1, True), (20, 5, 512, 512, 1, 1, True), (16, 33, 256, 3, 0, 1, False)])

@@ -119,6 +119,16 @@ def test_convolutions_whose_output_shares_memory_with_the_image_take_a_route_tha
         assert call(out) == kernel
 
 
+def test_few_output_channels_of_a_flat_image(conv_plan):
+    """1 x 1 over all pixels as a column, the way a projection is called: tiles of 16 x 32 pixels would be almost empty."""
+    assert conv_plan(65536, 1, 128, 3, 1) == conv_plan(262144, 1, 128, 16, 1) == conv_plan(1, 65536, 128, 28, 1) == ONE_BY_ONE
+    assert conv_plan(65536, 1, 64, 3, 1) == 0
+    assert conv_plan(65536, 1, 32, 3, 3, 1, 1, 1) == 0 and conv_plan(65536, 1, 128, 3, 3, 1, 1, 1) == FEW_OUT
+    assert conv_plan(128, 128, 128, 28, 1) == ONE_BY_ONE and conv_plan(128, 128, 64, 28, 1) == 0
+    for h, w in ((8, 8), (4096, 1), (100, 90), (512, 512), (1024, 1024)):
+        assert conv_plan(h, w, 128, 3, 1) == conv_plan(h, w, 128, 3, 3, 1, 1, 1) == conv_plan(h, w, 64, 7, 2, 1, 0, 1) == FEW_OUT
+
+
 # ------------------------------------------------------------------ row norms
 def test_row_norms_take_a_wave_per_row_where_rows_are_many_and_short_and_a_workgroup_elsewhere():
     lib = C.CDLL(iris_c_amd.LIB_PATH)
