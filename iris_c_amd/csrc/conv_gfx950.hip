@@ -927,6 +927,16 @@ bool few_out_pays(const ConvShape &s, long out_pixels, float copied_us) {
     return 3.0f + (float)((tiles + 511) / 512) * (2.7f + 0.036f * (float)s.cin) < copied_us;
 }
 
+/* About what k_conv_1x1 takes: every workgroup first brings all the weights of its channels into the LDS, 5 us per 128 input
+ * channels whatever the image, so a few thousand pixels of 256 and more channels are faster through a copy. Measured, us,
+ * k_conv_1x1 / copy: 256 -> 128 1000 pixels 16.7 / 13.3, 9216 17.4 / 16.0, 30000 19.1 / 21.9; 512 -> 128 4096 27.5 / 12.2, 16384
+ * 28.6 / 19.2, 65536 33.8 / 52.9; 384 -> 256 1000 22.1 / 21.0, 9216 23.4 / 25.8. With 128 input channels it is always faster. */
+float one_by_one_us(long pixels, int cin, int cout) {
+    const float weights = 6.0f + (cout <= 64 ? 3.6f : 5.2f) * (float)(cin / 128), memory = 4.0f * (float)pixels * (float)(cin + cout) / 5.0e6f;
+    const float chain = (pixels < 256 ? 0.6f : 1.0f) * weights + 1e-4f * (float)pixels;
+    return chain > memory ? chain : memory;
+}
+
 /* Which kernel a convolution takes, host arithmetic only. All of them store results while other workgroups still read the
  * image around them, so an output that shares memory with the image goes elsewhere: those routes copy the image first. */
 Route route(const ConvShape &s, const void *out, const void *in, const void *w) {
@@ -939,8 +949,8 @@ Route route(const ConvShape &s, const void *out, const void *in, const void *w) 
     if (s.k <= FO_MAX_K && s.k * s.k * s.cout <= FO_ROWS && s.stride == 1 && (s.cin == 32 || s.cin == 64 || s.cin == 128) && al16(in) && al16(w) &&
         few_out_pays(s, out_pixels, copied_us))
         return FEW_OUT;
-    if (plain && s.cin % 128 == 0 && s.cin <= C1_MAX_CIN && s.cout <= 2 * C1_N && al16(in) &&
-        ((uintptr_t)w & 7) == 0)
+    if (plain && s.cin % 128 == 0 && s.cin <= C1_MAX_CIN && s.cout <= 2 * C1_N && al16(in) && ((uintptr_t)w & 7) == 0 &&
+        (s.cin == 128 || one_by_one_us(out_pixels, s.cin, s.cout) < copied_us))
         return ONE_BY_ONE;
     /* a thread's byte offsets into image and weights are 32-bit */
     const bool offsets = in_bytes < ((size_t)1 << 32) && (size_t)s.cout * 9 * s.cin * 2 < ((size_t)1 << 32);

@@ -129,6 +129,18 @@ def test_few_output_channels_of_a_flat_image(conv_plan):
         assert conv_plan(h, w, 128, 3, 1) == conv_plan(h, w, 128, 3, 3, 1, 1, 1) == conv_plan(h, w, 64, 7, 2, 1, 0, 1) == FEW_OUT
 
 
+def test_one_by_one_convolutions_of_few_pixels_and_many_channels_go_through_a_copy(conv_plan):
+    for pixels in (256, 1000, 4096):
+        for cin, cout in ((256, 64), (256, 128), (384, 100), (512, 32), (512, 128), (512, 256)):
+            assert conv_plan(pixels, 1, cin, cout, 1) == 0, (pixels, cin, cout)
+        for cout in (64, 128, 256):
+            assert conv_plan(pixels, 1, 128, cout, 1) == ONE_BY_ONE
+    assert conv_plan(16384, 1, 512, 128, 1) == 0
+    for cin, cout in ((256, 64), (256, 128), (384, 100), (384, 256), (512, 32), (512, 128), (512, 256)):
+        assert conv_plan(256, 256, cin, cout, 1) == conv_plan(512, 512, cin, cout, 1) == ONE_BY_ONE, (cin, cout)
+    assert conv_plan(30000, 1, 256, 128, 1) == conv_plan(1000, 1, 256, 256, 1) == conv_plan(64, 1, 256, 128, 1) == ONE_BY_ONE
+
+
 # ------------------------------------------------------------------ row norms
 def test_row_norms_take_a_wave_per_row_where_rows_are_many_and_short_and_a_workgroup_elsewhere():
     lib = C.CDLL(iris_c_amd.LIB_PATH)
