@@ -937,6 +937,22 @@ float one_by_one_us(long pixels, int cin, int cout) {
     return chain > memory ? chain : memory;
 }
 
+inline long three_tiles(const ConvShape &s, int ty, int tx) {
+    return (long)((s.oh + ty - 1) / ty) * ((s.ow + tx - 1) / tx) * ((s.cout + C3_N - 1) / C3_N);
+}
+
+/* The 3 x 3 kernels multiply whole tiles. An image of a few rows or columns fills only part of each, and once its tiles no
+ * longer fit one round of the CUs a copy and a product over the pixels alone is faster: us, 1 x 4096 512 -> 512 190 / 113, 8 x 3000
+ * 150 / 132, 20000 x 1 128 -> 128 70 / 30, with stride 2 172 / 68 for 256 -> 256. Where tiles are at least two thirds full
+ * the copy never was; elsewhere the estimates decide. A tile takes 5.8 us per 64 channels (4.9 in a grid of one round),
+ * with stride 2 2.3 per 32. */
+bool three_pays(const ConvShape &s, int ty, int tx, float copied_us) {
+    const long tiles = three_tiles(s, ty, tx), rounds = (tiles + 255) / 256, n_tiles = (s.cout + C3_N - 1) / C3_N;
+    if (2 * tiles * ty * tx <= 3 * n_tiles * s.oh * s.ow) return true;
+    const float tile_us = s.stride == 1 ? 3.0f + (rounds > 1 ? 5.8f : 4.9f) * (float)(s.cin / 64) : 1.5f + 2.3f * (float)(s.cin / H3_C);
+    return 3.0f + (float)rounds * tile_us <= copied_us / 0.97f;
+}
+
 /* Which kernel a convolution takes, host arithmetic only. All of them store results while other workgroups still read the
  * image around them, so an output that shares memory with the image goes elsewhere: those routes copy the image first. */
 Route route(const ConvShape &s, const void *out, const void *in, const void *w) {
@@ -954,8 +970,12 @@ Route route(const ConvShape &s, const void *out, const void *in, const void *w) 
         return ONE_BY_ONE;
     /* a thread's byte offsets into image and weights are 32-bit */
     const bool offsets = in_bytes < ((size_t)1 << 32) && (size_t)s.cout * 9 * s.cin * 2 < ((size_t)1 << 32);
-    if (s.k == 3 && s.stride == 1 && s.cin % 64 == 0 && s.cout <= C3_MAX_COUT && al16(in) && al16(w) && offsets) return THREE;
-    if (s.k == 3 && s.stride == 2 && s.cin % H3_C == 0 && s.cout >= 128 && s.cout <= H3_MAX_COUT && al16(in) && al16(w) && offsets) return THREE_HALF;
+    if (s.k == 3 && s.stride == 1 && s.cin % 64 == 0 && s.cout <= C3_MAX_COUT && al16(in) && al16(w) && offsets &&
+        three_pays(s, C3_T, C3_T, copied_us))
+        return THREE;
+    if (s.k == 3 && s.stride == 2 && s.cin % H3_C == 0 && s.cout >= 128 && s.cout <= H3_MAX_COUT && al16(in) && al16(w) && offsets &&
+        three_pays(s, H3_TY, H3_TX, copied_us))
+        return THREE_HALF;
     return OTHER;
 }
 
@@ -971,7 +991,6 @@ void iris_hip_conv2d_plan(const void *out, const void *in, const void *w, int h,
     const int oh = (h + pad_before + pad_after - k) / stride + 1, ow = (width + pad_before + pad_after - k) / stride + 1;
     const ConvShape s = {h, width, cin, cout, k, stride, pad_before, oh, ow};
     const auto turns = [](long work, long takers) { return (int)((work + takers - 1) / takers); };
-    const auto tiles = [&](int ty, int tx) { return (long)((oh + ty - 1) / ty) * ((ow + tx - 1) / tx) * ((cout + C3_N - 1) / C3_N); };
     plan[0] = route(s, out, in, w);
     plan[1] = 1;
     if (plan[0] == FEW_IN) {
@@ -980,7 +999,7 @@ void iris_hip_conv2d_plan(const void *out, const void *in, const void *w, int h,
     } else if (plan[0] == ONE_BY_ONE) {
         plan[1] = turns(((long)h * width + 15) / 16, (long)one_by_one_slots(h * width, cout) * C1_WAVES);
     } else if (plan[0] == THREE || plan[0] == THREE_HALF) {
-        plan[1] = turns((plan[0] == THREE ? tiles(C3_T, C3_T) : tiles(H3_TY, H3_TX)), 256);
+        plan[1] = turns(plan[0] == THREE ? three_tiles(s, C3_T, C3_T) : three_tiles(s, H3_TY, H3_TX), 256);
     }
 }
 

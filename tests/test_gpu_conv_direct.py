@@ -95,3 +95,10 @@ def test_output_in_the_image_s_own_memory(dev, orc, h, w, cin, cout, k, stride, 
     got = dev.get(out, want.shape, np.float32)
     dev.free_all()
     np.testing.assert_allclose(got, want, atol=2e-5 * np.sqrt(k * k * cin))
+
+
+@pytest.mark.parametrize("h,w,cin,cout,stride,pb,pa", [(1, 9000, 64, 384, 1, 1, 1), (8, 1100, 128, 640, 1, 1, 1), (9000, 1, 64, 40, 1, 1, 1),
+                                                       (9000, 1, 128, 640, 2, 1, 1), (1, 2000, 128, 256, 1, 1, 1), (3, 700, 64, 256, 2, 0, 1)])
+def test_three_by_three_of_images_thinner_than_a_tile(dev, orc, h, w, cin, cout, stride, pb, pa):
+    """On both sides of the choice between the tiles and a copy of the image."""
+    conv_case(dev, orc, h, w, cin, cout, 3, stride, pb, pa)

@@ -141,6 +141,20 @@ def test_one_by_one_convolutions_of_few_pixels_and_many_channels_go_through_a_co
     assert conv_plan(30000, 1, 256, 128, 1) == conv_plan(1000, 1, 256, 256, 1) == conv_plan(64, 1, 256, 128, 1) == ONE_BY_ONE
 
 
+def test_three_by_three_convolutions_of_images_thinner_than_a_tile(conv_plan):
+    three = lambda h, w, cin, cout, stride=1: conv_plan(h, w, cin, cout, 3, stride, 1, 1)
+    for h, w in ((1, 4096), (4096, 1), (1, 20000), (20000, 1), (8, 3000), (3000, 8)):
+        assert three(h, w, 512, 512) == three(h, w, 128, 384) == 0, (h, w)
+    for cin, cout in ((64, 64), (64, 128), (128, 128), (256, 256), (512, 64), (1024, 1024)):
+        assert three(1, 20000, cin, cout) == three(20000, 1, cin, cout) == 0, (cin, cout)
+    assert three(4096, 1, 512, 512, 2) == three(20000, 1, 128, 128, 2) == three(1, 20000, 512, 512, 2) == 0
+    # tiles that fit one round of the CUs, and images that fill theirs
+    assert three(3, 1000, 512, 512) == three(1, 4096, 128, 128) == three(1000, 3, 256, 128) == THREE
+    assert three(1, 4096, 512, 512, 2) == three(4096, 1, 256, 128, 2) == THREE_HALF
+    for h, w in ((8, 8), (17, 17), (48, 48), (33, 500), (250, 130), (512, 512)):
+        assert three(h, w, 512, 512) == three(h, w, 128, 64) == THREE and three(h, w, 256, 256, 2) == THREE_HALF, (h, w)
+
+
 # ------------------------------------------------------------------ row norms
 def test_row_norms_take_a_wave_per_row_where_rows_are_many_and_short_and_a_workgroup_elsewhere():
     lib = C.CDLL(iris_c_amd.LIB_PATH)
