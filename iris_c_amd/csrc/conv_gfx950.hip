@@ -915,6 +915,17 @@ inline unsigned few_in_columns(int groups) { return groups < 1280 * FI_WAVES ? (
 
 enum Route { OTHER, FEW_IN, FEW_OUT, ONE_BY_ONE, THREE, THREE_HALF };
 
+/* Not where there is next to nothing to do per pixel: on large images the whole products of 16 pixels x 128 channels then take
+ * longer than a thread per output (1 x 1, 1 -> 1 over 1024 x 1024 45 us / 11, 4 -> 4 over 512 x 512 17 / 12; 3 x 3, 1 -> 1 44.7 / 43;
+ * from images of 8 channels and up, which are gathered in 16-byte pieces, 1 x 1, 32 -> 1 26 / 22). And not for 1 x 1 of 32 channels
+ * to 128 and more, where every load of a wave touches 64 different cache lines: 32 -> 512 over 256 x 256 135 us / 86, 16 x 16
+ * 11.2 / 10.4; on larger images the patches of the other side go through HBM (512 x 512 220 / 428). */
+bool few_in_pays(const ConvShape &s, long out_pixels) {
+    const int values = s.k * s.k * s.cin;
+    if (out_pixels > 131072) return values * s.cout > 16 && !(s.cin % 8 == 0 && 8 * s.cout <= values);
+    return !(s.k == 1 && s.cin == 32 && s.cout >= 128);
+}
+
 /* With 1 x 1 there are no taps to save, and a thread adds up and stores all the channels of its pixel: k_conv_1x1 or a copy are
  * faster from 5 channels on (128 -> 16 over 512 x 512 41 us against 33 in k_conv_1x1; 64 -> 28 over 128 x 128 13.5 / 10.2), with 64
  * input channels from 17 (64 -> 16 9.9 / 10.0). And where an image is not as wide as a tile, as one of width 1 that a
@@ -958,9 +969,9 @@ bool three_pays(const ConvShape &s, int ty, int tx, float copied_us) {
 Route route(const ConvShape &s, const void *out, const void *in, const void *w) {
     const size_t in_bytes = (size_t)s.h * s.w * s.cin * 4, out_bytes = (size_t)s.oh * s.ow * s.cout * 4;
     if (overlap(out, out_bytes, in, in_bytes)) return OTHER;
-    if (s.k * s.k * s.cin <= 32 && (long)s.oh * s.ow <= (1L << 30)) return FEW_IN;
     const bool plain = s.k == 1 && s.stride == 1 && s.oh == s.h && s.ow == s.w;
     const long out_pixels = (long)s.oh * s.ow;
+    if (s.k * s.k * s.cin <= 32 && out_pixels <= (1L << 30) && few_in_pays(s, out_pixels)) return FEW_IN;
     const float copied_us = iris_hip_conv2d_copied_us((long)s.h * s.w, out_pixels, s.cin, s.cout, s.k, plain);
     if (s.k <= FO_MAX_K && s.k * s.k * s.cout <= FO_ROWS && s.stride == 1 && (s.cin == 32 || s.cin == 64 || s.cin == 128) && al16(in) && al16(w) &&
         few_out_pays(s, out_pixels, copied_us))

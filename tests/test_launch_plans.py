@@ -155,6 +155,18 @@ def test_three_by_three_convolutions_of_images_thinner_than_a_tile(conv_plan):
         assert three(h, w, 512, 512) == three(h, w, 128, 64) == THREE and three(h, w, 256, 256, 2) == THREE_HALF, (h, w)
 
 
+def test_few_input_channels_with_next_to_nothing_to_do_per_pixel(conv_plan):
+    big = lambda cin, cout, k=1: conv_plan(1024, 1024, cin, cout, k, 1, k // 2, k // 2)
+    for cin, cout, k in ((1, 1, 1), (1, 4, 1), (4, 4, 1), (16, 1, 1), (24, 1, 1), (1, 1, 3)):
+        assert big(cin, cout, k) == 0, (cin, cout, k)
+    assert big(32, 1) == big(32, 4) == FEW_OUT
+    for cin, cout, k in ((3, 128, 3), (3, 3, 3), (2, 1, 3), (1, 2, 3), (8, 4, 1), (1, 32, 1), (32, 28, 1), (32, 512, 1)):
+        assert big(cin, cout, k) == FEW_IN, (cin, cout, k)
+    for h, w in ((16, 16), (256, 256)):
+        assert conv_plan(h, w, 32, 128, 1) == conv_plan(h, w, 32, 512, 1) == 0
+        assert conv_plan(h, w, 1, 1, 1) == conv_plan(h, w, 32, 4, 1) == conv_plan(h, w, 16, 512, 1) == conv_plan(h, w, 3, 128, 3, 1, 1, 1) == FEW_IN
+
+
 # ------------------------------------------------------------------ row norms
 def test_row_norms_take_a_wave_per_row_where_rows_are_many_and_short_and_a_workgroup_elsewhere():
     lib = C.CDLL(iris_c_amd.LIB_PATH)
