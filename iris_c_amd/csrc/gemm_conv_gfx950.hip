@@ -12,11 +12,11 @@
  * a single 16-byte (f32) or 8-byte (bf16) store.
  *
  * Products with too few 256-row tiles to fill the chip (short sequences) take k_gemm_tiles (gemm_tiles_gfx950.hip). For
- * the rest, three kernels. M, N >= 256 with K a multiple of 128 (every linear layer of the models at their
+ * the rest, three kernels. M, N >= 256 with K a multiple of 64 (every linear layer of the models at their
  * larger sequence lengths) take k_gemm_wide: tiles of 256 rows x 256 - 160 columns on eight waves, every memory
- * instruction in a gap between two products. Other shapes with M, N >= 256 and K a multiple of 64, and the convolutions
- * that have no kernel of their own, take k_gemm_dma: the same tiles with the loads and reads in groups. Both give the same
- * bits. Everything else with K a multiple of 8 takes k_gemm_bf16:
+ * instruction in a gap between two products. One, three, five or seven k tiles of 64, outputs whose rows are not 16-byte aligned, and
+ * the convolutions that have no kernel of their own take k_gemm_dma: the same tiles with the loads and reads in groups. Both
+ * give the same bits. Everything else with K a multiple of 8 takes k_gemm_bf16:
  * Workgroup = WM x WN waves (2 x 2 in use), tile 128 (m) x 128 (n), K in steps of 64; a wave owns
  * 64 x 64 = 4 x 4 accumulator blocks and reads 8 operands from LDS per 16 MFMAs. One
  * LDS stage of [W tile | x tile], rows padded to 160 B so that the 16 lanes the LDS
@@ -427,7 +427,7 @@ k_gemm_dma(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *
 }
 /* ---- tiles of 256 rows x 256, 224, 192 or 160 columns ----
  *
- * For M, N >= 256, K a multiple of 128: every linear layer of the models at their larger sequence lengths. Eight waves, two
+ * For M, N >= 256, K a multiple of 64: every linear layer of the models at their larger sequence lengths. Eight waves, two
  * per SIMD, 4 (rows of 64) x 2: a wave owns 64 rows x 16 NA columns = NA x 4 accumulator blocks (NA = 8, 7, 6, 5, so that the
  * launcher can pick the width whose grid fills the last round of the 256 CUs best). A k tile of 64 is four steps: k-step
  * 0 with the first and the second half of the columns, then k-step 1; the operands of a step are requested from the LDS
@@ -745,10 +745,12 @@ int launch_gemm_wide(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *
     return (int)hipGetLastError();
 }
 
-/* What that kernel takes: 16-byte stores, and 32-bit byte offsets into the operands. */
+/* What that kernel takes: 16-byte stores, and 32-bit byte offsets into the operands. It has no use for an even number of
+ * k tiles, but with one, three, five or seven k_gemm_dma is as fast or faster (4608 rows, -> 9216, us here / there: 64 24.0 / 22.6,
+ * 320 40.7 / 40.7, 448 50 / 50; 576 54.5 / 57.7, 1088 80 / 94, 3136 190 / 233). */
 static bool wide_shape(int M, int N, int K, size_t out_size) {
-    return M >= DT && N >= 256 && K % (2 * TK) == 0 && N % (16 / (int)out_size) == 0 && ((size_t)M * K * 2) >> 32 == 0 &&
-           ((size_t)N * K * 2) >> 32 == 0;
+    return M >= DT && N >= 256 && K % TK == 0 && (K % (2 * TK) == 0 || K >= 8 * TK) && N % (16 / (int)out_size) == 0 &&
+           ((size_t)M * K * 2) >> 32 == 0 && ((size_t)N * K * 2) >> 32 == 0;
 }
 
 /* The tile width (32 NA columns) whose grid wastes least of its last round of 256 workgroups: time goes with

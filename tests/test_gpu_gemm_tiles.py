@@ -9,6 +9,7 @@ import oracle as O
 from gpu_harness import Dev
 
 pytestmark = pytest.mark.gpu
+WIDE_ODD = [(513, 576, 17408), (600, 704, 20488), (2100, 1088, 6152), (512, 576, 19456)]
 TILES = [(128, 128), (128, 192), (128, 256), (64, 256), (160, 192), (160, 256)]
 
 
@@ -103,6 +104,21 @@ def test_wide_tiles_of_160_columns(dev, rows, k, out, bf16):
     dev.free_all()
     assert (got[rows * out:] == 7).all()
     check(got[:rows * out].reshape(rows, out), want, k, bf16)
+
+
+@pytest.mark.parametrize("rows,k,out", WIDE_ODD)
+@pytest.mark.parametrize("bf16", [False, True])
+def test_wide_tiles_of_an_odd_number_of_k_tiles(dev, rows, k, out, bf16):
+    plan = (C.c_int * 2)()
+    dev.lib.iris_hip_linear_plan(rows, k, out, 2 if bf16 else 4, plan)
+    assert plan[0] == 3
+    x, W, want = operands(rows, k, out)
+    dy = dev.alloc(rows * out * (2 if bf16 else 4))
+    (dev.lib.iris_dev_linear_bf16 if bf16 else dev.lib.iris_dev_linear_f32)(dy, dev.put(x), dev.put(W), rows, k, out)
+    dev.check()
+    got = dev.get(dy, (rows, out), np.uint16 if bf16 else np.float32)
+    dev.free_all()
+    check(got, want, k, bf16)
 
 
 def test_projection_with_norm_takes_the_same_kernel(dev):

@@ -85,6 +85,14 @@ def test_linear_layers_of_the_models_take_the_four_wave_kernel_in_the_width_that
     assert linear_plan(512, 256, 258, 4)[0] == 2             # f32 rows of 258 columns cannot take 16-byte stores
 
 
+def test_long_products_of_an_odd_number_of_k_tiles_take_the_wide_kernel_too(linear_plan):
+    for k in (576, 704, 1088, 2624, 3136):
+        for out in (3072, 9216):
+            assert linear_plan(4608, k, out)[0] == linear_plan(9000, k, out, 4)[0] == 3, (k, out)
+    for k in (64, 192, 320, 448):
+        assert linear_plan(4608, k, 9216)[0] == 2                  # the other kernel is as fast
+
+
 # ------------------------------------------------------------------ the convolutions' kernel choice
 FEW_IN, FEW_OUT, ONE_BY_ONE, THREE, THREE_HALF = 1, 2, 3, 4, 5
 
