@@ -490,22 +490,23 @@ k_gemm_wide(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t 
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const int r = 8 * (4 * wave + j) + (lane >> 3);
-        xoff[j] = ((uint32_t)min(m0 + r, M - 1) * (uint32_t)K + 8u * ((lane & 7) ^ ((r >> 1) & 7))) * 2u;
+        xoff[j] = ((uint32_t)(min(m0 + r, M - 1) - m0) * (uint32_t)K + 8u * ((lane & 7) ^ ((r >> 1) & 7))) * 2u;
     }
 #pragma unroll
     for (int j = 0; j < WP; j++) {
         wpiece[j] = min(WP * wave + j, TN / 8 - 1);
         const int r = 8 * wpiece[j] + (lane >> 3);
-        woff[j] = ((uint32_t)min(n0 + r, N - 1) * (uint32_t)K + 8u * ((lane & 7) ^ ((r >> 1) & 7))) * 2u;
+        woff[j] = ((uint32_t)(min(n0 + r, N - 1) - n0) * (uint32_t)K + 8u * ((lane & 7) ^ ((r >> 1) & 7))) * 2u;
     }
+    const uint16_t *x_tile = x + (size_t)m0 * K, *w_tile = W + (size_t)n0 * K;       /* offsets inside a tile fit 32 bits */
     const uint32_t lds0 = lds_address(dlds);
     auto request_x = [&](int j, int kt, uint32_t stage) {      /* stage: bytes into the LDS */
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                     ::"s"(lds0 + stage + (4 * wave + j) * 1024), "v"(xoff[j]), "s"(x + (size_t)kt * TK) : "memory", "m0");
+                     ::"s"(lds0 + stage + (4 * wave + j) * 1024), "v"(xoff[j]), "s"(x_tile + (size_t)kt * TK) : "memory", "m0");
     };
     auto request_w = [&](int j, int kt, uint32_t stage) {
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                     ::"s"(lds0 + stage + wpiece[j] * 1024), "v"(woff[j]), "s"(W + (size_t)kt * TK) : "memory", "m0");
+                     ::"s"(lds0 + stage + wpiece[j] * 1024), "v"(woff[j]), "s"(w_tile + (size_t)kt * TK) : "memory", "m0");
     };
 
     f32x4 acc[NA][4];                                          /* [16 columns][16 rows] */
@@ -745,12 +746,12 @@ int launch_gemm_wide(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *
     return (int)hipGetLastError();
 }
 
-/* What that kernel takes: 16-byte stores, and 32-bit byte offsets into the operands. It has no use for an even number of
+/* What that kernel takes: 16-byte stores, and 32-bit byte offsets into the rows of a tile. It has no use for an even number of
  * k tiles, but with one, three, five or seven k_gemm_dma is as fast or faster (4608 rows, -> 9216, us here / there: 64 24.0 / 22.6,
  * 320 40.7 / 40.7, 448 50 / 50; 576 54.5 / 57.7, 1088 80 / 94, 3136 190 / 233). */
 static bool wide_shape(int M, int N, int K, size_t out_size) {
     return M >= DT && N >= 256 && K % TK == 0 && (K % (2 * TK) == 0 || K >= 8 * TK) && N % (16 / (int)out_size) == 0 &&
-           ((size_t)M * K * 2) >> 32 == 0 && ((size_t)N * K * 2) >> 32 == 0;
+           ((size_t)DT * K * 2) >> 32 == 0;
 }
 
 /* The tile width (32 NA columns) whose grid wastes least of its last round of 256 workgroups: time goes with

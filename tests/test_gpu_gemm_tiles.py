@@ -121,6 +121,29 @@ def test_wide_tiles_of_an_odd_number_of_k_tiles(dev, rows, k, out, bf16):
     check(got, want, k, bf16)
 
 
+@pytest.mark.parametrize("rows,out", [(131400, 264), (264, 131400)])
+def test_wide_tiles_of_operands_beyond_four_gibibytes(dev, rows, out):
+    """x or W of 4.3 GB: rows on both sides of the byte that 32 bits no longer count, against float64 products on the device."""
+    import torch
+    k = 16384
+    plan = (C.c_int * 2)()
+    dev.lib.iris_hip_linear_plan(rows, k, out, 4, plan)
+    assert plan[0] == 3 and max(rows, out) * k * 2 > 1 << 32
+    torch.manual_seed(4)
+    x, W = torch.randn(rows, k, dtype=torch.bfloat16, device="cuda"), torch.randn(out, k, dtype=torch.bfloat16, device="cuda") * 0.05
+    y = torch.empty(rows, out, device="cuda")
+    torch.cuda.synchronize()
+    dev.lib.iris_dev_linear_f32(y.data_ptr(), x.data_ptr(), W.data_ptr(), rows, k, out)
+    dev.lib.iris_dev_sync()
+    dev.check()
+    pick = lambda n: torch.tensor(sorted({i % n for i in (0, 1, 255, 256, 131070, 131071, 131072, 131073, -257, -1)}), device="cuda")
+    m, n = pick(rows), pick(out)
+    want = x[m].double() @ W[n].double().t().contiguous()
+    assert float((y[m][:, n].double() - want).abs().max()) <= np.sqrt(k) * 0.05 * 2e-5
+    del x, W, y
+    torch.cuda.empty_cache()
+
+
 def test_projection_with_norm_takes_the_same_kernel(dev):
     """The projection that normalises its own columns, at a size whose plain layer takes these tiles: the bits of the two calls."""
     rows, k, heads = 320, 1024, 6

@@ -93,6 +93,11 @@ def test_long_products_of_an_odd_number_of_k_tiles_take_the_wide_kernel_too(line
         assert linear_plan(4608, k, 9216)[0] == 2                  # the other kernel is as fast
 
 
+def test_operands_of_four_gibibytes_and_more_take_the_wide_kernel(linear_plan):
+    assert linear_plan(140000, 16384, 512)[0] == linear_plan(512, 16384, 140000, 4)[0] == 3
+    assert linear_plan(300000, 8192, 300000)[0] == 3
+
+
 # ------------------------------------------------------------------ the convolutions' kernel choice
 FEW_IN, FEW_OUT, ONE_BY_ONE, THREE, THREE_HALF = 1, 2, 3, 4, 5
 
