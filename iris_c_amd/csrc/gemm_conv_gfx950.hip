@@ -771,6 +771,13 @@ static int wide_width(int M, int N) {
     return best;
 }
 
+/* workgroups of k_gemm_wide with tiles of 32 na columns, and the estimated time of that grid */
+static long wide_wgs(int M, int N, int na) { return (long)((M + DT - 1) / DT) * ((N + 32 * na - 1) / (32 * na)); }
+static float wide_us(int M, int N, int K, int na) {
+    const long wgs = wide_wgs(M, N, na), rounds = (wgs + 255) / 256;
+    return 4.0f + (float)rounds * ((float)(K / TK) * (wgs <= 128 ? 0.145f : 0.175f) * (float)na + 4.0f);
+}
+
 /* Which kernel a linear layer takes, host arithmetic only: 4 = k_gemm_tiles (gemm_tiles_gfx950.hip) with its tile `na` and
  * `splits` ranges of K, 3 = k_gemm_wide with tiles of 32 na columns, 2 = k_gemm_dma, 1 = k_gemm_bf16, 0 = k_gemm_scalar.
  *
@@ -786,12 +793,11 @@ static GemmPlan plan_gemm(int M, int N, int K, int out_size, bool operands_align
     if (K > 0 && K % TK == 0 && operands_aligned16 && M >= DT && N >= DT && (size_t)K * 2 * 8 < ((size_t)1 << 31)) {
         if (wide_shape(M, N, K, (size_t)out_size) && out_aligned16) {
             const int na = wide_width(M, N);
-            const long wgs = (long)((M + DT - 1) / DT) * ((N + 32 * na - 1) / (32 * na)), rounds = (wgs + 255) / 256;
-            const float us = 4.0f + (float)rounds * ((float)(K / TK) * (wgs <= 128 ? 0.145f : 0.175f) * (float)na + 4.0f);
+            const float us = wide_us(M, N, K, na);
             if (tiles_us < 0.0f || tiles_us >= us) return {3, na, 1, us};
             return {4, shape, splits, tiles_us};
         }
-        if (tiles_us < 0.0f) return {2, 8, 1, 0.0f};
+        if (tiles_us < 0.0f) return {2, 8, 1, wide_us(M, N, K, 8)};
     }
     if (tiles_us >= 0.0f) return {4, shape, splits, tiles_us};
     if (K > 0 && K % 8 == 0 && operands_aligned16) return {1, 0, 1, 0.0f};
@@ -894,27 +900,46 @@ int iris_hip_linear_bf16(void *stream, float *part, uint16_t *y, const uint16_t 
     return gemm<uint16_t>((hipStream_t)stream, y, x, W, rows, out, in, part, part ? IRIS_LINEAR_PART_BYTES : 0);
 }
 
+/* How the projection that normalises its own columns runs, host arithmetic only: 1 k_gemm_wide in tiles of 256 columns that
+ * normalises them in its epilogue (a tile holds two whole heads), 0 the plain layer in whatever tiles suit it and the norm
+ * kernel behind it, -1 neither (the norm kernel counts fewer than 2^24 vectors).
+ * Normalising tiles costs their workgroups 4 us a round, the pass over the stored columns 1.8 us and what they take at 7 TB/s, so
+ * the epilogue pays where the plain layer takes the same tiles anyway or close to them in a grid of several rounds. us,
+ * epilogue / two kernels: 4608 x 64 -> 9216 with 24 + 24 heads 35.6 / 41.9, 192 43.2 / 48.6, 576 67.6 / 73.6, 1024 92.4 / 94.9, 3072
+ * (224 columns suit the plain layer) 207 / 203; 2115 x 192 28.1 / 26.4; 512 x 3072 64 / 42. */
+static int qknorm_plan(int M, int N, int K, int q_cols, int k_cols, bool aligned, size_t part_bytes) {
+    const int heads = (q_cols + k_cols) / 128;
+    if (!aligned || K <= 0 || K % TK || ((size_t)DT * K * 2) >> 32 || M < DT || N < DT || N % 128 || q_cols < 0 || k_cols < 0 || q_cols % 128 ||
+        k_cols % 128 || q_cols + k_cols > N || heads == 0)
+        return -1;
+    if ((long long)M * heads >= (1 << 24) || heads >= 256) return 1;
+    const GemmPlan plan = plan_gemm(M, N, K, 2, true, true, part_bytes);
+    if (plan.kernel == 3 && plan.na == 8) return 1;
+    const long wgs = wide_wgs(M, N, 8);
+    const float norm_us = 1.8f + 4.0f * (float)M * (float)(q_cols + k_cols) / 7.0e6f;
+    return wgs > 512 && wide_us(M, N, K, 8) + 4.0f * (float)((wgs + 255) / 256) < plan.us + norm_us;
+}
+int iris_hip_linear_qknorm_plan(int rows, int in, int out, int q_cols, int k_cols) {
+    return qknorm_plan(rows, out, in, q_cols, k_cols, true, IRIS_LINEAR_PART_BYTES);
+}
+
 /* y = x W^T as bf16 with the per-head RMSNorm + rotary embedding (head_dim 128) of columns [0, q_cols) (weights
- * wq) and [q_cols, q_cols + k_cols) (weights wk): applied in the GEMM's epilogue where the plain layer takes 256-column
- * tiles of k_gemm_wide (a tile then holds two whole heads), by the norm kernel behind it elsewhere. Returns -2, with
- * nothing enqueued, for a shape it does not take: the caller then runs the two steps one after the other. */
+ * wq) and [q_cols, q_cols + k_cols) (weights wk). Returns -2, with nothing enqueued, for a shape it does not take: the
+ * caller then runs the two steps one after the other. */
 int iris_hip_linear_bf16_qknorm(void *stream, float *part, uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in, int out,
                                 int q_cols, int k_cols, const float *wq, const float *wk, const float *rope_cos,
                                 const float *rope_sin, float eps, int split_half) {
     const int M = rows, N = out, K = in;
     const uintptr_t all = (uintptr_t)x | (uintptr_t)W | (uintptr_t)y | (uintptr_t)wq | (uintptr_t)wk | (uintptr_t)rope_cos |
                           (uintptr_t)rope_sin;
-    const bool tiled = K > 0 && K % TK == 0 && (all & 15) == 0 && M >= DT && N >= DT && (size_t)K * 2 * 8 < ((size_t)1 << 31);
-    const int qh = q_cols / 128, kh = k_cols / 128;
-    if (!tiled || N % 128 || q_cols < 0 || k_cols < 0 || q_cols % 128 || k_cols % 128 || q_cols + k_cols > N ||
-        q_cols + k_cols == 0 || (long long)M * (qh + kh) >= (1 << 24) || qh + kh >= 256)
-        return -2;
     const size_t part_bytes = part ? IRIS_LINEAR_PART_BYTES : 0;
-    const GemmPlan plan = plan_gemm(M, N, K, 2, true, true, part_bytes);
-    if (plan.kernel == 3 && plan.na == 8) {
+    const int fused = qknorm_plan(M, N, K, q_cols, k_cols, (all & 15) == 0, part_bytes);
+    if (fused < 0) return -2;
+    if (fused) {
         const QkNorm qn = {wq, k_cols ? wk : wq, rope_cos, rope_sin, q_cols, q_cols + k_cols, eps, split_half};
         return launch_gemm_wide<uint16_t, 8, true>((hipStream_t)stream, y, x, W, M, N, K, nullptr, qn);
     }
+    const int qh = q_cols / 128, kh = k_cols / 128;
     const int e = gemm<uint16_t>((hipStream_t)stream, y, x, W, M, N, K, part, part_bytes);
     if (e) return e;
     return qh ? iris_hip_norm_rope_hd128(stream, y, kh ? y + q_cols : nullptr, N, wq, wk, rope_cos, rope_sin, M, qh, kh, eps, split_half)

@@ -147,6 +147,8 @@ float iris_hip_gemm_tiles_plan(int M, int N, int K, int out_size, size_t part_by
 int iris_hip_gemm_tiles(void *stream, void *y, int out_size, const uint16_t *x, const uint16_t *W, int M, int N, int K,
                         const float *bias, int shape, int splits, float *part);
 
+/* 1: the tiles normalise themselves, 0: the norm kernel runs behind the layer, -1: not taken; host arithmetic only */
+int iris_hip_linear_qknorm_plan(int rows, int in, int out, int q_cols, int k_cols);
 /* -2 = shape not taken, nothing enqueued */
 int iris_hip_linear_bf16_qknorm(void *stream, float *part, uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in,
                                 int out, int q_cols, int k_cols, const float *wq, const float *wk, const float *rope_cos,

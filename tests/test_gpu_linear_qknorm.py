@@ -2,8 +2,9 @@
 
 Two yardsticks. The CPU oracle's chain (its linear layer rounded to bf16, then its norm+rope on the Q and on
 the K columns: the three calls of iris_transformer_flux.c:3833-3837), to the relative bar of the other
-kernels. And the library's own two-call form on its own GEMM, bit for bit: the one-launch kernel rounds the
-projection to bf16 and then runs the same function as the stand-alone norm+rope kernel.
+kernels. And the library's own two-call form on its own GEMM, bit for bit: the tiles that normalise themselves round the
+projection to bf16 and then run the same function as the stand-alone norm+rope kernel. Small projections run as those
+two kernels; which of the two forms a size takes is iris_hip_linear_qknorm_plan's to say.
 """
 import numpy as np
 import pytest
@@ -70,16 +71,16 @@ def oracle_chain(orc, c, split):
 
 # rows, in, q heads, k heads, columns after K, pairing
 ONE_LAUNCH = [
-    (256, 64, 2, 2, 256, 0),        # whole tiles, the smallest the kernel takes
+    (256, 64, 2, 2, 256, 0),        # whole tiles, the smallest the entry takes
     (333, 384, 3, 3, 384 + 1536, 0),  # ragged rows; a tile that holds a Q head and a K head; FLUX single-block layout
     (600, 256, 2, 2, 256 + 1024, 1),  # split halves
     (700, 640, 8, 2, 256, 1),       # text encoder: 8 query heads on 2 kv heads, split halves
     (512, 128, 3, 0, 128, 0),       # Q only, and a last tile of 128 columns
     (300, 192, 0, 1, 128, 1),       # K only
     (1000, 512, 5, 5, 0, 0),        # nothing after K; 1280 columns = five tiles
-    (512, 256, 2, 2, 256, 0),       # whole tiles and in % 128 == 0: the four-wave kernel's epilogue
+    (512, 256, 2, 2, 256, 0),       # whole tiles, in a multiple of 128
     (768, 384, 3, 1, 0, 1),         # the same, split halves, three query heads on one kv head
-    (256, 128, 1, 1, 256, 1),       # its smallest case: two k tiles, one tile with a Q and a K head, one without
+    (256, 128, 1, 1, 256, 1),       # two k tiles
 ]
 
 
@@ -97,6 +98,30 @@ def test_one_launch_matches_oracle_chain_and_own_two_calls(dev, orc, rows, k, q_
     plain, _ = run(dev, dict(c, q_heads=0, k_heads=0), False, split, 1)
     assert np.array_equal(got[:, qk:], plain[:, qk:])
     assert not np.array_equal(got[:, :qk], plain[:, :qk])
+
+
+# rows, in, q heads, k heads, columns after K, pairing: tiles that normalise themselves
+FUSED = [
+    (525, 128, 24, 24, 12928, 0),     # ragged rows, a last tile of 128 columns
+    (525, 128, 24, 24, 12928, 1),
+    (512, 128, 3, 2, 18432, 0),       # whole tiles; a tile with a Q and a K head, one with a K head and plain columns
+    (700, 128, 5, 0, 18432, 1),       # Q only, ending inside a tile
+    (525, 128, 0, 7, 18176, 0),       # K only
+    (4000, 64, 24, 24, 3072, 0),      # a single k tile
+    (4352, 192, 24, 24, 3072, 1),     # three
+]
+
+
+@pytest.mark.parametrize("rows,k,q_heads,k_heads,extra,split", FUSED)
+def test_tiles_that_normalise_themselves_match_oracle_chain_and_own_two_calls(dev, orc, rows, k, q_heads, k_heads, extra, split):
+    c = make(rows + k + q_heads, rows, k, q_heads, k_heads, extra)
+    assert dev.lib.iris_hip_linear_qknorm_plan(rows, k, c["out"], 128 * q_heads, 128 * k_heads) == 1
+    got, kernel = run(dev, c, True, split, 1)
+    assert kernel == "linear_mfma_qknorm"
+    two, _ = run(dev, c, False, split, 1)
+    assert np.array_equal(got, two)
+    want = oracle_chain(orc, c, split)
+    assert_parity(bf16_to_f32(got), bf16_to_f32(want), f"rows {rows} in {k} heads {q_heads}+{k_heads}")
 
 
 def test_vendor_backend_against_oracle(dev, orc):

@@ -98,6 +98,19 @@ def test_operands_of_four_gibibytes_and_more_take_the_wide_kernel(linear_plan):
     assert linear_plan(300000, 8192, 300000)[0] == 3
 
 
+def test_projections_normalise_their_tiles_where_that_is_the_faster_form(linear_plan):
+    lib = C.CDLL(iris_c_amd.LIB_PATH)
+    plan = lambda rows, k, out, q, kv: lib.iris_hip_linear_qknorm_plan(rows, k, out, 128 * q, 128 * kv)
+    assert linear_plan(4608, 3072, 27648) == (3, 256) and plan(4608, 3072, 27648, 24, 24) == 1       # the plain layer's own tiles
+    for k in (64, 192, 448, 576):
+        assert plan(4608, k, 9216, 24, 24) == 1
+    for rows, k, out in ((320, 3072, 27648), (512, 3072, 9216), (2115, 192, 9216), (4608, 3072, 9216)):
+        assert plan(rows, k, out, 24, 24) == 0
+    assert plan(400000, 256, 6144, 24, 24) == 1          # more vectors than the norm kernel counts
+    for rows, k, out, q, kv in ((255, 64, 768, 2, 2), (300, 72, 768, 2, 2), (300, 64, 800, 2, 2), (300, 64, 768, 4, 3), (300, 64, 768, 0, 0)):
+        assert plan(rows, k, out, q, kv) == -1
+
+
 # ------------------------------------------------------------------ the convolutions' kernel choice
 FEW_IN, FEW_OUT, ONE_BY_ONE, THREE, THREE_HALF = 1, 2, 3, 4, 5
 
