@@ -28,15 +28,25 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 
 @functools.lru_cache(maxsize=None)
-def isa(name):
+def assembly(name):
     if not os.path.exists(HIPCC):
         pytest.skip("no hipcc here")
     r = subprocess.run([HIPCC, "-O3", "--offload-arch=gfx950", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
                         "-packed-fp32-ops", "-I" + CSRC, "-I" + os.path.join(ROOT, "include"), "--cuda-device-only", "-S",
                         "-o", "-", os.path.join(CSRC, name)], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-2000:]
-    ins = [l.strip() for l in r.stdout.splitlines()]
-    return [l for l in ins if l and not l.startswith((";", ".")) and not l.endswith(":")]
+    return [l.strip() for l in r.stdout.splitlines()]
+
+
+def isa(name, kernel=None):
+    """The instructions of a source, or of one of its kernels."""
+    ins = assembly(name)
+    if kernel:
+        begin = [i for i, l in enumerate(ins) if re.match(rf"_Z\w*\d{kernel}E\w*:", l)]
+        assert len(begin) == 1, (kernel, begin)
+        ins = ins[begin[0]:]
+        ins = ins[:next(i for i, l in enumerate(ins) if l.startswith(".Lfunc_end"))]
+    return [l for l in ins if l and not l.startswith((";", ".")) and not l.split(";")[0].strip().endswith(":")]
 
 
 def vregs(tok):
@@ -59,10 +69,21 @@ def operands(line):
     return [t.strip().split()[0] for t in line.split(None, 1)[1].split(",")] if " " in line else []
 
 
-@pytest.mark.parametrize("name,least", [("fa_fwd_hd512_gfx950.hip", 300), ("gemm_conv_gfx950.hip", 300)])
-def test_no_vector_instruction_feeds_an_asm_matrix_instruction_directly(name, least):
-    """The sources whose matrix products are asm statements."""
-    ins = isa(name)
+# where matrix products are asm statements: all of a source, or one kernel of it (the products of its others are the
+# compiler's, which places the wait states of its own instructions and need not keep to these stricter rules)
+ASM_PRODUCTS = [("fa_fwd_hd512_gfx950.hip", None, 300), ("conv_gfx950.hip", "k_conv_3x3", 288)]
+
+
+def test_every_source_with_asm_products_is_checked():
+    code = lambda f: re.sub(r"/\*.*?\*/|//[^\n]*", "", open(os.path.join(CSRC, f)).read(), flags=re.S)
+    found = {f for f in os.listdir(CSRC) if f.endswith((".hip", ".h")) and "v_mfma" in code(f)}
+    # microbench.hip times products whose results nobody reads
+    assert found == {name for name, _, _ in ASM_PRODUCTS} | {"microbench.hip"}
+
+
+@pytest.mark.parametrize("name,kernel,least", ASM_PRODUCTS)
+def test_no_vector_instruction_feeds_an_asm_matrix_instruction_directly(name, kernel, least):
+    ins = isa(name, kernel)
     products = 0
     for i, l in enumerate(ins):
         if not l.startswith("v_mfma"):
@@ -73,7 +94,7 @@ def test_no_vector_instruction_feeds_an_asm_matrix_instruction_directly(name, le
             p = ins[i - back]
             if p.startswith("v_") and not p.startswith("v_mfma"):
                 assert not (vregs(operands(p)[0]) & src), f"{name}: {p}  feeds  {l}"
-    assert products > least
+    assert products >= least
 
 
 @pytest.mark.parametrize("name", sorted(f for f in os.listdir(CSRC) if f.endswith(".hip")))
@@ -113,9 +134,9 @@ def test_data_registers_of_a_wide_store_are_left_alone_right_behind_it(name):
             waits += int(m.group(1)) + 1 if m else 1
 
 
-@pytest.mark.parametrize("name", ["fa_fwd_hd512_gfx950.hip", "gemm_conv_gfx950.hip"])
-def test_results_of_asm_matrix_instructions_are_left_alone_until_they_have_left_the_matrix_core(name):
-    ins = isa(name)
+@pytest.mark.parametrize("name,kernel,least", ASM_PRODUCTS)
+def test_results_of_asm_matrix_instructions_are_left_alone_until_they_have_left_the_matrix_core(name, kernel, least):
+    ins = isa(name, kernel)
     for i, l in enumerate(ins):
         if not l.startswith("v_mfma"):
             continue
