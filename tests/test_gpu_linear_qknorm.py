@@ -104,7 +104,7 @@ def test_one_launch_matches_oracle_chain_and_own_two_calls(dev, orc, rows, k, q_
 FUSED = [
     (525, 128, 24, 24, 12928, 0),     # ragged rows, a last tile of 128 columns
     (525, 128, 24, 24, 12928, 1),
-    (512, 128, 3, 2, 18432, 0),       # whole tiles; a tile with a Q and a K head, one with a K head and plain columns
+    (768, 128, 3, 2, 18560, 0),       # whole tiles; a tile with a Q and a K head, one with a K head and plain columns
     (700, 128, 5, 0, 18432, 1),       # Q only, ending inside a tile
     (525, 128, 0, 7, 18176, 0),       # K only
     (4000, 64, 24, 24, 3072, 0),      # a single k tile
@@ -120,8 +120,18 @@ def test_tiles_that_normalise_themselves_match_oracle_chain_and_own_two_calls(de
     assert kernel == "linear_mfma_qknorm"
     two, _ = run(dev, c, False, split, 1)
     assert np.array_equal(got, two)
-    want = oracle_chain(orc, c, split)
-    assert_parity(bf16_to_f32(got), bf16_to_f32(want), f"rows {rows} in {k} heads {q_heads}+{k_heads}")
+    got, want = bf16_to_f32(got), bf16_to_f32(oracle_chain(orc, c, split))
+    # The f32 sums are taken in another order, so a projected value may round to the neighbouring bf16 number, 2^-7 of it away at
+    # most. A normed one carries that of its pair, whose length the rotation keeps, that of the vector's root mean square,
+    # and rounds once more.
+    allowed = 2.0 ** -7 * np.abs(want) + 2e-5
+    heads = want[:, :128 * (q_heads + k_heads)].reshape(rows, -1, 2, 64) if split else \
+        want[:, :128 * (q_heads + k_heads)].reshape(rows, -1, 64, 2).swapaxes(2, 3)
+    length = np.broadcast_to(np.hypot(heads[:, :, 0], heads[:, :, 1])[:, :, None], heads.shape)
+    normed = 2.0 ** -7 * (length + 2 * np.abs(heads)) + 2e-5
+    allowed[:, :128 * (q_heads + k_heads)] = (normed if split else normed.swapaxes(2, 3)).reshape(rows, -1)
+    assert (np.abs(got - want) <= allowed).all()
+    assert np.abs(got - want).mean() <= 2.0 ** -9 * np.abs(want).mean()
 
 
 def test_vendor_backend_against_oracle(dev, orc):
