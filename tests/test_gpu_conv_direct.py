@@ -1,5 +1,8 @@
 """The convolutions that work straight on the f32 image (conv_gfx950.hip), at the sizes where their tiles and remainders
-begin and end, against the CPU oracle (bf16-rounded operands, f32 sums: the bar is the rounding of the sum's order)."""
+begin and end, against the CPU oracle (bf16-rounded operands, f32 sums: the bar is the rounding of the sum's order).
+Larger images against the same sums in float64."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -61,7 +64,7 @@ def test_three_by_three(dev, orc, h, w, cin, cout, pb, pa, bias):
 @pytest.mark.parametrize("h,w,cin,cout,bias", [(1, 1, 128, 128, True), (8, 4, 128, 128, True), (257, 1, 256, 130, False), (33, 31, 512, 64, True),
                                                (300, 1, 512, 1536, True), (2000, 1, 512, 1536, True), (90, 91, 384, 256, True), (17, 16, 64, 320, True), (9, 9, 128, 258, True), (128, 128, 128, 3, False)])
 def test_one_by_one(dev, orc, h, w, cin, cout, bias):
-    """One block of 16 pixels and less, more blocks than waves, one and two tiles of 128 channels, a ragged one; and what goes
+    """One block of 16 pixels and less, as many blocks as waves, one and two tiles of 128 channels, a ragged one; and what goes
     through the bf16 copy and a plain product with the bias in its epilogue or behind it."""
     conv_case(dev, orc, h, w, cin, cout, 1, 1, 0, 0, bias)
 
@@ -72,7 +75,7 @@ def test_one_by_one(dev, orc, h, w, cin, cout, bias):
     (150, 340, 128, 256, 0, 1, True)])
 def test_three_by_three_stride_two(dev, orc, h, w, cin, cout, pb, pa, bias):
     """Tile edges (8 x 16 output pixels, 128 channels), one to sixteen groups of 32 input channels (odd and even numbers of them),
-    padding of other widths, more tiles than workgroups."""
+    padding of other widths, nearly as many tiles as workgroups."""
     conv_case(dev, orc, h, w, cin, cout, 3, 2, pb, pa, bias)
 
 
@@ -102,3 +105,49 @@ def test_output_in_the_image_s_own_memory(dev, orc, h, w, cin, cout, k, stride, 
 def test_three_by_three_of_images_thinner_than_a_tile(dev, orc, h, w, cin, cout, stride, pb, pa):
     """On both sides of the choice between the tiles and a copy of the image."""
     conv_case(dev, orc, h, w, cin, cout, 3, stride, pb, pa)
+
+
+def conv_float64(img, wt, bias, h, w, k, stride, pb, pa):
+    """The definition, tap by tap in float64 on the bf16-rounded operands, on the device."""
+    import torch
+    cin, cout = img.shape[1], wt.shape[0]
+    oh, ow = (h + pb + pa - k) // stride + 1, (w + pb + pa - k) // stride + 1
+    x = torch.zeros(h + pb + pa, w + pb + pa, cin, dtype=torch.float64, device="cuda")
+    x[pb:pb + h, pb:pb + w] = torch.from_numpy(O.bf16_to_f32(O.f32_to_bf16(img)).reshape(h, w, cin)).cuda()
+    taps = torch.from_numpy(O.bf16_to_f32(wt).reshape(cout, k, k, cin)).cuda().double()
+    out = torch.from_numpy(bias).cuda().double().repeat(oh * ow, 1)
+    for ky in range(k):
+        for kx in range(k):
+            pixels = x[ky:ky + stride * (oh - 1) + 1:stride, kx:kx + stride * (ow - 1) + 1:stride].reshape(oh * ow, cin)
+            out += pixels @ taps[:, ky, kx].t().contiguous()
+    return out.cpu().numpy()
+
+
+FEW_IN, ONE_BY_ONE, THREE, THREE_HALF = 1, 3, 4, 5             # iris_hip_conv2d_plan
+
+
+@pytest.mark.parametrize("kernel,turns,h,w,cin,cout,k,stride,pb,pa", [
+    (FEW_IN, 2, 301, 290, 3, 128, 3, 1, 1, 1), (FEW_IN, 3, 500, 341, 3, 130, 3, 1, 1, 1), (FEW_IN, 2, 600, 580, 7, 260, 2, 2, 0, 0),
+    (ONE_BY_ONE, 2, 70001, 1, 128, 100, 1, 1, 0, 0), (ONE_BY_ONE, 2, 211, 193, 256, 200, 1, 1, 0, 0), (ONE_BY_ONE, 3, 301, 233, 384, 256, 1, 1, 0, 0),
+    (THREE, 2, 150, 250, 64, 260, 3, 1, 1, 1), (THREE, 2, 130, 270, 192, 130, 3, 1, 1, 1), (THREE, 4, 250, 270, 64, 384, 3, 1, 0, 1),
+    (THREE_HALF, 2, 150, 340, 128, 260, 3, 2, 0, 1), (THREE_HALF, 2, 180, 360, 96, 130, 3, 2, 0, 1), (THREE_HALF, 2, 190, 350, 64, 256, 3, 2, 1, 1),
+    (THREE_HALF, 3, 201, 399, 32, 400, 3, 2, 1, 0)])
+def test_work_taken_in_several_turns(dev, kernel, turns, h, w, cin, cout, k, stride, pb, pa):
+    """Waves and workgroups that go on to another piece, with what they keep between pieces: fetches ahead, another tile of
+    channels, operand sets that change places (odd and even numbers of channel groups), ragged last pieces."""
+    plan = (C.c_int * 2)()
+    dev.lib.iris_hip_conv2d_plan(C.c_void_p(1 << 44), C.c_void_p(1 << 40), C.c_void_p(1 << 46), h, w, cin, cout, k, stride, pb, pa, plan)
+    assert (plan[0], plan[1]) == (kernel, turns)
+    rng = np.random.default_rng(h + w + cout)
+    img = rng.standard_normal((h * w, cin), dtype=np.float32)
+    wt = O.f32_to_bf16((rng.standard_normal((cout, k * k * cin)) * 0.1).astype(np.float32))
+    b = rng.standard_normal(cout).astype(np.float32)
+    want = conv_float64(img, wt, b, h, w, k, stride, pb, pa)
+    guard = 64
+    out = dev.put(np.full(want.size + guard, 7.0, np.float32))
+    dev.lib.iris_dev_conv2d(out, dev.put(img), dev.put(wt), dev.put(b), h, w, cin, cout, k, stride, pb, pa)
+    dev.check()
+    got = dev.get(out, (want.size + guard,), np.float32)
+    dev.free_all()
+    assert (got[want.size:] == 7.0).all()
+    np.testing.assert_allclose(got[:want.size].reshape(want.shape), want, atol=2e-5 * np.sqrt(k * k * cin))
