@@ -151,3 +151,46 @@ def test_work_taken_in_several_turns(dev, kernel, turns, h, w, cin, cout, k, str
     dev.free_all()
     assert (got[want.size:] == 7.0).all()
     np.testing.assert_allclose(got[:want.size].reshape(want.shape), want, atol=2e-5 * np.sqrt(k * k * cin))
+
+
+ZERO_BYTES = 256                                             # IRIS_CONV_ZERO_BYTES
+
+
+# scratch: what it holds behind the page of zeros, in rows of the image, pixels or patches, as the route counts
+@pytest.mark.parametrize("route,h,w,cin,cout,k,stride,pb,pa,scratch", [
+    ("implicit", 37, 29, 64, 128, 5, 1, 2, 2, 9), ("implicit", 40, 33, 128, 260, 5, 2, 1, 3, 7), ("implicit", 30, 41, 192, 256, 2, 1, 0, 1, 2),
+    ("implicit", 41, 30, 64, 384, 2, 2, 1, 0, 5), ("implicit", 50, 37, 64, 130, 3, 3, 1, 1, 8), ("implicit", 23, 21, 128, 320, 5, 1, 2, 2, 64),
+    ("plain", 61, 13, 512, 320, 1, 1, 0, 0, 150), ("plain", 1000, 1, 576, 264, 1, 1, 0, 0, 333), ("plain", 20, 20, 512, 512, 1, 1, 0, 0, 400),
+    ("gathered", 30, 31, 24, 64, 3, 1, 1, 1, 100), ("gathered", 31, 30, 5, 40, 3, 2, 0, 1, 77), ("gathered", 25, 26, 64, 60, 5, 1, 2, 2, 7),
+    ("gathered", 19, 18, 72, 128, 2, 2, 0, 0, 1)])
+def test_routes_that_copy_the_image_in_chunks_of_the_scratch(dev, route, h, w, cin, cout, k, stride, pb, pa, scratch):
+    """The routes of gemm_conv_gfx950.hip with a scratch that holds only part of the copy (and once all of it): taps other than 3 x 3
+    through the implicit product, chunks of output rows with their halo, of pixels, of gathered patches, ragged last ones."""
+    row_bytes = {"implicit": w * cin, "plain": cin, "gathered": k * k * cin}[route] * 2
+    scratch_bytes, guard = ZERO_BYTES + scratch * row_bytes, 256
+    plan = (C.c_int * 2)()
+    dev.lib.iris_hip_conv2d_plan(C.c_void_p(1 << 44), C.c_void_p(1 << 40), C.c_void_p(1 << 46), h, w, cin, cout, k, stride, pb, pa, plan)
+    assert plan[0] == 0 and (route == "implicit") == (cin % 64 == 0 and cout >= 128 and k > 1)
+    if route == "plain":
+        dev.lib.iris_hip_linear_plan(min(h * w, scratch), cin, cout, 4, plan)
+        assert plan[0] == 4
+    rng = np.random.default_rng(h + w + cout)
+    img = rng.standard_normal((h * w, cin)).astype(np.float32)
+    wt = O.f32_to_bf16((rng.standard_normal((cout, k * k * cin)) * 0.1).astype(np.float32))
+    b = rng.standard_normal(cout).astype(np.float32)
+    want = conv_float64(img, wt, b, h, w, k, stride, pb, pa)
+    room = dev.put(np.full(scratch_bytes + guard, 0x5a, np.uint8))
+    out = dev.put(np.full(want.size + 64, 7.0, np.float32))
+    vp, ci = C.c_void_p, C.c_int
+    stream = vp(dev.lib.iris_dev_stream())
+    conv = dev.lib.iris_hip_conv2d
+    conv.argtypes = [vp, vp, C.c_size_t, vp, vp, vp, vp] + [ci] * 8
+    dev.lib.iris_hip_conv2d_prepare_scratch.argtypes = [vp, vp]
+    assert dev.lib.iris_hip_conv2d_prepare_scratch(stream, room) == 0
+    assert conv(stream, room, scratch_bytes, out, dev.put(img), dev.put(wt), dev.put(b), h, w, cin, cout, k, stride, pb, pa) == 0
+    dev.check()
+    got = dev.get(out, (want.size + 64,), np.float32)
+    page = dev.get(room, (scratch_bytes + guard,), np.uint8)
+    dev.free_all()
+    assert (got[want.size:] == 7.0).all() and (page[scratch_bytes:] == 0x5a).all() and not page[:ZERO_BYTES].any()
+    np.testing.assert_allclose(got[:want.size].reshape(want.shape), want, atol=2e-5 * np.sqrt(k * k * cin))

@@ -221,7 +221,7 @@ def test_swiglu(dev, orc, rows, cols, ldi, ldo):
 # ------------------------------------------------------------------ VAE layers
 @pytest.mark.parametrize("h,w,cin,cout,k,stride,pb,pa", [(6, 5, 8, 4, 3, 1, 1, 1), (7, 7, 3, 5, 3, 1, 1, 1), (8, 8, 16, 6, 3, 2, 0, 1),
                                                          (16, 16, 128, 128, 3, 1, 1, 1), (9, 9, 32, 64, 1, 1, 0, 0),
-                                                         # cin % 64 == 0 and cout >= 128: the implicit-GEMM path
+                                                         # cin % 64 == 0 and cout >= 128: whole tiles of the kernels for 3 x 3 and 1 x 1
                                                          (20, 17, 64, 128, 3, 1, 1, 1), (16, 16, 128, 256, 3, 1, 1, 1),
                                                          (33, 20, 64, 320, 3, 2, 0, 1), (12, 12, 128, 130, 1, 1, 0, 0),
                                                          (24, 40, 192, 128, 3, 1, 1, 1), (5, 4, 64, 512, 3, 1, 1, 1),
@@ -243,9 +243,9 @@ def test_conv2d(dev, orc, h, w, cin, cout, k, stride, pb, pa):
 
 
 def test_conv2d_large_image_in_chunks_sampled_pixels(dev):
-    """An image whose bf16 copy does not fit the library's 256 MB of convolution scratch is processed in
-    chunks of output rows with their halo rows. 1040 x 1024 x 128 -> 128, 3 x 3: sampled output pixels
-    (corners, edges, the rows around every possible chunk boundary, random ones) against the definition
+    """An image whose bf16 copy would not fit the library's 256 MB of convolution scratch: 1040 x 1024 x 128 -> 128, 3 x 3, which
+    needs no copy (the routes that do, in chunks of the scratch, are in test_gpu_conv_direct.py). Sampled output pixels
+    (corners, edges, rows at which a copy would have to be cut, random ones) against the definition
     in float64 on bf16-rounded inputs."""
     h, w, cin, cout, k = 1040, 1024, 128, 128, 3
     rng = np.random.default_rng(11)
