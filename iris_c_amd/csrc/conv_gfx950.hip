@@ -7,6 +7,8 @@
  * k_conv_1x1: cin a multiple of 128, at most 512, cout at most 256: the VAE's skip connections.
  * k_conv_3x3: 3 x 3, stride 1, cin a multiple of 64: every other layer of the VAE but the halving ones.
  * k_conv_3x3_half: 3 x 3, stride 2, cin a multiple of 32, cout at least 128: those.
+ * `route` says where each of them pays. The counts of workgroups in it, and in the launchers, are for the 256 CUs of an MI355X; on
+ * another number of them only the choice would be another, not the results.
  *
  * The first two are bound by memory: one side of the product is so thin that the image on the other side is all there
  * is to move. The image is rounded to bf16 on the way into the matrix core, products are summed in f32.
@@ -126,10 +128,12 @@ k_conv_few_in(float *__restrict__ out, const float *__restrict__ in, const uint1
  * The taps move from the reduction into the rows of the product: Z[(tap, channel)][pixel] = W[channel, tap] . image[pixel]
  * for every INPUT pixel, k * k * cout <= 28 rows (two A operands), cin long; the output pixel then adds its k * k entries of
  * Z. So a pixel goes through the matrix core once instead of once per tap, its B operand comes straight from global
- * memory (a k-step's 32 channels as two 16-byte loads a lane, channels 4 lg and 16 + 4 lg, so that a load covers 64 B of a pixel), and only Z passes through the LDS. A workgroup makes Z for the
- * (32 + k - 1) x (16 + k - 1) pixels under a 32 x 16 tile of the output (1.2 x, the overlap comes from the L2).
+ * memory (a k-step's 32 channels as two 16-byte loads a lane, channels 4 lg and 16 + 4 lg, so that a load covers 64 B of
+ * a pixel), and only Z passes through the LDS. A workgroup makes Z for the (32 + k - 1) x (16 + k - 1) pixels under a 32 x 16
+ * tile of the output (1.2 x, the overlap comes from the L2).
  * What bounds it is the read of the image. 128 -> 3 on 1024 x 1024 (537 MB in): 1383 us as patches + 128-wide product +
- * bias, 122 us here (5.3 TB/s with the overlap). Two workgroups per CU (Z and the weights take 78 KB of LDS), so that one adds while one reads. */
+ * bias, 122 us here (5.3 TB/s with the overlap). Two workgroups per CU (Z and the weights take 78 KB of LDS), so that one
+ * adds while one reads. */
 constexpr int FO_TX = 32, FO_TY = 16, FO_THREADS = 512, FO_ROWS = 28, FO_MAX_K = 3;
 constexpr int FO_PIXELS = (FO_TX + FO_MAX_K - 1) * (FO_TY + FO_MAX_K - 1), FO_MAX_CIN = 128;
 constexpr int FO_GROUPS = (FO_PIXELS + 15) / 16;
@@ -211,14 +215,15 @@ k_conv_few_out(float *__restrict__ out, const float *__restrict__ in, const uint
 /* ---- 1 x 1 ----
  *
  * A product of the image with a small matrix. A workgroup keeps the weights of 128 output channels in the LDS for as long as
- * it lives, as A operands in the order the waves read them, and its eight waves walk blocks of 32 pixels: a wave fetches
+ * it lives, as A operands in the order the waves read them, and its sixteen waves walk blocks of 16 pixels: a wave fetches
  * its pixels straight into registers as f32 (two 16-byte loads per k-step, so that a load covers 64 B of a pixel), rounds
- * them there and multiplies them with all 128 channels, half an LDS read per product. While a group of 128 input channels
+ * them there and multiplies them with all 128 channels, one LDS read per product. While a group of 128 input channels
  * is multiplied the next one, or the next block's first, is on its way. Nothing is shared between waves but the weights:
  * no barrier.
  * What bounds it is the image and the result: 512 x 512 pixels, 256 -> 128 channels 76 + 65 us as a bf16 copy and an implicit
- * product, 91 here (402 MB; eight waves of 32 pixels 93). With more than two tiles of channels the image is read once for
- * each (512 -> 1536 over 16384 pixels: 84 us against 61), so those stay with the copy and a plain product. */
+ * product, 91 here (402 MB; eight waves that take 32 pixels each, half an LDS read per product, 93). With more than two
+ * tiles of channels the image is read once for each (512 -> 1536 over 16384 pixels: 84 us against 61), so those go through a
+ * copy (gemm_conv_gfx950.hip), as do few pixels of many channels (one_by_one_us). */
 constexpr int C1_N = 128, C1_MAX_CIN = 512, C1_WAVES = 16, C1_OUT = 512;   /* output channels of a workgroup; f32 of LDS per wave for its stores */
 
 __global__ void __launch_bounds__(64 * C1_WAVES, 4)
@@ -353,9 +358,9 @@ int launch_1x1(hipStream_t st, float *out, const float *in, const uint16_t *W, c
  * Measured against a bf16 copy of the image + implicit product that fetches every tap from the L2 (copy + product), against
  * eight waves that did everything (and stood still while a tile's stores landed), and now: 512 x 512 pixels, 128 -> 128
  * 30 + 118, 79, 73 us (the image and the result alone take 50 us to move), 256 -> 128 76 + 214, 129, 123, 256 -> 256 88 + 290,
- * 253, 235 us (1320 TFLOP/s). With nothing to bring in, the products and stores of the last take 192 us; the image costs 42 of
- * the rest, the weights 25, all at a clock that the chip's power has brought down to 2.0 GHz. Pixels and weights on waves of
- * their own (three and one) 1 % slower. */
+ * 253, 235 us (1320 TFLOP/s). The first is bound by memory (matrix cores busy 43 % of its cycles), the last by the products at
+ * the clock that the chip's power leaves (63 % at 1.9 GHz of 2.4; counters, under the profiler). Pixels and weights on waves
+ * of their own (three and one) 1 % slower. */
 constexpr int C3_T = 16, C3_H = C3_T + 2, C3_PIXELS = C3_H * C3_H, C3_ROW = 80, C3_IMG = C3_PIXELS * C3_ROW;   /* elements */
 constexpr int C3_N = 128, C3_STAGE = C3_N * 64;
 constexpr int C3_MUL = 8, C3_BRING = 4, C3_THREADS = 64 * (C3_MUL + C3_BRING);           /* waves that multiply, that bring pixels and weights */

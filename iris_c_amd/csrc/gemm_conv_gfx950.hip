@@ -434,9 +434,8 @@ k_gemm_dma(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *
  * during the step before. What the kernel lives on:
  *  - every memory instruction stands in a gap of its own between two products. All waves of the CU leave a barrier
  *    together, so what is bunched behind it is not hidden by the other wave of the SIMD but added to the products;
- *  - no branches: a request past the end of K asks for the last tile again, into a stage that nobody reads. With a
- *    uniform branch around each request a k tile of 256 x 256 took 2550 cycles, without them 2230, of which the products
- *    are 2048;
+ *  - no branches: a request past the end of K asks for the last tile again, into a stage that nobody reads. Of a k tile of
+ *    256 x 256 the products are 2048 cycles; a variant with a uniform branch around each request took 14 % longer for it;
  *  - the LDS holds two stages of x and three of W (160 KB at 256 columns). The stage of x that a barrier sets free is
  *    requested at once (first gaps of step 3), W one step at a time in steps 0 - 2: rows from the L2 or HBM take as long
  *    as a whole k tile. x spread over two steps instead: 4608 x 12288 -> 3072 284 us, as it is 244.
@@ -444,8 +443,8 @@ k_gemm_dma(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *
  *
  * Against the kernel it replaces (four waves of 128 x 128, one per SIMD, staged through registers), weights from HBM, us:
  * 4608 x 3072 -> 9216 203 -> 188 (1390 TFLOP/s), -> 18432 408 -> 378, -> 27648 593 -> 566, 12288 -> 3072 257 -> 244, 9216 -> 3072
- * 195 -> 186. With everything in the L2 4096 x 8192 -> 4096 runs at 1530 TFLOP/s, 2060 on zeros: the rest is the chip's
- * power. Tried on it: k tiles of 32 in five stages (a direct load of sixteen 64 B rows takes longer than one of eight
+ * 195 -> 186. With everything in the L2 4096 x 8192 -> 4096, one round of workgroups, runs at 1530 TFLOP/s, 2060 on zeros: the
+ * rest is the chip's power (counters, under the profiler: matrix cores busy 80 % of all cycles, at 1.8 GHz of 2.4). Tried on it: k tiles of 32 in five stages (a direct load of sixteen 64 B rows takes longer than one of eight
  * 128 B rows: 1170 TFLOP/s), a second barrier that frees the stages earlier (2 - 4 % slower). */
 /* The per-head RMSNorm + rotary embedding of the leading columns of a projection, applied by the GEMM to its
  * own output tile (head_dim 128): columns [0, q_cols) are heads normalised with wq, [q_cols, qk_cols) with wk,
@@ -995,7 +994,8 @@ int iris_hip_conv2d(void *stream, uint16_t *scratch, size_t scratch_bytes, float
      * product. An attention block with 512 -> 1536 over 1024 pixels 82 -> 69 us, over 4096 122 -> 117. Over more pixels
      * k_gemm_wide on the copy is 4 us faster than the implicit product by itself (16384: 59 - 63 us with the copy against 64),
      * but the head_dim-512 attention kernel behind it then runs 20 - 30 us longer: the block 611 against 573, 14391 pixels
-     * 527 / 497, 9216 273 / 261, 7200 198 / 196. */
+     * 527 / 497, 9216 273 / 261, 7200 198 / 196. Only the times were measured; what slows the attention kernel there (its
+     * clock, or what the caches still hold) is not known. */
     const long rows = (long)(scratch_bytes / ((size_t)cin * sizeof(uint16_t)));
     const bool aligned_w = ((uintptr_t)w & 15) == 0 && ((uintptr_t)out & 15) == 0;
     if (k == 1 && stride == 1 && oh == h && ow == width && rows > 0 &&
