@@ -46,7 +46,7 @@ def run(dev, fn, outs):
                                         # the 256 x 256 kernel (rows, out >= 256, k % 64 == 0): ragged edges, and an `out` that
                                         # rules out 16-byte stores (its epilogue then stores straight from the accumulators)
                                         (300, 128, 258), (257, 64, 257), (512, 192, 256), (700, 256, 1000),
-                                        # whole 256 x 256 tiles and k % 128 == 0: the four-wave kernel (two k tiles at least)
+                                        # whole 256 x 256 tiles and k % 128 == 0: the wide kernel or the smaller tiles
                                         (256, 128, 256), (512, 256, 512), (768, 640, 1024)])
 @pytest.mark.parametrize("out_bf16", [False, True])
 @pytest.mark.parametrize("backend", ["library", "own"])
@@ -74,10 +74,10 @@ def test_linear(dev, orc, rows, k, out, out_bf16, backend):
 
 @pytest.mark.parametrize("rows,k,out,width", [(4608, 128, 9216, 224), (4608, 256, 3072, 224), (4608, 128, 27648, 256), (2048, 128, 2048, 192)])
 @pytest.mark.parametrize("out_bf16", [False, True])
-def test_four_wave_gemm_every_tile_width(dev, orc, rows, k, out, width, out_bf16):
-    """The four-wave kernel at each of its tile widths (192, 224, 256 columns), f32 and bf16 output, WHOLE output:
-    the widths the model projections take (4608 rows -> 9216 / 3072 columns: 224, with a last tile moved back because
-    9216 % 224 != 0; -> 27648: 256) with a short reduction so that the comparison stays cheap. Against a float64
+def test_wide_gemm_at_the_widths_of_the_models(dev, orc, rows, k, out, width, out_bf16):
+    """k_gemm_wide in tiles of 192, 224 and 256 columns (160: test_gpu_gemm_tiles.py), f32 and bf16 output, WHOLE output:
+    the widths the model projections take (4608 rows -> 9216 / 3072 columns: 224, with a last tile that ends past the
+    matrix because 9216 % 224 != 0; -> 27648: 256) with a short reduction so that the comparison stays cheap. Against a float64
     product of the same bf16 operands (numpy's BLAS, an independent routine; the f32 accumulation error over 128-256
     terms is far below the bar), and the oracle on sampled rows."""
     import ctypes as C

@@ -73,13 +73,13 @@ def linear_plan():
     return call
 
 
-def test_linear_layers_of_the_models_take_the_four_wave_kernel_in_the_width_that_fills_the_rounds(linear_plan):
+def test_linear_layers_of_the_models_take_the_wide_kernel_in_the_width_that_fills_the_rounds(linear_plan):
     assert linear_plan(4608, 3072, 9216) == (3, 224)        # 756 tiles = 2.95 rounds of 256 CUs (648 of 256 columns: 2.53)
     assert linear_plan(4608, 3072, 3072) == (3, 224)        # 252 tiles: one round (216 of 256 columns: also one, but wider)
     assert linear_plan(4608, 3072, 27648) == (3, 256)       # 1944 tiles = 7.6 rounds; narrower tiles need 9 or 11
     assert linear_plan(4608, 3072, 18432)[1] in (224, 192)  # 1296 tiles of 256 columns are 5.06 rounds
     for rows, k, out in ((300, 128, 258), (257, 64, 257), (512, 192, 256)):
-        assert linear_plan(rows, k, out)[0] == 2             # k not a multiple of 128, or rows of 2 bytes not 16-byte aligned
+        assert linear_plan(rows, k, out)[0] == 2             # rows of 2 bytes not 16-byte aligned, or three k tiles
     assert linear_plan(700, 256, 1000) == (3, 256) or linear_plan(700, 256, 1000)[0] == 3
     assert linear_plan(64, 128, 64)[0] == 1 and linear_plan(37, 27, 19)[0] == 0
     assert linear_plan(512, 256, 258, 4)[0] == 2             # f32 rows of 258 columns cannot take 16-byte stores
