@@ -444,7 +444,7 @@ k_gemm_dma(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *
  * Against the kernel it replaces (four waves of 128 x 128, one per SIMD, staged through registers), weights from HBM, us:
  * 4608 x 3072 -> 9216 203 -> 188 (1390 TFLOP/s), -> 18432 408 -> 378, -> 27648 593 -> 566, 12288 -> 3072 257 -> 244, 9216 -> 3072
  * 195 -> 186. With everything in the L2 4096 x 8192 -> 4096, one round of workgroups, runs at 1530 TFLOP/s, 2060 on zeros: the
- * rest is the chip's power (counters, under the profiler: matrix cores busy 80 % of all cycles, at 1.8 GHz of 2.4). Tried on it: k tiles of 32 in five stages (a direct load of sixteen 64 B rows takes longer than one of eight
+ * rest is the chip's power (counters, under the profiler: matrix cores busy 77 - 80 % of all cycles, 1.8 GHz of 2.4). Tried on it: k tiles of 32 in five stages (a direct load of sixteen 64 B rows takes longer than one of eight
  * 128 B rows: 1170 TFLOP/s), a second barrier that frees the stages earlier (2 - 4 % slower). */
 /* The per-head RMSNorm + rotary embedding of the leading columns of a projection, applied by the GEMM to its
  * own output tile (head_dim 128): columns [0, q_cols) are heads normalised with wq, [q_cols, qk_cols) with wk,
