@@ -359,8 +359,8 @@ int launch_1x1(hipStream_t st, float *out, const float *in, const uint16_t *W, c
  * eight waves that did everything (and stood still while a tile's stores landed), and now: 512 x 512 pixels, 128 -> 128
  * 30 + 118, 79, 73 us (the image and the result alone take 50 us to move), 256 -> 128 76 + 214, 129, 123, 256 -> 256 88 + 290,
  * 253, 235 us (1320 TFLOP/s). The first is bound by memory (matrix cores busy 43 - 45 % of its cycles), the last by the products
- * at the clock that the chip's power leaves (62 - 64 % at 1.9 - 2.0 GHz of 2.4; counters, under the profiler). Pixels and weights on waves
- * of their own (three and one) 1 % slower. */
+ * at the clock that the chip's power leaves (62 - 64 % at 1.9 - 2.0 GHz of 2.4; counters, under the profiler). Pixels and
+ * weights on waves of their own (three and one) 1 % slower. */
 constexpr int C3_T = 16, C3_H = C3_T + 2, C3_PIXELS = C3_H * C3_H, C3_ROW = 80, C3_IMG = C3_PIXELS * C3_ROW;   /* elements */
 constexpr int C3_N = 128, C3_STAGE = C3_N * 64;
 constexpr int C3_MUL = 8, C3_BRING = 4, C3_THREADS = 64 * (C3_MUL + C3_BRING);           /* waves that multiply, that bring pixels and weights */

@@ -5,9 +5,9 @@
  * accesses per lane where the pointers and sizes allow it, a scalar form of
  * the same kernel otherwise.
  *
- * Row normalisations use one workgroup per row, a wave for short rows, and
- * keep the row in registers between the statistics and the write (rows up to
- * 4096 floats; longer rows are read again, from cache).
+ * Row normalisations use one workgroup per row, a wave where rows are many and
+ * short (row_route), and keep the row in registers between the statistics and
+ * the write (rows up to 4096 floats; longer rows are read again, from cache).
  * Statistics follow the reference: LayerNorm takes the mean first and the
  * variance about it. Group norm takes its statistics in ONE pass over the
  * image (coalesced per-pixel reads, per-workgroup partial moments of every

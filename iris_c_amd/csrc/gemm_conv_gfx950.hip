@@ -6,7 +6,7 @@
  *
  * Both operands are K-contiguous, which is exactly what the matrix-core operand
  * layout wants (a lane holds 8 consecutive K elements of one row), so tiles go
- * HBM -> registers -> LDS unchanged. The product is issued transposed,
+ * from HBM to the LDS unchanged. The product is issued transposed,
  * D^T = W_tile x_tile^T with v_mfma_f32_16x16x32_bf16 (A = W rows, B = x rows): in
  * the 16x16 accumulator a lane then holds four consecutive n of one output row m,
  * a single 16-byte (f32) or 8-byte (bf16) store.
@@ -14,9 +14,9 @@
  * Products with too few 256-row tiles to fill the chip (short sequences) take k_gemm_tiles (gemm_tiles_gfx950.hip). For
  * the rest, three kernels. M, N >= 256 with K a multiple of 64 (every linear layer of the models at their
  * larger sequence lengths) take k_gemm_wide: tiles of 256 rows x 256 - 160 columns on eight waves, every memory
- * instruction in a gap between two products. One, three, five or seven k tiles of 64, outputs whose rows are not 16-byte aligned, and
- * the convolutions that have no kernel of their own take k_gemm_dma: the same tiles with the loads and reads in groups. Both
- * give the same bits. Everything else with K a multiple of 8 takes k_gemm_bf16:
+ * instruction in a gap between two products. One, three, five or seven k tiles of 64, outputs whose rows are not 16-byte
+ * aligned, and the convolutions that have no kernel of their own take k_gemm_dma: the same tiles with the loads and reads in
+ * groups. Both give the same bits. Everything else with K a multiple of 8 takes k_gemm_bf16:
  * Workgroup = WM x WN waves (2 x 2 in use), tile 128 (m) x 128 (n), K in steps of 64; a wave owns
  * 64 x 64 = 4 x 4 accumulator blocks and reads 8 operands from LDS per 16 MFMAs. One
  * LDS stage of [W tile | x tile], rows padded to 160 B so that the 16 lanes the LDS
@@ -28,7 +28,7 @@
  * of 8 with 16-byte aligned rows, otherwise the scalar kernel below takes over.
  *
  * Convolution with a handful of input or output channels (the VAE's first and last layers) has kernels of its own
- * (conv_gfx950.hip), and so has 3 x 3 with strides 1 and 2. Otherwise, with a multiple of 64 input channels it is an
+ * (conv_gfx950.hip), and so have 3 x 3 with strides 1 and 2 and 1 x 1, where these are the faster ones. Otherwise, with a multiple of 64 input channels it is an
  * implicit GEMM: the image is converted to bf16 once and k_gemm_dma fetches the pixels under each
  * tap itself, so the k x k patches are never written out. Other shapes gather the patches as bf16
  * rows into scratch (what the reference does for all of them, iris_cuda.cu:959-985) and run the
@@ -444,8 +444,9 @@ k_gemm_dma(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *
  * Against the kernel it replaces (four waves of 128 x 128, one per SIMD, staged through registers), weights from HBM, us:
  * 4608 x 3072 -> 9216 203 -> 188 (1390 TFLOP/s), -> 18432 408 -> 378, -> 27648 593 -> 566, 12288 -> 3072 257 -> 244, 9216 -> 3072
  * 195 -> 186. With everything in the L2 4096 x 8192 -> 4096, one round of workgroups, runs at 1530 TFLOP/s, 2060 on zeros: the
- * rest is the chip's power (counters, under the profiler: matrix cores busy 77 - 80 % of all cycles, 1.8 GHz of 2.4). Tried on it: k tiles of 32 in five stages (a direct load of sixteen 64 B rows takes longer than one of eight
- * 128 B rows: 1170 TFLOP/s), a second barrier that frees the stages earlier (2 - 4 % slower). */
+ * rest is the chip's power (counters, under the profiler: matrix cores busy 77 - 80 % of all cycles, 1.8 GHz of 2.4). Tried on
+ * it: k tiles of 32 in five stages (a direct load of sixteen 64 B rows takes longer than one of eight 128 B rows: 1170
+ * TFLOP/s), a second barrier that frees the stages earlier (2 - 4 % slower). */
 /* The per-head RMSNorm + rotary embedding of the leading columns of a projection, applied by the GEMM to its
  * own output tile (head_dim 128): columns [0, q_cols) are heads normalised with wq, [q_cols, qk_cols) with wk,
  * the rest is stored as it is. */

@@ -136,7 +136,7 @@ def test_tiles_that_normalise_themselves_match_oracle_chain_and_own_two_calls(de
 
 def test_vendor_backend_against_oracle(dev, orc):
     """With the vendor GEMM selected (2) and present the entry issues that GEMM and the norm kernel; without it the
-    one-launch kernel. Either way the oracle's chain is the yardstick."""
+    library's own form. Either way the oracle's chain is the yardstick."""
     c = make(5, 512, 256, 4, 4, 512)
     got, kernel = run(dev, c, True, 0, 2)
     assert kernel in ("norm_rope_hd128", "linear_mfma_qknorm")
