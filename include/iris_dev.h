@@ -139,7 +139,7 @@ void iris_dev_group_norm(float *out, const float *in, const float *gamma, const 
 /* No counterpart in the reference. The same operator for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc):
  * same arguments, same kernels and the same bits as iris_dev_group_norm, but its scratch (partial
- * moments and statistics, 787 KB) is an array inside the library instead of memory allocated at
+ * moments and statistics, 1.05 MB) is an array inside the library instead of memory allocated at
  * the first call, so this entry calls no hipMalloc / hipFree at all. groups <= 64; more is refused
  * with an error (use iris_dev_group_norm). All calls on a GPU share that one array: calls that
  * overlap in time would race, so keep them on the library's stream, which orders them. */

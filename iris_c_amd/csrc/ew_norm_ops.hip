@@ -9,18 +9,22 @@
  * short (row_route), and keep the row in registers between the statistics and
  * the write (rows up to 4096 floats; longer rows are read again, from cache).
  * Statistics follow the reference: LayerNorm takes the mean first and the
- * variance about it. Group norm takes its statistics in ONE pass over the
- * image (coalesced per-pixel reads, per-workgroup partial moments of every
- * group, merged in double by a small second kernel) and normalises in a
- * second pass; the partial moments and the final statistics live in a
- * scratch buffer the caller of the launcher provides.
+ * variance about it. Group norm of a large image is one launch that keeps
+ * what it can of the image on the chip between the statistics and the write.
+ * Of others it takes the statistics in ONE pass over the image (coalesced
+ * per-pixel reads, per-workgroup partial moments of every group, merged in
+ * double by a small second kernel) and normalises in a second pass. Moments
+ * and statistics live in a scratch buffer the caller of the launcher provides.
  */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "iris_kernels_hip.h"
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 namespace {
@@ -331,7 +335,7 @@ int launch_row_norm(hipStream_t st, uint16_t *out_bf, float *xres, const float *
 
 /* ---------------------------------------------------------------- group norm
  *
- * Two passes over the image in all: one for the statistics, one that normalises.
+ * Large images as one launch (k_gn_resident below); else two passes over the image, one for the statistics, one that normalises.
  *
  * Statistics in ONE pass: a thread sums (x - K) and (x - K)^2 over its share of a group, K being
  * the first value it reads. K is a sample of the data, so the sums stay of the size of the
@@ -505,6 +509,284 @@ k_gn_normalize(float *__restrict__ out, const float *__restrict__ in, const floa
     else out[i] = v[0];
 }
 
+/* ---- the whole norm as one launch, from 8 MB on ----
+ *
+ * One workgroup per CU: each reads its share of the image once, keeps as much of it as its registers and LDS hold (KEEP steps of
+ * 8 KB: 138 MB in all), leaves the moments of its share, waits for the image's statistics, and writes the share normalised; only
+ * what it could not keep is read a second time, the newest first, a part of which the Infinity Cache still holds. Step i of
+ * workgroup b is step 256 i + b of the image, so that the chip streams through one run of memory at any time (a run of memory per
+ * workgroup: 512 x 512 x 256 146 us, this way 143). Stores carry the streaming hint: they leave the L2 as they are issued and
+ * not at the end of the kernel (143 -> 114 us, 1024 x 1024 x 128 278 -> 247).
+ * Bound by the memory in both directions (134 MB read in 20 us), 5 - 6 us between the last value read and the first written, and
+ * the launch. Against statistics, their sum and normalising as three launches, f32 image from memory, us:
+ * 16384 x 512 26.7 -> 20.1, 65536 x 256 45 -> 30, 384 x 384 x 128 50 -> 33, 512 x 512 x 128 82 -> 52, 512 x 512 x 256 155 -> 114,
+ * 700 x 700 x 128 146 -> 109, 1024 x 1024 x 128 294 -> 247; 4096 x 512 (8 MB) 13.4 / 13.1, 1024 x 512 10.0 / 11.6: the line.
+ *
+ * Everything between workgroups is a word with the number of the launch in its high half (Tagged), so that no store has to be
+ * waited for and nothing is cleared between launches: a workgroup leaves the moments of its share, workgroup g < groups
+ * gathers those of group g and leaves the group's statistics, all wait for these. With fences of the memory model and every
+ * workgroup gathering all groups the wait took 25 us in place of 5.
+ *
+ * The wait is bounded and needs no workgroup to be resident beside another: one that has waited for `patience` ticks of 10 ns
+ * (another process may hold CUs) gives up its share: it notes that in the counter of arrivals and in its flag and ends. The
+ * counter takes such a note only while a workgroup is missing, so the one that arrives last knows how many there are, gathers
+ * all groups, as the workgroups meant to may be among them, and normalises their shares itself. What is on its way once all have
+ * arrived is looked for RES_LATE times, so that calls that share a scratch buffer and overlap, which the callers rule out, get
+ * wrong values and not a wait without end. */
+constexpr int RES_WGS = 256, RES_THREADS = 512, RES_REG = 48, RES_LDS = 18, RES_KEEP = RES_REG + RES_LDS, RES_BATCH = 8, RES_LDS_BATCH = 6;
+constexpr unsigned RES_STRIDE = RES_WGS * RES_THREADS;
+constexpr int RES_LDS_BYTES = RES_LDS * RES_THREADS * 16;
+constexpr int RES_MIN_GROUPS = 8, RES_MAX_GROUPS = 64;         /* a group's threads are at most a wave; a wave gathers the statistics */
+constexpr size_t RES_MIN_BYTES = (size_t)8 << 20;
+constexpr unsigned RES_PATIENCE = 1000000, RES_LATE = 1u << 20;
+struct Tagged { unsigned long long a, b; };                    /* two floats, each with the number of the launch in its high half */
+struct ResidentSync {
+    unsigned long long arrivals;                               /* of all launches; + 2^48 for each workgroup of this launch that gave up */
+    unsigned pad[30], gave_up[RES_WGS];
+    Tagged stat[RES_MAX_GROUPS], part[RES_MAX_GROUPS][RES_WGS];
+};
+constexpr size_t SYNC_FLOATS = sizeof(ResidentSync) / sizeof(float);
+
+__global__ void __launch_bounds__(ROW_THREADS)
+k_gn_clear(unsigned *sync) {
+    for (unsigned i = threadIdx.x; i < SYNC_FLOATS; i += ROW_THREADS) sync[i] = 0u;
+}
+
+template <typename T> __device__ __forceinline__ T agent_load(const T *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+template <typename T> __device__ __forceinline__ void agent_store(T *p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+template <bool SILU>
+__global__ void __launch_bounds__(RES_THREADS, 2)
+k_gn_resident(f32x4 *out, const f32x4 *in, const float *__restrict__ gamma, const float *__restrict__ beta, ResidentSync *sync,
+              unsigned total, int c, int cg, float eps, unsigned patience) {
+    extern __shared__ f32x4 kept[];                            /* [RES_LDS][RES_THREADS] */
+    __shared__ float2 sh[RES_THREADS];
+    __shared__ float stat[2 * RES_MAX_GROUPS];
+    __shared__ unsigned verdict, to_do;
+    const unsigned tid = threadIdx.x, b = blockIdx.x;
+    const int quads = c >> 2, q = tid % quads, groups = c / cg, group = 4 * q / cg;
+    /* a step is 512 quads in a row: whole pixels, so a thread keeps its quad of channels. n: this workgroup's steps */
+    const unsigned steps = (total + RES_THREADS - 1) / RES_THREADS;
+    auto steps_of = [&](unsigned w) { return w < steps ? (steps - w + RES_WGS - 1) / RES_WGS : 0; };
+    const unsigned n = steps_of(b), at0 = b * RES_THREADS + tid;
+    auto load = [&](unsigned i) { return in[min(at0 + i * RES_STRIDE, total - 1)]; };
+    constexpr unsigned long long ARRIVALS = (1ull << 48) - 1;
+    /* the number of this launch, the same in all workgroups as this one has not arrived yet */
+    const unsigned epoch = (unsigned)((agent_load(&sync->arrivals) & ARRIVALS) / RES_WGS) + 1;
+
+    /* moments of this thread's values, shifted by the first value of the workgroup's share of the group; sums of a batch at a time */
+    float k = 0.0f, s = 0.0f, ss = 0.0f;
+    if (n > 0) k = reinterpret_cast<const float *>(in)[(size_t)b * RES_THREADS * 4 + group * cg];
+    auto take = [&](const f32x4 *v, unsigned i0, auto batch) {
+        float bs = 0.0f, bss = 0.0f;
+#pragma unroll
+        for (int j = 0; j < batch(); j++)
+            if (i0 + j < n && at0 + (i0 + j) * RES_STRIDE < total) {
+                const float a0 = v[j][0] - k, a1 = v[j][1] - k, a2 = v[j][2] - k, a3 = v[j][3] - k;
+                bs += (a0 + a1) + (a2 + a3);
+                bss += (a0 * a0 + a1 * a1) + (a2 * a2 + a3 * a3);
+            }
+        s += bs;
+        ss += bss;
+    };
+    /* what cannot be kept, two batches in flight */
+    if (n > RES_KEEP) {
+        const std::integral_constant<int, RES_BATCH> batch;
+        unsigned i = RES_KEEP;
+        for (; (n - i) % RES_BATCH; i++) { const f32x4 v = load(i); take(&v, i, std::integral_constant<int, 1>{}); }
+        f32x4 v[2][RES_BATCH];
+        auto fetch = [&](f32x4 *dst, unsigned at) {
+#pragma unroll
+            for (int j = 0; j < RES_BATCH; j++) dst[j] = load(at + j);
+        };
+        if (i < n) {                                           /* no request behind a branch: the wait for it would be for all */
+            fetch(v[0], i);
+            for (; i + 2 * RES_BATCH < n; i += 2 * RES_BATCH) {
+                fetch(v[1], i + RES_BATCH);
+                take(v[0], i, batch);
+                fetch(v[0], i + 2 * RES_BATCH);
+                take(v[1], i + RES_BATCH, batch);
+            }
+            if (i + RES_BATCH < n) {
+                fetch(v[1], i + RES_BATCH);
+                take(v[0], i, batch);
+                take(v[1], i + RES_BATCH, batch);
+            } else {
+                take(v[0], i, batch);
+            }
+        }
+    }
+    f32x4 keep[RES_REG];
+    for (int g = 0; g < RES_LDS && RES_REG + g < n; g += RES_LDS_BATCH) {
+        f32x4 v[RES_LDS_BATCH];
+#pragma unroll
+        for (int j = 0; j < RES_LDS_BATCH; j++) v[j] = load(min(RES_REG + g + j, n - 1));
+#pragma unroll
+        for (int j = 0; j < RES_LDS_BATCH; j++) kept[(g + j) * RES_THREADS + tid] = v[j];
+        take(v, RES_REG + g, std::integral_constant<int, RES_LDS_BATCH>{});
+    }
+#pragma unroll
+    for (int g = 0; g < RES_REG; g += RES_BATCH)
+        if (g < n)
+#pragma unroll
+            for (int j = 0; j < RES_BATCH; j++) keep[g + j] = load(min(g + j, n - 1));
+#pragma unroll
+    for (int g = 0; g < RES_REG; g += RES_BATCH)
+        if (g < n) take(keep + g, g, std::integral_constant<int, RES_BATCH>{});
+
+    /* values of a group in the share of workgroup w; the last step may be a part of one */
+    auto values_of = [&](unsigned w) {
+        return (float)(steps_of(w) * RES_THREADS - ((steps - 1) % RES_WGS == w ? steps * RES_THREADS - total : 0)) * (4.0f / (float)groups);
+    };
+    auto put = [&](Tagged *t, float x, float y) {
+        agent_store(&t->a, (unsigned long long)epoch << 32 | __float_as_uint(x));
+        agent_store(&t->b, (unsigned long long)epoch << 32 | __float_as_uint(y));
+    };
+    const f32x4 ga = *reinterpret_cast<const f32x4 *>(gamma + 4 * q), be = *reinterpret_cast<const f32x4 *>(beta + 4 * q);
+    /* lanes: a power of two, at most a wave; the share's moments of group g */
+    const int lanes = RES_THREADS / groups, g = tid / lanes, l = tid % lanes;
+    sh[tid] = make_float2(s, ss);
+    if (4 * q == group * cg && tid < (unsigned)quads) stat[group] = k;
+    __syncthreads();
+    {
+        const int qpg = cg >> 2;
+        float2 t = sh[l / qpg * quads + g * qpg + l % qpg];
+        for (int off = lanes / 2; off > 0; off >>= 1) { t.x += __shfl_xor(t.x, off, 64); t.y += __shfl_xor(t.y, off, 64); }
+        if (l == 0) {
+            const float num = values_of(b), mean = t.x / num;
+            put(&sync->part[g][b], n > 0 ? stat[g] + mean : 0.0f, n > 0 ? fmaxf(t.y - t.x * mean, 0.0f) : 0.0f);
+        }
+    }
+    /* The first wave waits for the workgroup. */
+    unsigned quitters = 0;
+    if (tid < 64) {
+        unsigned long long before = 0;
+        if (tid == 0) before = __hip_atomic_fetch_add(&sync->arrivals, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned long long t0 = wall_clock64();
+        /* until the entry is this launch's in all lanes; false: this workgroup has given up its share */
+        auto wait = [&](const Tagged *t, bool wanted, auto &x, auto &y) {
+            constexpr int N = sizeof(x) / sizeof(float);
+            for (unsigned late = 0; late < RES_LATE;) {
+                unsigned long long va[N], vb[N];
+#pragma unroll
+                for (int i = 0; i < N; i++) {
+                    va[i] = vb[i] = 0;
+                    if (wanted) { va[i] = agent_load(&t[64 * i].a); vb[i] = agent_load(&t[64 * i].b); }
+                }
+                bool here = true;
+#pragma unroll
+                for (int i = 0; i < N; i++) {
+                    x[i] = __uint_as_float((unsigned)va[i]);
+                    y[i] = __uint_as_float((unsigned)vb[i]);
+                    here = here && (unsigned)(va[i] >> 32) == epoch && (unsigned)(vb[i] >> 32) == epoch;
+                }
+                if (__all(!wanted || here)) return true;
+                if (wall_clock64() - t0 < patience) continue;
+                int gave_up = 0;
+                if (tid == 0) {
+                    unsigned long long seen = agent_load(&sync->arrivals);
+                    while (!gave_up && (unsigned)((seen & ARRIVALS) / RES_WGS) != epoch)
+                        gave_up = __hip_atomic_compare_exchange_strong(&sync->arrivals, &seen, seen + (1ull << 48), __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (gave_up) agent_store(&sync->gave_up[b], 1u);
+                }
+                if (__any(gave_up)) return false;
+                late++;                                        /* all have arrived */
+            }
+            return true;
+        };
+        /* a group's statistics from the moments of all shares, in double */
+        auto finish = [&](unsigned gr) {
+            constexpr int N = RES_WGS / 64;
+            double sum = 0.0, sq = 0.0;
+            float m[N], m2[N];
+            if (!wait(&sync->part[gr][tid], true, m, m2)) return false;
+#pragma unroll
+            for (int i = 0; i < N; i++) {
+                const double weighted = (double)values_of(64 * i + tid) * (double)m[i];
+                sum += weighted;
+                sq += (double)m2[i] + weighted * (double)m[i];
+            }
+            sum = wave_sum64(sum);
+            sq = wave_sum64(sq);
+            const double num = (double)total * (4.0 / (double)groups), mean = sum / num;
+            if (tid == 0) put(&sync->stat[gr], (float)mean, (float)(1.0 / sqrt(fmax(sq / num - mean * mean, 0.0) + (double)eps)));
+            return true;
+        };
+        bool go = b >= (unsigned)groups || finish(b);
+            if (go) {
+            /* last to arrive: those that had given up by then (ARRIVALS is a multiple of the number less one) */
+            quitters = __builtin_amdgcn_readfirstlane((before + 1) % RES_WGS == 0 ? (unsigned)(before >> 48) : 0u);
+            if (quitters)
+                for (unsigned gr = 0; gr < (unsigned)groups; gr++) (void)finish(gr);          /* theirs may be among them */
+            float m[1], r[1];
+            go = wait(&sync->stat[tid], tid < (unsigned)groups, m, r);
+            if (tid < (unsigned)groups) { stat[tid] = m[0]; stat[RES_MAX_GROUPS + tid] = r[0]; }
+        }
+        if (tid == 0) { verdict = go; to_do = quitters; }
+    }
+    __syncthreads();
+    if (!verdict) return;
+    quitters = to_do;
+    const float mean = stat[group], rstd = stat[RES_MAX_GROUPS + group];
+    auto one = [&](float v, float g, float bt) { const float y = (v - mean) * rstd * g + bt; return SILU ? silu(y) : y; };
+    auto store = [&](unsigned at, const f32x4 v) {
+        if (at < total) __builtin_nontemporal_store(f32x4{one(v[0], ga[0], be[0]), one(v[1], ga[1], be[1]), one(v[2], ga[2], be[2]), one(v[3], ga[3], be[3])}, out + at);
+    };
+    /* steps first .. end - 1 from memory, the last first */
+    auto again = [&](unsigned first, unsigned end, unsigned at) {
+        if (first >= end) return;
+        f32x4 v[2][RES_BATCH];
+        auto fetch = [&](f32x4 *dst, unsigned from) {
+#pragma unroll
+            for (int j = 0; j < RES_BATCH; j++) dst[j] = in[min(at + (from + j) * RES_STRIDE, total - 1)];
+        };
+        auto put = [&](const f32x4 *src, unsigned from) {
+#pragma unroll
+            for (int j = RES_BATCH - 1; j >= 0; j--) store(at + (from + j) * RES_STRIDE, src[j]);
+        };
+        for (; (end - first) % RES_BATCH; end--) store(at + (end - 1) * RES_STRIDE, in[min(at + (end - 1) * RES_STRIDE, total - 1)]);
+        if (first >= end) return;
+        fetch(v[0], end - RES_BATCH);
+        for (; end - first > 2 * RES_BATCH; end -= 2 * RES_BATCH) {
+            fetch(v[1], end - 2 * RES_BATCH);
+            put(v[0], end - RES_BATCH);
+            fetch(v[0], end - 3 * RES_BATCH);
+            put(v[1], end - 2 * RES_BATCH);
+        }
+        if (end - first > RES_BATCH) {
+            fetch(v[1], first);
+            put(v[0], end - RES_BATCH);
+            put(v[1], first);
+        } else {
+            put(v[0], first);
+        }
+    };
+#pragma unroll
+    for (int g = 0; g < RES_REG; g++)
+        if (g < n) store(at0 + g * RES_STRIDE, keep[g]);
+    for (int g = 0; g < RES_LDS && RES_REG + g < n; g++) store(at0 + (RES_REG + g) * RES_STRIDE, kept[g * RES_THREADS + tid]);
+    again(RES_KEEP, n, at0);
+
+    if (quitters) {
+        if (tid == 0) __hip_atomic_fetch_add(&sync->arrivals, -((unsigned long long)quitters << 48), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        unsigned left = quitters;
+        for (unsigned sweep = 0; left > 0 && sweep < RES_LATE; sweep++)
+            for (unsigned w = 0; w < RES_WGS; w++) {
+                if (tid == 0) {
+                    const unsigned f = agent_load(&sync->gave_up[w]);
+                    if (f) agent_store(&sync->gave_up[w], 0u);
+                    verdict = f;
+                }
+                __syncthreads();
+                const unsigned f = verdict;
+                __syncthreads();
+                if (!f) continue;
+                left--;
+                again(0, steps_of(w), w * RES_THREADS + tid);
+            }
+    }
+}
+
 }  // namespace
 
 extern "C" {
@@ -573,16 +855,46 @@ int iris_hip_rms_norm_residual(void *stream, float *x, const float *a, const flo
     return launch_row_norm<RMS_NORM_RESIDUAL>((hipStream_t)stream, nullptr, x, a, w, gate, rows, dim, eps);
 }
 
-size_t iris_hip_group_norm_scratch_floats(int groups) { return 3 * (size_t)groups * GN_MAX_BLOCKS + 2 * (size_t)groups; }
+size_t iris_hip_group_norm_scratch_floats(int groups) { return SYNC_FLOATS + 3 * (size_t)groups * GN_MAX_BLOCKS + 2 * (size_t)groups; }
 
-/* scratch: iris_hip_group_norm_scratch_floats(groups) floats of device memory. Every slot a call
- * reads (partial moments [group][workgroup], statistics [2][group]) is written by that call first. */
+/* Once for a new scratch buffer: the counters of k_gn_resident, zero between calls. */
+int iris_hip_group_norm_prepare_scratch(void *stream, float *scratch) {
+    hipLaunchKernelGGL(k_gn_clear, dim3(1), dim3(ROW_THREADS), 0, (hipStream_t)stream, reinterpret_cast<unsigned *>(scratch));
+    return (int)hipGetLastError();
+}
+
+/* The norm as one launch: -2, with nothing enqueued, for what it does not take: it wants a thread to keep one quad of channels
+ * through all its steps, and 32-bit byte offsets. scratch as below; patience in ticks of 10 ns. */
+int iris_hip_group_norm_resident(void *stream, float *scratch, float *out, const float *in, const float *gamma, const float *beta,
+                                 int hw, int c, int groups, float eps, int do_silu, unsigned patience) {
+    if (hw <= 0 || c <= 0 || groups < RES_MIN_GROUPS || groups > RES_MAX_GROUPS || c % groups) return -2;
+    const int cg = c / groups;
+    const size_t total = (size_t)hw * c / 4;
+    if (cg % 4 || RES_THREADS % (c / 4) || !al16(in) || !al16(out) || !al16(gamma) || !al16(beta) || total >= 1u << 28) return -2;
+    auto go = [&](auto kernel) {
+        static const hipError_t configured =
+            hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, RES_LDS_BYTES);
+        if (configured != hipSuccess) return (int)configured;
+        hipLaunchKernelGGL(kernel, dim3(RES_WGS), dim3(RES_THREADS), RES_LDS_BYTES, (hipStream_t)stream, reinterpret_cast<f32x4 *>(out),
+                           reinterpret_cast<const f32x4 *>(in), gamma, beta, reinterpret_cast<ResidentSync *>(scratch), (unsigned)total, c, cg, eps,
+                           patience);
+        return (int)hipGetLastError();
+    };
+    return do_silu ? go(k_gn_resident<true>) : go(k_gn_resident<false>);
+}
+
+/* scratch: iris_hip_group_norm_scratch_floats(groups) floats of device memory, prepared once. Behind the counters every slot a
+ * call reads (partial moments [group][workgroup], statistics [2][group]) is written by that call first. */
 int iris_hip_group_norm(void *stream, float *scratch, float *out, const float *in, const float *gamma,
                         const float *beta, int hw, int c, int groups, float eps, int do_silu) {
     if (hw <= 0 || c <= 0) return 0;
+    if ((size_t)hw * c * sizeof(float) >= RES_MIN_BYTES) {
+        const int e = iris_hip_group_norm_resident(stream, scratch, out, in, gamma, beta, hw, c, groups, eps, do_silu, RES_PATIENCE);
+        if (e != -2) return e;
+    }
     hipStream_t st = (hipStream_t)stream;
-    Moments *part = reinterpret_cast<Moments *>(scratch);
-    float *stats = scratch + 3 * (size_t)groups * GN_MAX_BLOCKS;
+    Moments *part = reinterpret_cast<Moments *>(scratch + SYNC_FLOATS);
+    float *stats = scratch + SYNC_FLOATS + 3 * (size_t)groups * GN_MAX_BLOCKS;
     const int cg = c / groups;
     const bool quads_form = c % 4 == 0 && cg % 4 == 0 && c / 4 <= ROW_THREADS && ROW_THREADS % (c / 4) == 0 && al16(in);
     int nblocks;
@@ -617,8 +929,8 @@ int iris_hip_group_norm(void *stream, float *scratch, float *out, const float *i
  * get the address that call returned, kept per device. Calls on one GPU share the array: they must
  * not overlap (the library issues everything on one stream, which orders them). */
 constexpr int GN_STATIC_MAX_GROUPS = 64;
-constexpr size_t GN_STATIC_FLOATS = 3 * (size_t)GN_STATIC_MAX_GROUPS * GN_MAX_BLOCKS + 2 * (size_t)GN_STATIC_MAX_GROUPS;
-static __device__ __align__(256) float scratch[GN_STATIC_FLOATS];          /* 786,944 B */
+constexpr size_t GN_STATIC_FLOATS = SYNC_FLOATS + 3 * (size_t)GN_STATIC_MAX_GROUPS * GN_MAX_BLOCKS + 2 * (size_t)GN_STATIC_MAX_GROUPS;
+static __device__ __align__(256) float scratch[GN_STATIC_FLOATS];          /* 1,051,264 B, zero when the library is loaded */
 
 constexpr int GN_STATIC_MAX_DEVICES = 64;
 static float *scratch_address[GN_STATIC_MAX_DEVICES];                        /* per device; null = not looked up yet */

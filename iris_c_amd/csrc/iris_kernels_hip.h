@@ -118,9 +118,12 @@ int iris_hip_rms_norm_mod(void *stream, uint16_t *out, const float *x, const flo
                           const float *scale, int rows, int dim, float eps);
 int iris_hip_rms_norm_residual(void *stream, float *x, const float *a, const float *w,
                                const float *gate, int rows, int dim, float eps);
-/* group norm needs iris_hip_group_norm_scratch_floats(groups) floats of device scratch;
- * requires c % groups == 0 */
+/* group norm needs iris_hip_group_norm_scratch_floats(groups) floats of device scratch, prepared once;
+ * requires c % groups == 0. The resident form (-2: not taken) is the one launch that large images take. */
 size_t iris_hip_group_norm_scratch_floats(int groups);
+int iris_hip_group_norm_prepare_scratch(void *stream, float *scratch);
+int iris_hip_group_norm_resident(void *stream, float *scratch, float *out, const float *in, const float *gamma,
+                                 const float *beta, int hw, int c, int groups, float eps, int do_silu, unsigned patience);
 int iris_hip_group_norm(void *stream, float *scratch, float *out, const float *in, const float *gamma,
                         const float *beta, int hw, int c, int groups, float eps, int do_silu);
 

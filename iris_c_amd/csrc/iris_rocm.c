@@ -608,6 +608,13 @@ void iris_dev_group_norm(float *out, const float *in, const float *gamma, const 
             fail(-1, "group_norm", "scratch allocation failed");
             return;
         }
+        int e = iris_hip_group_norm_prepare_scratch(g_stream, g_gn_scratch);
+        if (e) {
+            check((hipError_t)e, "group_norm scratch");
+            check(hipFree(g_gn_scratch), "free");
+            g_gn_scratch = NULL;
+            return;
+        }
         g_gn_scratch_floats = need;
     }
     int err = iris_hip_group_norm(g_stream, g_gn_scratch, out, in, gamma, beta, hw, c, groups, eps, silu != 0);

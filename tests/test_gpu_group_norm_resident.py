@@ -1,0 +1,134 @@
+"""Group norm as one launch (k_gn_resident), through its launcher so that every size takes it, against float64: workgroups with
+no, one and all steps kept, in registers, in the LDS and beyond both, images that end inside a step, in place, and workgroups
+that give up their share at once (patience 0: the last one to arrive does theirs) between ordinary calls on the same scratch."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from gpu_harness import Dev
+
+pytestmark = pytest.mark.gpu
+WGS, REG, KEEP, BATCH = 256, 48, 66, 8                         # workgroups; steps of 2048 floats kept in registers, in all; read at a time
+NOT_TAKEN = -2
+
+
+@pytest.fixture(scope="module")
+def dev():
+    d = Dev()
+    d.lib.iris_hip_group_norm_scratch_floats.restype = C.c_size_t
+    d.stream = C.c_void_p(d.lib.iris_dev_stream())
+    d.scratch = C.c_void_p(d.lib.iris_dev_alloc(4 * d.lib.iris_hip_group_norm_scratch_floats(64)))
+    assert d.lib.iris_hip_group_norm_prepare_scratch(d.stream, d.scratch) == 0
+    return d
+
+
+def resident(dev, out, img, gamma, beta, hw, c, groups, silu, patience=1000000):
+    ptrs = [C.c_void_p(p) for p in (out, img, gamma, beta)]
+    return dev.lib.iris_hip_group_norm_resident(dev.stream, dev.scratch, *ptrs, hw, c, groups, C.c_float(1e-6), silu, C.c_uint(patience))
+
+
+def data(hw, c):
+    rng = np.random.default_rng(hw + c)
+    x = rng.standard_normal((hw, c), dtype=np.float32) * 2 + 0.5 + 0.01 * np.arange(c, dtype=np.float32)
+    return x, (1 + 0.1 * rng.standard_normal(c)).astype(np.float32), (0.1 * rng.standard_normal(c)).astype(np.float32)
+
+
+def expected(x, gamma, beta, groups, silu):
+    hw, c = x.shape
+    y = x.astype(np.float64).reshape(hw, groups, c // groups)
+    y -= y.mean(axis=(0, 2), keepdims=True)
+    y /= np.sqrt((y ** 2).mean(axis=(0, 2), keepdims=True) + 1e-6)
+    y = y.reshape(hw, c) * gamma + beta
+    return y / (1 + np.exp(-y)) if silu else y
+
+
+def compare(got, want):
+    # f32: the mean, three products and a sum of values up to 6 are each off by half a unit in the last place, 2^-22 there, and
+    # the statistics by a few 2^-24
+    np.testing.assert_allclose(got, want, atol=6 * 2.0 ** -20)
+
+
+def steps(n, c):
+    """pixels of n steps"""
+    return n * 2048 // c
+
+
+# hw, c, groups, silu
+CASES = [(1, 128, 32, 1), (15, 128, 32, 0), (17, 128, 32, 1), (steps(255, 512) + 1, 512, 32, 0), (steps(WGS, 128) - 3, 128, 32, 1),
+         (steps(WGS * BATCH, 64) + 5, 64, 16, 0), (steps(WGS * BATCH + 1, 64), 64, 8, 1), (steps(WGS * 9, 256) + 3, 256, 64, 1),
+         (steps(WGS * REG, 128), 128, 32, 0), (steps(WGS * REG + 7, 128) + 1, 128, 32, 1), (steps(WGS * (REG + 7), 256), 256, 32, 1),
+         (steps(WGS * KEEP, 128), 128, 32, 1), (steps(WGS * KEEP, 128) + 1, 128, 32, 0), (steps(WGS * (KEEP + 1) + 40, 128) + 3, 128, 32, 1),
+         (steps(WGS * (KEEP + BATCH) + 9, 512), 512, 32, 1), (steps(WGS * (KEEP + 3 * BATCH + 3), 128) + 7, 128, 32, 1)]
+
+
+@pytest.mark.parametrize("hw,c,groups,silu", CASES)
+def test_sizes(dev, hw, c, groups, silu):
+    x, gamma, beta = data(hw, c)
+    dx, dg, db = dev.put(x), dev.put(gamma), dev.put(beta)
+    dout = dev.put(np.full((hw + 1, c), np.nan, np.float32))
+    assert resident(dev, dout, dx, dg, db, hw, c, groups, silu) == 0
+    assert resident(dev, dx, dx, dg, db, hw, c, groups, silu) == 0                           # in place
+    got, same = dev.get(dout, (hw + 1, c), np.float32), dev.get(dx, (hw, c), np.float32)
+    dev.free_all()
+    compare(got[:hw], expected(x, gamma, beta, groups, silu))
+    assert np.isnan(got[hw]).all()                                                           # nothing behind the image
+    np.testing.assert_array_equal(got[:hw], same)
+
+
+@pytest.mark.parametrize("hw,c", [(5, 128), (steps(WGS * 2 + 9, 128) + 3, 128), (steps(WGS * (KEEP + 1) + 5, 128) + 1, 128)])
+def test_shares_that_are_given_up(dev, hw, c):
+    """Counters and flags as an ordinary call leaves them: the same bits before, with and after impatient calls."""
+    x, gamma, beta = data(hw, c)
+    dx, dg, db, dout = dev.put(x), dev.put(gamma), dev.put(beta), dev.alloc(hw * c * 4)
+    outs = []
+    for patience in (1000000, 0, 0, 1000000, 0):
+        dev.dev.lib.iris_dev_upload(dout, np.full((hw, c), np.nan, np.float32).ctypes.data_as(C.c_void_p), hw * c * 4)
+        assert resident(dev, dout, dx, dg, db, hw, c, 32, 1, patience) == 0
+        outs.append(dev.get(dout, (hw, c), np.float32))
+    dev.free_all()
+    compare(outs[0], expected(x, gamma, beta, 32, 1))
+    for o in outs[1:]:
+        np.testing.assert_array_equal(outs[0], o)
+
+
+def test_what_it_does_not_take(dev):
+    hw = 64
+    p = dev.alloc(hw * 512 * 4 + 16)
+    for c, groups, shift in ((96, 32, 0), (128, 4, 0), (512, 128, 0), (64, 32, 0), (128, 32, 4), (4096, 32, 0)):
+        assert resident(dev, p + shift, p, p, p, hw, c, groups, 0) == NOT_TAKEN, (c, groups, shift)
+    assert resident(dev, p, p, p, p, (1 << 28) // 32, 128, 32, 0) == NOT_TAKEN               # 4 GiB
+    dev.free_all()
+
+
+@pytest.mark.parametrize("hw", [16383, 16384])                 # 8 MB: the first size that takes it, and the last that does not
+def test_both_sides_of_the_line(dev, hw):
+    x, gamma, beta = data(hw, 128)
+    dx, dg, db, dout = dev.put(x), dev.put(gamma), dev.put(beta), dev.alloc(hw * 128 * 4)
+    dev.lib.iris_dev_group_norm(dout, dx, dg, db, hw, 128, 32, 1e-6, 1)
+    dev.check()
+    got = dev.get(dout, (hw, 128), np.float32)
+    dev.free_all()
+    compare(got, expected(x, gamma, beta, 32, 1))
+
+
+def test_replayed_from_a_graph(dev):
+    from test_gpu_graph import Graphs
+    hw, c, lib, g = 20000, 128, dev.lib, Graphs()
+    x, gamma, beta = data(hw, c)
+    dx, dg, db, dout, deager = dev.put(x), dev.put(gamma), dev.put(beta), dev.alloc(hw * c * 4), dev.alloc(hw * c * 4)
+    norm = lambda out: lib.iris_dev_group_norm_noalloc(out, dx, dg, db, hw, c, 32, 1e-6, 1)
+    norm(deager)
+    want = dev.get(deager, (hw, c), np.float32)
+    run = g.capture(dev.stream, lambda: norm(dout))
+    for _ in range(4):
+        lib.iris_dev_upload(dout, np.full((hw, c), np.nan, np.float32).ctypes.data_as(C.c_void_p), hw * c * 4)
+        assert g.rt.hipGraphLaunch(run, dev.stream) == 0
+        lib.iris_dev_sync()
+        np.testing.assert_array_equal(dev.get(dout, (hw, c), np.float32), want)
+        norm(deager)
+        np.testing.assert_array_equal(dev.get(deager, (hw, c), np.float32), want)
+    g.rt.hipGraphExecDestroy(run)
+    dev.check()
+    dev.free_all()
+    compare(want, expected(x, gamma, beta, 32, 1))
