@@ -480,6 +480,12 @@ k_gemm_wide(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t 
     const int band_rows = min(tiles_m - band * BAND, BAND);
     const int m0 = (band * BAND + in_band % band_rows) * TM, n0 = in_band / band_rows * TN;
     const int last_tile = K / TK - 1;
+    /* The workgroups that share rows of W or x run in step; they take the k tiles of a group of four in different orders, so
+     * that one of them brings a line from HBM and the others find it in the L2 (gemm_tiles_gfx950.hip has the reasons); by the
+     * tile row alone, so that all widths add in the same order. All in one order / turned, us: 512 x 2560 -> 19456 49.1 / 47.4,
+     * 512 x 3072 -> 27648 73.8 / 71.2, 1024 x 2560 -> 19456 96.3 / 92.5; 4608 rows within 1 %. */
+    const int turn = (m0 / TM) & 3, turned = (last_tile + 1) & ~3;
+    auto source = [&](int kt) { return (size_t)(kt < turned ? kt ^ turn : kt) * TK; };
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4, wm = wave & 3, wn = wave >> 2;
 
@@ -502,11 +508,11 @@ k_gemm_wide(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t 
     const uint32_t lds0 = lds_address(dlds);
     auto request_x = [&](int j, int kt, uint32_t stage) {      /* stage: bytes into the LDS */
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                     ::"s"(lds0 + stage + (4 * wave + j) * 1024), "v"(xoff[j]), "s"(x_tile + (size_t)kt * TK) : "memory", "m0");
+                     ::"s"(lds0 + stage + (4 * wave + j) * 1024), "v"(xoff[j]), "s"(x_tile + source(kt)) : "memory", "m0");
     };
     auto request_w = [&](int j, int kt, uint32_t stage) {
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                     ::"s"(lds0 + stage + wpiece[j] * 1024), "v"(woff[j]), "s"(w_tile + (size_t)kt * TK) : "memory", "m0");
+                     ::"s"(lds0 + stage + wpiece[j] * 1024), "v"(woff[j]), "s"(w_tile + source(kt)) : "memory", "m0");
     };
 
     f32x4 acc[NA][4];                                          /* [16 columns][16 rows] */

@@ -9,13 +9,27 @@
  * K into ranges that different workgroups multiply: each leaves f32 partial sums in a workspace and k_gemm_sum adds
  * them in order (no atomics: a call gives the same bits every time).
  *
- * A workgroup is WM x WN waves of 16 NB rows x 16 NA columns, in KG groups: with KG = 2 both halves of the workgroup
+ * A workgroup is WM x WN waves (eight, or four) of 16 NB rows x 16 NA columns, in KG groups: with KG = 2 both halves of the workgroup
  * own the same outputs and take one k-step of 32 each of every k tile of 64, and add their sums through the LDS at the
  * end. That keeps 64 x 64 outputs per wave, i.e. half an LDS read per product, on a tile of 128 x 128. W and x rows go
  * from memory straight into a ring of STAGES LDS stages (128 B rows, 16 B chunk c of row r in slot c ^ ((r >> 1) & 7),
  * which keeps the 128-bit reads off each other's banks, see k_gemm_dma); weights come from HBM here, so the ring is as
  * deep as the LDS allows. In front of the barrier of a k tile a wave waits for its own share of the next tile and for
  * its last operand reads of this one; behind it the stage is free and is requested again, STAGES tiles ahead.
+ *
+ * What bounds it is the fetch of the weights. A CU has at most the 32 KB of its vector cache in flight: rows from HBM
+ * come at 50 GB/s a CU, rows from the L2 at 125 (direct loads by themselves, 32 to 64 workgroups on their own lines), and a
+ * workgroup that only fetched its tiles and multiplied nothing took nine tenths of the whole kernel's time. The workgroups that
+ * share W rows (one column of tiles) or x rows run in step, so each of them would wait for HBM for the same lines. Instead
+ * they take the k tiles of a group of four in different orders (tile kt of the order is k tile kt ^ turn, turn = the tile's
+ * row ^ its column, mod 4): a line is brought from HBM by one of them and found in the L2 by the others. Weights from HBM,
+ * us, all in one order / turned: 512 x 2560 -> 6144 29.5 / 23.0, 512 x 3072 -> 9216 38.0 / 34.8, 512 x 9728 -> 2560 39.5 / 35.6,
+ * 320 x 3072 -> 27648 59.1 / 55.5; with weights in the Infinity Cache 1 - 3 % slower. Turns over eight tiles, or turned by pairs
+ * and fours of tiles, gave the same or less; four waves that only fetch beside the eight that multiply changed nothing.
+ * Then comes the LDS: a wave's 64 x 64 outputs read 8 KB of operands for 16 products. The 160-row tiles of 256 and 224 columns
+ * run on four waves of 80 x 128 and 80 x 112 (12 KB for 35 products; 512 registers to a wave): 320 x 3072 -> 27648 in tiles of
+ * 256 58.0 on eight waves / 56.5, 1024 x 3072 -> 9216 62.2 / 53.5; in tiles of 224, which fill 248 CUs instead of 216, 53.6.
+ * Tiles of 128 x 256, 160 x 192 and 128 x 192 on four waves were as fast as on eight.
  */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -57,12 +71,12 @@ struct Tile {
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"                          /* M0 in a clobber list */
 template <typename OUT, int NB, int WM, int NA, int WN, int KG, int STAGES>
-__global__ void __launch_bounds__(64 * WM * WN * KG, 2)
+__global__ void __launch_bounds__(64 * WM * WN * KG, WM * WN * KG / 4)
 k_gemm_tiles(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *__restrict__ W, int M, int N, int K,
              const float *__restrict__ bias, int tiles_m, int tiles_n, int splits, int total, int per_xcd) {
     using T = Tile<NB, WM, NA, WN, KG, STAGES>;
     constexpr int TM = T::TM, TN = T::TN, STAGE = T::STAGE, PIECES = T::PIECES;
-    static_assert(T::LDS <= 160 * 1024 && NA <= 4 && (KG == 1 || (KG == 2 && NB % 2 == 0)), "");
+    static_assert(T::LDS <= 160 * 1024 && NA <= 8 && (KG == 1 || (KG == 2 && NB % 2 == 0)), "");
     extern __shared__ __align__(16) uint16_t lds[];
     /* An XCD (own L2) takes a contiguous range of the work list: K ranges outermost, then bands of 8 tile rows, inside a
      * band m fastest: its 32 CUs share the W tiles and each other's x rows. */
@@ -77,6 +91,8 @@ k_gemm_tiles(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;
+    /* the order of this workgroup's k tiles, see above: tile kt of the order is k tile kt ^ turn inside whole groups of four */
+    const int turn = (m0 / TM ^ n0 / TN) & 3, turned = nk & ~3;
     const int wm = wave % WM, wn = wave / WM % WN, kg = wave / (WM * WN);
 
     /* this wave's pieces of a stage: row 8 (PIECES wave + j) + lane / 8 of [W tile | x tile]; rows past the end of a matrix
@@ -91,7 +107,7 @@ k_gemm_tiles(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t
         off[j] = ((uint32_t)row * (uint32_t)K + 8u * ((lane & 7) ^ ((r >> 1) & 7))) * 2u;
     }
     auto request_one = [&](int j, int kt, uint16_t *stage) {
-        const uint16_t *src = (piece[j] < TN / 8 ? W : x) + (size_t)(kt0 + kt) * TK;
+        const uint16_t *src = (piece[j] < TN / 8 ? W : x) + (size_t)(kt0 + (kt < turned ? kt ^ turn : kt)) * TK;
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                      ::"s"(lds_address(stage + piece[j] * 8 * TK)), "v"(off[j]), "s"(src) : "memory", "m0");
     };
@@ -126,8 +142,8 @@ k_gemm_tiles(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t
         }
     };
     /* A k-step's products with the memory instructions of later steps dealt out between them, at most one per gap: first
-     * the operands of the next k-step (from `rd`, where `reads`), then pieces [first, last) of a later k tile (`wanted`). A wave issues
-     * in order, and the eight waves leave a barrier together: bunched in front of the products the same instructions
+     * the operands of the next k-step (from `rd`, where `reads`), then, evenly, pieces [first, last) of a later k tile (`wanted`).
+     * A wave issues in order, and the waves leave a barrier together: bunched in front of the products the same instructions
      * were not hidden by the other wave of the SIMD but added to it (128 x 256 tile: 1024 cycles of products, 1171 with
      * nothing else, 1477 with the operand reads, 1754 with the pieces too). */
     auto products = [&](int set, auto reads, const uint16_t *rd, int rd_ks, int first, int last, auto wanted, int kt, uint16_t *stage) {
@@ -136,10 +152,9 @@ k_gemm_tiles(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t
         for (int g = 0; g < GAPS; g++) {
             acc[g / NB][g % NB] = mfma(av[set][g / NB], bv[set][g % NB], acc[g / NB][g % NB]);
             if (decltype(reads)::value && g < READS) operand(rd, set ^ 1, rd_ks, g);
-#pragma unroll
-            for (int j = first; j < last; j++)
-                if (g == READS + (j - first) * (GAPS - READS) / (last - first))
-                    if (wanted) request_one(j, kt, stage);
+            const int gap = g - READS, span = GAPS - READS, count = last - first, j = gap * count / span;
+            if (gap >= 0 && count && (gap == 0 || (gap - 1) * count / span != j))
+                if (wanted) request_one(first + j, kt, stage);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -219,36 +234,41 @@ k_gemm_tiles(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t
     OUT *dst = y + (size_t)split * M * N;
     const int mw = m0 + 16 * (NB * wm + b0), nw = n0 + 16 * NA * wn;
     uint16_t *mine = lds + wave * (NBS * 16 * 128);
-    if constexpr (sizeof(OUT) == 4) {
-        float *buf = reinterpret_cast<float *>(mine);          /* 16 B chunk c of row r in slot c ^ (r % 16) */
+    /* up to 64 columns at a time */
 #pragma unroll
-        for (int b = 0; b < NBS; b++)
+    for (int c0 = 0; c0 < NA; c0 += 4) {
+        const int na = min(NA - c0, 4), nc = nw + 16 * c0;
+        if constexpr (sizeof(OUT) == 4) {
+            float *buf = reinterpret_cast<float *>(mine);      /* 16 B chunk c of row r in slot c ^ (r % 16) */
 #pragma unroll
-            for (int a = 0; a < NA; a++) *reinterpret_cast<f32x4 *>(&buf[(16 * b + li) * 64 + 4 * ((4 * a + lg) ^ li)]) = acc[a][b];
+            for (int b = 0; b < NBS; b++)
 #pragma unroll
-        for (int it = 0; it < 4 * NBS; it++) {
-            const int row = 4 * it + (lane >> 4), c = lane & 15, m = mw + row, n = nw + 4 * c;
-            f32x4 v = *reinterpret_cast<const f32x4 *>(&buf[row * 64 + 4 * (c ^ (row & 15))]);
-            if (c < 4 * NA && m < M && n < N) {
-                if (bias) v += *reinterpret_cast<const f32x4 *>(bias + n);
-                *reinterpret_cast<f32x4 *>(dst + (size_t)m * N + n) = v;
+                for (int a = 0; a < na; a++) *reinterpret_cast<f32x4 *>(&buf[(16 * b + li) * 64 + 4 * ((4 * a + lg) ^ li)]) = acc[c0 + a][b];
+#pragma unroll
+            for (int it = 0; it < 4 * NBS; it++) {
+                const int row = 4 * it + (lane >> 4), c = lane & 15, m = mw + row, n = nc + 4 * c;
+                f32x4 v = *reinterpret_cast<const f32x4 *>(&buf[row * 64 + 4 * (c ^ (row & 15))]);
+                if (c < 4 * na && m < M && n < N) {
+                    if (bias) v += *reinterpret_cast<const f32x4 *>(bias + n);
+                    *reinterpret_cast<f32x4 *>(dst + (size_t)m * N + n) = v;
+                }
             }
-        }
-    } else {
-        uint16_t *buf = mine;                                  /* chunk c of row r in slot c ^ (r % 8) */
+        } else {
+            uint16_t *buf = mine;                              /* chunk c of row r in slot c ^ (r % 8) */
 #pragma unroll
-        for (int b = 0; b < NBS; b++)
+            for (int b = 0; b < NBS; b++)
 #pragma unroll
-            for (int a = 0; a < NA; a++) {
-                const int chunk = 2 * a + (lg >> 1);
-                *reinterpret_cast<uint2 *>(&buf[(16 * b + li) * 64 + 8 * (chunk ^ (li & 7)) + 4 * (lg & 1)]) =
-                    make_uint2(pack_bf16(acc[a][b][0], acc[a][b][1]), pack_bf16(acc[a][b][2], acc[a][b][3]));
+                for (int a = 0; a < na; a++) {
+                    const int chunk = 2 * a + (lg >> 1);
+                    *reinterpret_cast<uint2 *>(&buf[(16 * b + li) * 64 + 8 * (chunk ^ (li & 7)) + 4 * (lg & 1)]) =
+                        make_uint2(pack_bf16(acc[c0 + a][b][0], acc[c0 + a][b][1]), pack_bf16(acc[c0 + a][b][2], acc[c0 + a][b][3]));
+                }
+#pragma unroll
+            for (int it = 0; it < 2 * NBS; it++) {
+                const int row = 8 * it + (lane >> 3), c = lane & 7, m = mw + row, n = nc + 8 * c;
+                const u32x4 v = *reinterpret_cast<const u32x4 *>(&buf[row * 64 + 8 * (c ^ (row & 7))]);
+                if (c < 2 * na && m < M && n < N) *reinterpret_cast<u32x4 *>(dst + (size_t)m * N + n) = v;
             }
-#pragma unroll
-        for (int it = 0; it < 2 * NBS; it++) {
-            const int row = 8 * it + (lane >> 3), c = lane & 7, m = mw + row, n = nw + 8 * c;
-            const u32x4 v = *reinterpret_cast<const u32x4 *>(&buf[row * 64 + 8 * (c ^ (row & 7))]);
-            if (c < 2 * NA && m < M && n < N) *reinterpret_cast<u32x4 *>(dst + (size_t)m * N + n) = v;
         }
     }
 }
@@ -294,8 +314,8 @@ int launch_tiles(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, i
  * grid of one round, where the chip is not at its power limit, `step_full` in a longer one. A workgroup's first tiles and
  * its epilogue take 3.5 us more. */
 struct Shape { int tm, tn; float step, step_full; };
-constexpr Shape SHAPES[] = {{128, 128, 0.50f, 0.55f}, {128, 192, 0.62f, 0.65f}, {128, 256, 0.74f, 0.82f},
-                            {64, 256, 0.61f, 0.62f},  {160, 192, 0.66f, 0.74f}, {160, 256, 0.86f, 0.94f}};
+constexpr Shape SHAPES[] = {{128, 128, 0.44f, 0.50f}, {128, 192, 0.58f, 0.62f}, {128, 256, 0.72f, 0.80f}, {64, 256, 0.60f, 0.61f},
+                            {160, 192, 0.67f, 0.72f}, {160, 256, 0.90f, 0.93f}, {160, 224, 0.84f, 0.87f}};
 constexpr int NSHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
 
 template <typename OUT>
@@ -306,7 +326,8 @@ int launch_shape(hipStream_t st, int shape, OUT *y, const uint16_t *x, const uin
     case 2: return launch_tiles<OUT, 4, 2, 4, 4, 1, 3>(st, y, x, W, M, N, K, bias, splits);
     case 3: return launch_tiles<OUT, 4, 1, 4, 4, 2, 4>(st, y, x, W, M, N, K, bias, splits);
     case 4: return launch_tiles<OUT, 5, 2, 3, 4, 1, 3>(st, y, x, W, M, N, K, bias, splits);
-    case 5: return launch_tiles<OUT, 5, 2, 4, 4, 1, 3>(st, y, x, W, M, N, K, bias, splits);
+    case 5: return launch_tiles<OUT, 5, 2, 8, 2, 1, 3>(st, y, x, W, M, N, K, bias, splits);
+    case 6: return launch_tiles<OUT, 5, 2, 7, 2, 1, 3>(st, y, x, W, M, N, K, bias, splits);
     default: return (int)hipErrorInvalidValue;
     }
 }

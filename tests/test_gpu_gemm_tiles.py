@@ -56,6 +56,38 @@ def test_every_tile(dev, shape, more_rows, more_cols, k, splits, bf16):
     check(got[:rows * out].reshape(rows, out), want, k, bf16)
 
 
+def one_layer(dev, shape, rows, k, out, splits, bf16):
+    x, W, want = operands(rows, k, out)
+    lib = dev.lib
+    lib.iris_hip_gemm_tiles.restype = C.c_int
+    lib.iris_hip_gemm_tiles.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p] + [C.c_int] * 3 + [C.c_void_p] + [C.c_int] * 2 + [C.c_void_p]
+    fill = np.full(rows * out + 512, 7, np.uint16 if bf16 else np.float32)
+    dy, part = dev.put(fill), dev.alloc(splits * rows * out * 4)
+    assert lib.iris_hip_gemm_tiles(lib.iris_dev_stream(), dy, 2 if bf16 else 4, dev.put(x), dev.put(W), rows, out, k, None, shape, splits, part) == 0
+    dev.check()
+    got = dev.get(dy, fill.shape, fill.dtype)
+    dev.free_all()
+    assert (got[rows * out:] == 7).all()
+    check(got[:rows * out].reshape(rows, out), want, k, bf16)
+
+
+# the tile of 160 x 224 at the same edges
+@pytest.mark.parametrize("more_rows,more_cols,k,splits", [(0, 0, 64, 1), (1, 8, 128, 1), (-1, -8, 192, 1), (0, 72, 256, 1), (33, 0, 320, 1),
+                                                          (-63, 8, 704, 3), (0, 0, 640, 2), (1, 8, 832, 6)])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_tile_of_224_columns(dev, more_rows, more_cols, k, splits, bf16):
+    one_layer(dev, 6, 160 + more_rows, k, 224 + more_cols, splits, bf16)
+
+
+# five by five tiles, whose workgroups take the k tiles in four different orders: no whole group of four, one, several, and
+# some left over; ranges of K with all of these
+@pytest.mark.parametrize("shape", range(7))
+@pytest.mark.parametrize("k_tiles,splits", [(3, 1), (4, 1), (7, 1), (13, 1), (16, 1), (19, 4)])
+def test_orders_of_the_k_tiles(dev, shape, k_tiles, splits):
+    tm, tn = (TILES + [(160, 224)])[shape]
+    one_layer(dev, shape, 5 * tm - 3, 64 * k_tiles, 5 * tn - 8, splits, k_tiles % 2 == 0)
+
+
 @pytest.mark.parametrize("rows,k,out", [(1, 512, 128), (77, 2048, 1544), (130, 1536, 136), (300, 4096, 640), (500, 1024, 3072)])
 @pytest.mark.parametrize("bf16", [False, True])
 def test_linear_layers_that_take_it(dev, rows, k, out, bf16):
