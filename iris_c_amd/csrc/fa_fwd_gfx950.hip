@@ -332,11 +332,12 @@ __device__ __forceinline__ void norm_rope_q_fragment(bf16x8 (&qb)[4], const QNor
 }
 
 
-/* The walk of one wave over the key tiles of its workgroup. WAVES and GROUP belong to the workgroup (pieces of a
- * tile per wave, tiles between two barriers, stages); NB, the blocks of 16 queries the wave carries, may differ
+/* The walk of one wave over the key tiles of its workgroup. WAVES, GROUP and PARTS belong to the workgroup (pieces of a
+ * tile per wave, tiles between two barriers, stages, waves that share their queries); with PARTS = 2 the two tiles of a group
+ * go to the two halves of the workgroup, which hold the same queries and merge what they have at the end; NB, the blocks of 16 queries the wave carries, may differ
  * between the waves of a workgroup as long as every wave passes the same barriers: the tile count depends on the
  * workgroup's queries q0 .. q0 + bm - 1 only. wq0 is the wave's first query. */
-template <int WAVES, int NB, int GROUP, bool CAUSAL, bool MASK>
+template <int WAVES, int NB, int GROUP, bool CAUSAL, bool MASK, int PARTS = 1>
 __device__ __forceinline__ void
 fa_walk_hd128(uint16_t *__restrict__ lds, uint16_t *__restrict__ out, int ldo, const uint16_t *__restrict__ q,
               const uint16_t *__restrict__ k, const uint16_t *__restrict__ v, int ldi,
@@ -344,6 +345,7 @@ fa_walk_hd128(uint16_t *__restrict__ lds, uint16_t *__restrict__ out, int ldo, c
               float scale_log2, const int *__restrict__ key_mask, const QNorm &qnorm) {
     constexpr int NI = (32 + WAVES - 1) / WAVES;         /* pieces of a tile per wave (the last waves may have one fewer) */
     constexpr int NSTAGE = 2 * GROUP;                    /* the group in use and the group on its way */
+    static_assert(PARTS == 1 || (PARTS == 2 && GROUP == 2), "");
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;       /* 16x16 block: column li, row group lg */
@@ -484,13 +486,15 @@ fa_walk_hd128(uint16_t *__restrict__ lds, uint16_t *__restrict__ out, int ldo, c
             wait_vmcnt<0>();
             lds_barrier();
         }
+        if (PARTS == 2) lds_barrier();                   /* the merge of the others */
         return;
     }
+    const int part = PARTS == 2 ? wave / (WAVES / 2) : 0;
 
     for (int g0 = 0, half = 0; g0 < ntiles_run; g0 += GROUP, half ^= 1) {
 #pragma unroll
-      for (int h = 0; h < GROUP; h++) {
-        const int it = g0 + h;
+      for (int step = 0; step < GROUP / PARTS; step++) {
+        const int h = PARTS == 2 ? part : step, it = g0 + h;
         if (it >= ntiles_run) break;                     /* wave-uniform */
         const int k0 = it * BN;
         uint16_t *cur = lds + (half * GROUP + h) * STAGE;
@@ -537,7 +541,7 @@ fa_walk_hd128(uint16_t *__restrict__ lds, uint16_t *__restrict__ out, int ldo, c
          * the barrier: there every wave would issue its requests before its first operand read,
          * with the matrix cores of the whole CU idle meanwhile. It still has the rest of the
          * group's time to land. */
-        if (h == 0) {
+        if (step == 0) {
 #pragma unroll
             for (int t = 0; t < GROUP; t++) request(g0 + GROUP + t, (half ^ 1) * GROUP + t);
             __builtin_amdgcn_sched_barrier(0);
@@ -679,6 +683,39 @@ fa_walk_hd128(uint16_t *__restrict__ lds, uint16_t *__restrict__ out, int ldo, c
 
     wait_vmcnt<0>();       /* nothing may still be on its way into the LDS when it is given back (the loop ends with this wait too) */
 
+    if constexpr (PARTS == 2) {
+        /* The two waves of the same queries hand each other half of the dims: part 0 keeps the dim blocks 0 - 3 and part 1
+         * the blocks 4 - 7. Behind the last barrier of the loop nobody reads the stages any more. */
+        constexpr int REGION = (4 * NB * 4 + 2 * NB) * 64;                   /* floats a wave hands over */
+        float *mine = reinterpret_cast<float *>(lds) + wave * REGION, *theirs = reinterpret_cast<float *>(lds) + (wave ^ (WAVES / 2)) * REGION;
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) {
+#pragma unroll
+            for (int d = 0; d < 4; d++) *reinterpret_cast<f32x4 *>(mine + ((4 * nb + d) * 64 + lane) * 4) = part ? o[d][nb] : o[4 + d][nb];
+            mine[16 * NB * 64 + (2 * nb) * 64 + lane] = m_run[nb];
+            mine[16 * NB * 64 + (2 * nb + 1) * 64 + lane] = l_acc[nb][0];
+        }
+        lds_barrier();
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) {
+            const float m_other = theirs[16 * NB * 64 + (2 * nb) * 64 + lane], l_other = theirs[16 * NB * 64 + (2 * nb + 1) * 64 + lane];
+            const float m_all = fmaxf(m_run[nb], m_other), base = m_all == -INFINITY ? 0.0f : m_all;
+            const float fa = __builtin_amdgcn_exp2f(m_run[nb] - base), fb = __builtin_amdgcn_exp2f(m_other - base);
+            const float l_tot = l_acc[nb][0] * fa + l_other * fb;
+            const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+            const int qrow = qrow0 + 16 * nb;
+            uint16_t *op = out + (size_t)qrow * ldo + (size_t)head * HD + 64 * part + 4 * lg;
+#pragma unroll
+            for (int d = 0; d < 4; d++) {
+                const f32x4 other = *reinterpret_cast<const f32x4 *>(theirs + ((4 * nb + d) * 64 + lane) * 4), own = part ? o[4 + d][nb] : o[d][nb];
+                f32x4 sum;
+#pragma unroll
+                for (int r = 0; r < 4; r++) sum[r] = (own[r] * fa + other[r] * fb) * inv;
+                if (qrow < seq_q) *reinterpret_cast<uint2 *>(op + 16 * d) = make_uint2(pack_bf16(sum[0], sum[1]), pack_bf16(sum[2], sum[3]));
+            }
+        }
+        return;
+    }
     /* ---- normalise and store: the lane holds dims 16db + 4lg + {0..3} of its queries ---- */
 #pragma unroll
     for (int nb = 0; nb < NB; nb++) {
@@ -699,7 +736,7 @@ fa_walk_hd128(uint16_t *__restrict__ lds, uint16_t *__restrict__ out, int ldo, c
 }
 
 /* Workgroups of WAVES waves that all carry NB blocks of 16 queries. */
-template <int WAVES, int NB, bool CAUSAL, bool MASK>
+template <int WAVES, int NB, bool CAUSAL, bool MASK, int PARTS = 1>
 __global__ void __launch_bounds__(64 * WAVES, 2)
 k_fa_fwd_hd128(uint16_t *__restrict__ out, int ldo, const uint16_t *__restrict__ q,
                const uint16_t *__restrict__ k, const uint16_t *__restrict__ v, int ldi,
@@ -707,11 +744,11 @@ k_fa_fwd_hd128(uint16_t *__restrict__ out, int ldo, const uint16_t *__restrict__
                int kv_group, float scale_log2, const int *__restrict__ key_mask, QNorm qnorm) {
     extern __shared__ __align__(16) uint16_t lds[];     /* 2 GROUP stages of [K tile | V tile] */
     constexpr int WQ = 16 * NB;                          /* queries per wave */
-    constexpr int BM = WQ * WAVES;
+    constexpr int BM = WQ * WAVES / PARTS;
     /* Key tiles between two barriers. Two for the 8-wave shape (one workgroup per CU, so the LDS
      * has room for four stages): the waves of a workgroup then only meet every other tile, and
      * the faster ones do not stand at a barrier while the slower ones finish every single tile. */
-    constexpr int GROUP = WAVES * NB >= 12 ? 2 : 1;
+    constexpr int GROUP = WAVES * NB >= 12 || PARTS == 2 ? 2 : 1;
 
     /* XCD-aware numbering: hardware deals workgroups round-robin to the 8
      * XCDs, so id%8 is the XCD; give each XCD a contiguous slice of the
@@ -723,8 +760,8 @@ k_fa_fwd_hd128(uint16_t *__restrict__ out, int ldo, const uint16_t *__restrict__
     if (CAUSAL) qt = q_tiles - 1 - qt;             /* longest rows first */
     const int q0 = qt * BM;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    fa_walk_hd128<WAVES, NB, GROUP, CAUSAL, MASK>(lds, out, ldo, q, k, v, ldi, seq_q, seq_k, head, head / kv_group, q0, BM,
-                                                  q0 + wave * WQ, scale_log2, key_mask, qnorm);
+    fa_walk_hd128<WAVES, NB, GROUP, CAUSAL, MASK, PARTS>(lds, out, ldo, q, k, v, ldi, seq_q, seq_k, head, head / kv_group, q0, BM,
+                                                         q0 + wave % (WAVES / PARTS) * WQ, scale_log2, key_mask, qnorm);
 }
 
 /* The last, partly filled round of the kernel above leaves CUs idle: 432 workgroups on 256 CUs run as 256 + 176.
@@ -1085,7 +1122,7 @@ k_fa_short_hd128(uint16_t *__restrict__ out, int ldo, const uint16_t *__restrict
 }
 #pragma clang diagnostic pop
 
-template <int W, int NB> constexpr size_t stage_bytes() { return (W * NB >= 12 ? 4 : 2) * STAGE * sizeof(uint16_t); }
+template <int W, int NB, int PARTS = 1> constexpr size_t stage_bytes() { return (W * NB >= 12 || PARTS == 2 ? 4 : 2) * STAGE * sizeof(uint16_t); }
 constexpr size_t LDS_MAX = 160 * 1024;
 
 /* Compute units of the current device (256 on an MI355X in its single-partition mode); 256 where no device answers,
@@ -1106,24 +1143,25 @@ int cu_count() {
     return n;
 }
 
-template <int W, int NB, bool C, bool M>
+template <int W, int NB, bool C, bool M, int PARTS = 1>
 int launch(hipStream_t st, uint16_t *out, int ldo, const uint16_t *q, const uint16_t *k,
            const uint16_t *v, int ldi, int seq_q, int seq_k, int heads, int kv_heads,
            float scale, const int *key_mask, const QNorm &qn) {
     static bool configured = false;
     if (!configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_fa_fwd_hd128<W, NB, C, M>),
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_fa_fwd_hd128<W, NB, C, M, PARTS>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_MAX);
         if (e != hipSuccess) return (int)e;
         configured = true;
     }
-    const int q_tiles = (seq_q + 16 * NB * W - 1) / (16 * NB * W);
+    constexpr int BM = 16 * NB * W / PARTS;
+    const int q_tiles = (seq_q + BM - 1) / BM;
     const int total = q_tiles * heads;
     const int per_xcd = (total + XCDS - 1) / XCDS;
     /* the stages, and for a key mask one 64-bit word per key tile behind them */
-    const size_t lds_bytes = stage_bytes<W, NB>() + (M ? 8 * (size_t)((seq_k + BN - 1) / BN) : 0);
+    const size_t lds_bytes = stage_bytes<W, NB, PARTS>() + (M ? 8 * (size_t)((seq_k + BN - 1) / BN) : 0);
     if (lds_bytes > LDS_MAX) return (int)hipErrorInvalidValue;       /* the caller keeps masked seq_k below the limit */
-    hipLaunchKernelGGL((k_fa_fwd_hd128<W, NB, C, M>), dim3(per_xcd * XCDS), dim3(64 * W), lds_bytes, st, out, ldo,
+    hipLaunchKernelGGL((k_fa_fwd_hd128<W, NB, C, M, PARTS>), dim3(per_xcd * XCDS), dim3(64 * W), lds_bytes, st, out, ldo,
                        q, k, v, ldi, seq_q, seq_k, q_tiles, total, per_xcd, heads / kv_heads,
                        scale * 1.4426950408889634f, key_mask, qn);
     return (int)hipGetLastError();
@@ -1152,16 +1190,18 @@ int launch_two_sizes(hipStream_t st, uint16_t *out, int ldo, const uint16_t *q, 
     return (int)hipGetLastError();
 }
 
-template <int W, int NB = 2>
+template <int W, int NB = 2, int PARTS = 1>
 int launch_w(hipStream_t st, uint16_t *out, int ldo, const uint16_t *q, const uint16_t *k,
              const uint16_t *v, int ldi, int seq_q, int seq_k, int heads, int kv_heads, float scale,
              int causal, const int *key_mask, const QNorm &qn) {
     if (causal) {
-        if (key_mask) return launch<W, NB, true, true>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, key_mask, qn);
-        return launch<W, NB, true, false>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, key_mask, qn);
+        if constexpr (PARTS == 2) {                          /* plan_hd128 */
+            if (key_mask) return (int)hipErrorInvalidValue;
+        } else if (key_mask) return launch<W, NB, true, true, PARTS>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, key_mask, qn);
+        return launch<W, NB, true, false, PARTS>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, key_mask, qn);
     }
-    if (key_mask) return launch<W, NB, false, true>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, key_mask, qn);
-    return launch<W, NB, false, false>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, key_mask, qn);
+    if (key_mask) return launch<W, NB, false, true, PARTS>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, key_mask, qn);
+    return launch<W, NB, false, false, PARTS>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, key_mask, qn);
 }
 
 template <int S, bool C, bool M>
@@ -1238,11 +1278,12 @@ static long two_sizes_cost(long n_full, long n_tail) {
     return worst;
 }
 
-/* Which kernel a call takes: kind 0 = k_fa_fwd_hd128<waves, nb>, 1 = k_fa_fwd_hd128_two_sizes with `full` workgroups
+/* Which kernel a call takes: kind 0 = k_fa_fwd_hd128<waves, nb>, with `split` = 2 that kernel with twice the waves, of which
+ * two take the tiles of the same queries in turn (PARTS = 2), 1 = k_fa_fwd_hd128_two_sizes with `full` workgroups
  * of 256 queries per head, 2 = k_fa_short_hd128<split>. Host arithmetic only. */
 struct FaPlan { int kind, waves, nb, split, full; };
 
-static FaPlan plan_hd128(int seq_q, int seq_k, int heads, int causal) {
+static FaPlan plan_hd128(int seq_q, int seq_k, int heads, int causal, bool masked) {
     /* Three regimes, by the number of waves of 16 queries the problem makes (heads x ceil(seq_q / 16)).
      *
      * Up to 2048 of them (one wave per SIMD and CU slot, or fewer): a workgroup walks its key tiles one after the
@@ -1274,6 +1315,18 @@ static FaPlan plan_hd128(int seq_q, int seq_k, int heads, int causal) {
         const long tiles = (keys + BN - 1) / BN;
         const long cost_chain = tiles * (w <= 2 ? 65 : w == 4 ? 92 : 108);           /* 0.01 us */
         if (q_tiles32 * heads <= CUS && ((tiles + 3) / 4) * 145 + 150 < cost_chain) return {2, 4, 2, 4, 0};   /* from 7 tiles on */
+        /* Two waves that take the tiles of 16 queries in turn halve the chain: 1.0 us per two tiles on 2 x 2 waves, 1.5 on
+         * 4 x 2, and 0.5 for the merge. Their four stages fill the LDS, so every workgroup needs a CU of its own, and with
+         * one, two or three tiles there is no chain to halve. us, one wave / two: 24 heads x 256 tokens 7.0 / 6.5, x 320 8.0 /
+         * 7.6, x 384 10.8 / 9.0 (288 workgroups of 32 queries become 144 of 64), x 512 11.4 / 10.5, x 640 13.5 / 12.1; 32 heads x
+         * 320 9.5 / 8.3, x 512 causal 11.6 / 10.4; and where it is not taken 32 heads x 160 6.0 / 6.2, 24 heads x 720 17.9 / 24.2.
+         * Eight waves of 32 queries (128 a workgroup) in place of eight of 16 beyond that: within 3 %. A causal call with a key
+         * mask is a prompt padded to a fixed length: its walk ends at the last valid key, mostly after two or three tiles (32
+         * heads x 512, 118 valid keys 7.3 / 8.0), so it keeps one wave. */
+        if (w > 1 && w < 8 && tiles >= 4 && !(causal && masked)) {
+            if (w == 2 && q_tiles32 * heads <= CUS) return {0, 2, 1, 2, 0};
+            if ((long)((seq_q + 63) / 64) * heads <= CUS) return {0, 4, 1, 2, 0};
+        }
         return {0, w, 1, 0, 0};
     }
     const long wg256 = (long)((seq_q + 255) / 256) * heads, wg128 = (long)((seq_q + 127) / 128) * heads;
@@ -1304,7 +1357,7 @@ static FaPlan plan_hd128(int seq_q, int seq_k, int heads, int causal) {
 static int launch_any_width(hipStream_t st, uint16_t *out, int ldo, const uint16_t *q, const uint16_t *k,
                             const uint16_t *v, int ldi, int seq_q, int seq_k, int heads, int kv_heads, float scale,
                             int causal, const int *key_mask, const QNorm &qn) {
-    const FaPlan p = plan_hd128(seq_q, seq_k, heads, causal);
+    const FaPlan p = plan_hd128(seq_q, seq_k, heads, causal, key_mask != nullptr);
     if (p.kind == 2) return launch_short_cm<4>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, causal, key_mask, qn);
     if (p.kind == 1) {
         if (key_mask) return launch_two_sizes<false, true>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, key_mask, qn, p.full);
@@ -1312,6 +1365,8 @@ static int launch_any_width(hipStream_t st, uint16_t *out, int ldo, const uint16
     }
     if (p.nb == 1) {
         if (p.waves == 1) return launch_w<1, 1>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, causal, key_mask, qn);
+        if (p.split == 2 && p.waves == 2) return launch_w<4, 1, 2>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, causal, key_mask, qn);
+        if (p.split == 2) return launch_w<8, 1, 2>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, causal, key_mask, qn);
         if (p.waves == 2) return launch_w<2, 1>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, causal, key_mask, qn);
         if (p.waves == 4) return launch_w<4, 1>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, causal, key_mask, qn);
         return launch_w<8, 1>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, causal, key_mask, qn);
@@ -1321,10 +1376,10 @@ static int launch_any_width(hipStream_t st, uint16_t *out, int ldo, const uint16
 }
 
 /* The launcher's choice for a head_dim-128 call, without launching anything (no GPU needed): plan[0] = kind (0 one
- * size, 1 two sizes, 2 keys split over the waves), plan[1] = waves per workgroup, plan[2] = blocks of 16 queries per
+ * size, 1 two sizes, 2 keys split over the waves), plan[1] = waves per workgroup with queries of their own, plan[2] = blocks of 16 queries per
  * wave, plan[3] = 256-query workgroups per head of the two-size grid, plan[4] = its 192-query workgroups per head. */
 extern "C" void iris_hip_fa_hd128_plan(int seq_q, int seq_k, int heads, int causal, int *plan) {
-    const FaPlan p = plan_hd128(seq_q, seq_k, heads, causal);
+    const FaPlan p = plan_hd128(seq_q, seq_k, heads, causal, false);
     plan[0] = p.kind; plan[1] = p.waves; plan[2] = p.nb; plan[3] = p.full;
     plan[4] = p.kind == 1 ? (seq_q - 256 * p.full + 191) / 192 : 0;
 }
