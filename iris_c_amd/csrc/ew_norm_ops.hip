@@ -519,8 +519,8 @@ k_gn_normalize(float *__restrict__ out, const float *__restrict__ in, const floa
  * not at the end of the kernel (143 -> 114 us, 1024 x 1024 x 128 278 -> 247).
  * Bound by the memory in both directions (134 MB read in 20 us), 5 - 6 us between the last value read and the first written, and
  * the launch. Against statistics, their sum and normalising as three launches, f32 image from memory, us:
- * 16384 x 512 26.7 -> 20.1, 65536 x 256 45 -> 30, 384 x 384 x 128 50 -> 33, 512 x 512 x 128 82 -> 52, 512 x 512 x 256 155 -> 114,
- * 700 x 700 x 128 146 -> 109, 1024 x 1024 x 128 294 -> 247; 4096 x 512 (8 MB) 13.4 / 13.1, 1024 x 512 10.0 / 11.6: the line.
+ * 16384 x 512 26.7 -> 20.1, 65536 x 256 45 -> 30, 384 x 384 x 128 50 -> 33, 512 x 512 x 128 82 -> 51, 512 x 512 x 256 155 -> 108,
+ * 700 x 700 x 128 146 -> 101, 1024 x 1024 x 128 294 -> 232; 4096 x 512 (8 MB) 13.4 / 13.1, 1024 x 512 10.0 / 11.6: the line.
  *
  * Everything between workgroups is a word with the number of the launch in its high half (Tagged), so that no store has to be
  * waited for and nothing is cleared between launches: a workgroup leaves the moments of its share, workgroup g < groups
@@ -555,7 +555,12 @@ k_gn_clear(unsigned *sync) {
 template <typename T> __device__ __forceinline__ T agent_load(const T *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 template <typename T> __device__ __forceinline__ void agent_store(T *p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
-template <bool SILU>
+/* ONCE: what is read for the last time is read with the streaming hint, in images of RES_ONCE_BYTES and more; smaller ones may still be in the
+ * Infinity Cache. us without / with: 512 x 512 x 128 (134 MB) 53.2 / 51.6, 512 x 512 x 256 115 / 108, 700 x 700 x 128 108 / 101,
+ * 1024 x 1024 x 128 258 / 232; 256 x 256 x 256 (67 MB) 31.8 / 31.6, 16384 x 512 20.8 / 21.9. With the hint on what is read
+ * again later too: 117, 110 and 257. */
+constexpr size_t RES_ONCE_BYTES = (size_t)96 << 20;
+template <bool SILU, bool ONCE>
 __global__ void __launch_bounds__(RES_THREADS, 2)
 k_gn_resident(f32x4 *out, const f32x4 *in, const float *__restrict__ gamma, const float *__restrict__ beta, ResidentSync *sync,
               unsigned total, int c, int cg, float eps, unsigned patience) {
@@ -570,6 +575,7 @@ k_gn_resident(f32x4 *out, const f32x4 *in, const float *__restrict__ gamma, cons
     auto steps_of = [&](unsigned w) { return w < steps ? (steps - w + RES_WGS - 1) / RES_WGS : 0; };
     const unsigned n = steps_of(b), at0 = b * RES_THREADS + tid;
     auto load = [&](unsigned i) { return in[min(at0 + i * RES_STRIDE, total - 1)]; };
+    auto last_load = [&](unsigned at) { return ONCE ? __builtin_nontemporal_load(in + min(at, total - 1)) : in[min(at, total - 1)]; };
     constexpr unsigned long long ARRIVALS = (1ull << 48) - 1;
     /* the number of this launch, the same in all workgroups as this one has not arrived yet */
     const unsigned epoch = (unsigned)((agent_load(&sync->arrivals) & ARRIVALS) / RES_WGS) + 1;
@@ -620,7 +626,7 @@ k_gn_resident(f32x4 *out, const f32x4 *in, const float *__restrict__ gamma, cons
     for (int g = 0; g < RES_LDS && RES_REG + g < n; g += RES_LDS_BATCH) {
         f32x4 v[RES_LDS_BATCH];
 #pragma unroll
-        for (int j = 0; j < RES_LDS_BATCH; j++) v[j] = load(min(RES_REG + g + j, n - 1));
+        for (int j = 0; j < RES_LDS_BATCH; j++) v[j] = last_load(at0 + min(RES_REG + g + j, n - 1) * RES_STRIDE);
 #pragma unroll
         for (int j = 0; j < RES_LDS_BATCH; j++) kept[(g + j) * RES_THREADS + tid] = v[j];
         take(v, RES_REG + g, std::integral_constant<int, RES_LDS_BATCH>{});
@@ -629,7 +635,7 @@ k_gn_resident(f32x4 *out, const f32x4 *in, const float *__restrict__ gamma, cons
     for (int g = 0; g < RES_REG; g += RES_BATCH)
         if (g < n)
 #pragma unroll
-            for (int j = 0; j < RES_BATCH; j++) keep[g + j] = load(min(g + j, n - 1));
+            for (int j = 0; j < RES_BATCH; j++) keep[g + j] = last_load(at0 + min(g + j, n - 1) * RES_STRIDE);
 #pragma unroll
     for (int g = 0; g < RES_REG; g += RES_BATCH)
         if (g < n) take(keep + g, g, std::integral_constant<int, RES_BATCH>{});
@@ -738,7 +744,7 @@ k_gn_resident(f32x4 *out, const f32x4 *in, const float *__restrict__ gamma, cons
         f32x4 v[2][RES_BATCH];
         auto fetch = [&](f32x4 *dst, unsigned from) {
 #pragma unroll
-            for (int j = 0; j < RES_BATCH; j++) dst[j] = in[min(at + (from + j) * RES_STRIDE, total - 1)];
+            for (int j = 0; j < RES_BATCH; j++) dst[j] = last_load(at + (from + j) * RES_STRIDE);
         };
         auto put = [&](const f32x4 *src, unsigned from) {
 #pragma unroll
@@ -871,8 +877,9 @@ int iris_hip_group_norm_resident(void *stream, float *scratch, float *out, const
     const int cg = c / groups;
     const size_t total = (size_t)hw * c / 4;
     if (cg % 4 || RES_THREADS % (c / 4) || !al16(in) || !al16(out) || !al16(gamma) || !al16(beta) || total >= 1u << 28) return -2;
-    auto go = [&](auto kernel) {
-        static const hipError_t configured =
+    auto go = [&](auto silu, auto once) {
+        constexpr auto kernel = k_gn_resident<decltype(silu)::value, decltype(once)::value>;
+        static const hipError_t configured =                   /* one for each kernel: the arguments' types tell them apart */
             hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, RES_LDS_BYTES);
         if (configured != hipSuccess) return (int)configured;
         hipLaunchKernelGGL(kernel, dim3(RES_WGS), dim3(RES_THREADS), RES_LDS_BYTES, (hipStream_t)stream, reinterpret_cast<f32x4 *>(out),
@@ -880,7 +887,10 @@ int iris_hip_group_norm_resident(void *stream, float *scratch, float *out, const
                            patience);
         return (int)hipGetLastError();
     };
-    return do_silu ? go(k_gn_resident<true>) : go(k_gn_resident<false>);
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
+    if (total * 16 >= RES_ONCE_BYTES) return do_silu ? go(yes, yes) : go(no, yes);
+    return do_silu ? go(yes, no) : go(no, no);
 }
 
 /* scratch: iris_hip_group_norm_scratch_floats(groups) floats of device memory, prepared once. Behind the counters every slot a

@@ -194,3 +194,25 @@ def test_routes_that_copy_the_image_in_chunks_of_the_scratch(dev, route, h, w, c
     dev.free_all()
     assert (got[want.size:] == 7.0).all() and (page[scratch_bytes:] == 0x5a).all() and not page[:ZERO_BYTES].any()
     np.testing.assert_allclose(got[:want.size].reshape(want.shape), want, atol=2e-5 * np.sqrt(k * k * cin))
+
+
+def test_one_by_one_of_large_images(dev):
+    """192 MB of pixels are read with the streaming hint, a pixel less without: the same bits, and those of the definition."""
+    h, cin, cout = (192 << 20) // (384 * 4), 384, 100
+    rng = np.random.default_rng(5)
+    img = rng.standard_normal((h, cin), dtype=np.float32)
+    wt = O.f32_to_bf16((rng.standard_normal((cout, cin)) * 0.1).astype(np.float32))
+    b = rng.standard_normal(cout).astype(np.float32)
+    dimg, dw, db = dev.put(img), dev.put(wt), dev.put(b)
+    got = []
+    for n in (h, h - 1):
+        out = dev.put(np.full((h + 1, cout), 7.0, np.float32))
+        dev.lib.iris_dev_conv2d(out, dimg, dw, db, n, 1, cin, cout, 1, 1, 0, 0)
+        dev.check()
+        got.append(dev.get(out, (h + 1, cout), np.float32))
+        assert (got[-1][n:] == 7.0).all()
+    dev.free_all()
+    np.testing.assert_array_equal(got[0][:h - 1], got[1][:h - 1])
+    rows = np.unique(np.r_[0:40, h - 40:h, rng.integers(0, h, 400)])
+    want = O.bf16_to_f32(O.f32_to_bf16(img[rows])).astype(np.float64) @ O.bf16_to_f32(wt).astype(np.float64).T + b
+    np.testing.assert_allclose(got[0][rows], want, atol=2e-5 * np.sqrt(cin))
