@@ -274,24 +274,33 @@ k_gemm_tiles(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t
 }
 #pragma clang diagnostic pop
 
-/* y[i] = part[0][i] + part[1][i] + ..., eight values a thread (n a multiple of 8) */
-template <typename OUT>
+/* y[i] = part[0][i] + part[1][i] + ..., four values a thread (n a multiple of 8). AT_ONCE (at most `splits`) sums are requested
+ * before the first is used: what bounds it is the launch and one trip to memory, and one range after the other was a trip each. With
+ * the layer in front of it, us, eight values a thread and one after the other / now: 512 x 9728 -> 2560 (6 ranges) 36.5 / 36.0,
+ * 512 x 9216 -> 3072 (4) 39.7 / 38.9, 700 x 12288 -> 3072 (3) 62.2 / 61.1, 1000 x 9728 -> 2560 (3) 56.4 / 54.9; 100 and 320 rows the same. */
+constexpr int SUM_MOST = 8;
+template <typename OUT, int AT_ONCE>
 __global__ void __launch_bounds__(256)
 k_gemm_sum(OUT *__restrict__ y, const float *__restrict__ part, size_t n, int splits) {
-    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8;
+    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= n) return;
-    f32x4 lo = *reinterpret_cast<const f32x4 *>(part + i), hi = *reinterpret_cast<const f32x4 *>(part + i + 4);
+    f32x4 v[AT_ONCE];
+#pragma unroll
+    for (int s = 0; s < AT_ONCE; s++) v[s] = *reinterpret_cast<const f32x4 *>(part + s * n + i);
+#pragma unroll
+    for (int s = 1; s < AT_ONCE; s++) v[0] += v[s];
 #pragma unroll 4
-    for (int s = 1; s < splits; s++) {
-        lo += *reinterpret_cast<const f32x4 *>(part + s * n + i);
-        hi += *reinterpret_cast<const f32x4 *>(part + s * n + i + 4);
-    }
-    if constexpr (sizeof(OUT) == 4) {
-        *reinterpret_cast<f32x4 *>(y + i) = lo;
-        *reinterpret_cast<f32x4 *>(y + i + 4) = hi;
-    } else {
-        *reinterpret_cast<u32x4 *>(y + i) = u32x4{pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3])};
-    }
+    for (int s = AT_ONCE; s < splits; s++) v[0] += *reinterpret_cast<const f32x4 *>(part + s * n + i);
+    if constexpr (sizeof(OUT) == 4) *reinterpret_cast<f32x4 *>(y + i) = v[0];
+    else *reinterpret_cast<uint2 *>(y + i) = make_uint2(pack_bf16(v[0][0], v[0][1]), pack_bf16(v[0][2], v[0][3]));
+}
+
+template <typename OUT, int AT_ONCE = SUM_MOST>
+int launch_sum(hipStream_t st, OUT *y, const float *part, size_t n, int splits) {
+    if constexpr (AT_ONCE > 2)
+        if (splits < AT_ONCE) return launch_sum<OUT, AT_ONCE - 1>(st, y, part, n, splits);
+    hipLaunchKernelGGL((k_gemm_sum<OUT, AT_ONCE>), dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, st, y, part, n, splits);
+    return (int)hipGetLastError();
 }
 
 template <typename OUT, int NB, int WM, int NA, int WN, int KG, int STAGES>
@@ -369,10 +378,7 @@ int iris_hip_gemm_tiles(void *stream, void *y, int out_size, const uint16_t *x, 
     int e = launch_shape<float>(st, shape, part, x, W, M, N, K, nullptr, splits);
     if (e) return e;
     const size_t n = (size_t)M * N;
-    const dim3 grid((unsigned)((n / 8 + 255) / 256));
-    if (out_size == 2) hipLaunchKernelGGL(k_gemm_sum<uint16_t>, grid, dim3(256), 0, st, (uint16_t *)y, part, n, splits);
-    else hipLaunchKernelGGL(k_gemm_sum<float>, grid, dim3(256), 0, st, (float *)y, part, n, splits);
-    return (int)hipGetLastError();
+    return out_size == 2 ? launch_sum(st, (uint16_t *)y, part, n, splits) : launch_sum(st, (float *)y, part, n, splits);
 }
 
 }  // extern "C"

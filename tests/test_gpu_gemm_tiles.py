@@ -88,6 +88,13 @@ def test_orders_of_the_k_tiles(dev, shape, k_tiles, splits):
     one_layer(dev, shape, 5 * tm - 3, 64 * k_tiles, 5 * tn - 8, splits, k_tiles % 2 == 0)
 
 
+# up to eight partial sums are requested at once, more one after the other; the last workgroup is not full
+@pytest.mark.parametrize("splits", [2, 3, 4, 5, 6, 7, 8, 9, 13])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_numbers_of_partial_sums(dev, splits, bf16):
+    one_layer(dev, 0, 131, 64 * 13, 136, splits, bf16)
+
+
 @pytest.mark.parametrize("rows,k,out", [(1, 512, 128), (77, 2048, 1544), (130, 1536, 136), (300, 4096, 640), (500, 1024, 3072)])
 @pytest.mark.parametrize("bf16", [False, True])
 def test_linear_layers_that_take_it(dev, rows, k, out, bf16):
