@@ -30,6 +30,10 @@
  * run on four waves of 80 x 128 and 80 x 112 (12 KB for 35 products; 512 registers to a wave): 320 x 3072 -> 27648 in tiles of
  * 256 58.0 on eight waves / 56.5, 1024 x 3072 -> 9216 62.2 / 53.5; in tiles of 224, which fill 248 CUs instead of 216, 53.6.
  * Tiles of 128 x 256, 160 x 192 and 128 x 192 on four waves were as fast as on eight.
+ * A tile of 128 x 96 is there for what its width fills the chip with: 512 x 2560 -> 6144 takes 256 workgroups instead of 192 of
+ * 128 x 128, each of which fetches 224 rows instead of 256. Weights from HBM, us, without / with it: 512 x 2560 -> 6144 24.2 / 22.9,
+ * 320 rows 25.3 / 22.6, 512 x 3072 -> 3072 22.4 / 20.2 (two ranges of K instead of three), 700 rows 26.0 / 23.2, 1000 x 4096 -> 2560
+ * 32.2 / 30.2, 100 x 2560 -> 19456 33.0 / 30.7; no slower at any of the 60 sizes from 100 to 1000 rows where it is chosen.
  */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -324,7 +328,7 @@ int launch_tiles(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, i
  * its epilogue take 3.5 us more. */
 struct Shape { int tm, tn; float step, step_full; };
 constexpr Shape SHAPES[] = {{128, 128, 0.44f, 0.50f}, {128, 192, 0.58f, 0.62f}, {128, 256, 0.72f, 0.80f}, {64, 256, 0.60f, 0.61f},
-                            {160, 192, 0.67f, 0.72f}, {160, 256, 0.90f, 0.93f}, {160, 224, 0.84f, 0.87f}};
+                            {160, 192, 0.67f, 0.72f}, {160, 256, 0.90f, 0.93f}, {160, 224, 0.84f, 0.87f}, {128, 96, 0.39f, 0.45f}};
 constexpr int NSHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
 
 template <typename OUT>
@@ -337,6 +341,7 @@ int launch_shape(hipStream_t st, int shape, OUT *y, const uint16_t *x, const uin
     case 4: return launch_tiles<OUT, 5, 2, 3, 4, 1, 3>(st, y, x, W, M, N, K, bias, splits);
     case 5: return launch_tiles<OUT, 5, 2, 8, 2, 1, 3>(st, y, x, W, M, N, K, bias, splits);
     case 6: return launch_tiles<OUT, 5, 2, 7, 2, 1, 3>(st, y, x, W, M, N, K, bias, splits);
+    case 7: return launch_tiles<OUT, 4, 2, 3, 2, 2, 4>(st, y, x, W, M, N, K, bias, splits);
     default: return (int)hipErrorInvalidValue;
     }
 }
