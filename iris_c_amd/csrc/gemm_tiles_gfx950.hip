@@ -26,9 +26,10 @@
  * us, all in one order / turned: 512 x 2560 -> 6144 29.5 / 23.0, 512 x 3072 -> 9216 38.0 / 34.8, 512 x 9728 -> 2560 39.5 / 35.6,
  * 320 x 3072 -> 27648 59.1 / 55.5; with weights in the Infinity Cache 1 - 3 % slower. Turns over eight tiles, or turned by pairs
  * and fours of tiles, gave the same or less; four waves that only fetch beside the eight that multiply changed nothing.
- * Then comes the LDS: a wave's 64 x 64 outputs read 8 KB of operands for 16 products. The 160-row tiles of 256 and 224 columns
- * run on four waves of 80 x 128 and 80 x 112 (12 KB for 35 products; 512 registers to a wave): 320 x 3072 -> 27648 in tiles of
- * 256 58.0 on eight waves / 56.5, 1024 x 3072 -> 9216 62.2 / 53.5; in tiles of 224, which fill 248 CUs instead of 216, 53.6.
+ * Then comes the LDS: a wave's 64 x 64 outputs read 8 KB of operands for 16 products. The tile of 160 x 224 runs on four waves of 80 x 112
+ * (12 KB for 35 products; 512 registers to a wave) and fills 248 CUs with 320 x 3072 -> 27648 instead of 216: 58.0 us / 53.6. Tiles of
+ * 160 x 256 on four waves are no faster than on eight, and their ends longer: 1000 x 3072 -> 9216 52.2 us on four / 52.1, -> 18432 105.6 / 103.8,
+ * 11700 x 512 -> 1536 31.6 / 30.7, 1024 x 512 -> 1536 13.8 / 12.9.
  * Tiles of 128 x 256, 160 x 192 and 128 x 192 on four waves were as fast as on eight.
  * A tile of 128 x 96 is there for what its width fills the chip with: 512 x 2560 -> 6144 takes 256 workgroups instead of 192 of
  * 128 x 128, each of which fetches 224 rows instead of 256. Weights from HBM, us, without / with it: 512 x 2560 -> 6144 24.2 / 22.9,
@@ -339,7 +340,7 @@ int launch_shape(hipStream_t st, int shape, OUT *y, const uint16_t *x, const uin
     case 2: return launch_tiles<OUT, 4, 2, 4, 4, 1, 3>(st, y, x, W, M, N, K, bias, splits);
     case 3: return launch_tiles<OUT, 4, 1, 4, 4, 2, 4>(st, y, x, W, M, N, K, bias, splits);
     case 4: return launch_tiles<OUT, 5, 2, 3, 4, 1, 3>(st, y, x, W, M, N, K, bias, splits);
-    case 5: return launch_tiles<OUT, 5, 2, 8, 2, 1, 3>(st, y, x, W, M, N, K, bias, splits);
+    case 5: return launch_tiles<OUT, 5, 2, 4, 4, 1, 3>(st, y, x, W, M, N, K, bias, splits);
     case 6: return launch_tiles<OUT, 5, 2, 7, 2, 1, 3>(st, y, x, W, M, N, K, bias, splits);
     case 7: return launch_tiles<OUT, 4, 2, 3, 2, 2, 4>(st, y, x, W, M, N, K, bias, splits);
     default: return (int)hipErrorInvalidValue;
