@@ -51,6 +51,7 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 namespace {
 
 constexpr int TK = 64;
+constexpr size_t L2_BYTES = (size_t)4 << 20;                             /* of one XCD */
 
 __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
     f32x2 p = {lo, hi};
@@ -96,8 +97,9 @@ k_gemm_tiles(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;
-    /* the order of this workgroup's k tiles, see above: tile kt of the order is k tile kt ^ turn inside whole groups of four */
-    const int turn = (m0 / TM ^ n0 / TN) & 3, turned = nk & ~3;
+    /* the order of this workgroup's k tiles, see above: tile kt of the order is k tile kt ^ turn inside whole groups of four. Not where
+     * the weights fit an XCD's L2, as under the VAE's attention: its block at 128 x 128 582 us turned / 576, at 120 x 124 527 / 513 */
+    const int turn = (size_t)N * K * 2 > L2_BYTES ? (m0 / TM ^ n0 / TN) & 3 : 0, turned = nk & ~3;
     const int wm = wave % WM, wn = wave / WM % WN, kg = wave / (WM * WN);
 
     /* this wave's pieces of a stage: row 8 (PIECES wave + j) + lane / 8 of [W tile | x tile]; rows past the end of a matrix

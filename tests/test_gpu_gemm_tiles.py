@@ -96,6 +96,18 @@ def test_orders_of_the_k_tiles(dev, shape, k_tiles, splits):
     one_layer(dev, shape, 5 * tm - 3, 64 * k_tiles, 5 * tn - 8, splits, k_tiles % 2 == 0)
 
 
+# the same with weights of more than the 4 MB of an L2, the only ones that are taken in different orders; just below them
+@pytest.mark.parametrize("shape", range(8))
+@pytest.mark.parametrize("more,splits", [(-2, 1), (1, 1), (2, 1), (3, 1), (4, 5)])
+def test_orders_of_the_k_tiles_of_large_weights(dev, shape, more, splits):
+    tm, tn = (TILES + [(160, 224), (128, 96)])[shape]
+    out = 5 * tn - 8
+    k = ((1 << 21) // out // 256 * 4 + more) * 64            # whole groups of four k tiles up to 4 MB, and `more` k tiles
+    k += 256 * (more > 0 and k * out <= 1 << 21)
+    assert (k * out > 1 << 21) == (more > 0)
+    one_layer(dev, shape, 5 * tm - 3, k, out, splits, more % 2 == 0)
+
+
 # up to eight partial sums are requested at once, more one after the other; the last workgroup is not full
 @pytest.mark.parametrize("splits", [2, 3, 4, 5, 6, 7, 8, 9, 13])
 @pytest.mark.parametrize("bf16", [False, True])
