@@ -567,7 +567,7 @@ k_gn_resident(f32x4 *out, const f32x4 *in, const float *__restrict__ gamma, cons
     extern __shared__ f32x4 kept[];                            /* [RES_LDS][RES_THREADS] */
     __shared__ float2 sh[RES_THREADS];
     __shared__ float stat[2 * RES_MAX_GROUPS];
-    __shared__ unsigned verdict, to_do;
+    __shared__ unsigned verdict, to_do, found;
     const unsigned tid = threadIdx.x, b = blockIdx.x;
     const int quads = c >> 2, q = tid % quads, groups = c / cg, group = 4 * q / cg;
     /* a step is 512 quads in a row: whole pixels, so a thread keeps its quad of channels. n: this workgroup's steps */
@@ -719,7 +719,7 @@ k_gn_resident(f32x4 *out, const f32x4 *in, const float *__restrict__ gamma, cons
             return true;
         };
         bool go = b >= (unsigned)groups || finish(b);
-            if (go) {
+        if (go) {
             /* last to arrive: those that had given up by then (ARRIVALS is a multiple of the number less one) */
             quitters = __builtin_amdgcn_readfirstlane((before + 1) % RES_WGS == 0 ? (unsigned)(before >> 48) : 0u);
             if (quitters)
@@ -781,10 +781,10 @@ k_gn_resident(f32x4 *out, const f32x4 *in, const float *__restrict__ gamma, cons
                 if (tid == 0) {
                     const unsigned f = agent_load(&sync->gave_up[w]);
                     if (f) agent_store(&sync->gave_up[w], 0u);
-                    verdict = f;
+                    found = f;                                 /* not verdict: other waves may not have read that yet */
                 }
                 __syncthreads();
-                const unsigned f = verdict;
+                const unsigned f = found;
                 __syncthreads();
                 if (!f) continue;
                 left--;

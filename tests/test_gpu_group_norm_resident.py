@@ -92,6 +92,23 @@ def test_shares_that_are_given_up(dev, hw, c):
         np.testing.assert_array_equal(outs[0], o)
 
 
+@pytest.mark.parametrize("hw,c", [(steps(WGS * 3, 128), 128), (steps(WGS + 40, 512) + 3, 512)])
+def test_every_wave_stores_its_part_where_shares_are_given_up(dev, hw, c):
+    """The last workgroup goes from its own share straight on to the others': its waves still have to know that it did not give
+    up itself. Its share is another one in each call."""
+    x, gamma, beta = data(hw, c)
+    dx, dg, db, want = dev.put(x), dev.put(gamma), dev.put(beta), None
+    douts = [dev.put(np.full((hw, c), np.nan, np.float32)) for _ in range(12)]
+    for i, dout in enumerate(douts):
+        assert resident(dev, dout, dx, dg, db, hw, c, 32, 1, 0 if i else 1000000) == 0
+    for dout in douts:
+        got = dev.get(dout, (hw, c), np.float32)
+        want = got if want is None else want
+        np.testing.assert_array_equal(got, want)
+    dev.free_all()
+    compare(want, expected(x, gamma, beta, 32, 1))
+
+
 def test_what_it_does_not_take(dev):
     hw = 64
     p = dev.alloc(hw * 512 * 4 + 16)
