@@ -142,7 +142,9 @@ void iris_dev_group_norm(float *out, const float *in, const float *gamma, const 
  * moments and statistics, 1.05 MB) is an array inside the library instead of memory allocated at
  * the first call, so this entry calls no hipMalloc / hipFree at all. groups <= 64; more is refused
  * with an error (use iris_dev_group_norm). All calls on a GPU share that one array: calls that
- * overlap in time would race, so keep them on the library's stream, which orders them. */
+ * overlap in time would race, so keep them on the library's stream, which orders them: the overlapping
+ * calls give wrong values and may take seconds; later ones are not affected. The same holds for calls of
+ * iris_dev_group_norm, which share a scratch of their own. */
 void iris_dev_group_norm_noalloc(float *out, const float *in, const float *gamma, const float *beta,
                                  int hw, int c, int groups, float eps, int silu);
 /* nearest-neighbour 2x upsampling of [h * w, c] into [2h * 2w, c] (reference iris_dev.h:128-129) */

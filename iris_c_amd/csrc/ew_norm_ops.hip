@@ -529,20 +529,26 @@ k_gn_normalize(float *__restrict__ out, const float *__restrict__ in, const floa
  *
  * The wait is bounded and needs no workgroup to be resident beside another: one that has waited for `patience` ticks of 10 ns
  * (another process may hold CUs) gives up its share: it notes that in the counter of arrivals and in its flag and ends. The
- * counter takes such a note only while a workgroup is missing, so the one that arrives last knows how many there are, gathers
- * all groups, as the workgroups meant to may be among them, and normalises their shares itself. What is on its way once all have
- * arrived is looked for RES_LATE times, so that calls that share a scratch buffer and overlap, which the callers rule out, get
- * wrong values and not a wait without end. */
+ * counter takes such a note only while a workgroup of its launch is missing, so the one that arrives last knows how many there are,
+ * gathers all groups, as the workgroups meant to may be among them, and normalises their shares itself.
+ *
+ * Calls that share a scratch buffer must not overlap, and the callers rule it out. If they do they get wrong values, but neither a
+ * wait without end nor anything that a later call would suffer from: what is on its way once all have arrived is looked for a
+ * bounded number of times; every launch adds RES_WGS arrivals, whatever happens; nothing is taken off the counter again, the
+ * last to arrive notes how far it was instead (`closed`, which only grows); and flags carry the number of the launch. So when
+ * everything has ended the counter is a multiple of RES_WGS, `closed` holds its state, and no word carries the next number. */
 constexpr int RES_WGS = 256, RES_THREADS = 512, RES_REG = 48, RES_LDS = 18, RES_KEEP = RES_REG + RES_LDS, RES_BATCH = 8, RES_LDS_BATCH = 6;
 constexpr unsigned RES_STRIDE = RES_WGS * RES_THREADS;
 constexpr int RES_LDS_BYTES = RES_LDS * RES_THREADS * 16;
 constexpr int RES_MIN_GROUPS = 8, RES_MAX_GROUPS = 64;         /* a group's threads are at most a wave; a wave gathers the statistics */
 constexpr size_t RES_MIN_BYTES = (size_t)8 << 20;
-constexpr unsigned RES_PATIENCE = 1000000, RES_LATE = 1u << 20;
+constexpr unsigned RES_PATIENCE = 1000000, RES_LATE = 1u << 20, RES_SWEEPS = 1u << 12;         /* a second or so each */
 struct Tagged { unsigned long long a, b; };                    /* two floats, each with the number of the launch in its high half */
 struct ResidentSync {
-    unsigned long long arrivals;                               /* of all launches; + 2^48 for each workgroup of this launch that gave up */
-    unsigned pad[30], gave_up[RES_WGS];
+    unsigned long long arrivals;                               /* of all launches; in the upper 16 bits those that gave up, modulo 2^16 */
+    unsigned long long closed;                                 /* the last launch that all arrived in * 2^16 + those upper bits then */
+    unsigned pad[28];
+    unsigned long long gave_up[RES_WGS];                       /* the launch whose share this workgroup has given up */
     Tagged stat[RES_MAX_GROUPS], part[RES_MAX_GROUPS][RES_WGS];
 };
 constexpr size_t SYNC_FLOATS = sizeof(ResidentSync) / sizeof(float);
@@ -577,8 +583,10 @@ k_gn_resident(f32x4 *out, const f32x4 *in, const float *__restrict__ gamma, cons
     auto load = [&](unsigned i) { return in[min(at0 + i * RES_STRIDE, total - 1)]; };
     auto last_load = [&](unsigned at) { return ONCE ? __builtin_nontemporal_load(in + min(at, total - 1)) : in[min(at, total - 1)]; };
     constexpr unsigned long long ARRIVALS = (1ull << 48) - 1;
-    /* the number of this launch, the same in all workgroups as this one has not arrived yet */
-    const unsigned epoch = (unsigned)((agent_load(&sync->arrivals) & ARRIVALS) / RES_WGS) + 1;
+    /* the number of this launch, the same in all workgroups as this one has not arrived yet; words carry 31 bits of it and a one,
+     * as a new scratch is all zeros */
+    const unsigned long long closed = agent_load(&sync->closed), launch = (agent_load(&sync->arrivals) & ARRIVALS) / RES_WGS + 1;
+    const unsigned epoch = (unsigned)launch | 1u << 31;
 
     /* moments of this thread's values, shifted by the first value of the workgroup's share of the group; sums of a batch at a time */
     float k = 0.0f, s = 0.0f, ss = 0.0f;
@@ -691,9 +699,9 @@ k_gn_resident(f32x4 *out, const f32x4 *in, const float *__restrict__ gamma, cons
                 int gave_up = 0;
                 if (tid == 0) {
                     unsigned long long seen = agent_load(&sync->arrivals);
-                    while (!gave_up && (unsigned)((seen & ARRIVALS) / RES_WGS) != epoch)
+                    while (!gave_up && (seen & ARRIVALS) / RES_WGS < launch)
                         gave_up = __hip_atomic_compare_exchange_strong(&sync->arrivals, &seen, seen + (1ull << 48), __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    if (gave_up) agent_store(&sync->gave_up[b], 1u);
+                    if (gave_up) agent_store(&sync->gave_up[b], launch);
                 }
                 if (__any(gave_up)) return false;
                 late++;                                        /* all have arrived */
@@ -721,7 +729,12 @@ k_gn_resident(f32x4 *out, const f32x4 *in, const float *__restrict__ gamma, cons
         bool go = b >= (unsigned)groups || finish(b);
         if (go) {
             /* last to arrive: those that had given up by then (ARRIVALS is a multiple of the number less one) */
-            quitters = __builtin_amdgcn_readfirstlane((before + 1) % RES_WGS == 0 ? (unsigned)(before >> 48) : 0u);
+            if (tid == 0 && (before + 1) % RES_WGS == 0) {
+                const unsigned long long all = ((before & ARRIVALS) + 1) / RES_WGS, gone = before >> 48;
+                if (closed >> 16 == all - 1) quitters = (unsigned)(gone - closed) & 0xffffu;
+                (void)__hip_atomic_fetch_max(&sync->closed, all << 16 | gone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            quitters = __builtin_amdgcn_readfirstlane(quitters);
             if (quitters)
                 for (unsigned gr = 0; gr < (unsigned)groups; gr++) (void)finish(gr);          /* theirs may be among them */
             float m[1], r[1];
@@ -774,13 +787,12 @@ k_gn_resident(f32x4 *out, const f32x4 *in, const float *__restrict__ gamma, cons
     again(RES_KEEP, n, at0);
 
     if (quitters) {
-        if (tid == 0) __hip_atomic_fetch_add(&sync->arrivals, -((unsigned long long)quitters << 48), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         unsigned left = quitters;
-        for (unsigned sweep = 0; left > 0 && sweep < RES_LATE; sweep++)
+        for (unsigned sweep = 0; left > 0 && sweep < RES_SWEEPS; sweep++)
             for (unsigned w = 0; w < RES_WGS; w++) {
                 if (tid == 0) {
-                    const unsigned f = agent_load(&sync->gave_up[w]);
-                    if (f) agent_store(&sync->gave_up[w], 0u);
+                    const unsigned f = agent_load(&sync->gave_up[w]) == launch;
+                    if (f) agent_store(&sync->gave_up[w], 0ull);
                     found = f;                                 /* not verdict: other waves may not have read that yet */
                 }
                 __syncthreads();
@@ -940,7 +952,7 @@ int iris_hip_group_norm(void *stream, float *scratch, float *out, const float *i
  * not overlap (the library issues everything on one stream, which orders them). */
 constexpr int GN_STATIC_MAX_GROUPS = 64;
 constexpr size_t GN_STATIC_FLOATS = SYNC_FLOATS + 3 * (size_t)GN_STATIC_MAX_GROUPS * GN_MAX_BLOCKS + 2 * (size_t)GN_STATIC_MAX_GROUPS;
-static __device__ __align__(256) float scratch[GN_STATIC_FLOATS];          /* 1,051,264 B, zero when the library is loaded */
+static __device__ __align__(256) float scratch[GN_STATIC_FLOATS];          /* 1,052,288 B, zero when the library is loaded */
 
 constexpr int GN_STATIC_MAX_DEVICES = 64;
 static float *scratch_address[GN_STATIC_MAX_DEVICES];                        /* per device; null = not looked up yet */

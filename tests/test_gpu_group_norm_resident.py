@@ -109,6 +109,28 @@ def test_every_wave_stores_its_part_where_shares_are_given_up(dev, hw, c):
     compare(want, expected(x, gamma, beta, 32, 1))
 
 
+# words of 64 bits at the front of the scratch: arrivals of all launches with the number of those that gave up above bit 48, the
+# last launch that all arrived in with that number in its low 16 bits; from byte 128 on the launch a workgroup gave up in
+@pytest.mark.parametrize("launches,gone,flags", [(3, 0, 0), (3, 7, 3), (3, 7, 1), (1000, 65535, 1000), (1 << 32, 12, 1 << 32), ((1 << 32) - 1, 300, 5)])
+def test_counters_that_calls_have_left_behind(dev, launches, gone, flags):
+    """Shares given up in earlier launches, however many, are no business of this one: not normalised a second time in place."""
+    hw, c = steps(WGS + 9, 128) + 3, 128
+    x, gamma, beta = data(hw, c)
+    dx, dg, db, dout = dev.put(x), dev.put(gamma), dev.put(beta), dev.alloc(hw * c * 4)
+    words = np.zeros(16 + WGS, np.uint64)
+    words[0], words[1], words[16:] = launches * WGS + (gone << 48), (launches << 16) + gone, flags
+    dev.dev.lib.iris_dev_upload(dev.scratch, words.ctypes.data_as(C.c_void_p), words.nbytes)
+    for patience in (1000000, 0):
+        assert resident(dev, dout, dx, dg, db, hw, c, 32, 1, patience) == 0
+        compare(dev.get(dout, (hw, c), np.float32), expected(x, gamma, beta, 32, 1))
+    words = dev.get(dev.scratch, (16 + WGS,), np.uint64)
+    assert words[0] % (1 << 48) == (launches + 2) * WGS and words[1] >> 16 == launches + 2 and words[1] % 65536 == words[0] >> 48
+    assert resident(dev, dx, dx, dg, db, hw, c, 32, 1) == 0
+    compare(dev.get(dx, (hw, c), np.float32), expected(x, gamma, beta, 32, 1))
+    dev.free_all()
+    assert dev.lib.iris_hip_group_norm_prepare_scratch(dev.stream, dev.scratch) == 0
+
+
 def test_what_it_does_not_take(dev):
     hw = 64
     p = dev.alloc(hw * 512 * 4 + 16)
