@@ -540,7 +540,7 @@ k_gn_normalize(float *__restrict__ out, const float *__restrict__ in, const floa
 constexpr int RES_WGS = 256, RES_THREADS = 512, RES_REG = 48, RES_LDS = 18, RES_KEEP = RES_REG + RES_LDS, RES_BATCH = 8, RES_LDS_BATCH = 6;
 constexpr unsigned RES_STRIDE = RES_WGS * RES_THREADS;
 constexpr int RES_LDS_BYTES = RES_LDS * RES_THREADS * 16;
-constexpr int RES_MIN_GROUPS = 8, RES_MAX_GROUPS = 64;         /* a group's threads are at most a wave; a wave gathers the statistics */
+constexpr int RES_MIN_GROUPS = 8, RES_MAX_GROUPS = IRIS_GN_MOST_GROUPS;        /* a group's threads are at most a wave; a wave gathers the statistics */
 constexpr size_t RES_MIN_BYTES = (size_t)8 << 20;
 constexpr unsigned RES_PATIENCE = 1000000, RES_LATE = 1u << 20, RES_SWEEPS = 1u << 12;         /* a second or so each */
 struct Tagged { unsigned long long a, b; };                    /* two floats, each with the number of the launch in its high half */
@@ -950,7 +950,7 @@ int iris_hip_group_norm(void *stream, float *scratch, float *out, const float *i
  * process ends. In host code the array's name is only a handle for hipGetSymbolAddress; kernels
  * get the address that call returned, kept per device. Calls on one GPU share the array: they must
  * not overlap (the library issues everything on one stream, which orders them). */
-constexpr int GN_STATIC_MAX_GROUPS = 64;
+constexpr int GN_STATIC_MAX_GROUPS = IRIS_GN_MOST_GROUPS;
 constexpr size_t GN_STATIC_FLOATS = SYNC_FLOATS + 3 * (size_t)GN_STATIC_MAX_GROUPS * GN_MAX_BLOCKS + 2 * (size_t)GN_STATIC_MAX_GROUPS;
 static __device__ __align__(256) float scratch[GN_STATIC_FLOATS];          /* 1,052,288 B, zero when the library is loaded */
 

@@ -118,8 +118,9 @@ int iris_hip_rms_norm_mod(void *stream, uint16_t *out, const float *x, const flo
                           const float *scale, int rows, int dim, float eps);
 int iris_hip_rms_norm_residual(void *stream, float *x, const float *a, const float *w,
                                const float *gate, int rows, int dim, float eps);
-/* group norm needs iris_hip_group_norm_scratch_floats(groups) floats of device scratch, prepared once;
- * requires c % groups == 0. The resident form (-2: not taken) is the one launch that large images take. */
+/* group norm needs iris_hip_group_norm_scratch_floats(groups) floats of device scratch, prepared once if groups is at most
+ * IRIS_GN_MOST_GROUPS; requires c % groups == 0. The resident form (-2: not taken) is the one launch that large images take. */
+#define IRIS_GN_MOST_GROUPS 64
 size_t iris_hip_group_norm_scratch_floats(int groups);
 int iris_hip_group_norm_prepare_scratch(void *stream, float *scratch);
 int iris_hip_group_norm_resident(void *stream, float *scratch, float *out, const float *in, const float *gamma,

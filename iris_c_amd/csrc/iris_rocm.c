@@ -28,15 +28,16 @@ static hipStream_t g_stream = NULL;
 static int g_last_error = 0;
 static const char *g_last_kernel = "none";
 /* private scratch, allocated on first use and kept until cleanup (as the reference backend
- * does, iris_cuda.cu:149-173): convolution patches and group-norm partial sums */
+ * does, iris_cuda.cu:149-173): convolution patches, group-norm partial moments of many groups */
 #ifndef IRIS_DEV_PATH_ONLY
 #define CONV_SCRATCH_BYTES ((size_t)256 << 20)
 static uint16_t *g_conv_scratch = NULL;
 /* partial sums of linear layers whose K is cut into ranges; allocated at initialisation, so that a linear layer never
  * allocates */
 static float *g_linear_part = NULL;
-static float *g_gn_scratch = NULL;
-static size_t g_gn_scratch_floats = 0;
+/* group norm of up to 64 groups, which keeps counters there: allocated and cleared once, by iris_dev_init; and of more */
+static float *g_gn_scratch = NULL, *g_gn_more = NULL;
+static size_t g_gn_more_floats = 0;
 #endif
 /* normalised copy of Q for the iris_dev_attention_qnorm calls that the matrix-core kernel does not take */
 static uint16_t *g_q_scratch = NULL;
@@ -71,6 +72,21 @@ static int need_ready(const char *what) {
 }
 
 #ifndef IRIS_DEV_PATH_ONLY
+/* At initialisation, as the first call may come inside a capture, where the clearing would be recorded and not run. A call that
+ * finds none, there having been no memory then, tries again outside a capture. */
+static int gn_scratch_setup(void) {
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (g_gn_scratch) return 1;
+    if (hipStreamIsCapturing(g_stream, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) return 0;
+    if (hipMalloc((void **)&g_gn_scratch, iris_hip_group_norm_scratch_floats(IRIS_GN_MOST_GROUPS) * sizeof(float)) == hipSuccess) {
+        if (iris_hip_group_norm_prepare_scratch(g_stream, g_gn_scratch) == 0 && hipStreamSynchronize(g_stream) == hipSuccess) return 1;
+        (void)hipFree(g_gn_scratch);
+    }
+    (void)hipGetLastError();
+    g_gn_scratch = NULL;
+    return 0;
+}
+
 int iris_dev_init(void) {
     if (g_ready) return 1;
     int count = 0;
@@ -91,6 +107,7 @@ int iris_dev_init(void) {
         g_linear_part = NULL;
     }
     if (hipStreamCreate(&g_stream) != hipSuccess) return 0;
+    (void)gn_scratch_setup();
     /* address of the in-library scratch of iris_dev_group_norm_noalloc on this device; if the lookup
      * fails here the entry point tries again at its first call and reports it there */
     (void)iris_hip_group_norm_static_setup();
@@ -122,6 +139,7 @@ void iris_dev_cleanup(void) {
     if (g_linear_part) check(hipFree(g_linear_part), "free");
     g_linear_part = NULL;
     if (g_gn_scratch) check(hipFree(g_gn_scratch), "free");
+    if (g_gn_more) check(hipFree(g_gn_more), "free");
     if (g_rope_stage) check(hipFree(g_rope_stage), "free");
     if (g_q_scratch) check(hipFree(g_q_scratch), "free");
     if (g_pack) check(hipFree(g_pack), "free");
@@ -134,8 +152,8 @@ void iris_dev_cleanup(void) {
     g_q_scratch_bytes = 0;
     iris_lt_release();
     g_conv_scratch = NULL;
-    g_gn_scratch = NULL;
-    g_gn_scratch_floats = 0;
+    g_gn_scratch = g_gn_more = NULL;
+    g_gn_more_floats = 0;
     g_rope_stage = NULL;
     g_rope_stage_bytes = 0;
     check(hipStreamDestroy(g_stream), "stream destroy");
@@ -594,30 +612,32 @@ void iris_dev_group_norm(float *out, const float *in, const float *gamma, const 
     if (!need_ready("group_norm")) return;
     if (hw <= 0 || c <= 0) return;
     if (groups <= 0 || c % groups != 0) { fail(-1, "group_norm", "need c % groups == 0"); return; }
-    size_t need = iris_hip_group_norm_scratch_floats(groups);
-    if (need > g_gn_scratch_floats) {
-        if (g_gn_scratch) {
-            check(hipStreamSynchronize(g_stream), "sync");
-            check(hipFree(g_gn_scratch), "free");
+    float *scratch;
+    if (groups > IRIS_GN_MOST_GROUPS) {                        /* no counters: every slot is written before it is read */
+        size_t need = iris_hip_group_norm_scratch_floats(groups);
+        if (need > g_gn_more_floats) {
+            if (g_gn_more) {
+                check(hipStreamSynchronize(g_stream), "sync");
+                check(hipFree(g_gn_more), "free");
+            }
+            g_gn_more = NULL;
+            g_gn_more_floats = 0;
+            if (hipMalloc((void **)&g_gn_more, need * sizeof(float)) != hipSuccess) {
+                (void)hipGetLastError();
+                g_gn_more = NULL;
+                fail(-1, "group_norm", "scratch allocation failed");
+                return;
+            }
+            g_gn_more_floats = need;
         }
-        g_gn_scratch = NULL;
-        g_gn_scratch_floats = 0;
-        if (hipMalloc((void **)&g_gn_scratch, need * sizeof(float)) != hipSuccess) {
-            (void)hipGetLastError();
-            g_gn_scratch = NULL;
-            fail(-1, "group_norm", "scratch allocation failed");
-            return;
-        }
-        int e = iris_hip_group_norm_prepare_scratch(g_stream, g_gn_scratch);
-        if (e) {
-            check((hipError_t)e, "group_norm scratch");
-            check(hipFree(g_gn_scratch), "free");
-            g_gn_scratch = NULL;
-            return;
-        }
-        g_gn_scratch_floats = need;
+        scratch = g_gn_more;
+    } else if (!gn_scratch_setup()) {
+        fail(-1, "group_norm", "scratch allocation failed");
+        return;
+    } else {
+        scratch = g_gn_scratch;
     }
-    int err = iris_hip_group_norm(g_stream, g_gn_scratch, out, in, gamma, beta, hw, c, groups, eps, silu != 0);
+    int err = iris_hip_group_norm(g_stream, scratch, out, in, gamma, beta, hw, c, groups, eps, silu != 0);
     if (err) check((hipError_t)err, "group_norm launch");
 }
 

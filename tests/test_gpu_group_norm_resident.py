@@ -171,3 +171,40 @@ def test_replayed_from_a_graph(dev):
     dev.check()
     dev.free_all()
     compare(want, expected(x, gamma, beta, 32, 1))
+
+
+def test_first_call_of_a_process_inside_a_relaxed_capture(tmp_path):
+    """The counters are cleared by then: an eager call before the first replay, the replays and eager calls between them all give
+    the same. A copy of the library, so that the call is its first."""
+    import shutil
+    import iris_c_amd
+    from test_gpu_graph import Graphs
+    lib = C.CDLL(shutil.copy(iris_c_amd.LIB_PATH, tmp_path / "first_call.so"))
+    for name, (res, args) in iris_c_amd.ABI.items():
+        getattr(lib, name).restype, getattr(lib, name).argtypes = res, args
+    assert lib.iris_dev_init() == 1
+    g, stream = Graphs(), C.c_void_p(lib.iris_dev_stream())
+    hw, c = 40000, 128
+    x, gamma, beta = data(hw, c)
+    def put(a):
+        p = lib.iris_dev_alloc(a.nbytes)
+        lib.iris_dev_upload(p, a.ctypes.data_as(C.c_void_p), a.nbytes)
+        return p
+    dx, dg, db, captured, eager = put(x), put(gamma), put(beta), lib.iris_dev_alloc(x.nbytes), lib.iris_dev_alloc(x.nbytes)
+    graph, run = C.c_void_p(), C.c_void_p()
+    assert g.rt.hipStreamBeginCapture(stream, 2) == 0                                          # hipStreamCaptureModeRelaxed
+    lib.iris_dev_group_norm(captured, dx, dg, db, hw, c, 32, 1e-6, 1)
+    assert g.rt.hipStreamEndCapture(stream, C.byref(graph)) == 0 and graph
+    assert lib.iris_dev_last_error() == 0
+    assert g.rt.hipGraphInstantiate(C.byref(run), graph, None, None, 0) == 0
+    g.rt.hipGraphDestroy(graph)
+    got = np.empty_like(x)
+    for _ in range(3):
+        lib.iris_dev_group_norm(eager, dx, dg, db, hw, c, 32, 1e-6, 1)
+        assert g.rt.hipGraphLaunch(run, stream) == 0
+        lib.iris_dev_sync()
+        for out in (eager, captured):
+            lib.iris_dev_download(got.ctypes.data_as(C.c_void_p), out, got.nbytes)
+            compare(got, expected(x, gamma, beta, 32, 1))
+    g.rt.hipGraphExecDestroy(run)
+    lib.iris_dev_cleanup()
