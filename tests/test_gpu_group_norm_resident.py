@@ -131,6 +131,32 @@ def test_counters_that_calls_have_left_behind(dev, launches, gone, flags):
     assert dev.lib.iris_hip_group_norm_prepare_scratch(dev.stream, dev.scratch) == 0
 
 
+@pytest.mark.parametrize("c,per_group", [(128, 4), (512, 16), (256, 32)])
+@pytest.mark.parametrize("what", ["a hot pixel", "hot pixels", "a very hot pixel", "a hot row", "an offset", "a step"])
+def test_values_far_from_the_rest(dev, c, per_group, what):
+    """Where the sums of a thread start says nothing about the rest: images with pixels far off at the front of one workgroup's share
+    or of all, with a large mean, with two levels."""
+    hw = steps(WGS * 9, c)
+    x, gamma, beta = data(hw, c)
+    share = 2048 // c                                           # pixels from the front of a workgroup's share to that of the next
+    if what == "a hot pixel": x[37 * share] += 600.0
+    if what == "hot pixels": x[0:WGS * share:share] += 600.0
+    if what == "a very hot pixel": x[37 * share] += 20000.0
+    if what == "a hot row": x[:share] *= 30.0
+    if what == "an offset": x += 1000.0
+    if what == "a step": x[hw // 2:] += 200.0
+    want = expected(x, gamma, beta, c // per_group, 0)
+    dx, dg, db, dout = dev.put(x), dev.put(gamma), dev.put(beta), dev.alloc(hw * c * 4)
+    assert resident(dev, dout, dx, dg, db, hw, c, c // per_group, 0) == 0
+    got = dev.get(dout, (hw, c), np.float32)
+    dev.free_all()
+    # A thread adds 36 values and their squares about its first one, d of it away: M2 loses at most 36 d^2 x 2^-24, and d^2 is at
+    # most what M2 of the group has anyway. Half of it in the reciprocal root, once more for the merging; the mean is a float.
+    rel = 36 * 2.0 ** -24 + 2.0 ** -20
+    spread = x.astype(np.float64).std()
+    np.testing.assert_allclose(got, want, rtol=rel, atol=6 * 2.0 ** -20 + np.abs(x.mean(dtype=np.float64)) / spread * 1.5 * 2.0 ** -23)
+
+
 def test_what_it_does_not_take(dev):
     hw = 64
     p = dev.alloc(hw * 512 * 4 + 16)
