@@ -707,22 +707,23 @@ k_gn_resident(f32x4 *out, const f32x4 *in, const float *__restrict__ gamma, cons
             }
             return true;
         };
-        /* a group's statistics from the moments of all shares, in double */
+        /* a group's statistics from the moments of all shares, in double as k_gn_finish takes them: nothing turns what is not a
+         * number into one */
         auto finish = [&](unsigned gr) {
             constexpr int N = RES_WGS / 64;
-            double sum = 0.0, sq = 0.0;
             float m[N], m2[N];
             if (!wait(&sync->part[gr][tid], true, m, m2)) return false;
+            double sum = 0.0, sq = 0.0;
+#pragma unroll
+            for (int i = 0; i < N; i++) sum += (double)values_of(64 * i + tid) * (double)m[i];
+            const double num = (double)total * (4.0 / (double)groups), mean = wave_sum64(sum) / num;
 #pragma unroll
             for (int i = 0; i < N; i++) {
-                const double weighted = (double)values_of(64 * i + tid) * (double)m[i];
-                sum += weighted;
-                sq += (double)m2[i] + weighted * (double)m[i];
+                const double d = (double)m[i] - mean, count = (double)values_of(64 * i + tid);
+                if (count > 0.0) sq += (double)m2[i] + count * d * d;
             }
-            sum = wave_sum64(sum);
             sq = wave_sum64(sq);
-            const double num = (double)total * (4.0 / (double)groups), mean = sum / num;
-            if (tid == 0) put(&sync->stat[gr], (float)mean, (float)(1.0 / sqrt(fmax(sq / num - mean * mean, 0.0) + (double)eps)));
+            if (tid == 0) put(&sync->stat[gr], (float)mean, (float)(1.0 / sqrt(sq / num + (double)eps)));
             return true;
         };
         bool go = b >= (unsigned)groups || finish(b);

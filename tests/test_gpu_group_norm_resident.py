@@ -157,6 +157,26 @@ def test_values_far_from_the_rest(dev, c, per_group, what):
     np.testing.assert_allclose(got, want, rtol=rel, atol=6 * 2.0 ** -20 + np.abs(x.mean(dtype=np.float64)) / spread * 1.5 * 2.0 ** -23)
 
 
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("pixel", [0, 16, -1])
+@pytest.mark.parametrize("steps_each", [0.125, 3])
+def test_infinities_and_nan_spoil_their_group_only(dev, value, pixel, steps_each):
+    """As the definition has it (x - mean is infinite or not a number, the variance is not a number), and the other form. The last
+    pixel is all that its workgroup has of the last step, or of the image."""
+    hw, c, groups = steps(int(WGS * steps_each), 128) + 1, 128, 32
+    x, gamma, beta = data(hw, c)
+    x[pixel, 13] = value                                        # group 3
+    x[pixel, 40], x[pixel - 1, 41] = value, -value              # group 10
+    dx, dg, db, dout = dev.put(x), dev.put(gamma), dev.put(beta), dev.alloc(hw * c * 4)
+    assert resident(dev, dout, dx, dg, db, hw, c, groups, 0) == 0
+    got = dev.get(dout, (hw, c), np.float32)
+    dev.free_all()
+    spoilt = np.isin(np.arange(c) // 4, (3, 10))
+    assert np.isnan(got[:, spoilt]).all()
+    x[:, spoilt] = 0.0
+    compare(got[:, ~spoilt], expected(x, gamma, beta, groups, 0)[:, ~spoilt])
+
+
 def test_what_it_does_not_take(dev):
     hw = 64
     p = dev.alloc(hw * 512 * 4 + 16)
