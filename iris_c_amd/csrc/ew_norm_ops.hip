@@ -530,7 +530,7 @@ k_gn_normalize(float *__restrict__ out, const float *__restrict__ in, const floa
  * workgroup gathering all groups the wait took 25 us in place of 5.
  *
  * The wait is bounded and needs no workgroup to be resident beside another: one that has waited for `patience` ticks of 10 ns
- * (another process may hold CUs) gives up its share: it notes that in the counter of arrivals and in its flag and ends. The
+ * (another process, or work on another stream, may hold CUs) gives up its share: it notes that in the counter of arrivals and in its flag and ends. The
  * counter takes such a note only while a workgroup of its launch is missing, so the one that arrives last knows how many there are,
  * gathers all groups, as the workgroups meant to may be among them, and normalises their shares itself.
  *
@@ -558,6 +558,17 @@ constexpr size_t SYNC_FLOATS = sizeof(ResidentSync) / sizeof(float);
 __global__ void __launch_bounds__(ROW_THREADS)
 k_gn_clear(unsigned *sync) {
     for (unsigned i = threadIdx.x; i < SYNC_FLOATS; i += ROW_THREADS) sync[i] = 0u;
+}
+
+/* compute units of the current device: 256 on an MI355X that is not partitioned */
+int cu_count() {
+    static const int n = [] {
+        int dev = 0, cus = 0;
+        if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess) return cus;
+        (void)hipGetLastError();
+        return 0;
+    }();
+    return n;
 }
 
 template <typename T> __device__ __forceinline__ T agent_load(const T *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -881,14 +892,24 @@ int iris_hip_group_norm_prepare_scratch(void *stream, float *scratch) {
     return (int)hipGetLastError();
 }
 
-/* The norm as one launch: -2, with nothing enqueued, for what it does not take: it wants a thread to keep one quad of channels
- * through all its steps, and 32-bit byte offsets. scratch as below; patience in ticks of 10 ns. */
+/* What k_gn_resident takes: a thread keeps one quad of channels through all its steps, and byte offsets have 32 bits. */
+static bool resident_shape(int hw, int c, int groups) {
+    return hw > 0 && c > 0 && groups >= RES_MIN_GROUPS && groups <= RES_MAX_GROUPS && c % groups == 0 && c / groups % 4 == 0 &&
+           RES_THREADS % (c / 4) == 0 && (size_t)hw * c / 4 < 1u << 28;
+}
+
+/* 1: an image of this size is normalised by one launch, on a device of `cus` CUs, on which its workgroups all find room at once. On
+ * fewer (a partition of the device) those that do would hold their CUs until their patience ends, 10 ms at a time. Host arithmetic only. */
+int iris_hip_group_norm_plan(int hw, int c, int groups, int cus) {
+    return resident_shape(hw, c, groups) && (size_t)hw * c * sizeof(float) >= RES_MIN_BYTES && cus >= RES_WGS;
+}
+
+/* The norm as one launch: -2, with nothing enqueued, for what it does not take. scratch as below; patience in ticks of 10 ns. */
 int iris_hip_group_norm_resident(void *stream, float *scratch, float *out, const float *in, const float *gamma, const float *beta,
                                  int hw, int c, int groups, float eps, int do_silu, unsigned patience) {
-    if (hw <= 0 || c <= 0 || groups < RES_MIN_GROUPS || groups > RES_MAX_GROUPS || c % groups) return -2;
+    if (!resident_shape(hw, c, groups) || !al16(in) || !al16(out) || !al16(gamma) || !al16(beta)) return -2;
     const int cg = c / groups;
     const size_t total = (size_t)hw * c / 4;
-    if (cg % 4 || RES_THREADS % (c / 4) || !al16(in) || !al16(out) || !al16(gamma) || !al16(beta) || total >= 1u << 28) return -2;
     auto go = [&](auto silu, auto once) {
         constexpr auto kernel = k_gn_resident<decltype(silu)::value, decltype(once)::value>;
         static const hipError_t configured =                   /* one for each kernel: the arguments' types tell them apart */
@@ -910,7 +931,7 @@ int iris_hip_group_norm_resident(void *stream, float *scratch, float *out, const
 int iris_hip_group_norm(void *stream, float *scratch, float *out, const float *in, const float *gamma,
                         const float *beta, int hw, int c, int groups, float eps, int do_silu) {
     if (hw <= 0 || c <= 0) return 0;
-    if ((size_t)hw * c * sizeof(float) >= RES_MIN_BYTES) {
+    if (iris_hip_group_norm_plan(hw, c, groups, cu_count())) {
         const int e = iris_hip_group_norm_resident(stream, scratch, out, in, gamma, beta, hw, c, groups, eps, do_silu, RES_PATIENCE);
         if (e != -2) return e;
     }

@@ -123,6 +123,7 @@ int iris_hip_rms_norm_residual(void *stream, float *x, const float *a, const flo
 #define IRIS_GN_MOST_GROUPS 64
 size_t iris_hip_group_norm_scratch_floats(int groups);
 int iris_hip_group_norm_prepare_scratch(void *stream, float *scratch);
+int iris_hip_group_norm_plan(int hw, int c, int groups, int cus);
 int iris_hip_group_norm_resident(void *stream, float *scratch, float *out, const float *in, const float *gamma,
                                  const float *beta, int hw, int c, int groups, float eps, int do_silu, unsigned patience);
 int iris_hip_group_norm(void *stream, float *scratch, float *out, const float *in, const float *gamma,

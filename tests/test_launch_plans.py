@@ -229,3 +229,23 @@ def test_profile_summaries_say_which_source_they_were_taken_on():
     import bench
     nbytes, source, stale = bench.traffic_on_file()
     assert nbytes and nbytes > 113_246_208 and source.endswith("hbm_traffic.txt") and stale in (True, False)
+
+
+# ------------------------------------------------------------------ group norm as one launch
+@pytest.fixture(scope="module")
+def norm_plan():
+    return C.CDLL(iris_c_amd.LIB_PATH).iris_hip_group_norm_plan
+
+
+def test_group_norm_is_one_launch_only_where_all_its_workgroups_find_a_cu(norm_plan):
+    for hw, c in ((1 << 20, 128), (512 * 512, 256), (128 * 128, 512)):
+        assert norm_plan(hw, c, 32, 256) == norm_plan(hw, c, 32, 304) == 1
+        for cus in (0, 32, 64, 128, 255):
+            assert norm_plan(hw, c, 32, cus) == 0
+
+
+def test_group_norm_is_one_launch_for_the_shapes_it_takes(norm_plan):
+    for c, groups, takes in ((128, 32, 1), (64, 8, 1), (2048, 64, 1), (128, 4, 0), (96, 8, 0), (512, 128, 0), (64, 32, 0), (4096, 32, 0), (130, 32, 0)):
+        assert norm_plan((64 << 20) // (4 * c), c, groups, 256) == takes, (c, groups)
+    assert norm_plan((1 << 28) // 32, 128, 32, 256) == 0 and norm_plan((1 << 28) // 32 - 1, 128, 32, 256) == 1     # 4 GiB
+    assert norm_plan(100, 128, 32, 256) == 0
