@@ -509,7 +509,7 @@ k_gn_normalize(float *__restrict__ out, const float *__restrict__ in, const floa
     else out[i] = v[0];
 }
 
-/* ---- the whole norm as one launch, from 8 MB on ----
+/* ---- the whole norm as one launch, from 10 MB on ----
  *
  * One workgroup per CU: each reads its share of the image once, keeps as much of it as its registers and LDS hold (KEEP steps of
  * 8 KB: 138 MB in all), leaves the moments of its share, waits for the image's statistics, and writes the share normalised; only
@@ -520,7 +520,9 @@ k_gn_normalize(float *__restrict__ out, const float *__restrict__ in, const floa
  * Bound by the memory in both directions (134 MB read in 20 us), 5 - 6 us between the last value read and the first written, and
  * the launch. Against statistics, their sum and normalising as three launches, f32 image from memory, us:
  * 16384 x 512 26.7 -> 20.1, 65536 x 256 45 -> 30, 384 x 384 x 128 50 -> 33, 512 x 512 x 128 82 -> 51, 512 x 512 x 256 155 -> 108,
- * 700 x 700 x 128 146 -> 101, 1024 x 1024 x 128 294 -> 232; 4096 x 512 (8 MB) 13.4 / 13.1, 1024 x 512 10.0 / 11.6: the line.
+ * 700 x 700 x 128 146 -> 101, 1024 x 1024 x 128 294 -> 235. The line is where an image that the operator in front has left in the
+ * Infinity Cache is as fast either way (from memory / cached, three launches -> one): 512 channels, 8.5 MB 13.8 -> 13.5 / 12.7 -> 13.4,
+ * 9.5 MB 14.4 -> 13.7 / 13.2 -> 13.5, 10.5 MB 14.7 -> 13.9 / 13.5 -> 13.5, 16 MB 16.6 -> 15.3 / 15.8 -> 14.5.
  *
  * Everything between workgroups is a word with the number of the launch in its high half (Tagged), so that no store has to be
  * waited for and nothing is cleared between launches: a workgroup leaves the moments of its share, merged from its threads' as in
@@ -543,7 +545,7 @@ constexpr int RES_WGS = 256, RES_THREADS = 512, RES_REG = 48, RES_LDS = 18, RES_
 constexpr unsigned RES_STRIDE = RES_WGS * RES_THREADS;
 constexpr int RES_LDS_BYTES = RES_LDS * RES_THREADS * 16;
 constexpr int RES_MIN_GROUPS = 8, RES_MAX_GROUPS = IRIS_GN_MOST_GROUPS;        /* a group's threads are at most a wave; a wave gathers the statistics */
-constexpr size_t RES_MIN_BYTES = (size_t)8 << 20;
+constexpr size_t RES_MIN_BYTES = (size_t)10 << 20;
 constexpr unsigned RES_PATIENCE = 1000000, RES_LATE = 1u << 20, RES_SWEEPS = 1u << 12;         /* a second or so each */
 struct Tagged { unsigned long long a, b; };                    /* two floats, each with the number of the launch in its high half */
 struct ResidentSync {

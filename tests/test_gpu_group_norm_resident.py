@@ -186,7 +186,7 @@ def test_what_it_does_not_take(dev):
     dev.free_all()
 
 
-@pytest.mark.parametrize("hw", [16383, 16384])                 # 8 MB: the first size that takes it, and the last that does not
+@pytest.mark.parametrize("hw", [16383, 16384, 20479, 20480])   # 10 MB: the first size that takes it, and the last that does not
 def test_both_sides_of_the_line(dev, hw):
     x, gamma, beta = data(hw, 128)
     dx, dg, db, dout = dev.put(x), dev.put(gamma), dev.put(beta), dev.alloc(hw * 128 * 4)

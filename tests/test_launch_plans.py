@@ -249,3 +249,9 @@ def test_group_norm_is_one_launch_for_the_shapes_it_takes(norm_plan):
         assert norm_plan((64 << 20) // (4 * c), c, groups, 256) == takes, (c, groups)
     assert norm_plan((1 << 28) // 32, 128, 32, 256) == 0 and norm_plan((1 << 28) // 32 - 1, 128, 32, 256) == 1     # 4 GiB
     assert norm_plan(100, 128, 32, 256) == 0
+
+
+def test_group_norm_is_one_launch_from_ten_megabytes_on(norm_plan):
+    for c in (128, 256, 512):
+        n = (10 << 20) // (4 * c)
+        assert norm_plan(n, c, 32, 256) == 1 and norm_plan(n - 1, c, 32, 256) == 0
