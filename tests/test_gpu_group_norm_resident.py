@@ -199,7 +199,7 @@ def test_both_sides_of_the_line(dev, hw):
 
 def test_replayed_from_a_graph(dev):
     from test_gpu_graph import Graphs
-    hw, c, lib, g = 20000, 128, dev.lib, Graphs()
+    hw, c, lib, g = 21000, 128, dev.lib, Graphs()
     x, gamma, beta = data(hw, c)
     dx, dg, db, dout, deager = dev.put(x), dev.put(gamma), dev.put(beta), dev.alloc(hw * c * 4), dev.alloc(hw * c * 4)
     norm = lambda out: lib.iris_dev_group_norm_noalloc(out, dx, dg, db, hw, c, 32, 1e-6, 1)
