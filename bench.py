@@ -95,17 +95,17 @@ def traffic_on_file():
 def attention_kernel_name(lib, c):
     """The __global__ function an iris_dev_attention call of configuration c launches, from the launcher's own
     planner (host arithmetic, nothing launched)."""
-    plan = (C.c_int * 5)()
-    lib.iris_hip_fa_hd128_plan.argtypes = [C.c_int, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int)]
-    lib.iris_hip_fa_hd128_plan.restype = None
-    lib.iris_hip_fa_hd128_plan(c["seq"], c["seq"], c["heads"], int(c["causal"]), plan)
+    plan = (C.c_int * 6)()
+    lib.iris_hip_fa_hd128_route.argtypes = [C.c_int] * 5 + [C.POINTER(C.c_int)]
+    lib.iris_hip_fa_hd128_route.restype = None
+    lib.iris_hip_fa_hd128_route(c["seq"], c["seq"], c["heads"], int(c["causal"]), int(c["key_mask"] is not None), plan)
     flags = f"{'true' if c['causal'] else 'false'}, {'true' if c['key_mask'] is not None else 'false'}"
-    kind, waves, nb = plan[0], plan[1], plan[2]
+    kind, waves, nb, parts = plan[0], plan[1], plan[2], plan[5]
     if kind == 1:
         return f"k_fa_fwd_hd128_two_sizes<{flags}>", {"workgroups_of_256_queries_per_head": plan[3], "workgroups_of_192_queries_per_head": plan[4]}
     if kind == 2:
         return f"k_fa_short_hd128<4, {flags}>", {}
-    return f"k_fa_fwd_hd128<{waves}, {nb}, {flags}>", {"queries_per_workgroup": 16 * nb * waves}
+    return f"k_fa_fwd_hd128<{waves * parts}, {nb}, {flags}, {parts}>", {"queries_per_workgroup": 16 * nb * waves}
 
 NORM_ROPE_PROFILE = os.path.join("profiles", "k_norm_rope_hd128__c2__kernel_trace.txt")
 

@@ -1377,11 +1377,20 @@ static int launch_any_width(hipStream_t st, uint16_t *out, int ldo, const uint16
 
 /* The launcher's choice for a head_dim-128 call, without launching anything (no GPU needed): plan[0] = kind (0 one
  * size, 1 two sizes, 2 keys split over the waves), plan[1] = waves per workgroup with queries of their own, plan[2] = blocks of 16 queries per
- * wave, plan[3] = 256-query workgroups per head of the two-size grid, plan[4] = its 192-query workgroups per head. */
-extern "C" void iris_hip_fa_hd128_plan(int seq_q, int seq_k, int heads, int causal, int *plan) {
-    const FaPlan p = plan_hd128(seq_q, seq_k, heads, causal, false);
+ * wave, plan[3] = 256-query workgroups per head of the two-size grid, plan[4] = its 192-query workgroups per head, plan[5] =
+ * waves that take the tiles of the same queries in turn (kind 0: 1 or 2; 4 in kind 2). */
+extern "C" void iris_hip_fa_hd128_route(int seq_q, int seq_k, int heads, int causal, int masked, int *plan) {
+    const FaPlan p = plan_hd128(seq_q, seq_k, heads, causal, masked != 0);
     plan[0] = p.kind; plan[1] = p.waves; plan[2] = p.nb; plan[3] = p.full;
     plan[4] = p.kind == 1 ? (seq_q - 256 * p.full + 191) / 192 : 0;
+    plan[5] = p.split ? p.split : 1;
+}
+
+/* the first five of these for a call without a key mask */
+extern "C" void iris_hip_fa_hd128_plan(int seq_q, int seq_k, int heads, int causal, int *plan) {
+    int route[6];
+    iris_hip_fa_hd128_route(seq_q, seq_k, heads, causal, 0, route);
+    for (int i = 0; i < 5; i++) plan[i] = route[i];
 }
 
 extern "C" int iris_hip_fa_hd128(void *stream, uint16_t *out, int ldo, const uint16_t *q,

@@ -60,7 +60,8 @@ int iris_hip_fa_hd128_qnorm(void *stream, uint16_t *out, int ldo, const uint16_t
 /* What iris_hip_fa_hd128 would launch for these sizes, host arithmetic only (no GPU needed): plan[0] = 0 one size
  * of workgroup, 1 two sizes (256 queries, then 192), 2 keys split over the waves of a workgroup; plan[1] = waves per
  * workgroup with queries of their own; plan[2] = blocks of 16 queries per wave; plan[3], plan[4] = 256- and 192-query workgroups per head of
- * the two-size grid. */
+ * the two-size grid; plan[5] = waves that take the key tiles of the same queries in turn. The second: the first five without a key mask. */
+void iris_hip_fa_hd128_route(int seq_q, int seq_k, int heads, int causal, int masked, int *plan);
 void iris_hip_fa_hd128_plan(int seq_q, int seq_k, int heads, int causal, int *plan);
 
 /* head_dim 512 (the VAE's call; key mask and causal limit as options): one wave per SIMD owns 32 queries and all 512

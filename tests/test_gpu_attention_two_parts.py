@@ -1,6 +1,8 @@
 """Attention of head_dim 128 whose workgroups give the two tiles of a group to two halves of their waves (k_fa_fwd_hd128 with
 PARTS = 2: 197 - 640 rows of 24 heads), against the oracle at the bar of the other attention tests: odd and even numbers of tiles,
 waves and tiles without queries or keys, rows whose keys all lie in one half's tiles, no valid key at all."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -21,6 +23,9 @@ def call(dev, orc, heads, kv, seq_q, seq_k, causal, mask, amp=1.0):
     ldi, rows = q + 2 * kvd, max(seq_q, seq_k)
     buf = O.f32_to_bf16((rng.standard_normal((rows, ldi)) * amp).astype(np.float32))
     scale = 128 ** -0.5
+    route = (C.c_int * 6)()
+    dev.lib.iris_hip_fa_hd128_route(seq_q, seq_k, heads, int(causal), int(mask is not None), route)
+    assert route[0] == 0 and route[5] == 2
     out, kernel = dev.attention(buf, ldi, 0, q, q + kvd, seq_q, seq_k, heads, kv, 128, scale, causal, mask)
     assert kernel == "fa_hd128"
     want = orc.attention_bf16(buf, ldi, 0, q, q + kvd, seq_q, seq_k, heads, kv, 128, scale, causal, mask)

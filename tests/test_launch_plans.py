@@ -59,6 +59,29 @@ def test_exact_rounds_keep_one_size(plan):
         assert plan(seq, seq, heads)["kind"] == 0, (heads, seq)
 
 
+@pytest.fixture(scope="module")
+def parts():
+    lib = C.CDLL(iris_c_amd.LIB_PATH)
+    lib.iris_hip_fa_hd128_route.argtypes = [C.c_int] * 5 + [C.POINTER(C.c_int)]
+    lib.iris_hip_fa_hd128_route.restype = None
+
+    def call(seq_q, seq_k, heads, causal=0, masked=0):
+        """waves with queries of their own, and that share theirs, of the kernel with one size of workgroups"""
+        out = (C.c_int * 6)()
+        lib.iris_hip_fa_hd128_route(seq_q, seq_k, heads, causal, masked, out)
+        return (out[1], out[5]) if out[0] == 0 else None
+    return call
+
+
+def test_two_waves_share_their_queries_where_that_halves_a_chain_and_every_workgroup_has_a_cu(parts):
+    assert parts(192, 192, 24) == (2, 1) and parts(193, 193, 24) == (2, 2)               # three key tiles; four
+    assert parts(320, 320, 24) == (2, 2) and parts(321, 321, 24) == (4, 2)               # 240 workgroups of 32 queries; 264: 144 of 64
+    assert parts(640, 640, 24) == (4, 2) and parts(641, 641, 24) == (4, 1)               # 240 workgroups of 64 queries; 264
+    assert parts(320, 320, 24, 1) == (2, 2) and parts(512, 512, 32, 1) == (4, 2)
+    assert parts(512, 512, 32, 1, 1) == (4, 1)                                           # a prompt padded to a fixed length
+    assert parts(4352, 4352, 30) == (8, 1) and parts(64, 64, 24) == (1, 1)
+
+
 # ------------------------------------------------------------------ the linear layers' kernel choice
 @pytest.fixture(scope="module")
 def linear_plan():
