@@ -1194,13 +1194,13 @@ template <int W, int NB = 2, int PARTS = 1>
 int launch_w(hipStream_t st, uint16_t *out, int ldo, const uint16_t *q, const uint16_t *k,
              const uint16_t *v, int ldi, int seq_q, int seq_k, int heads, int kv_heads, float scale,
              int causal, const int *key_mask, const QNorm &qn) {
-    if (causal) {
-        if constexpr (PARTS == 2) {                          /* plan_hd128 */
-            if (key_mask) return (int)hipErrorInvalidValue;
-        } else if (key_mask) return launch<W, NB, true, true, PARTS>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, key_mask, qn);
-        return launch<W, NB, true, false, PARTS>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, key_mask, qn);
+    if constexpr (PARTS == 2) {                              /* plan_hd128 */
+        if (key_mask) return (int)hipErrorInvalidValue;
+    } else if (key_mask) {
+        return causal ? launch<W, NB, true, true>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, key_mask, qn)
+                      : launch<W, NB, false, true>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, key_mask, qn);
     }
-    if (key_mask) return launch<W, NB, false, true, PARTS>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, key_mask, qn);
+    if (causal) return launch<W, NB, true, false, PARTS>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, key_mask, qn);
     return launch<W, NB, false, false, PARTS>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, key_mask, qn);
 }
 
@@ -1320,12 +1320,14 @@ static FaPlan plan_hd128(int seq_q, int seq_k, int heads, int causal, bool maske
          * one, two or three tiles there is no chain to halve. us, one wave / two: 24 heads x 256 tokens 7.0 / 6.5, x 320 8.0 /
          * 7.6, x 384 10.8 / 9.0 (288 workgroups of 32 queries become 144 of 64), x 512 11.4 / 10.5, x 640 13.5 / 12.1; 32 heads x
          * 320 9.5 / 8.3, x 512 causal 11.6 / 10.4; and where it is not taken 32 heads x 160 6.0 / 6.2, 24 heads x 720 17.9 / 24.2.
-         * Eight waves of 32 queries (128 a workgroup) in place of eight of 16 beyond that: within 3 %. A causal call with a key
-         * mask is a prompt padded to a fixed length: its walk ends at the last valid key, mostly after two or three tiles (32
-         * heads x 512, 118 valid keys 7.3 / 8.0), so it keeps one wave. */
-        if (w > 1 && w < 8 && tiles >= 4 && !(causal && masked)) {
+         * Eight waves of 32 queries (128 a workgroup) in place of eight of 16 beyond that: within 3 %. With 64 queries a workgroup
+         * and causal, the last rows alone have four tiles while the last one is short, and three in two steps are no gain: 40 heads
+         * x 200 causal 6.8 / 7.3, x 224 7.6 / 7.3, x 240 8.9 / 7.5; 48 heads x 224 7.1 / 7.5. Calls with a key mask keep one wave: the walk
+         * ends at the last valid key, and how many tiles that leaves is not known here: 24 heads x 512, 509 valid 11.6 / 10.9, 296 9.3 /
+         * 9.6, 168 7.9 / 8.6, 40 6.3 / 7.4; x 200, 168 valid 6.7 / 7.2. */
+        if (w > 1 && w < 8 && tiles >= 4 && !masked) {
             if (w == 2 && q_tiles32 * heads <= CUS) return {0, 2, 1, 2, 0};
-            if ((long)((seq_q + 63) / 64) * heads <= CUS) return {0, 4, 1, 2, 0};
+            if ((long)((seq_q + 63) / 64) * heads <= CUS && !(causal && keys <= 4 * BN - BN / 2)) return {0, 4, 1, 2, 0};
         }
         return {0, w, 1, 0, 0};
     }

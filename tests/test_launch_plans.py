@@ -78,8 +78,18 @@ def test_two_waves_share_their_queries_where_that_halves_a_chain_and_every_workg
     assert parts(320, 320, 24) == (2, 2) and parts(321, 321, 24) == (4, 2)               # 240 workgroups of 32 queries; 264: 144 of 64
     assert parts(640, 640, 24) == (4, 2) and parts(641, 641, 24) == (4, 1)               # 240 workgroups of 64 queries; 264
     assert parts(320, 320, 24, 1) == (2, 2) and parts(512, 512, 32, 1) == (4, 2)
-    assert parts(512, 512, 32, 1, 1) == (4, 1)                                           # a prompt padded to a fixed length
     assert parts(4352, 4352, 30) == (8, 1) and parts(64, 64, 24) == (1, 1)
+
+
+def test_two_waves_share_their_queries_only_where_the_number_of_tiles_is_known_and_enough(parts):
+    for heads, seq in ((24, 200), (24, 320), (24, 512), (30, 350), (32, 512), (40, 320)):
+        assert parts(seq, seq, heads)[1] == 2
+        for causal in (0, 1):
+            assert parts(seq, seq, heads, causal, 1)[1] == 1                             # the walk ends at the last valid key
+    for heads in (40, 48, 64):                                                           # 64 queries a workgroup, three tiles and a short fourth
+        assert [parts(seq, seq, heads, 1)[1] for seq in (193, 208, 224, 225, 256)] == [1, 1, 1, 2, 2]
+        assert parts(193, 193, heads)[1] == 2
+    assert parts(193, 193, 24, 1) == (2, 2)
 
 
 # ------------------------------------------------------------------ the linear layers' kernel choice
