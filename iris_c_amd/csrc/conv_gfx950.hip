@@ -221,16 +221,13 @@ k_conv_few_out(float *__restrict__ out, const float *__restrict__ in, const uint
  * is multiplied the next one, or the next block's first, is on its way. Nothing is shared between waves but the weights:
  * no barrier.
  * What bounds it is the image and the result: 512 x 512 pixels, 256 -> 128 channels 76 + 65 us as a bf16 copy and an implicit
- * product, 80 here (402 MB; eight waves that take 32 pixels each, half an LDS read per product, 93). With more than two
+ * product, 85 here (402 MB; eight waves that take 32 pixels each, half an LDS read per product, 2 more; pixels of images of 192 MB
+ * and more read with the streaming hint 80, but other channels 10 - 20 % slower: 512 x 512, 256 -> 64 66 / 69, 202 MB, 384 -> 100 62 / 78,
+ * and 256 -> 256, where two workgroups read every pixel, 116 / 141). With more than two
  * tiles of channels the image is read once for each (512 -> 1536 over 16384 pixels: 84 us against 61), so those go through a
  * copy (gemm_conv_gfx950.hip), as do few pixels of many channels (one_by_one_us). */
 constexpr int C1_N = 128, C1_MAX_CIN = 512, C1_WAVES = 16, C1_OUT = 512;   /* output channels of a workgroup; f32 of LDS per wave for its stores */
 
-/* ONCE: the pixels are read with the streaming hint, for images of 192 MB and more, of which little can be in the 256 MB Infinity Cache:
- * 512 x 512, 256 -> 128 (268 MB) 84.7 -> 80.1 us, image cached as far as it goes 84.6 -> 80.0; 256 x 256 (67 MB), where it is not
- * taken, 28.2 -> 26.4 from memory but 21.5 -> 26.3 cached. */
-constexpr size_t C1_ONCE_BYTES = (size_t)192 << 20;
-template <bool ONCE>
 __global__ void __launch_bounds__(64 * C1_WAVES, 4)
 k_conv_1x1(float *__restrict__ out, const float *__restrict__ in, const uint16_t *__restrict__ W, const float *__restrict__ bias,
            int pixels, int cin, int cout, int tiles_n, int total, int per_xcd) {
@@ -272,10 +269,7 @@ k_conv_1x1(float *__restrict__ out, const float *__restrict__ in, const uint16_t
         const int p = min(16 * block + li, pixels - 1);
         const float *src = in + (size_t)p * cin + 128 * group + 4 * lg;
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const f32x4 *p4 = reinterpret_cast<const f32x4 *>(src + 16 * i);
-            raw[i] = ONCE ? __builtin_nontemporal_load(p4) : *p4;
-        }
+        for (int i = 0; i < 8; i++) raw[i] = *reinterpret_cast<const f32x4 *>(src + 16 * i);
     };
     int block = slot * C1_WAVES + wave;
     if (block < blocks) fetch(block, 0);
@@ -327,17 +321,16 @@ int one_by_one_slots(int pixels, int cout) {
     return slots < 1 ? 1 : slots < most ? slots : most;
 }
 
-template <bool ONCE>
 int launch_1x1(hipStream_t st, float *out, const float *in, const uint16_t *W, const float *bias, int pixels, int cin, int cout) {
     static bool configured = false;
     if (!configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_conv_1x1<ONCE>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_conv_1x1), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (e != hipSuccess) return (int)e;
         configured = true;
     }
     const int tiles_n = (cout + C1_N - 1) / C1_N, slots = one_by_one_slots(pixels, cout);
     const int total = slots * tiles_n, per_xcd = (total + 7) / 8;
-    hipLaunchKernelGGL(k_conv_1x1<ONCE>, dim3((unsigned)per_xcd * 8), dim3(64 * C1_WAVES), C1_WAVES * C1_OUT * 4 + cin * 256, st, out, in, W, bias, pixels,
+    hipLaunchKernelGGL(k_conv_1x1, dim3((unsigned)per_xcd * 8), dim3(64 * C1_WAVES), C1_WAVES * C1_OUT * 4 + cin * 256, st, out, in, W, bias, pixels,
                        cin, cout, tiles_n, total, per_xcd);
     return (int)hipGetLastError();
 }
@@ -1044,9 +1037,7 @@ int iris_hip_conv2d_direct(void *stream, float *out, const float *in, const uint
     case FEW_OUT:
         return cin == 32 ? launch_few_out<1>(st, out, in, w, bias, s) : cin == 64 ? launch_few_out<2>(st, out, in, w, bias, s)
                                                                                : launch_few_out<4>(st, out, in, w, bias, s);
-    case ONE_BY_ONE:
-        return (size_t)h * width * cin * sizeof(float) >= C1_ONCE_BYTES ? launch_1x1<true>(st, out, in, w, bias, h * width, cin, cout)
-                                                                        : launch_1x1<false>(st, out, in, w, bias, h * width, cin, cout);
+    case ONE_BY_ONE: return launch_1x1(st, out, in, w, bias, h * width, cin, cout);
     case THREE: return launch_3x3(st, out, in, w, bias, s);
     case THREE_HALF: return launch_3x3_half(st, out, in, w, bias, s);
     default: return -2;

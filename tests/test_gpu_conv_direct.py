@@ -197,7 +197,7 @@ def test_routes_that_copy_the_image_in_chunks_of_the_scratch(dev, route, h, w, c
 
 
 def test_one_by_one_of_large_images(dev):
-    """192 MB of pixels are read with the streaming hint, a pixel less without: the same bits, and those of the definition."""
+    """192 MB of pixels and a pixel less: the same bits, and those of the definition."""
     h, cin, cout = (192 << 20) // (384 * 4), 384, 100
     rng = np.random.default_rng(5)
     img = rng.standard_normal((h, cin), dtype=np.float32)
