@@ -467,7 +467,7 @@ struct Wide {
 template <typename OUT, int NA, bool QKN>
 __global__ void __launch_bounds__(512, 2)
 k_gemm_wide(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *__restrict__ W, int M, int N, int K,
-            int tiles_m, int total, int per_xcd, QkNorm qn, const float *__restrict__ bias, int streaming_out) {
+            int tiles_m, int total, int per_xcd, int turns, QkNorm qn, const float *__restrict__ bias, int streaming_out) {
     using T = Wide<NA>;
     constexpr int TM = T::TM, TN = T::TN, XS = T::XS, WS = T::WS, WP = T::WP, H0 = (NA + 1) / 2, H1 = NA / 2;
     static_assert(WP <= 4 && H1 >= 2, "");
@@ -481,10 +481,10 @@ k_gemm_wide(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t 
     const int m0 = (band * BAND + in_band % band_rows) * TM, n0 = in_band / band_rows * TN;
     const int last_tile = K / TK - 1;
     /* The workgroups that share rows of W or x run in step; they take the k tiles of a group of four in different orders, so
-     * that one of them brings a line from HBM and the others find it in the L2 (gemm_tiles_gfx950.hip has the reasons); by the
-     * tile row alone, so that all widths add in the same order. All in one order / turned, us: 512 x 2560 -> 19456 49.1 / 47.4,
+     * that one of them brings a line from HBM and the others find it in the L2 (gemm_tiles_gfx950.hip has the reasons, and where
+     * not); by the tile row alone, so that all widths add in the same order. All in one order / turned, us: 512 x 2560 -> 19456 49.1 / 47.4,
      * 512 x 3072 -> 27648 73.8 / 71.2, 1024 x 2560 -> 19456 96.3 / 92.5; 4608 rows within 1 %. */
-    const int turn = (m0 / TM) & 3, turned = (last_tile + 1) & ~3;
+    const int turn = (m0 / TM) & turns, turned = (last_tile + 1) & ~3;
     auto source = [&](int kt) { return (size_t)(kt < turned ? kt ^ turn : kt) * TK; };
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4, wm = wave & 3, wn = wave >> 2;
@@ -731,6 +731,10 @@ k_gemm_scalar(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_
     store4(y + i, v, 1);
 }
 
+/* workgroups of k_gemm_wide with tiles of 32 na columns */
+static long wide_wgs(int M, int N, int na) { return (long)((M + DT - 1) / DT) * ((N + 32 * na - 1) / (32 * na)); }
+
+/* the order of the k tiles goes by the grid of 256-column tiles, whatever the width */
 template <typename OUT, int NA, bool QKN = false>
 int launch_gemm_wide(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, const float *bias, const QkNorm &qn = QkNorm{}) {
     static bool configured = false;
@@ -748,7 +752,7 @@ int launch_gemm_wide(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *
      * them cached for the operator that reads them next). */
     const int streaming_out = (size_t)M * N * sizeof(OUT) >= ((size_t)192 << 20);
     hipLaunchKernelGGL((k_gemm_wide<OUT, NA, QKN>), dim3((unsigned)per_xcd * 8), dim3(512), Wide<NA>::LDS, st, y, x, W, M, N, K,
-                       tiles_m, total, per_xcd, qn, bias, streaming_out);
+                       tiles_m, total, per_xcd, iris_hip_gemm_turns(wide_wgs(M, N, 8), M, (size_t)N * K * 2), qn, bias, streaming_out);
     return (int)hipGetLastError();
 }
 
@@ -777,8 +781,7 @@ static int wide_width(int M, int N) {
     return best;
 }
 
-/* workgroups of k_gemm_wide with tiles of 32 na columns, and the estimated time of that grid */
-static long wide_wgs(int M, int N, int na) { return (long)((M + DT - 1) / DT) * ((N + 32 * na - 1) / (32 * na)); }
+/* the estimated time of a grid of k_gemm_wide with tiles of 32 na columns */
 static float wide_us(int M, int N, int K, int na) {
     const long wgs = wide_wgs(M, N, na), rounds = (wgs + 255) / 256;
     return 4.0f + (float)rounds * ((float)(K / TK) * (wgs <= 128 ? 0.145f : 0.175f) * (float)na + 4.0f);

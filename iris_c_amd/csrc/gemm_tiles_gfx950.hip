@@ -24,7 +24,7 @@
  * they take the k tiles of a group of four in different orders (tile kt of the order is k tile kt ^ turn, turn = the tile's
  * row ^ its column, mod 4): a line is brought from HBM by one of them and found in the L2 by the others. Weights from HBM,
  * us, all in one order / turned: 512 x 2560 -> 6144 29.5 / 23.0, 512 x 3072 -> 9216 38.0 / 34.8, 512 x 9728 -> 2560 39.5 / 35.6,
- * 320 x 3072 -> 27648 59.1 / 55.5; with weights in the Infinity Cache 1 - 3 % slower. Turns over eight tiles, or turned by pairs
+ * 320 x 3072 -> 27648 59.1 / 55.5; with weights in the Infinity Cache 1 - 3 % slower, so not everywhere (iris_hip_gemm_turns). Turns over eight tiles, or turned by pairs
  * and fours of tiles, gave the same or less; four waves that only fetch beside the eight that multiply changed nothing.
  * Then comes the LDS: a wave's 64 x 64 outputs read 8 KB of operands for 16 products. The tile of 160 x 224 runs on four waves of 80 x 112
  * (12 KB for 35 products; 512 registers to a wave) and fills 248 CUs with 320 x 3072 -> 27648 instead of 216: 58.0 us / 53.6. Tiles of
@@ -51,7 +51,6 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 namespace {
 
 constexpr int TK = 64;
-constexpr size_t L2_BYTES = (size_t)4 << 20;                             /* of one XCD */
 
 __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
     f32x2 p = {lo, hi};
@@ -79,7 +78,7 @@ struct Tile {
 template <typename OUT, int NB, int WM, int NA, int WN, int KG, int STAGES>
 __global__ void __launch_bounds__(64 * WM * WN * KG, WM * WN * KG / 4)
 k_gemm_tiles(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *__restrict__ W, int M, int N, int K,
-             const float *__restrict__ bias, int tiles_m, int tiles_n, int splits, int total, int per_xcd) {
+             const float *__restrict__ bias, int tiles_m, int tiles_n, int splits, int total, int per_xcd, int turns) {
     using T = Tile<NB, WM, NA, WN, KG, STAGES>;
     constexpr int TM = T::TM, TN = T::TN, STAGE = T::STAGE, PIECES = T::PIECES;
     static_assert(T::LDS <= 160 * 1024 && NA <= 8 && (KG == 1 || (KG == 2 && NB % 2 == 0)), "");
@@ -97,9 +96,8 @@ k_gemm_tiles(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;
-    /* the order of this workgroup's k tiles, see above: tile kt of the order is k tile kt ^ turn inside whole groups of four. Not where
-     * the weights fit an XCD's L2, as under the VAE's attention: its block at 128 x 128 582 us turned / 576, at 120 x 124 527 / 513 */
-    const int turn = (size_t)N * K * 2 > L2_BYTES ? (m0 / TM ^ n0 / TN) & 3 : 0, turned = nk & ~3;
+    /* the order of this workgroup's k tiles, see above: tile kt of the order is k tile kt ^ turn inside whole groups of four */
+    const int turn = (m0 / TM ^ n0 / TN) & turns, turned = nk & ~3;
     const int wm = wave % WM, wn = wave / WM % WN, kg = wave / (WM * WN);
 
     /* this wave's pieces of a stage: row 8 (PIECES wave + j) + lane / 8 of [W tile | x tile]; rows past the end of a matrix
@@ -322,7 +320,7 @@ int launch_tiles(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, i
     }
     const int tiles_m = (M + T::TM - 1) / T::TM, tiles_n = (N + T::TN - 1) / T::TN, total = tiles_m * tiles_n * splits, per_xcd = (total + 7) / 8;
     hipLaunchKernelGGL((k_gemm_tiles<OUT, NB, WM, NA, WN, KG, STAGES>), dim3((unsigned)per_xcd * 8), dim3(T::THREADS), T::LDS, st, y, x, W, M, N, K,
-                       bias, tiles_m, tiles_n, splits, total, per_xcd);
+                       bias, tiles_m, tiles_n, splits, total, per_xcd, iris_hip_gemm_turns(total, M, (size_t)N * K * 2));
     return (int)hipGetLastError();
 }
 
@@ -352,6 +350,19 @@ int launch_shape(hipStream_t st, int shape, OUT *y, const uint16_t *x, const uin
 }  // namespace
 
 extern "C" {
+
+/* 3: the workgroups of a product take the k tiles of a group of four in different orders (the mask of the turn), 0: all in one.
+ * The first brings new lines from HBM once; on lines that are already on the chip it is only a cost. So the weights have to be
+ * larger than an XCD's L2 (4 MB) even in a grid of one round, larger than 14 MB in a longer one, whose later rounds find smaller
+ * ones on the chip, and 80 MB where many rows use them again and again. Weights from HBM, us, one order / turned: 512 x 1536 -> 4096
+ * (12 MB, one round) 16.3 / 13.9, 1500 x 2560 -> 2560 29.0 / 24.5, 512 x 1024 -> 4096 (8 MB) 11.7 / 10.7; more rounds:
+ * 3000 x 512 -> 8192 (8 MB) 29.5 / 30.8, 9000 x 768 -> 6272 81.3 / 83.2, 14650 x 512 -> 6912 109.1 / 111.6, 3179 x 512 -> 15488 (15 MB)
+ * 61.7 / 57.2, 2692 x 1024 -> 18944 106.8 / 103.4; 2 MB, 14391 x 512 -> 1536 31.6 / 32.5, and the VAE's attention block on weights
+ * of 1.5 MB 576 / 582; many rows: 14650 x 1536 -> 6912 (20 MB) 249 / 251, 11538 x 4096 -> 8832 (69 MB) 624.5 / 627.7,
+ * 12600 x 12288 -> 4096 (96 MB) 1013 / 980. The other way: 2115 x 512 -> 8192 27.3 / 25.2. */
+int iris_hip_gemm_turns(long wgs, int rows, size_t weight_bytes) {
+    return weight_bytes > (size_t)(wgs <= 256 ? 4 : rows <= 10240 ? 14 : 80) << 20 ? 3 : 0;
+}
 
 /* The cheapest tile and number of K ranges for a product, and its estimated time in us; negative where these kernels do
  * not take it: they want rows of 16-byte chunks (N % 8), whole k tiles and enough of them to fill the ring, and 32-bit

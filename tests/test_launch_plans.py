@@ -131,6 +131,15 @@ def test_operands_of_four_gibibytes_and_more_take_the_wide_kernel(linear_plan):
     assert linear_plan(300000, 8192, 300000)[0] == 3
 
 
+def test_orders_of_the_k_tiles_go_by_what_of_the_weights_the_chip_already_holds(linear_plan):
+    lib = C.CDLL(iris_c_amd.LIB_PATH)
+    lib.iris_hip_gemm_turns.argtypes = [C.c_long, C.c_int, C.c_size_t]
+    turned = lambda wgs, rows, mb: lib.iris_hip_gemm_turns(wgs, rows, int(mb * (1 << 20)) + (mb % 1 > 0)) == 3
+    assert not turned(256, 500, 4) and turned(256, 500, 4.1) and turned(1, 50000, 4.1)                # one round: more than an L2
+    assert not turned(257, 500, 14) and turned(257, 500, 14.1) and turned(5000, 10240, 14.1)          # several
+    assert not turned(257, 10241, 80) and turned(257, 10241, 80.1)                                    # and many rows
+
+
 def test_projections_normalise_their_tiles_where_that_is_the_faster_form(linear_plan):
     lib = C.CDLL(iris_c_amd.LIB_PATH)
     plan = lambda rows, k, out, q, kv: lib.iris_hip_linear_qknorm_plan(rows, k, out, 128 * q, 128 * kv)
