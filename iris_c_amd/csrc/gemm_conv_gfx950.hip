@@ -734,9 +734,10 @@ k_gemm_scalar(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_
 /* workgroups of k_gemm_wide with tiles of 32 na columns */
 static long wide_wgs(int M, int N, int na) { return (long)((M + DT - 1) / DT) * ((N + 32 * na - 1) / (32 * na)); }
 
-/* the order of the k tiles goes by the grid of 256-column tiles, whatever the width */
+/* in_order: all workgroups take the k tiles in one order; otherwise that goes by the grid of 256-column tiles, whatever the width */
 template <typename OUT, int NA, bool QKN = false>
-int launch_gemm_wide(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, const float *bias, const QkNorm &qn = QkNorm{}) {
+int launch_gemm_wide(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, const float *bias, const QkNorm &qn = QkNorm{},
+                     bool in_order = false) {
     static bool configured = false;
     if (!configured) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_gemm_wide<OUT, NA, QKN>),
@@ -752,7 +753,7 @@ int launch_gemm_wide(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *
      * them cached for the operator that reads them next). */
     const int streaming_out = (size_t)M * N * sizeof(OUT) >= ((size_t)192 << 20);
     hipLaunchKernelGGL((k_gemm_wide<OUT, NA, QKN>), dim3((unsigned)per_xcd * 8), dim3(512), Wide<NA>::LDS, st, y, x, W, M, N, K,
-                       tiles_m, total, per_xcd, iris_hip_gemm_turns(wide_wgs(M, N, 8), M, (size_t)N * K * 2), qn, bias, streaming_out);
+                       tiles_m, total, per_xcd, in_order ? 0 : iris_hip_gemm_turns(wide_wgs(M, N, 8), (size_t)N * K * 2), qn, bias, streaming_out);
     return (int)hipGetLastError();
 }
 
@@ -910,8 +911,10 @@ int iris_hip_linear_bf16(void *stream, float *part, uint16_t *y, const uint16_t 
 }
 
 /* How the projection that normalises its own columns runs, host arithmetic only: 1 k_gemm_wide in tiles of 256 columns that
- * normalises them in its epilogue (a tile holds two whole heads), 0 the plain layer in whatever tiles suit it and the norm
- * kernel behind it, -1 neither (the norm kernel counts fewer than 2^24 vectors).
+ * normalises them in its epilogue (a tile holds two whole heads), 2 the same with all k tiles in one order, 0 the plain layer in
+ * whatever tiles suit it and the norm kernel behind it, -1 neither (the norm kernel counts fewer than 2^24 vectors).
+ * The bits are to be the plain layer's, so the epilogue is taken where that adds in the same order: k_gemm_wide of any width as
+ * it is, k_gemm_dma and the tiles that add in order with 2.
  * Normalising tiles costs their workgroups 4 us a round, the pass over the stored columns 1.8 us and what they take at 7 TB/s, so
  * the epilogue pays where the plain layer takes the same tiles anyway or close to them in a grid of several rounds. us,
  * epilogue / two kernels: 4608 x 64 -> 9216 with 24 + 24 heads 35.6 / 41.9, 192 43.2 / 48.6, 576 67.6 / 73.6, 1024 92.4 / 94.9, 3072
@@ -921,15 +924,17 @@ static int qknorm_plan(int M, int N, int K, int q_cols, int k_cols, bool aligned
     if (!aligned || K <= 0 || K % TK || ((size_t)DT * K * 2) >> 32 || M < DT || N < DT || N % 128 || q_cols < 0 || k_cols < 0 || q_cols % 128 ||
         k_cols % 128 || q_cols + k_cols > N || heads == 0)
         return -1;
-    if ((long long)M * heads >= (1 << 24) || heads >= 256) return 1;
     const GemmPlan plan = plan_gemm(M, N, K, 2, true, true, part_bytes);
-    if (plan.kernel == 3 && plan.na == 8) return 1;
+    const int epilogue = plan.kernel == 3 ? 1 : plan.kernel == 2 || (plan.kernel == 4 && iris_hip_gemm_tiles_in_order(plan.na, plan.splits, M, N, K)) ? 2 : 0;
+    if ((long long)M * heads >= (1 << 24) || heads >= 256) return epilogue ? epilogue : -1;
+    if (plan.kernel == 3 && plan.na == 8) return epilogue;
     const long wgs = wide_wgs(M, N, 8);
     const float norm_us = 1.8f + 4.0f * (float)M * (float)(q_cols + k_cols) / 7.0e6f;
-    return wgs > 512 && wide_us(M, N, K, 8) + 4.0f * (float)((wgs + 255) / 256) < plan.us + norm_us;
+    return wgs > 512 && wide_us(M, N, K, 8) + 4.0f * (float)((wgs + 255) / 256) < plan.us + norm_us ? epilogue : 0;
 }
 int iris_hip_linear_qknorm_plan(int rows, int in, int out, int q_cols, int k_cols) {
-    return qknorm_plan(rows, out, in, q_cols, k_cols, true, IRIS_LINEAR_PART_BYTES);
+    const int plan = qknorm_plan(rows, out, in, q_cols, k_cols, true, IRIS_LINEAR_PART_BYTES);
+    return plan < 1 ? plan : 1;
 }
 
 /* y = x W^T as bf16 with the per-head RMSNorm + rotary embedding (head_dim 128) of columns [0, q_cols) (weights
@@ -946,7 +951,7 @@ int iris_hip_linear_bf16_qknorm(void *stream, float *part, uint16_t *y, const ui
     if (fused < 0) return -2;
     if (fused) {
         const QkNorm qn = {wq, k_cols ? wk : wq, rope_cos, rope_sin, q_cols, q_cols + k_cols, eps, split_half};
-        return launch_gemm_wide<uint16_t, 8, true>((hipStream_t)stream, y, x, W, M, N, K, nullptr, qn);
+        return launch_gemm_wide<uint16_t, 8, true>((hipStream_t)stream, y, x, W, M, N, K, nullptr, qn, fused == 2);
     }
     const int qh = q_cols / 128, kh = k_cols / 128;
     const int e = gemm<uint16_t>((hipStream_t)stream, y, x, W, M, N, K, part, part_bytes);

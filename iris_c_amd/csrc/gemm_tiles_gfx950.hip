@@ -308,6 +308,13 @@ int launch_sum(hipStream_t st, OUT *y, const float *part, size_t n, int splits) 
     return (int)hipGetLastError();
 }
 
+/* The order of the k tiles, a mask as iris_hip_gemm_turns gives it. In a grid of more than 512 tiles of 256 x 256 a projection may be
+ * issued as k_gemm_wide that normalises its own tiles (iris_hip_linear_qknorm_plan), whose bits are to be those of the plain
+ * layer: all k tiles in one order there. It gives up 2627 x 3072 -> 18432 258 -> 249 us, 1600 x 2560 -> 19456 143 -> 135. */
+static int turns(int M, int N, int K, int wgs) {
+    return (long)((M + 255) / 256) * ((N + 255) / 256) > 512 ? 0 : iris_hip_gemm_turns(wgs, (size_t)N * K * 2);
+}
+
 template <typename OUT, int NB, int WM, int NA, int WN, int KG, int STAGES>
 int launch_tiles(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, const float *bias, int splits) {
     using T = Tile<NB, WM, NA, WN, KG, STAGES>;
@@ -320,7 +327,7 @@ int launch_tiles(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, i
     }
     const int tiles_m = (M + T::TM - 1) / T::TM, tiles_n = (N + T::TN - 1) / T::TN, total = tiles_m * tiles_n * splits, per_xcd = (total + 7) / 8;
     hipLaunchKernelGGL((k_gemm_tiles<OUT, NB, WM, NA, WN, KG, STAGES>), dim3((unsigned)per_xcd * 8), dim3(T::THREADS), T::LDS, st, y, x, W, M, N, K,
-                       bias, tiles_m, tiles_n, splits, total, per_xcd, iris_hip_gemm_turns(total, M, (size_t)N * K * 2));
+                       bias, tiles_m, tiles_n, splits, total, per_xcd, turns(M, N, K, total));
     return (int)hipGetLastError();
 }
 
@@ -354,14 +361,18 @@ extern "C" {
 /* 3: the workgroups of a product take the k tiles of a group of four in different orders (the mask of the turn), 0: all in one.
  * The first brings new lines from HBM once; on lines that are already on the chip it is only a cost. So the weights have to be
  * larger than an XCD's L2 (4 MB) even in a grid of one round, larger than 14 MB in a longer one, whose later rounds find smaller
- * ones on the chip, and 80 MB where many rows use them again and again. Weights from HBM, us, one order / turned: 512 x 1536 -> 4096
+ * ones on the chip. Weights from HBM, us, one order / turned: 512 x 1536 -> 4096
  * (12 MB, one round) 16.3 / 13.9, 1500 x 2560 -> 2560 29.0 / 24.5, 512 x 1024 -> 4096 (8 MB) 11.7 / 10.7; more rounds:
  * 3000 x 512 -> 8192 (8 MB) 29.5 / 30.8, 9000 x 768 -> 6272 81.3 / 83.2, 14650 x 512 -> 6912 109.1 / 111.6, 3179 x 512 -> 15488 (15 MB)
  * 61.7 / 57.2, 2692 x 1024 -> 18944 106.8 / 103.4; 2 MB, 14391 x 512 -> 1536 31.6 / 32.5, and the VAE's attention block on weights
- * of 1.5 MB 576 / 582; many rows: 14650 x 1536 -> 6912 (20 MB) 249 / 251, 11538 x 4096 -> 8832 (69 MB) 624.5 / 627.7,
- * 12600 x 12288 -> 4096 (96 MB) 1013 / 980. The other way: 2115 x 512 -> 8192 27.3 / 25.2. */
-int iris_hip_gemm_turns(long wgs, int rows, size_t weight_bytes) {
-    return weight_bytes > (size_t)(wgs <= 256 ? 4 : rows <= 10240 ? 14 : 80) << 20 ? 3 : 0;
+ * of 1.5 MB 576 / 582. The other way: 2115 x 512 -> 8192 27.3 / 25.2. */
+int iris_hip_gemm_turns(long wgs, size_t weight_bytes) { return weight_bytes > (size_t)(wgs <= 256 ? 4 : 14) << 20 ? 3 : 0; }
+
+/* 1: this tile adds the products of an output one k-step after the other, as k_gemm_wide does in one order (KG = 1, K whole) */
+int iris_hip_gemm_tiles_in_order(int shape, int splits, int M, int N, int K) {
+    constexpr bool two_groups[NSHAPES] = {true, false, false, true, false, false, false, true};
+    const long wgs = (long)((M + SHAPES[shape].tm - 1) / SHAPES[shape].tm) * ((N + SHAPES[shape].tn - 1) / SHAPES[shape].tn);
+    return splits == 1 && !two_groups[shape] && turns(M, N, K, (int)(wgs < 1 << 30 ? wgs : 1 << 30)) == 0;
 }
 
 /* The cheapest tile and number of K ranges for a product, and its estimated time in us; negative where these kernels do

@@ -149,7 +149,8 @@ int iris_hip_linear_bf16(void *stream, float *part, uint16_t *y, const uint16_t 
  * short sequences, 3 the 256-row tiles of k_gemm_wide, 2 those of k_gemm_dma, 1 the 128 x 128 kernel, 0 the scalar kernel;
  * plan[1] = the tile width of k_gemm_wide (256, 224, 192 or 160 columns), the number of K ranges of the first. */
 void iris_hip_linear_plan(int rows, int in, int out, int out_bytes, int *plan);
-int iris_hip_gemm_turns(long wgs, int rows, size_t weight_bytes);
+int iris_hip_gemm_turns(long wgs, size_t weight_bytes);
+int iris_hip_gemm_tiles_in_order(int shape, int splits, int M, int N, int K);
 float iris_hip_gemm_tiles_plan(int M, int N, int K, int out_size, size_t part_bytes, int *shape, int *splits);
 int iris_hip_gemm_tiles(void *stream, void *y, int out_size, const uint16_t *x, const uint16_t *W, int M, int N, int K,
                         const float *bias, int shape, int splits, float *part);

@@ -112,6 +112,23 @@ FUSED = [
 ]
 
 
+# where the plain layer takes other kernels: tiles of 160 x 256 (weights of 10, 15, 15 and 71 MB), 128 x 256, and k_gemm_dma with weights of
+# 14 MB and 7 and 5 k tiles. Random bits stand for the data: only the two forms are compared
+@pytest.mark.parametrize("rows,k,heads,out", [(7003, 704, 25, 7424), (6668, 512, 24, 15232), (8613, 640, 24, 12032), (5890, 2560, 32, 14592),
+                                              (1640, 2048, 48, 24832), (2389, 448, 32, 16512), (2048, 320, 64, 23040)])
+def test_tiles_that_normalise_themselves_have_the_bits_of_the_plain_layers_other_kernels(dev, rows, k, heads, out):
+    g = np.random.default_rng(rows + k)
+    bits = lambda n, m: (g.integers(0, 1 << 16, (n, m), dtype=np.uint16) & 0x87ff) | 0x3800             # +-2^-15 .. 2
+    ang = g.uniform(-3.0, 3.0, (rows, 64)).astype(np.float32)
+    c = dict(rows=rows, k=k, out=out, q_heads=heads, k_heads=heads, hd=128, x=bits(rows, k), w=bits(out, k), wq=np.ones(128, np.float32),
+             wk=np.ones(128, np.float32), cos=np.cos(ang), sin=np.sin(ang))
+    assert dev.lib.iris_hip_linear_qknorm_plan(rows, k, out, 128 * heads, 128 * heads) == 1
+    one, kernel = run(dev, c, True, 0, 1)
+    assert kernel == "linear_mfma_qknorm"
+    two, _ = run(dev, c, False, 0, 1)
+    assert np.array_equal(one, two)
+
+
 @pytest.mark.parametrize("rows,k,q_heads,k_heads,extra,split", FUSED)
 def test_tiles_that_normalise_themselves_match_oracle_chain_and_own_two_calls(dev, orc, rows, k, q_heads, k_heads, extra, split):
     c = make(rows + k + q_heads, rows, k, q_heads, k_heads, extra)

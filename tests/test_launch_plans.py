@@ -133,11 +133,29 @@ def test_operands_of_four_gibibytes_and_more_take_the_wide_kernel(linear_plan):
 
 def test_orders_of_the_k_tiles_go_by_what_of_the_weights_the_chip_already_holds(linear_plan):
     lib = C.CDLL(iris_c_amd.LIB_PATH)
-    lib.iris_hip_gemm_turns.argtypes = [C.c_long, C.c_int, C.c_size_t]
-    turned = lambda wgs, rows, mb: lib.iris_hip_gemm_turns(wgs, rows, int(mb * (1 << 20)) + (mb % 1 > 0)) == 3
-    assert not turned(256, 500, 4) and turned(256, 500, 4.1) and turned(1, 50000, 4.1)                # one round: more than an L2
-    assert not turned(257, 500, 14) and turned(257, 500, 14.1) and turned(5000, 10240, 14.1)          # several
-    assert not turned(257, 10241, 80) and turned(257, 10241, 80.1)                                    # and many rows
+    lib.iris_hip_gemm_turns.argtypes = [C.c_long, C.c_size_t]
+    turned = lambda wgs, mb: lib.iris_hip_gemm_turns(wgs, int(mb * (1 << 20))) == 3
+    assert not turned(256, 4) and turned(256, 4.1) and turned(1, 4.1)                                 # one round: more than an L2
+    assert not turned(257, 14) and turned(257, 14.1) and turned(5000, 14.1)                           # several
+
+
+def test_projections_that_normalise_their_tiles_add_as_the_plain_layer_does(linear_plan):
+    """Where the epilogue is taken, the plain layer is k_gemm_wide, k_gemm_dma, or tiles that take K whole, in one group and in order."""
+    lib = C.CDLL(iris_c_amd.LIB_PATH)
+    lib.iris_hip_gemm_tiles_plan.restype = C.c_float
+    lib.iris_hip_gemm_tiles_plan.argtypes = [C.c_int] * 4 + [C.c_size_t] + [C.POINTER(C.c_int)] * 2
+    seen = 0
+    for heads in (8, 24, 32, 48, 100):
+        for k in (64, 192, 320, 448, 512, 704, 1024, 2048, 2560, 4096):
+            for out in range(256 * heads, 40000, 1408):
+                for rows in list(range(300, 2000, 211)) + list(range(2000, 20000, 1117)):
+                    if lib.iris_hip_linear_qknorm_plan(rows, k, out, 128 * heads, 128 * heads) != 1 or linear_plan(rows, k, out)[0] in (2, 3):
+                        continue
+                    shape, splits = C.c_int(), C.c_int()
+                    lib.iris_hip_gemm_tiles_plan(rows, out, k, 2, 64 << 20, shape, splits)
+                    assert lib.iris_hip_gemm_tiles_in_order(shape, splits, rows, out, k) == 1, (rows, k, out, heads)
+                    seen += 1
+    assert seen > 10
 
 
 def test_projections_normalise_their_tiles_where_that_is_the_faster_form(linear_plan):
