@@ -332,11 +332,14 @@ int launch_tiles(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, i
 }
 
 /* The tiles, and what a workgroup's k tile of 64 costs in us. Measured on 80 - 2115 rows with weights from HBM: `step` in a
- * grid of one round, where the chip is not at its power limit, `step_full` in a longer one. A workgroup's first tiles and
- * its epilogue take 3.5 us more. */
-struct Shape { int tm, tn; float step, step_full; };
-constexpr Shape SHAPES[] = {{128, 128, 0.44f, 0.50f}, {128, 192, 0.58f, 0.62f}, {128, 256, 0.72f, 0.80f}, {64, 256, 0.60f, 0.61f},
-                            {160, 192, 0.67f, 0.72f}, {160, 256, 0.90f, 0.93f}, {160, 224, 0.84f, 0.87f}, {128, 96, 0.39f, 0.45f}};
+ * grid of one round, where the chip is not at its power limit, `step_two` in two. `step_more`, for longer ones, is what decides
+ * between these tiles and k_gemm_wide, which is the faster one there unless its tiles fit badly; with the figures of two rounds
+ * these tiles were taken for 12800 x 12288 -> 3072 (752 us on k_gemm_wide, 819 here), 9280 x 12288 -> 4096 (749 / 808),
+ * 7176 x 16384 -> 4096 (734 / 804), 3680 x 4096 -> 36864 (862 / 900). A workgroup's first tiles and its epilogue take 3.5 us more. */
+struct Shape { int tm, tn; float step, step_two, step_more; };
+constexpr Shape SHAPES[] = {{128, 128, 0.44f, 0.50f, 0.55f}, {128, 192, 0.58f, 0.62f, 0.65f}, {128, 256, 0.72f, 0.80f, 0.82f},
+                            {64, 256, 0.60f, 0.61f, 0.62f},  {160, 192, 0.67f, 0.72f, 0.74f}, {160, 256, 0.90f, 0.93f, 0.94f},
+                            {160, 224, 0.84f, 0.87f, 0.89f}, {128, 96, 0.39f, 0.45f, 0.50f}};
 constexpr int NSHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
 
 template <typename OUT>
@@ -387,7 +390,7 @@ float iris_hip_gemm_tiles_plan(int M, int N, int K, int out_size, size_t part_by
         const long tiles = (long)((M + SHAPES[i].tm - 1) / SHAPES[i].tm) * ((N + SHAPES[i].tn - 1) / SHAPES[i].tn);
         for (int s = 1; s == 1 || (s * MIN_TILES <= nk && (size_t)s * M * N * 4 <= part_bytes && tiles * s <= 512); s++) {
             const long wgs = tiles * s, rounds = (wgs + 255) / 256;
-            const float step = rounds > 1 ? SHAPES[i].step_full : SHAPES[i].step;
+            const float step = rounds > 2 ? SHAPES[i].step_more : rounds > 1 ? SHAPES[i].step_two : SHAPES[i].step;
             /* the sum: a launch, and its reads at 5 TB/s */
             const float sum = s > 1 ? 3.0f + ((float)s * 4.0f + (float)out_size) * (float)M * (float)N / 5e6f : 0.0f;
             const float cost = 4.0f + (float)rounds * ((float)((nk + s - 1) / s) * step + 3.5f) + sum;

@@ -131,6 +131,14 @@ def test_operands_of_four_gibibytes_and_more_take_the_wide_kernel(linear_plan):
     assert linear_plan(300000, 8192, 300000)[0] == 3
 
 
+def test_long_grids_of_large_products_take_the_wide_kernel(linear_plan):
+    for rows, k, out, size in ((12800, 12288, 3072, 4), (12304, 9216, 3072, 4), (9280, 12288, 4096, 4), (9000, 16384, 4096, 4), (7176, 16384, 4096, 4),
+                               (6100, 16384, 4096, 4), (6000, 12288, 4096, 4), (3640, 4096, 36864, 2), (4630, 3072, 18432, 2), (9500, 9728, 2560, 4)):
+        assert linear_plan(rows, k, out, size)[0] == 3, (rows, k, out)
+    for rows, k, out, size in ((5760, 9216, 3072, 4), (4160, 12288, 4096, 4), (12600, 4096, 4096, 4), (3640, 3072, 27648, 2)):
+        assert linear_plan(rows, k, out, size)[0] == 4, (rows, k, out)                  # two rounds; wide tiles that fit badly
+
+
 def test_orders_of_the_k_tiles_go_by_what_of_the_weights_the_chip_already_holds(linear_plan):
     lib = C.CDLL(iris_c_amd.LIB_PATH)
     lib.iris_hip_gemm_turns.argtypes = [C.c_long, C.c_size_t]
