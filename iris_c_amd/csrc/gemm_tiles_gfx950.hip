@@ -335,11 +335,12 @@ int launch_tiles(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, i
  * grid of one round, where the chip is not at its power limit, `step_two` in two. `step_more`, for longer ones, is what decides
  * between these tiles and k_gemm_wide, which is the faster one there unless its tiles fit badly; with the figures of two rounds
  * these tiles were taken for 12800 x 12288 -> 3072 (752 us on k_gemm_wide, 819 here), 9280 x 12288 -> 4096 (749 / 808),
- * 7176 x 16384 -> 4096 (734 / 804), 3680 x 4096 -> 36864 (862 / 900). A workgroup's first tiles and its epilogue take 3.5 us more. */
+ * 7176 x 16384 -> 4096 (734 / 804), 3680 x 4096 -> 36864 (862 / 900). A workgroup's first tiles and its epilogue take 3.5 us more.
+ * Three digits where sizes are decided by them: 528 - 640 x 4096 -> 2560 24.4 us in four ranges of 160 x 192, 26.2 in five of 128 x 256. */
 struct Shape { int tm, tn; float step, step_two, step_more; };
-constexpr Shape SHAPES[] = {{128, 128, 0.44f, 0.50f, 0.55f}, {128, 192, 0.58f, 0.62f, 0.65f}, {128, 256, 0.72f, 0.80f, 0.82f},
-                            {64, 256, 0.60f, 0.61f, 0.62f},  {160, 192, 0.67f, 0.72f, 0.74f}, {160, 256, 0.90f, 0.93f, 0.94f},
-                            {160, 224, 0.84f, 0.87f, 0.89f}, {128, 96, 0.39f, 0.45f, 0.50f}};
+constexpr Shape SHAPES[] = {{128, 128, 0.44f, 0.50f, 0.55f}, {128, 192, 0.58f, 0.62f, 0.65f}, {128, 256, 0.736f, 0.80f, 0.82f},
+                            {64, 256, 0.60f, 0.61f, 0.62f},  {160, 192, 0.665f, 0.72f, 0.74f}, {160, 256, 0.90f, 0.93f, 0.94f},
+                            {160, 224, 0.836f, 0.87f, 0.89f}, {128, 96, 0.39f, 0.45f, 0.50f}};
 constexpr int NSHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
 
 template <typename OUT>
@@ -390,10 +391,14 @@ float iris_hip_gemm_tiles_plan(int M, int N, int K, int out_size, size_t part_by
         const long tiles = (long)((M + SHAPES[i].tm - 1) / SHAPES[i].tm) * ((N + SHAPES[i].tn - 1) / SHAPES[i].tn);
         for (int s = 1; s == 1 || (s * MIN_TILES <= nk && (size_t)s * M * N * 4 <= part_bytes && tiles * s <= 512); s++) {
             const long wgs = tiles * s, rounds = (wgs + 255) / 256;
+            /* Rows of a multiple of 32 KB cut into ranges of a multiple of 4 KB: the lines that a single row of tiles fetches at a time
+             * lie as far apart, and come slower. 112 x 16384 -> 4096 in eight ranges of 128 x 128 41.7 us, 16448 -> 4096 36.6; in
+             * sixteen of 128 x 256 36.9. */
+            const float far_apart = M <= SHAPES[i].tm && K % 16384 == 0 && ((nk + s - 1) / s) % 32 == 0 ? 1.3f : 1.0f;
             const float step = rounds > 2 ? SHAPES[i].step_more : rounds > 1 ? SHAPES[i].step_two : SHAPES[i].step;
             /* the sum: a launch, and its reads at 5 TB/s */
             const float sum = s > 1 ? 3.0f + ((float)s * 4.0f + (float)out_size) * (float)M * (float)N / 5e6f : 0.0f;
-            const float cost = 4.0f + (float)rounds * ((float)((nk + s - 1) / s) * step + 3.5f) + sum;
+            const float cost = 4.0f + (float)rounds * ((float)((nk + s - 1) / s) * step * far_apart + 3.5f) + sum;
             if (best < 0.0f || cost < best) { best = cost; *shape = i; *splits = s; }
         }
     }

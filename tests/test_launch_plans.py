@@ -139,6 +139,14 @@ def test_long_grids_of_large_products_take_the_wide_kernel(linear_plan):
         assert linear_plan(rows, k, out, size)[0] == 4, (rows, k, out)                  # two rounds; wide tiles that fit badly
 
 
+def test_ranges_of_k_of_short_products(linear_plan):
+    for rows in (528, 584, 640):
+        assert linear_plan(rows, 4096, 2560, 4) == (4, 4)
+    for rows in (80, 104, 128):
+        assert linear_plan(rows, 16384, 4096, 4) == (4, 16)                             # ranges of 2 KB of a row, not of 4
+    assert linear_plan(112, 16448, 4096, 4) == (4, 8)
+
+
 def test_orders_of_the_k_tiles_go_by_what_of_the_weights_the_chip_already_holds(linear_plan):
     lib = C.CDLL(iris_c_amd.LIB_PATH)
     lib.iris_hip_gemm_turns.argtypes = [C.c_long, C.c_size_t]
