@@ -792,10 +792,11 @@ static float wide_us(int M, int N, int K, int na) {
  * `splits` ranges of K, 3 = k_gemm_wide with tiles of 32 na columns, 2 = k_gemm_dma, 1 = k_gemm_bf16, 0 = k_gemm_scalar.
  *
  * Between 4 and 3 the estimated times decide: a k tile costs a workgroup of k_gemm_wide 0.175 us per 32 columns (0.145 in a
- * grid that leaves most CUs idle), its ends 4 us a round. Measured, weights from HBM, us of 4 against 3 at its best width:
- * 512 x 9728 -> 2560 38 against 138, 512 x 3072 -> 9216 38 / 50, 1000 x 12288 -> 3072 76 / 175, 2115 x 9216 -> 3072 104 / 122,
- * 2115 x 3072 -> 9216 100 / 104; and where 3 is taken 512 x 3072 -> 18432 79 / 58, 1000 x 3072 -> 27648 156 / 136,
- * 2115 x 3072 -> 18432 209 / 194, 2912 x 12288 -> 4096 265 / 224. */
+ * grid that leaves most CUs idle), its ends 4 us a round. (Its order of k tiles made it 2 - 4 % faster on new weights; the
+ * figures are left, a little on the side of the tiles that 80 - 640 rows need.) Measured, weights from HBM, us of 4 against 3:
+ * 512 x 9728 -> 2560 37 against 134, 512 x 3072 -> 9216 36 / 48, 1000 x 12288 -> 3072 79 / 161, 2115 x 9216 -> 3072 106 / 135,
+ * 2115 x 3072 -> 9216 100 / 105; and where 3 is taken 512 x 3072 -> 18432 72 / 51, 1000 x 3072 -> 27648 154 / 133,
+ * 2115 x 3072 -> 18432 212 / 190, 2912 x 12288 -> 4096 254 / 223. */
 struct GemmPlan { int kernel, na, splits; float us; };       /* us: estimate, where there is one */
 static GemmPlan plan_gemm(int M, int N, int K, int out_size, bool operands_aligned16, bool out_aligned16, size_t part_bytes) {
     int shape = 0, splits = 1;

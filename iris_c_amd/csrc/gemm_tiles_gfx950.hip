@@ -24,7 +24,8 @@
  * they take the k tiles of a group of four in different orders (tile kt of the order is k tile kt ^ turn, turn = the tile's
  * row ^ its column, mod 4): a line is brought from HBM by one of them and found in the L2 by the others. Weights from HBM,
  * us, all in one order / turned: 512 x 2560 -> 6144 29.5 / 23.0, 512 x 3072 -> 9216 38.0 / 34.8, 512 x 9728 -> 2560 39.5 / 35.6,
- * 320 x 3072 -> 27648 59.1 / 55.5; with weights in the Infinity Cache 1 - 3 % slower, so not everywhere (iris_hip_gemm_turns). Turns over eight tiles, or turned by pairs
+ * 320 x 3072 -> 27648 59.1 / 55.5; with weights in the Infinity Cache 1 - 3 % slower, so not everywhere (iris_hip_gemm_turns).
+ * The f32 sums of a row are then taken in an order that goes by its tile's place. Turns over eight tiles, or turned by pairs
  * and fours of tiles, gave the same or less; four waves that only fetch beside the eight that multiply changed nothing.
  * Then comes the LDS: a wave's 64 x 64 outputs read 8 KB of operands for 16 products. The tile of 160 x 224 runs on four waves of 80 x 112
  * (12 KB for 35 products; 512 registers to a wave) and fills 248 CUs with 320 x 3072 -> 27648 instead of 216: 58.0 us / 53.6. Tiles of

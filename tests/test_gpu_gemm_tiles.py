@@ -79,7 +79,7 @@ def test_tile_of_224_columns(dev, more_rows, more_cols, k, splits, bf16):
     one_layer(dev, 6, 160 + more_rows, k, 224 + more_cols, splits, bf16)
 
 
-# the tile of 128 x 96 at the same edges, and the orders of its k tiles
+# the tile of 128 x 96 at the same edges, and whole and partial groups of four k tiles (weights of at most 1 MB: in one order)
 @pytest.mark.parametrize("rows,k,out,splits", [(128, 64, 96, 1), (129, 128, 104, 1), (127, 192, 88, 1), (128, 256, 168, 1), (161, 320, 96, 1), (65, 704, 104, 3),
                                                (128, 640, 96, 2), (129, 832, 104, 6), (637, 192, 472, 1), (637, 448, 472, 1), (637, 1216, 472, 4)])
 @pytest.mark.parametrize("bf16", [False, True])
@@ -87,8 +87,8 @@ def test_tile_of_96_columns(dev, rows, k, out, splits, bf16):
     one_layer(dev, 7, rows, k, out, splits, bf16)
 
 
-# five by five tiles, whose workgroups take the k tiles in four different orders: no whole group of four, one, several, and
-# some left over; ranges of K with all of these
+# five by five tiles: no whole group of four k tiles, one, several, and some left over; ranges of K with all of these. The weights are
+# at most 3 MB, so all workgroups take them in one order: the different orders are the next test's
 @pytest.mark.parametrize("shape", range(7))
 @pytest.mark.parametrize("k_tiles,splits", [(3, 1), (4, 1), (7, 1), (13, 1), (16, 1), (19, 4)])
 def test_orders_of_the_k_tiles(dev, shape, k_tiles, splits):
