@@ -101,8 +101,9 @@ def attention_kernel_name(lib, c):
     lib.iris_hip_fa_hd128_route(c["seq"], c["seq"], c["heads"], int(c["causal"]), int(c["key_mask"] is not None), plan)
     flags = f"{'true' if c['causal'] else 'false'}, {'true' if c['key_mask'] is not None else 'false'}"
     kind, waves, nb, parts = plan[0], plan[1], plan[2], plan[5]
-    if kind == 1:
-        return f"k_fa_fwd_hd128_two_sizes<{flags}>", {"workgroups_of_256_queries_per_head": plan[3], "workgroups_of_192_queries_per_head": plan[4]}
+    if kind in (1, 3):
+        tail = 192 if kind == 1 else 64
+        return f"k_fa_fwd_hd128_two_sizes<{flags}, {tail}>", {"workgroups_of_256_queries_per_head": plan[3], f"workgroups_of_{tail}_queries_per_head": plan[4]}
     if kind == 2:
         return f"k_fa_short_hd128<4, {flags}>", {}
     return f"k_fa_fwd_hd128<{waves * parts}, {nb}, {flags}, {parts}>", {"queries_per_workgroup": 16 * nb * waves}

@@ -90,6 +90,7 @@
  */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 #include "iris_kernels_hip.h"
 #include "norm_rope_math.h"
@@ -766,17 +767,19 @@ k_fa_fwd_hd128(uint16_t *__restrict__ out, int ldo, const uint16_t *__restrict__
 
 /* The last, partly filled round of the kernel above leaves CUs idle: 432 workgroups on 256 CUs run as 256 + 176.
  * Here a call is cut into workgroups of two sizes instead, so that its last round uses every CU for a shorter
- * time: per head `full_tiles` workgroups of 256 queries as above, and behind them `tail_tiles` workgroups of 192
- * queries, in which waves 0-3 carry 32 queries and waves 4-7 carry 16 (every SIMD then has three blocks of 16
- * queries instead of four). The 256-query workgroups of all heads are numbered first, so they are dispatched
- * first; each XCD takes its slice of both lists. */
-template <bool CAUSAL, bool MASK>
+ * time: per head `full_tiles` workgroups of 256 queries as above, and behind them `tail_tiles` workgroups of TAIL
+ * queries: 192, of which waves 0-3 carry 32 and waves 4-7 carry 16 (every SIMD then has three blocks of 16
+ * queries instead of four), or 64, of which a wave carries 16 and takes every other key tile (PARTS = 2): a third of the
+ * time of a 256-query one, for grids that are a few workgroups more than whole rounds. The 256-query workgroups of all
+ * heads are numbered first, so they are dispatched first; each XCD takes its slice of both lists. */
+template <bool CAUSAL, bool MASK, int TAIL>
 __global__ void __launch_bounds__(512, 2)
 k_fa_fwd_hd128_two_sizes(uint16_t *__restrict__ out, int ldo, const uint16_t *__restrict__ q,
                          const uint16_t *__restrict__ k, const uint16_t *__restrict__ v, int ldi,
                          int seq_q, int seq_k, int full_tiles, int total_full, int full_per_xcd,
                          int tail_tiles, int total_tail, int tail_per_xcd,
                          int kv_group, float scale_log2, const int *__restrict__ key_mask, QNorm qnorm) {
+    static_assert(TAIL == 192 || TAIL == 64, "");
     extern __shared__ __align__(16) uint16_t lds[];     /* four stages of [K tile | V tile] */
     const int xcd = blockIdx.x % XCDS, slot = blockIdx.x / XCDS;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -792,9 +795,9 @@ k_fa_fwd_hd128_two_sizes(uint16_t *__restrict__ out, int ldo, const uint16_t *__
         const int work = xcd * tail_per_xcd + slot - full_per_xcd;
         if (work >= total_tail) return;
         head = work / tail_tiles;
-        q0 = full_tiles * 256 + (work - head * tail_tiles) * 192; bm = 192;
-        two_blocks = wave < 4;
-        wq0 = two_blocks ? q0 + 32 * wave : q0 + 128 + 16 * (wave - 4);
+        q0 = full_tiles * 256 + (work - head * tail_tiles) * TAIL; bm = TAIL;
+        two_blocks = TAIL == 192 && wave < 4;
+        wq0 = TAIL == 64 ? q0 + 16 * (wave & 3) : two_blocks ? q0 + 32 * wave : q0 + 128 + 16 * (wave - 4);
     }
     /* Waves 0-3 and 4-7 of a 192-query workgroup run two instantiations of the walk and meet at its barriers.
      * INVARIANT: every barrier of fa_walk_hd128 is passed the same number of times by both, i.e. no barrier may sit
@@ -805,7 +808,7 @@ k_fa_fwd_hd128_two_sizes(uint16_t *__restrict__ out, int ldo, const uint16_t *__
         fa_walk_hd128<8, 2, 2, CAUSAL, MASK>(lds, out, ldo, q, k, v, ldi, seq_q, seq_k, head, head / kv_group, q0, bm, wq0,
                                              scale_log2, key_mask, qnorm);
     else
-        fa_walk_hd128<8, 1, 2, CAUSAL, MASK>(lds, out, ldo, q, k, v, ldi, seq_q, seq_k, head, head / kv_group, q0, bm, wq0,
+        fa_walk_hd128<8, 1, 2, CAUSAL, MASK, TAIL == 64 ? 2 : 1>(lds, out, ldo, q, k, v, ldi, seq_q, seq_k, head, head / kv_group, q0, bm, wq0,
                                              scale_log2, key_mask, qnorm);
 }
 
@@ -1167,24 +1170,24 @@ int launch(hipStream_t st, uint16_t *out, int ldo, const uint16_t *q, const uint
     return (int)hipGetLastError();
 }
 
-template <bool C, bool M>
+template <bool C, bool M, int TAIL>
 int launch_two_sizes(hipStream_t st, uint16_t *out, int ldo, const uint16_t *q, const uint16_t *k,
                      const uint16_t *v, int ldi, int seq_q, int seq_k, int heads, int kv_heads,
                      float scale, const int *key_mask, const QNorm &qn, int full_tiles) {
     static bool configured = false;
     if (!configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_fa_fwd_hd128_two_sizes<C, M>),
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_fa_fwd_hd128_two_sizes<C, M, TAIL>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_MAX);
         if (e != hipSuccess) return (int)e;
         configured = true;
     }
     const int rest = seq_q - 256 * full_tiles;
-    const int tail_tiles = rest > 0 ? (rest + 191) / 192 : 0;
+    const int tail_tiles = rest > 0 ? (rest + TAIL - 1) / TAIL : 0;
     const int total_full = full_tiles * heads, total_tail = tail_tiles * heads;
     const int full_per_xcd = (total_full + XCDS - 1) / XCDS, tail_per_xcd = (total_tail + XCDS - 1) / XCDS;
     const size_t lds_bytes = stage_bytes<8, 2>() + (M ? 8 * (size_t)((seq_k + BN - 1) / BN) : 0);
     if (lds_bytes > LDS_MAX) return (int)hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_fa_fwd_hd128_two_sizes<C, M>), dim3((full_per_xcd + tail_per_xcd) * XCDS), dim3(512), lds_bytes, st,
+    hipLaunchKernelGGL((k_fa_fwd_hd128_two_sizes<C, M, TAIL>), dim3((full_per_xcd + tail_per_xcd) * XCDS), dim3(512), lds_bytes, st,
                        out, ldo, q, k, v, ldi, seq_q, seq_k, full_tiles, total_full, full_per_xcd, tail_tiles, total_tail,
                        tail_per_xcd, heads / kv_heads, scale * 1.4426950408889634f, key_mask, qn);
     return (int)hipGetLastError();
@@ -1267,12 +1270,12 @@ static long makespan(long n_full, long n_tail, long tail_cost, long cus) {
 
 /* The two-size grid (k_fa_fwd_hd128_two_sizes) on its most loaded XCD, the first: workgroups k = 0 .. fx - 1 of the
  * XCD are the 256-query ones, k = fx .. fx + tx - 1 the 192-query ones, and k % 4 is the shader engine. */
-static long two_sizes_cost(long n_full, long n_tail) {
+static long two_sizes_cost(long n_full, long n_tail, long tail_cost) {
     const long fx = (n_full + XCDS - 1) / XCDS, tx = (n_tail + XCDS - 1) / XCDS;
     long worst = 0;
     for (long s = 0; s < 4; s++) {
         const long full = fx > s ? (fx - s + 3) / 4 : 0, both = fx + tx > s ? (fx + tx - s + 3) / 4 : 0;
-        const long c = makespan(full, both - full, 78, cu_count() / XCDS / 4);
+        const long c = makespan(full, both - full, tail_cost, cu_count() / XCDS / 4);
         if (c > worst) worst = c;
     }
     return worst;
@@ -1280,7 +1283,7 @@ static long two_sizes_cost(long n_full, long n_tail) {
 
 /* Which kernel a call takes: kind 0 = k_fa_fwd_hd128<waves, nb>, with `split` = 2 that kernel with twice the waves, of which
  * two take the tiles of the same queries in turn (PARTS = 2), 1 = k_fa_fwd_hd128_two_sizes with `full` workgroups
- * of 256 queries per head, 2 = k_fa_short_hd128<split>. Host arithmetic only. */
+ * of 256 queries per head and then 192-query ones, 3 = with 64-query ones, 2 = k_fa_short_hd128<split>. Host arithmetic only. */
 struct FaPlan { int kind, waves, nb, split, full; };
 
 static FaPlan plan_hd128(int seq_q, int seq_k, int heads, int causal, bool masked) {
@@ -1345,13 +1348,29 @@ static FaPlan plan_hd128(int seq_q, int seq_k, int heads, int causal, bool maske
          * heads, 2304 to 8704 tokens) the choice made here is within 2 % of the best of the 4-wave kernel, the 8-wave
          * kernel and every f on 70 of them and within 5 % on all. Beyond ten rounds the last one no longer matters. */
         long best_cost = (cost8 <= cost4 ? cost8 : cost4) * 97 / 100;
-        int best_full = -1;
+        int best_full = -1, best_tail = 0;
         for (int f = seq_q / 256; f >= 0; f--) {
-            const long tails = (seq_q - 256 * f + 191) / 192;
-            const long c = two_sizes_cost((long)f * heads, tails * heads);
-            if (c < best_cost) { best_cost = c; best_full = f; }
+            const long rest = seq_q - 256 * f;
+            const long c192 = two_sizes_cost((long)f * heads, (rest + 191) / 192 * heads, 78);
+            if (c192 < best_cost) { best_cost = c192; best_full = f; best_tail = 192; }
         }
-        if (best_full >= 0) return {1, 8, 2, 0, best_full};
+        /* 64-query workgroups behind them instead: their waves share LDS reads of K and V with fewer queries, so their time is
+         * more than their share, and the start of a workgroup weighs more in it the shorter the sequence is: about 0.33 + 2 /
+         * key tiles of a 256-query one (40 tiles 0.38 - 0.44, 68 0.31, 88 0.30). A lead of 5 % is wanted (with 2 - 3 % 24 heads x 9536 was
+         * 939 us without them and 944 with, 30 x 5440 407 / 405). us, without / with: 24 heads x 2704 127 / 110, x 3000 133 / 117, x 3264
+         * 141 / 126, x 8720 827 / 782, 30 x 2192 102 / 88, x 2624 117 / 103, x 4816 337 / 315, 32 x 2064 97 / 84, x 2560 114 / 103, 8 x 8208
+         * 340 / 292, 48 x 1296 67 / 57. With a key mask the walk may end early and the starts of the more workgroups be what counts, which
+         * in grids of more than two rounds is no gain: 700 / 100 valid keys 30 x 2400 48.4 -> 43.8 / 27.2 -> 25.4, but 40 x 3136
+         * 64.2 -> 63.9 / 36.7 -> 40.0. Workgroups of 128 queries were the best at none of 18 sizes. */
+        const long cost64 = 33 + 200 / ((seq_k + BN - 1) / BN);
+        if (!masked || cost8 <= 200) {
+            best_cost = (best_full >= 0 ? best_cost : best_cost * 100 / 97) * 95 / 100;
+            for (int f = seq_q / 256; f >= 0; f--) {
+                const long c64 = two_sizes_cost((long)f * heads, (long)((seq_q - 256 * f + 63) / 64) * heads, cost64);
+                if (c64 < best_cost) { best_cost = c64; best_full = f; best_tail = 64; }
+            }
+        }
+        if (best_full >= 0) return {best_tail == 64 ? 3 : 1, 8, 2, 0, best_full};
     }
     return {0, cost8 <= cost4 ? 8 : 4, 2, 0, 0};
 }
@@ -1361,9 +1380,15 @@ static int launch_any_width(hipStream_t st, uint16_t *out, int ldo, const uint16
                             int causal, const int *key_mask, const QNorm &qn) {
     const FaPlan p = plan_hd128(seq_q, seq_k, heads, causal, key_mask != nullptr);
     if (p.kind == 2) return launch_short_cm<4>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, causal, key_mask, qn);
-    if (p.kind == 1) {
-        if (key_mask) return launch_two_sizes<false, true>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, key_mask, qn, p.full);
-        return launch_two_sizes<false, false>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, key_mask, qn, p.full);
+    if (p.kind == 1 || p.kind == 3) {
+        auto go = [&](auto tail, auto masked) {
+            return launch_two_sizes<false, decltype(masked)::value, decltype(tail)::value>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale,
+                                                                                            key_mask, qn, p.full);
+        };
+        const std::integral_constant<int, 192> t192{};
+        const std::integral_constant<int, 64> t64{};
+        if (p.kind == 3) return key_mask ? go(t64, std::true_type{}) : go(t64, std::false_type{});
+        return key_mask ? go(t192, std::true_type{}) : go(t192, std::false_type{});
     }
     if (p.nb == 1) {
         if (p.waves == 1) return launch_w<1, 1>(st, out, ldo, q, k, v, ldi, seq_q, seq_k, heads, kv_heads, scale, causal, key_mask, qn);
@@ -1378,13 +1403,13 @@ static int launch_any_width(hipStream_t st, uint16_t *out, int ldo, const uint16
 }
 
 /* The launcher's choice for a head_dim-128 call, without launching anything (no GPU needed): plan[0] = kind (0 one
- * size, 1 two sizes, 2 keys split over the waves), plan[1] = waves per workgroup with queries of their own, plan[2] = blocks of 16 queries per
- * wave, plan[3] = 256-query workgroups per head of the two-size grid, plan[4] = its 192-query workgroups per head, plan[5] =
- * waves that take the tiles of the same queries in turn (kind 0: 1 or 2; 4 in kind 2). */
+ * size, 1 two sizes, 256 and 192 queries, 3 the same with 256 and 64, 2 keys split over the waves), plan[1] = waves per workgroup with
+ * queries of their own (of the 256-query ones in a two-size grid), plan[2] = blocks of 16 queries per wave, plan[3] = 256-query workgroups per
+ * head of the two-size grid, plan[4] = its smaller workgroups per head, plan[5] = waves that take the tiles of the same queries in turn (kind 0: 1 or 2; 4 in kind 2). */
 extern "C" void iris_hip_fa_hd128_route(int seq_q, int seq_k, int heads, int causal, int masked, int *plan) {
     const FaPlan p = plan_hd128(seq_q, seq_k, heads, causal, masked != 0);
     plan[0] = p.kind; plan[1] = p.waves; plan[2] = p.nb; plan[3] = p.full;
-    plan[4] = p.kind == 1 ? (seq_q - 256 * p.full + 191) / 192 : 0;
+    plan[4] = p.kind == 1 ? (seq_q - 256 * p.full + 191) / 192 : p.kind == 3 ? (seq_q - 256 * p.full + 63) / 64 : 0;
     plan[5] = p.split ? p.split : 1;
 }
 

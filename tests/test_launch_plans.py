@@ -54,6 +54,36 @@ def test_two_size_grids_cover_every_query_and_never_lose_to_one_size(plan, heads
         assert plan(seq, seq, heads, 1)["kind"] == 0                                      # causal calls keep one size
 
 
+def test_a_few_workgroups_over_a_round_become_small_ones(plan):
+    """256-query workgroups and 64-query ones behind them: every query in one of them, no empty workgroup"""
+    for heads, seq in ((24, 2704), (24, 3264), (30, 2400), (32, 2064), (32, 2560), (16, 4112), (8, 8208), (48, 1296), (64, 1100), (30, 4864)):
+        p = plan(seq, seq, heads)
+        assert p["kind"] == 3 and p["waves"] == 8 and 256 * p["full"] <= seq, (heads, seq, p)
+        assert 64 * (p["tails"] - 1) < seq - 256 * p["full"] <= 64 * p["tails"], (heads, seq, p)
+    for heads, seq in ((24, 2627), (24, 3584), (24, 4608), (30, 5440), (24, 9536), (32, 4352), (24, 12800)):
+        assert plan(seq, seq, heads)["kind"] in (0, 1), (heads, seq)
+
+
+def test_small_workgroups_behind_a_key_mask_only_in_two_rounds(masked_kind):
+    for heads, seq in ((24, 2816), (30, 2400), (32, 2304), (40, 1700)):
+        assert masked_kind(heads, seq, 0) == masked_kind(heads, seq, 1) == 3
+    for heads, seq in ((40, 3136), (30, 4816), (48, 2600)):
+        assert masked_kind(heads, seq, 0) == 3 and masked_kind(heads, seq, 1) != 3
+
+
+@pytest.fixture(scope="module")
+def masked_kind():
+    lib = C.CDLL(iris_c_amd.LIB_PATH)
+    lib.iris_hip_fa_hd128_route.argtypes = [C.c_int] * 5 + [C.POINTER(C.c_int)]
+    lib.iris_hip_fa_hd128_route.restype = None
+
+    def call(heads, seq, masked):
+        out = (C.c_int * 6)()
+        lib.iris_hip_fa_hd128_route(seq, seq, heads, 0, masked, out)
+        return out[0]
+    return call
+
+
 def test_exact_rounds_keep_one_size(plan):
     for heads, seq in ((16, 4096), (32, 2048), (8, 8192), (32, 4096), (30, 4352)):
         assert plan(seq, seq, heads)["kind"] == 0, (heads, seq)
