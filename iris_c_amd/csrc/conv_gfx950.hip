@@ -45,45 +45,80 @@ struct ConvShape {
  * output channels, B = 16 pixels. A wave keeps the weights of 128 output channels (eight A operands) in
  * registers and walks groups of 16 consecutive pixels: a lane gathers its eight patch values (cached: neighbouring
  * pixels share them), eight products, and the 16 x 128 results leave through the LDS as whole 512-byte rows.
- * What bounds it is the output stream. 3 -> 128 on 512 x 512 (134 MB out): 902 us as patches + scalar product + bias,
- * 40 us here (3.4 TB/s). */
-constexpr int FI_WAVES = 4, FI_COLS = 128;
+ * What bounds it is the output stream, as long as little else is done: a workgroup puts its weights and the places of the
+ * patch's values together once in the LDS (a thread of the form before read 64 weights one by one and divided eight times), and
+ * a group that lies inside the image adds eight offsets to one address and tests nothing. 3 -> 128 on 512 x 512 (134 MB out): 902 us
+ * as patches + scalar product + bias, 32 - 39 us with every value tested and divided for (image cached / from memory), 25 - 30 now (5.4 TB/s);
+ * 256 x 256 20 -> 10 - 12, 301 x 290 24 -> 14, 1024 x 1024 123 -> 108, 400 x 400, 3 -> 256 50 -> 37, 512 x 512, 3 -> 64 with stride 2 14 -> 9. */
+constexpr int FI_WAVES = 4, FI_COLS = 128, FI_BEYOND = 1 << 28;
+/* Whole 512-byte pieces of a row are written through as they are stored, as long as the result is neither too small to gain by it nor
+ * larger than the Infinity Cache: us, plain / through, 64 x 64, 3 -> 128 (2 MB) 6.2 / 7.4, 128 x 128 7.1 / 7.6, 180 x 180 (17 MB) 9.3 / 8.5,
+ * 512 x 512 35 / 30, 1024 x 1024 (537 MB) 108 / 115; rows that are not made of such pieces 512 x 512, 3 -> 64 24.9 / 26.4, 7 -> 260 34 / 40. */
+constexpr size_t FI_THROUGH_LEAST = (size_t)12 << 20, FI_THROUGH_MOST = (size_t)256 << 20;
 
-template <bool ALIGNED>
+/* p / ow for p < 2^30: umulhi(p, magic) >> shift, magic = ceil(2^(32 + shift) / ow) with 2^shift < ow <= 2^(shift + 1); 0: ow is 1 */
+struct RowOf { unsigned magic, shift; };
+inline RowOf row_of(unsigned ow) {
+    if (ow < 2) return {0, 0};
+    unsigned shift = 0;
+    while (2ull << shift < ow) shift++;
+    return {(unsigned)(((1ull << (32 + shift)) + ow - 1) / ow), shift};
+}
+
+template <bool ALIGNED, bool THROUGH>
 __global__ void __launch_bounds__(64 * FI_WAVES, 4)
 k_conv_few_in(float *__restrict__ out, const float *__restrict__ in, const uint16_t *__restrict__ W, const float *__restrict__ bias,
-              ConvShape s, int groups) {
+              ConvShape s, RowOf row_of, int small, int groups) {
     __shared__ __align__(16) float lds[FI_WAVES * 16 * FI_COLS];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, lg = lane >> 4;
-    const int n0 = blockIdx.y * FI_COLS, row_len = s.k * s.k * s.cin, pixels = s.oh * s.ow;
+    const int column = blockIdx.x, columns = gridDim.x, n0 = blockIdx.y * FI_COLS;
+    const int row_len = s.k * s.k * s.cin, pixels = s.oh * s.ow;
     float *buf = lds + wave * 16 * FI_COLS;
 
+    /* rows of 32 weights, zeros behind the patch; and for patch value r its tap's row and column (row FI_BEYOND: beyond the patch,
+     * never inside the image) and its offset from the patch's first value */
+    uint16_t *w_lds = reinterpret_cast<uint16_t *>(lds);
+    int *tap_y = reinterpret_cast<int *>(lds + FI_COLS * 16), *tap_x = tap_y + 32, *tap_off = tap_y + 64;
+#pragma unroll
+    for (int i = 0; i < FI_COLS * 32 / (64 * FI_WAVES); i++) {
+        const int e = threadIdx.x + 64 * FI_WAVES * i, n = n0 + (e >> 5), j = e & 31;
+        w_lds[e] = n < s.cout && j < row_len ? W[(size_t)n * row_len + j] : (uint16_t)0;
+    }
+    if (threadIdx.x < 32) {
+        const int r = threadIdx.x, tap = r / s.cin, c = r - tap * s.cin, y = tap / s.k, x = tap - y * s.k;
+        tap_y[r] = r < row_len ? y : FI_BEYOND;
+        tap_x[r] = x;
+        tap_off[r] = r < row_len ? (y * s.w + x) * s.cin + c : 0;
+    }
+    __syncthreads();
     u32x4 av[8];
 #pragma unroll
-    for (int a = 0; a < 8; a++) {
-        const int n = n0 + 16 * a + li;
-        uint16_t e[8];
+    for (int a = 0; a < 8; a++) av[a] = *reinterpret_cast<const u32x4 *>(&w_lds[(16 * a + li) * 32 + 8 * lg]);
+    int dy[8], dx[8], off[8];                                  /* of patch values 8 lg + j */
 #pragma unroll
-        for (int j = 0; j < 8; j++) e[j] = n < s.cout && 8 * lg + j < row_len ? W[(size_t)n * row_len + 8 * lg + j] : (uint16_t)0;
-        av[a] = u32x4{e[0] | (uint32_t)e[1] << 16, e[2] | (uint32_t)e[3] << 16, e[4] | (uint32_t)e[5] << 16, e[6] | (uint32_t)e[7] << 16};
-    }
+    for (int j = 0; j < 8; j++) { dy[j] = tap_y[8 * lg + j]; dx[j] = tap_x[8 * lg + j]; off[j] = tap_off[8 * lg + j]; }
+    const int c = lane & 31, n = n0 + 4 * c;
     f32x4 bv = {0, 0, 0, 0};                                   /* of the four channels this lane stores */
-    for (int r = 0; r < 4; r++)
-        if (bias && n0 + 4 * (lane & 31) + r < s.cout) bv[r] = bias[n0 + 4 * (lane & 31) + r];
-    /* patch value 8 lg + j of a pixel: (dy, dx) of its tap and its offset from the patch's first value */
-    int dy[8], dx[8], off[8];
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const int r = 8 * lg + j, tap = r / s.cin, c = r - tap * s.cin;
-        dy[j] = r < row_len ? tap / s.k : 1 << 28;              /* beyond the patch: never inside the image */
-        dx[j] = tap % s.k;
-        off[j] = (tap / s.k * s.w + dx[j]) * s.cin + c;
-    }
+    for (int r = 0; r < 4; r++)
+        if (bias && n + r < s.cout) bv[r] = bias[n + r];
+    __syncthreads();                                           /* the LDS is the waves' from here on */
 
     float v[8];
     auto fetch = [&](int g) {
         const int p = 16 * g + li;
-        const int oy = p / s.ow, y0 = oy * s.stride - s.pad, x0 = (p - oy * s.ow) * s.stride - s.pad;
+        const int oy = row_of.magic ? (int)(__umulhi((unsigned)p, row_of.magic) >> row_of.shift) : p;
+        const int y0 = oy * s.stride - s.pad, x0 = (p - oy * s.ow) * s.stride - s.pad;
+        const bool whole = p < pixels && y0 >= 0 && y0 + s.k <= s.h && x0 >= 0 && x0 + s.k <= s.w;
+        if (small && __all(whole)) {
+            const unsigned base = (unsigned)(y0 * s.w + x0) * (unsigned)s.cin;
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[j] = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(in) + 4u * (base + (unsigned)off[j]));
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                if (dy[j] == FI_BEYOND) v[j] = 0.0f;
+            return;
+        }
         const long base = ((long)y0 * s.w + x0) * s.cin;
 #pragma unroll
         for (int j = 0; j < 8; j++) {
@@ -93,9 +128,9 @@ k_conv_few_in(float *__restrict__ out, const float *__restrict__ in, const uint1
             v[j] = inside ? t : 0.0f;
         }
     };
-    int g = blockIdx.x * FI_WAVES + wave;
+    int g = column * FI_WAVES + wave;
     if (g < groups) fetch(g);
-    for (; g < groups; g += gridDim.x * FI_WAVES) {
+    for (; g < groups; g += columns * FI_WAVES) {
         const u32x4 b = {pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7])};
         /* lane: channels 16 a + 4 lg .. + 3 of pixel li. 16-byte chunk c of pixel r in slot (c & 16) | ((c ^ r) & 15): the
          * writes (16 pixels, one chunk) and the reads (32 chunks of a pixel) both spread over all banks. A wave's own
@@ -105,14 +140,17 @@ k_conv_few_in(float *__restrict__ out, const float *__restrict__ in, const uint1
             const int chunk = 4 * a + lg;
             *reinterpret_cast<f32x4 *>(&buf[li * FI_COLS + 4 * ((chunk & 16) | ((chunk ^ li) & 15))]) = mfma(av[a], b, f32x4{0, 0, 0, 0});
         }
-        if (g + gridDim.x * FI_WAVES < groups) fetch(g + gridDim.x * FI_WAVES);     /* on its way while this group is stored */
+        if (g + columns * FI_WAVES < groups) fetch(g + columns * FI_WAVES);         /* on its way while this group is stored */
+        float *first = out + (size_t)(16 * g) * s.cout + n0;    /* the same for the wave */
 #pragma unroll
         for (int it = 0; it < 8; it++) {
-            const int row = 2 * it + (lane >> 5), c = lane & 31, m = 16 * g + row, n = n0 + 4 * c;
+            const int row = 2 * it + (lane >> 5);
             const f32x4 r = *reinterpret_cast<const f32x4 *>(&buf[row * FI_COLS + 4 * ((c & 16) | ((c ^ row) & 15))]) + bv;
-            float *dst = out + (size_t)m * s.cout + n;
-            if (m >= pixels) continue;
-            if (ALIGNED) {
+            float *dst = first + (unsigned)(row * s.cout + 4 * c);
+            if (16 * g + row >= pixels) continue;
+            if (ALIGNED && THROUGH) {                          /* the wait states: the compiler does not know that this is a store */
+                if (n < s.cout) asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"(dst), "v"(r) : "memory");
+            } else if (ALIGNED) {
                 if (n < s.cout) *reinterpret_cast<f32x4 *>(dst) = r;
             } else {
 #pragma unroll
@@ -917,8 +955,13 @@ inline bool overlap(const void *a, size_t a_bytes, const void *b, size_t b_bytes
     return (uintptr_t)a < (uintptr_t)b + b_bytes && (uintptr_t)b < (uintptr_t)a + a_bytes;
 }
 
-/* five workgroups of k_conv_few_in a CU (32 KB of LDS each); a wave fetches its weights once for all its groups */
-inline unsigned few_in_columns(int groups) { return groups < 1280 * FI_WAVES ? (unsigned)(groups + FI_WAVES - 1) / FI_WAVES : 1280u; }
+/* Workgroups of k_conv_few_in per tile of channels. Four run on a CU at once, and one fetches its weights once for all its groups, so
+ * 1024 in all: with 1280 512 x 512 pixels, 3 -> 128 take 38 us in place of 30, with 1024 for each of four tiles (1 x 1, 4 -> 512 over
+ * 200 x 200) 26 in place of 21. Of two or three tiles twice as many, within a tenth of the time (400 x 400, 3 -> 256 38 us / 34). */
+inline unsigned few_in_columns(int groups, int cout) {
+    const int tiles_n = (cout + FI_COLS - 1) / FI_COLS, most = tiles_n == 1 ? 1024 : tiles_n < 4 ? 2048 / tiles_n : tiles_n < 1024 ? 1024 / tiles_n : 1;
+    return groups < most * FI_WAVES ? (unsigned)(groups + FI_WAVES - 1) / FI_WAVES : (unsigned)most;
+}
 
 enum Route { OTHER, FEW_IN, FEW_OUT, ONE_BY_ONE, THREE, THREE_HALF };
 
@@ -1013,7 +1056,7 @@ void iris_hip_conv2d_plan(const void *out, const void *in, const void *w, int h,
     plan[1] = 1;
     if (plan[0] == FEW_IN) {
         const int groups = (int)(((long)oh * ow + 15) / 16);
-        plan[1] = turns(groups, (long)few_in_columns(groups) * FI_WAVES);
+        plan[1] = turns(groups, (long)few_in_columns(groups, cout) * FI_WAVES);
     } else if (plan[0] == ONE_BY_ONE) {
         plan[1] = turns(((long)h * width + 15) / 16, (long)one_by_one_slots(h * width, cout) * C1_WAVES);
     } else if (plan[0] == THREE || plan[0] == THREE_HALF) {
@@ -1029,9 +1072,16 @@ int iris_hip_conv2d_direct(void *stream, float *out, const float *in, const uint
     switch (route(s, out, in, w)) {
     case FEW_IN: {
         const int groups = (int)(((long)oh * ow + 15) / 16);
-        const dim3 grid(few_in_columns(groups), (unsigned)((cout + FI_COLS - 1) / FI_COLS));
-        if (cout % 4 == 0 && al16(out)) hipLaunchKernelGGL(k_conv_few_in<true>, grid, dim3(64 * FI_WAVES), 0, st, out, in, w, bias, s, groups);
-        else hipLaunchKernelGGL(k_conv_few_in<false>, grid, dim3(64 * FI_WAVES), 0, st, out, in, w, bias, s, groups);
+        const int tiles_n = (cout + FI_COLS - 1) / FI_COLS;
+        const dim3 grid(few_in_columns(groups, cout), (unsigned)tiles_n);
+        const RowOf rows = row_of((unsigned)ow);
+        const int small = (size_t)h * width * cin * 4 < (size_t)1 << 31;          /* 32-bit byte offsets */
+        const size_t out_bytes = (size_t)oh * ow * cout * 4;
+        const bool through = cout % FI_COLS == 0 && out_bytes >= FI_THROUGH_LEAST && out_bytes <= FI_THROUGH_MOST;
+        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(64 * FI_WAVES), 0, st, out, in, w, bias, s, rows, small, groups); };
+        if (cout % 4 || !al16(out)) go(k_conv_few_in<false, false>);
+        else if (through) go(k_conv_few_in<true, true>);
+        else go(k_conv_few_in<true, false>);
         return (int)hipGetLastError();
     }
     case FEW_OUT:
