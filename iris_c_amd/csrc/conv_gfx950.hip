@@ -411,6 +411,8 @@ constexpr int C3_MAX_COUT = (160 * 1024 - 2 * C3_BIAS) / 4 / C3_N * C3_N;
 __device__ constexpr int c3_first(int t) { return t < 1 ? 0 : t < 4 ? 2 * (t - 1) : t + 2; }
 __device__ constexpr int c3_units(int t) { return c3_first(t + 1) - c3_first(t); }
 static_assert(c3_first(9) == C3_UNITS && c3_units(0) == 0, "");
+/* the tap of a step: down the columns of the 3 x 3 */
+__device__ constexpr int c3_tap(int t) { return t % 3 * 3 + t / 3; }
 
 __device__ __forceinline__ uint32_t lds_address(const uint16_t *p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
@@ -449,12 +451,12 @@ k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t
             }
         };
         const uint32_t stages = lds_address(lds + 2 * C3_IMG + C3_PIECES * bw * 8 * 64);
-        auto request = [&](int tap, int c0) {                  /* the stage of a tap: tap % 3 */
-            const uint16_t *src = W + (size_t)tap * s.cin + c0;
+        auto request = [&](int t, int c0) {                    /* the stage of step t: t % 3 */
+            const uint16_t *src = W + (size_t)c3_tap(t) * s.cin + c0;
 #pragma unroll
             for (int j = 0; j < C3_PIECES; j++)
                 asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                             ::"s"(stages + 2 * (tap % 3 * C3_STAGE + 8 * j * 64)), "v"(woff[j]), "s"(src) : "memory", "m0");
+                             ::"s"(stages + 2 * (t % 3 * C3_STAGE + 8 * j * 64)), "v"(woff[j]), "s"(src) : "memory", "m0");
         };
         /* pixels: unit u of this thread is channels 8 (bt % 8) .. + 7 of pixel bt / 8 + 32 u of the rimmed tile; a pixel
          * outside the image reads the first one and is zeroed */
@@ -570,20 +572,22 @@ k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t
 #pragma unroll
     for (int ks = 0; ks < 2; ks++) a_rd[ks] = 2 * C3_IMG + (64 * wn + li) * 64 + 8 * ((4 * ks + lg) ^ (li >> 1));
     const int b_rd = (4 * wm * C3_H + li) * C3_ROW + 8 * lg;
-    /* operand i of a half step, in the order its products use them; stage of a tap: tap % 3, nine steps per channel group */
-    auto operand = [&](int img, int tap, int ks, int i) {
+    /* operand i of a half of step t, in the order its products use them. Row r of pixels, counted from the wave's first in the rimmed
+     * tile, is kept in bv[ks][r % 4]: three steps go down a column of taps, and of the second and third only the last row is new. */
+    auto operand = [&](int img, int t, int ks, int i) {
         if (i == 0 || i > 4) {
             const int a = i == 0 ? 0 : i - 4;
-            av[ks][a] = *reinterpret_cast<const u32x4 *>(&lds[a_rd[ks] + (tap % 3) * C3_STAGE + 16 * a * 64]);
-        } else {
-            bv[ks][i - 1] = *reinterpret_cast<const u32x4 *>(&lds[img + b_rd + ((i - 1 + tap / 3) * C3_H + tap % 3) * C3_ROW + 32 * ks]);
+            av[ks][a] = *reinterpret_cast<const u32x4 *>(&lds[a_rd[ks] + (t % 3) * C3_STAGE + 16 * a * 64]);
+        } else if (t % 3 == 0 || i == 4) {
+            const int r = i - 1 + t % 3;
+            bv[ks][r % 4] = *reinterpret_cast<const u32x4 *>(&lds[img + b_rd + (r * C3_H + t / 3) * C3_ROW + 32 * ks]);
         }
     };
-    auto products = [&](int ks, int img, int tap) {            /* img, tap: of the operands read on the way */
+    auto products = [&](int ks, int t, int img, int next) {    /* of step t; img, next: of the operands read on the way */
 #pragma unroll
         for (int i = 0; i < 16; i++) {
-            asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc[i / 4][i % 4]) : "v"(av[ks][i / 4]), "v"(bv[ks][i % 4]));
-            if (i < 8) operand(img, tap, ks ^ 1, i);
+            asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc[i / 4][i % 4]) : "v"(av[ks][i / 4]), "v"(bv[ks][(i + t % 3) % 4]));
+            if (i < 8) operand(img, next, ks ^ 1, i);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -635,9 +639,9 @@ k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t
     for (int img = 0, g = 0; work < xcd_end; img = C3_IMG - img) {
 #pragma unroll
         for (int t = 0; t < 9; t++) {
-            products(0, img, t);
+            products(0, t, img, t);
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            products(1, t < 8 ? img : C3_IMG - img, t < 8 ? t + 1 : 0);
+            products(1, t, t < 8 ? img : C3_IMG - img, t < 8 ? t + 1 : 0);
         }
         if (++g == groups) {
             settle();
