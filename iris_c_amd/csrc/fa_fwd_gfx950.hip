@@ -1292,7 +1292,14 @@ static FaPlan plan_hd128(int seq_q, int seq_k, int heads, int causal, bool maske
      * Up to 2048 of them (one wave per SIMD and CU slot, or fewer): a workgroup walks its key tiles one after the
      * other, so a short sequence is bound by that chain, and the chain is shortest when a wave carries ONE block
      * of 16 queries (NB = 1: half the products per tile and wave, twice the waves): 1, 2, 4 or 8 such waves per
-     * workgroup so that the workgroups about fill the 256 CUs. Measured, clocks settled, rows in the L2, against
+     * workgroup so that the workgroups about fill the 256 CUs. Where the last rows make workgroups of eight more than one per CU and
+     * each walks all keys, the next regime's are faster (24 heads x 1281 - 1360 are 264 of them: us, these / those, x 1290 43.5 / 34.3,
+     * x 1355 52.4 / 35.4, 1255 valid keys 50.1 / 34.1; 30 x 1030 43.6 / 29.8, 343 valid 24.4 / 17.9). Not with causal, where a workgroup walks half of the keys on
+     * average and those behind the first round are the short ones: there these go on to half as many waves again (us, the next
+     * regime's / these, 32 heads x 1100 33.7 / 23.9, x 1280 39.8 / 31.5, 24 x 1400 40.0 / 30.0, x 2040 58.1 / 51.0, 16 x 3000 77.0 / 52.7; below 1024
+     * queries 40 x 900 30.2 / 32.8). Behind a key mask, which may end all walks early, only up to an eighth over a round: 32 x 1100 with 118,
+     * 550, 1100 valid keys 14.6 / 16.0, 25.4 / 22.1, 35.5 / 24.2; 24 x 1400, 350 valid 21.2 / 18.7; but x 1600, 400 valid 23.6 / 24.9.
+     * Measured, clocks settled, rows in the L2, against
      * 32 queries per wave: 32 heads on 8 x 512 tokens causal + mask 11.9 us against 15.5; 24 heads x 320 tokens
      * 7.7 against 10.5, x 576 11.8 against 15.2, x 768 17.4 against 20.2, x 1280 26.0 against 29.8 (x 1536: 56 against
      * 45, the other way round); same bits either way. About 0.65 us per key tile with up to two waves per
@@ -1311,7 +1318,9 @@ static FaPlan plan_hd128(int seq_q, int seq_k, int heads, int causal, bool maske
      * heads, 256 .. 12800 tokens, clocks settled. */
     const long CUS = cu_count();
     const long waves16 = (long)((seq_q + 15) / 16) * heads;
-    if (waves16 <= 8 * CUS) {
+    const long wg128 = (long)((seq_q + 127) / 128) * heads;
+    const bool longer_causal = causal && seq_q >= 1024 && (masked ? wg128 <= CUS + CUS / 8 : waves16 <= 12 * CUS);
+    if (longer_causal || (waves16 <= 8 * CUS && (causal || waves16 <= 4 * CUS || wg128 <= CUS))) {
         const int w = waves16 <= CUS ? 1 : waves16 <= 640 ? 2 : waves16 <= 4 * CUS ? 4 : 8;
         const long q_tiles32 = (seq_q + 31) / 32;
         const long keys = causal ? (seq_k < 32 * q_tiles32 ? seq_k : 32 * q_tiles32) : seq_k;
@@ -1334,7 +1343,7 @@ static FaPlan plan_hd128(int seq_q, int seq_k, int heads, int causal, bool maske
         }
         return {0, w, 1, 0, 0};
     }
-    const long wg256 = (long)((seq_q + 255) / 256) * heads, wg128 = (long)((seq_q + 127) / 128) * heads;
+    const long wg256 = (long)((seq_q + 255) / 256) * heads;
     const long cost8 = 100 * ((wg256 + CUS - 1) / CUS);
     const long rest4 = wg128 % (2 * CUS);
     const long cost4 = 110 * (wg128 / (2 * CUS)) + (rest4 == 0 ? 0 : rest4 <= CUS ? 60 : 110);
