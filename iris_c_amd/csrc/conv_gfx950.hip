@@ -414,23 +414,57 @@ static_assert(c3_first(9) == C3_UNITS && c3_units(0) == 0, "");
 /* the tap of a step: down the columns of the 3 x 3 */
 __device__ constexpr int c3_tap(int t) { return t % 3 * 3 + t / 3; }
 
+constexpr int C3_SLOTS = 32, C3_PART = 4096;                   /* CUs of an XCD; floats of a wave's sums */
+static_assert((size_t)16 * C3_SLOTS * C3_MUL * C3_PART * 4 <= IRIS_LINEAR_PART_BYTES, "two places a workgroup");
+
 __device__ __forceinline__ uint32_t lds_address(const uint16_t *p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
 }
+
+/* What a workgroup takes of its XCD's tiles [first, ..): whole ones up to rest_first, every slots-th; and, where the last round is cut,
+ * channel groups [u0, u1) of the `rest` tiles behind them, counted through those tiles, of which every taker has one at least. As
+ * rest < slots, these are at most a tile's number of groups and lie in at most two tiles. */
+struct C3Share { int first, rest_first, rest, takers, u0, u1; };
+__host__ __device__ inline C3Share c3_share(int xcd, int slot, int slots, int total, int per_xcd, int groups, bool cut) {
+    const int first = xcd * per_xcd < total ? xcd * per_xcd : total, end = first + per_xcd < total ? first + per_xcd : total;
+    if (!cut) return {first, end, 0, 0, 0, 0};
+    const int rest = (end - first) % slots, all = rest * groups, takers = all < slots ? all : slots;
+    return {first, end - rest, rest, takers, slot < takers ? all * slot / takers : all, slot < takers ? all * (slot + 1) / takers : all};
+}
+/* The workgroup that has channel group `unit` of the rest: the last with all * slot / takers < unit + 1 */
+__host__ __device__ inline int c3_taker(const C3Share &sh, int groups, int unit) { return ((unit + 1) * sh.takers - 1) / (sh.rest * groups); }
 
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"                /* M0 in a clobber list */
 __global__ void __launch_bounds__(C3_THREADS, 3)
 k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t *__restrict__ W, const float *__restrict__ bias,
-           ConvShape s, int tiles_x, int tiles_n, int total, int per_xcd) {
+           ConvShape s, int tiles_x, int tiles_n, int total, int per_xcd, float *__restrict__ part) {
     extern __shared__ __align__(16) uint16_t lds[];            /* image, image, weights, weights, weights, bias */
     /* an XCD takes a contiguous range of the tiles, the channel tiles of a pixel tile next to each other (they share the
-     * image in its L2), dealt out to its workgroups in turn */
-    const int xcd_end = min((int)(blockIdx.x % 8 + 1) * per_xcd, total), stride = gridDim.x / 8;
-    int work = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-    if (work >= xcd_end) return;
+     * image in its L2), dealt out to its workgroups in turn; with `part`, those of its last, incomplete round in ranges of channel groups */
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int groups = s.cin / 64;
+    const int groups = s.cin / 64, slot = blockIdx.x / 8, slots = gridDim.x / 8;
+    const C3Share sh = c3_share(blockIdx.x % 8, slot, slots, total, per_xcd, groups, part != nullptr);
+    /* the grid has C3_SLOTS workgroups an XCD, or one per tile of it */
+    const int wholes = slot >= sh.rest_first - sh.first ? 0 : slots == C3_SLOTS ? (sh.rest_first - sh.first - slot + C3_SLOTS - 1) / C3_SLOTS : 1;
+    const int units = wholes * groups + sh.u1 - sh.u0;         /* channel groups of tiles that this workgroup takes */
+    if (units == 0) return;
+    int p_w = sh.rest_first, p_g = 0;                          /* where its range begins */
+    if (part) {
+        p_w += sh.u0 / groups;
+        p_g = sh.u0 % groups;
+    }
+    const int w_first = wholes ? sh.first + slot : p_w, g_first = wholes ? 0 : p_g;
+    auto next = [&](int &w, int &g) {
+        if (++g < groups) return;
+        g = 0;
+        if (w >= sh.rest_first) {
+            w++;
+        } else if ((w += slots) >= sh.rest_first) {
+            w = p_w;
+            g = p_g;
+        }
+    };
     float *bias_lds = reinterpret_cast<float *>(lds + C3_BIAS);
     for (int i = tid; i < tiles_n * C3_N; i += C3_THREADS) bias_lds[i] = bias && i < s.cout ? bias[i] : 0.0f;
 
@@ -461,8 +495,8 @@ k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t
         /* pixels: unit u of this thread is channels 8 (bt % 8) .. + 7 of pixel bt / 8 + 32 u of the rimmed tile; a pixel
          * outside the image reads the first one and is zeroed */
         uint32_t off[C3_UNITS], inside = 0, held = 0;          /* bytes from the channel group's first value; bit u: in the image */
-        int w = work, g = 0;                                   /* where the next loads come from */
-        const float *src = in;
+        int w = w_first, g = g_first, left = units;            /* where the next loads come from */
+        const float *src = in + 64 * g;
         auto aim = [&]() {
             const int tile = w / tiles_n, ty = tile / tiles_x * C3_T - s.pad, tx = tile % tiles_x * C3_T - s.pad;
             int first = px0;
@@ -477,20 +511,16 @@ k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t
             }
         };
         auto advance = [&]() {
-            if (g + 1 < groups) {
-                g++;
-                src += 64;
-            } else {
+            if (--left > 0) {
+                const int tile = w;
+                next(w, g);
+                src = in + 64 * g;
+                if (w != tile) aim();
+            } else {                                           /* nothing comes next: the same loads, of a few cached bytes that nobody uses */
                 src = in;
-                g = 0;
-                w += stride;
-                if (w < xcd_end) {
-                    aim();
-                } else {                                       /* nothing comes next: the same loads, of a few cached bytes that nobody uses */
-                    inside = 0;
+                inside = 0;
 #pragma unroll
-                    for (int u = 0; u < C3_UNITS; u++) off[u] = 32u * (bt & 7);
-                }
+                for (int u = 0; u < C3_UNITS; u++) off[u] = 32u * (bt & 7);
             }
         };
         f32x4 xr[C3_UNITS][2];
@@ -506,9 +536,9 @@ k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t
             if (u + 1 < C3_UNITS || px0 < C3_PIXELS - 8 * C3_BRING * (C3_UNITS - 1))
                 *reinterpret_cast<u32x4 *>(&lds[img + (px0 + 8 * C3_BRING * u) * C3_ROW + 8 * (bt & 7)]) = v;
         };
-        aim_weights(work);
-        request(0, 0);
-        request(1, 0);
+        aim_weights(w);
+        request(0, 64 * g);
+        request(1, 64 * g);
         aim();
 #pragma unroll
         for (int u = 0; u < C3_UNITS; u++) load(u);
@@ -522,15 +552,18 @@ k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t
         }
         /* everything older than the loads just issued is there */
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * C3_UNITS) : "memory");
-        for (int img = 0, gg = 0; work < xcd_end; img = C3_IMG - img) {
-            const bool last = gg + 1 == groups;
+        int cw = w_first, cg = g_first;                        /* what is multiplied meanwhile */
+        for (int img = 0, unit = 0; unit < units; unit++, img = C3_IMG - img) {
+            const bool more = unit + 1 < units;
+            int nw = cw, ng = cg;
+            next(nw, ng);
             held = inside;
             advance();
 #pragma unroll
             for (int t = 0; t < 9; t++) {
-                if (t == 7 && last && work + stride < xcd_end) aim_weights(work + stride);
-                if (t < 7) request(t + 2, 64 * gg);
-                else request(t - 7, last ? 0 : 64 * (gg + 1));
+                if (t == 7 && more && nw != cw) aim_weights(nw);
+                if (t < 7) request(t + 2, 64 * cg);
+                else request(t - 7, more ? 64 * ng : 0);
 #pragma unroll
                 for (int u = c3_first(t); u < c3_first(t + 1); u++) {
                     put(C3_IMG - img, u);
@@ -543,8 +576,8 @@ k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t
                              ::"n"(2 * (c3_units(t > 0 ? t - 1 : 8) + c3_units(t)) + C3_PIECES) : "memory");
                 __builtin_amdgcn_sched_barrier(0);
             }
-            gg = last ? 0 : gg + 1;
-            if (last) work += stride;
+            cw = nw;
+            cg = ng;
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       /* no load into the LDS is left when it is given up */
         return;
@@ -596,8 +629,8 @@ k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t
      * it behind the next barrier; 4 KB per wave, a row of 16 pixels at a time), so that a store instruction covers four
      * pixels x 256 B. */
     const bool chunks = s.cout % 4 == 0 && ((uintptr_t)out & 15) == 0;
-    auto epilogue = [&](int img) {
-        const int tile = work / tiles_n, n0 = (work - tile * tiles_n) * C3_N, ty0 = tile / tiles_x * C3_T, tx0 = tile % tiles_x * C3_T;
+    auto epilogue = [&](int img, int w) {
+        const int tile = w / tiles_n, n0 = (w - tile * tiles_n) * C3_N, ty0 = tile / tiles_x * C3_T, tx0 = tile % tiles_x * C3_T;
         float *buf = reinterpret_cast<float *>(lds + img) + wave * 1024;
         int li = lane & 15, lg = lane >> 4;
         asm volatile("" : "+v"(li), "+v"(lg));                 /* the addresses are worked out here: kept over the loop they spill */
@@ -632,29 +665,103 @@ k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t
         }
     };
 
+    /* the sums of a range of channel groups, as the registers hold them: 128 KB, two places a workgroup */
+    auto store_part = [&](int w) {
+        float *dst = part + ((size_t)(2 * blockIdx.x + (w != p_w)) * C3_MUL + wave) * C3_PART;
+#pragma unroll
+        for (int a = 0; a < 4; a++)
+#pragma unroll
+            for (int b = 0; b < 4; b++) *reinterpret_cast<f32x4 *>(dst + ((4 * a + b) * 64 + lane) * 4) = acc[a][b];
+    };
+
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     clear();
 #pragma unroll
     for (int i = 0; i < 8; i++) operand(0, 0, 0, i);
-    for (int img = 0, g = 0; work < xcd_end; img = C3_IMG - img) {
+    int w = w_first, g = g_first;
+    bool from_start = g == 0;
+    for (int img = 0, unit = 0; unit < units; unit++, img = C3_IMG - img) {
 #pragma unroll
         for (int t = 0; t < 9; t++) {
             products(0, t, img, t);
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
             products(1, t, t < 8 ? img : C3_IMG - img, t < 8 ? t + 1 : 0);
         }
-        if (++g == groups) {
+        int nw = w, ng = g;
+        next(nw, ng);
+        if (nw != w || unit + 1 == units) {
             settle();
-            epilogue(img);
+            if (from_start && g + 1 == groups) epilogue(img, w);
+            else store_part(w);
             clear();
-            g = 0;
-            work += stride;
+            from_start = ng == 0;
         }
+        w = nw;
+        g = ng;
     }
 }
 #pragma clang diagnostic pop
 
-int launch_3x3(hipStream_t st, float *out, const float *in, const uint16_t *W, const float *bias, const ConvShape &s) {
+/* Adds the ranges of the tiles that were cut, in the order of their channels, and the bias. A workgroup takes what one wave of
+ * k_conv_3x3 left of a tile, on the XCD that made it. */
+__global__ void __launch_bounds__(256)
+k_conv_3x3_sum(float *__restrict__ out, const float *__restrict__ part, const float *__restrict__ bias, ConvShape s, int tiles_x, int tiles_n, int total,
+               int per_xcd) {
+    const int xcd = blockIdx.x % 8, wave = blockIdx.x / 8 % C3_MUL, t = blockIdx.x / 8 / C3_MUL, groups = s.cin / 64;
+    const C3Share sh = c3_share(xcd, 0, C3_SLOTS, total, per_xcd, groups, true);
+    if (t >= sh.rest) return;
+    const int first = c3_taker(sh, groups, t * groups), ranges = c3_taker(sh, groups, (t + 1) * groups - 1) - first + 1, w = sh.rest_first + t;
+    if (ranges == 1) return;                                   /* one workgroup took all of it, and has stored it */
+    const int place = c3_share(xcd, first, C3_SLOTS, total, per_xcd, groups, true).u0 < t * groups;
+    const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4, ab0 = threadIdx.x >> 6;
+    const auto at = [&](int r) {
+        return part + ((size_t)(2 * (8 * (first + r) + xcd) + (r == 0 ? place : 0)) * C3_MUL + wave) * C3_PART + threadIdx.x * 4;
+    };
+    f32x4 v[4];
+    const float *p = at(0);
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] = *reinterpret_cast<const f32x4 *>(p + i * 1024);
+#pragma unroll 2
+    for (int r = 1; r < ranges; r++) {
+        p = at(r);
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] += *reinterpret_cast<const f32x4 *>(p + i * 1024);
+    }
+    const int tile = w / tiles_n, n0 = (w - tile * tiles_n) * C3_N + 64 * (wave >> 2) + 4 * lg;
+    const int x = tile % tiles_x * C3_T + li, y0 = tile / tiles_x * C3_T + 4 * (wave & 3);
+    const bool chunks = s.cout % 4 == 0 && ((uintptr_t)out & 15) == 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int n = n0 + 16 * i, y = y0 + ab0;               /* block 4 i + ab0 of the wave's: channels 16 i, pixel row ab0 */
+        if (x >= s.ow || y >= s.oh || n >= s.cout) continue;
+        float *dst = out + ((size_t)y * s.ow + x) * s.cout + n;
+        if (chunks) {
+            if (bias) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[i][e] += bias[n + e];
+            }
+            *reinterpret_cast<f32x4 *>(dst) = v[i];
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (n + e < s.cout) dst[e] = v[i][e] + (bias ? bias[n + e] : 0.0f);
+        }
+    }
+}
+
+/* Whether the last round is worth cutting. It saves channel groups of 5.3 us, and costs a launch and the partial sums' way through memory,
+ * 128 KB a piece and about 0.25 us for one on each XCD. us, whole / cut: 512 -> 256 64 x 69 43.7 / 29.6, 84 x 89 44.8 / 36.6, 100 x 107 46.7 / 44.1,
+ * 124 x 133 47.9 / 52.0, 174 x 187 (one tile over a round on most XCDs) 91.3 / 71.3, 194 x 207 99.3 / 93.2, 217 x 233 101.9 / 112.9; 512 -> 512
+ * 122 x 131 92.5 / 75.1, 174 x 187 143.3 / 122.5; 256 -> 256 64 x 69 26.3 / 20.1, 82 x 87 27.2 / 30.0, 242 x 259 81.1 / 74.6; 256 -> 128 249 x 267
+ * 57.6 / 46.5; 128 -> 128 169 x 181 19.0 / 32.3, 249 x 267 37.0 / 34.3, which the rule leaves whole. */
+bool three_ranges(const ConvShape &s, int per_xcd) {
+    const int groups = s.cin / 64, rest = per_xcd % C3_SLOTS, units = (rest * groups + C3_SLOTS - 1) / C3_SLOTS;
+    if (rest == 0) return false;
+    const int pieces = rest * groups < C3_SLOTS ? rest * groups : C3_SLOTS + rest;
+    return 5.3f * (float)(groups - units) > 6.0f + 0.25f * (float)pieces;
+}
+
+int launch_3x3(hipStream_t st, float *part, float *out, const float *in, const uint16_t *W, const float *bias, const ConvShape &s) {
     static bool configured = false;
     if (!configured) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_conv_3x3), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -665,7 +772,17 @@ int launch_3x3(hipStream_t st, float *out, const float *in, const uint16_t *W, c
     const int total = tiles_x * ((s.oh + C3_T - 1) / C3_T) * tiles_n, per_xcd = (total + 7) / 8;
     const unsigned lds = 2 * C3_BIAS + 4 * C3_N * (unsigned)tiles_n;
     /* one workgroup per CU (its LDS): 32 per XCD, each walking the XCD's tiles */
-    hipLaunchKernelGGL(k_conv_3x3, dim3((unsigned)(per_xcd < 32 ? per_xcd : 32) * 8), dim3(C3_THREADS), lds, st, out, in, W, bias, s, tiles_x, tiles_n, total, per_xcd);
+    if (!three_ranges(s, per_xcd)) part = nullptr;
+    hipLaunchKernelGGL(k_conv_3x3, dim3((unsigned)(part || per_xcd >= C3_SLOTS ? C3_SLOTS : per_xcd) * 8), dim3(C3_THREADS), lds, st, out, in, W, bias, s,
+                       tiles_x, tiles_n, total, per_xcd, part);
+    int rest = 0;                                              /* of the XCD that has most of it: the last one may have fewer tiles */
+    for (int x = 0; part && x < 8; x++) {
+        const int r = c3_share(x, 0, C3_SLOTS, total, per_xcd, s.cin / 64, true).rest;
+        rest = r > rest ? r : rest;
+    }
+    if (part)
+        hipLaunchKernelGGL(k_conv_3x3_sum, dim3((unsigned)rest * 8 * C3_MUL), dim3(256), 0, st, out, part, bias, s, tiles_x, tiles_n,
+                           total, per_xcd);
     return (int)hipGetLastError();
 }
 
@@ -1048,6 +1165,20 @@ Route route(const ConvShape &s, const void *out, const void *in, const void *w) 
 
 extern "C" {
 
+/* How k_conv_3x3 cuts the last round of `total` tiles of `groups` channel groups, for tests: share = first, rest_first, rest, u0 and u1 of a
+ * workgroup; returns the workgroup of the XCD that has channel group `unit` of the rest (-1: it has none). */
+int iris_hip_conv2d_share(int xcd, int slot, int total, int groups, int unit, int *share) {
+    const C3Share sh = c3_share(xcd, slot, C3_SLOTS, total, (total + 7) / 8, groups, true);
+    share[0] = sh.first; share[1] = sh.rest_first; share[2] = sh.rest; share[3] = sh.u0; share[4] = sh.u1;
+    return unit < sh.rest * groups ? c3_taker(sh, groups, unit) : -1;
+}
+
+/* whether k_conv_3x3 does so for an output of this size where it has a workspace */
+int iris_hip_conv2d_cut(int oh, int ow, int cin, int cout) {
+    const ConvShape s = {oh, ow, cin, cout, 3, 1, 1, oh, ow};
+    return three_ranges(s, (int)((three_tiles(s, C3_T, C3_T) + 7) / 8));
+}
+
 /* plan[0] = the kernel such a convolution takes: 1 k_conv_few_in, 2 k_conv_few_out, 3 k_conv_1x1, 4 k_conv_3x3, 5 k_conv_3x3_half,
  * 0 none of them; plan[1] = how many pieces of work its busiest wave (1, 3) or workgroup takes one after the other.
  * No GPU needed: the addresses are only compared. */
@@ -1068,8 +1199,9 @@ void iris_hip_conv2d_plan(const void *out, const void *in, const void *w, int h,
     }
 }
 
-/* The shapes these kernels take; -2, with nothing enqueued, for any other. */
-int iris_hip_conv2d_direct(void *stream, float *out, const float *in, const uint16_t *w, const float *bias, int h, int width,
+/* The shapes these kernels take; -2, with nothing enqueued, for any other. part: IRIS_LINEAR_PART_BYTES of private workspace, 16-byte
+ * aligned, or null: no tile's input channels are then cut into ranges. */
+int iris_hip_conv2d_direct(void *stream, float *part, float *out, const float *in, const uint16_t *w, const float *bias, int h, int width,
                            int cin, int cout, int k, int stride, int pad_before, int oh, int ow) {
     hipStream_t st = (hipStream_t)stream;
     const ConvShape s = {h, width, cin, cout, k, stride, pad_before, oh, ow};
@@ -1092,7 +1224,7 @@ int iris_hip_conv2d_direct(void *stream, float *out, const float *in, const uint
         return cin == 32 ? launch_few_out<1>(st, out, in, w, bias, s) : cin == 64 ? launch_few_out<2>(st, out, in, w, bias, s)
                                                                                : launch_few_out<4>(st, out, in, w, bias, s);
     case ONE_BY_ONE: return launch_1x1(st, out, in, w, bias, h * width, cin, cout);
-    case THREE: return launch_3x3(st, out, in, w, bias, s);
+    case THREE: return launch_3x3(st, part, out, in, w, bias, s);
     case THREE_HALF: return launch_3x3_half(st, out, in, w, bias, s);
     default: return -2;
     }

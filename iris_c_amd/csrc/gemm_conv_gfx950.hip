@@ -997,7 +997,7 @@ int iris_hip_conv2d(void *stream, uint16_t *scratch, size_t scratch_bytes, float
     const int ow = (width + pad_before + pad_after - k) / stride + 1;
     if (oh <= 0 || ow <= 0) return 0;
     const int ohw = oh * ow, row_len = k * k * cin;
-    const int direct = iris_hip_conv2d_direct(stream, out, in, w, bias, h, width, cin, cout, k, stride, pad_before, oh, ow);
+    const int direct = iris_hip_conv2d_direct(stream, nullptr, out, in, w, bias, h, width, cin, cout, k, stride, pad_before, oh, ow);
     if (direct != -2) return direct;
 
     if (scratch_bytes <= IRIS_CONV_ZERO_BYTES) return (int)hipErrorInvalidValue;

@@ -171,8 +171,9 @@ int iris_hip_conv2d(void *stream, uint16_t *scratch, size_t scratch_bytes, float
                     int stride, int pad_before, int pad_after);
 
 /* Convolution of the shapes that need neither scratch nor a patch matrix (conv_gfx950.hip); -2 = not one of them, nothing
- * enqueued. oh, ow: output size. */
-int iris_hip_conv2d_direct(void *stream, float *out, const float *in, const uint16_t *w, const float *bias, int h, int width,
+ * enqueued. oh, ow: output size. part: IRIS_LINEAR_PART_BYTES of private workspace, 16-byte aligned, that the stream orders with its
+ * other users, or null (no tile's input channels are then cut into ranges). */
+int iris_hip_conv2d_direct(void *stream, float *part, float *out, const float *in, const uint16_t *w, const float *bias, int h, int width,
                            int cin, int cout, int k, int stride, int pad_before, int oh, int ow);
 /* an estimate of its other routes (those that copy the image first); plain: 1 x 1, no stride and no padding */
 float iris_hip_conv2d_copied_us(long in_pixels, long out_pixels, int cin, int cout, int k, int plain);

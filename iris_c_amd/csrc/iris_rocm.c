@@ -602,7 +602,12 @@ void iris_dev_conv2d(float *out, const float *in, const uint16_t *w, const float
         int e = iris_hip_conv2d_prepare_scratch(g_stream, g_conv_scratch);
         if (e) { check((hipError_t)e, "conv2d scratch"); return; }
     }
-    int err = iris_hip_conv2d(g_stream, g_conv_scratch, CONV_SCRATCH_BYTES, out, in, w, bias, h, width, cin, cout,
+    /* the kernels that need no scratch, of which one may use the workspace of the linear layers; the others */
+    int oh = (h + pad_before + pad_after - k) / stride + 1, ow = (width + pad_before + pad_after - k) / stride + 1, err = -2;
+    if (oh > 0 && ow > 0)
+        err = iris_hip_conv2d_direct(g_stream, linear_part(), out, in, w, bias, h, width, cin, cout, k, stride, pad_before, oh, ow);
+    if (err == -2)
+        err = iris_hip_conv2d(g_stream, g_conv_scratch, CONV_SCRATCH_BYTES, out, in, w, bias, h, width, cin, cout,
                               k, stride, pad_before, pad_after);
     if (err) check((hipError_t)err, "conv2d launch");
 }

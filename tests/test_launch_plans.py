@@ -299,6 +299,41 @@ def test_few_input_channels_with_next_to_nothing_to_do_per_pixel(conv_plan):
         assert conv_plan(h, w, 1, 1, 1) == conv_plan(h, w, 32, 4, 1) == conv_plan(h, w, 16, 512, 1) == conv_plan(h, w, 3, 128, 3, 1, 1, 1) == FEW_IN
 
 
+@pytest.mark.parametrize("groups", [1, 2, 3, 8, 16])
+def test_the_last_round_of_a_three_by_three_convolution_is_cut_into_ranges_that_cover_it_once(groups):
+    share = C.CDLL(iris_c_amd.LIB_PATH).iris_hip_conv2d_share
+    for total in (1, 2, 7, 8, 9, 31, 100, 255, 256, 257, 259, 288, 400, 511, 513, 1000, 1023, 2051):
+        tiles = set()
+        for xcd in range(8):
+            shares = []
+            for slot in range(32):
+                s = (C.c_int * 5)()
+                share(xcd, slot, total, groups, 0, s)
+                shares.append(tuple(s))
+            first, rest_first, rest = shares[0][:3]
+            assert rest < 32 and (rest_first - first) % 32 == 0 and all(s[:3] == shares[0][:3] for s in shares)
+            tiles |= set(range(first, rest_first + rest))
+            at = 0
+            for slot, (*_, u0, u1) in enumerate(shares):
+                assert u0 == at and u1 - u0 <= groups and (u1 == u0 or (u1 - 1) // groups - u0 // groups <= 1)
+                assert u1 > u0 or u0 == rest * groups                       # the workgroups that have a range come first
+                for unit in range(u0, u1):
+                    assert share(xcd, 0, total, groups, unit, (C.c_int * 5)()) == slot
+                at = u1
+            assert at == rest * groups
+        assert tiles == set(range(total))
+
+
+def test_the_last_round_is_cut_where_that_is_the_faster_form():
+    cut = C.CDLL(iris_c_amd.LIB_PATH).iris_hip_conv2d_cut
+    for oh, ow, cin, cout in CUT: assert cut(oh, ow, cin, cout) == 1, (oh, ow, cin, cout)
+    for oh, ow, cin, cout in WHOLE: assert cut(oh, ow, cin, cout) == 0, (oh, ow, cin, cout)
+
+
+CUT = [(64, 69, 512, 512), (64, 69, 512, 256), (122, 131, 512, 512), (177, 189, 512, 256), (16, 16, 512, 512)]
+WHOLE = [(256, 256, 512, 512), (512, 512, 256, 256), (512, 512, 128, 128), (200, 200, 128, 128), (111, 119, 512, 512), (40, 40, 64, 64)]
+
+
 # ------------------------------------------------------------------ row norms
 def test_row_norms_take_a_wave_per_row_where_rows_are_many_and_short_and_a_workgroup_elsewhere():
     lib = C.CDLL(iris_c_amd.LIB_PATH)
