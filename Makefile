@@ -56,7 +56,7 @@ oracle/libiris_oracle.so:
 iris_c_amd/libiris_microbench.so: $(CSRC)/microbench.hip
 	$(HIPCC) $(HIPFLAGS) -shared -o $@ $<
 
-$(CSRC)/%.o: $(CSRC)/%.hip $(CSRC)/iris_kernels_hip.h $(CSRC)/norm_rope_math.h
+$(CSRC)/%.o: $(CSRC)/%.hip $(CSRC)/iris_kernels_hip.h $(CSRC)/norm_rope_math.h $(CSRC)/write_through.h
 	$(HIPCC) $(HIPFLAGS) -c $< -o $@
 
 $(CSRC)/iris_rocm.o: $(CSRC)/iris_rocm.c $(HOST_HDRS)

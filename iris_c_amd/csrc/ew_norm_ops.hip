@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "iris_kernels_hip.h"
+#include "write_through.h"
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -43,19 +44,11 @@ __device__ __forceinline__ float bf_lo(uint32_t u) { return __uint_as_float(u <<
 __device__ __forceinline__ float bf_hi(uint32_t u) { return __uint_as_float(u & 0xffff0000u); }
 __device__ __forceinline__ float silu(float v) { return v / (1.0f + __expf(-v)); }
 
-/* 16 or 8 bytes, written through: the results leave the L2 as they are stored, while others are still read, and not at the end of
- * the kernel, in front of the next. us, plain / written through, operands from memory: LayerNorm 1000 x 2560 6.3 / 5.7, 2115 x 3072 11.1 /
+/* Written through, while others are still read: us, plain / written through, operands from memory: LayerNorm 1000 x 2560 6.3 / 5.7, 2115 x 3072 11.1 /
  * 10.7, residual 1000 x 2560 8.0 / 7.5, 4608 x 3072 31.2 / 29.3, f32 -> bf16 2115 x 3072 9.1 / 8.6; operands in the Infinity Cache: LayerNorm
  * 2115 x 3072 8.1 / 6.8, residual 12.3 / 8.8, SwiGLU 512 x 9728 5.6 / 4.3. A text-encoder layer of 512 rows 166.5 / 165.1, a single-stream
  * block of 320 rows 118.6 / 117.6, a double-stream block of 2627 803 / 800. Only where the result is what another operator reads:
- * rms_norm_residual and add_bias, called again on the same rows, find them in the L2 (12800 x 3072 76 / 86, 16384 x 512 7.7 / 10.4).
- * The compiler does not know that the statement is a store: the wait states stand for those it would place before the
- * registers are written again. */
-template <typename V> __device__ __forceinline__ void store_through(void *p, V v) {
-    if constexpr (sizeof(V) == 16) asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
-    else asm volatile("global_store_dwordx2 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
-}
-
+ * rms_norm_residual and add_bias, called again on the same rows, find them in the L2 (12800 x 3072 76 / 86, 16384 x 512 7.7 / 10.4). */
 inline unsigned blocks_for(size_t n, int per_block) { return (unsigned)((n + per_block - 1) / per_block); }
 
 /* ---------------------------------------------------------------- elementwise */
