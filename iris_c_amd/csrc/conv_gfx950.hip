@@ -18,6 +18,7 @@
 #include <type_traits>
 
 #include "iris_kernels_hip.h"
+#include "write_through.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -148,8 +149,8 @@ k_conv_few_in(float *__restrict__ out, const float *__restrict__ in, const uint1
             const f32x4 r = *reinterpret_cast<const f32x4 *>(&buf[row * FI_COLS + 4 * ((c & 16) | ((c ^ row) & 15))]) + bv;
             float *dst = first + (unsigned)(row * s.cout + 4 * c);
             if (16 * g + row >= pixels) continue;
-            if (ALIGNED && THROUGH) {                          /* the wait states: the compiler does not know that this is a store */
-                if (n < s.cout) asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"(dst), "v"(r) : "memory");
+            if (ALIGNED && THROUGH) {
+                if (n < s.cout) store_through(dst, r);
             } else if (ALIGNED) {
                 if (n < s.cout) *reinterpret_cast<f32x4 *>(dst) = r;
             } else {
@@ -384,7 +385,9 @@ int launch_1x1(hipStream_t st, float *out, const float *in, const uint16_t *W, c
  *  - Waves 0 - 7 multiply: 4 (rows of four pixels) x 2 (64 channels), a wave owns 64 pixels x 64 channels = 4 x 4
  *    accumulator blocks, and a step is 32 products: 16 of the first half of the step's channels, the barrier, 16 of the
  *    second half. The operands of a half are read from the LDS in the gaps between the products of the half before, one to
- *    a gap, across the barrier too. They issue no load and wait for none, so a tile's stores drain under the next tile.
+ *    a gap, across the barrier too: four of weights, and of a tap's four rows of pixels one where the tap before was the one above
+ *    it, which the order of the taps makes two of three (all four read for every tap: 512 x 512, 256 -> 256 249 us / 243, 256 -> 128
+ *    135.7 / 131.9, 256 x 256, 512 -> 512 228 / 222). They issue no load and wait for none, so a tile's stores drain under the next tile.
  *  - Waves 8 - 11 bring everything in. The image: 2592 units of 8 channels x pixel per group of 64 channels, 11 a thread,
  *    all of them in registers on their way while the group before is multiplied. One or two a step are rounded and written
  *    to the image buffer that the last group has left (the epilogue borrows it until the barrier of step 0), and
@@ -395,8 +398,13 @@ int launch_1x1(hipStream_t st, float *out, const float *in, const uint16_t *W, c
  * tap starts at, they fall into distinct bank windows; a tap's shift is an immediate offset. Weight rows are swizzled as
  * in gemm_conv_gfx950.hip. A workgroup takes 152 KB of LDS, so a CU runs one, and it is persistent.
  *
+ * A tile of 512 input channels takes 44 us on however few CUs, and a round of few tiles as long as a full one. So the tiles of an XCD
+ * behind its whole rounds may be cut into ranges of channel groups, dealt to its 32 CUs in equal shares (c3_share); what lies in a
+ * range is a tile like any other, but leaves its sums in a workspace, and k_conv_3x3_sum adds the ranges in order. `three_ranges` says
+ * where that is the faster form. A convolution under capture, which may be replayed on any stream, has no workspace and keeps its tiles whole.
+ *
  * Measured against a bf16 copy of the image + implicit product that fetches every tap from the L2 (copy + product), against
- * eight waves that did everything (and stood still while a tile's stores landed), and now: 512 x 512 pixels, 128 -> 128
+ * eight waves that did everything (and stood still while a tile's stores landed), and these roles: 512 x 512 pixels, 128 -> 128
  * 30 + 118, 79, 73 us (the image and the result alone take 50 us to move), 256 -> 128 76 + 214, 129, 123, 256 -> 256 88 + 290,
  * 253, 235 us (1320 TFLOP/s). The first is bound by memory (matrix cores busy 43 - 45 % of its cycles), the last by the products
  * at the clock that the chip's power leaves (62 - 64 % at 1.9 - 2.0 GHz of 2.4; counters, under the profiler). Pixels and
@@ -414,6 +422,10 @@ static_assert(c3_first(9) == C3_UNITS && c3_units(0) == 0, "");
 /* the tap of a step: down the columns of the 3 x 3 */
 __device__ constexpr int c3_tap(int t) { return t % 3 * 3 + t / 3; }
 
+/* Results of up to 64 MB are written through (write_through.h), larger ones stay for the operator that reads them next: us, plain /
+ * through, a decoder stage 64 x 70, 512 -> 512 298.7 / 293.1, the first encoder stage 150 x 200 106.7 / 105.0, 256 x 256 143.0 / 141.7, 320 x 330 (54 MB)
+ * 204.5 / 203.3, 512 x 512 (134 MB) 399.3 / 408.0. */
+constexpr size_t C3_THROUGH_MOST = (size_t)64 << 20;
 constexpr int C3_SLOTS = 32, C3_PART = 4096;                   /* CUs of an XCD; floats of a wave's sums */
 static_assert((size_t)16 * C3_SLOTS * C3_MUL * C3_PART * 4 <= IRIS_LINEAR_PART_BYTES, "two places a workgroup");
 
@@ -438,7 +450,7 @@ __host__ __device__ inline int c3_taker(const C3Share &sh, int groups, int unit)
 #pragma clang diagnostic ignored "-Winline-asm"                /* M0 in a clobber list */
 __global__ void __launch_bounds__(C3_THREADS, 3)
 k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t *__restrict__ W, const float *__restrict__ bias,
-           ConvShape s, int tiles_x, int tiles_n, int total, int per_xcd, float *__restrict__ part) {
+           ConvShape s, int tiles_x, int tiles_n, int total, int per_xcd, float *__restrict__ part, int through) {
     extern __shared__ __align__(16) uint16_t lds[];            /* image, image, weights, weights, weights, bias */
     /* an XCD takes a contiguous range of the tiles, the channel tiles of a pixel tile next to each other (they share the
      * image in its L2), dealt out to its workgroups in turn; with `part`, those of its last, incomplete round in ranges of channel groups */
@@ -649,7 +661,10 @@ k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t
                 v[it] = *reinterpret_cast<const f32x4 *>(&buf[row * 64 + 4 * (c ^ row)]) + bias4;
             }
             float *dst = out + ((size_t)y * s.ow + tx0 + lg) * s.cout + n;
-            if (whole) {
+            if (whole && through) {
+#pragma unroll
+                for (int it = 0; it < 4; it++) store_through(dst + (size_t)(4 * it) * s.cout, v[it]);
+            } else if (whole) {
 #pragma unroll
                 for (int it = 0; it < 4; it++) *reinterpret_cast<f32x4 *>(dst + (size_t)(4 * it) * s.cout) = v[it];
             } else if (y < s.oh) {
@@ -671,7 +686,7 @@ k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t
 #pragma unroll
         for (int a = 0; a < 4; a++)
 #pragma unroll
-            for (int b = 0; b < 4; b++) *reinterpret_cast<f32x4 *>(dst + ((4 * a + b) * 64 + lane) * 4) = acc[a][b];
+            for (int b = 0; b < 4; b++) store_through(dst + ((4 * a + b) * 64 + lane) * 4, acc[a][b]);
     };
 
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -774,7 +789,7 @@ int launch_3x3(hipStream_t st, float *part, float *out, const float *in, const u
     /* one workgroup per CU (its LDS): 32 per XCD, each walking the XCD's tiles */
     if (!three_ranges(s, per_xcd)) part = nullptr;
     hipLaunchKernelGGL(k_conv_3x3, dim3((unsigned)(part || per_xcd >= C3_SLOTS ? C3_SLOTS : per_xcd) * 8), dim3(C3_THREADS), lds, st, out, in, W, bias, s,
-                       tiles_x, tiles_n, total, per_xcd, part);
+                       tiles_x, tiles_n, total, per_xcd, part, (size_t)s.oh * s.ow * s.cout * 4 <= C3_THROUGH_MOST);
     int rest = 0;                                              /* of the XCD that has most of it: the last one may have fewer tiles */
     for (int x = 0; part && x < 8; x++) {
         const int r = c3_share(x, 0, C3_SLOTS, total, per_xcd, s.cin / 64, true).rest;
@@ -1000,7 +1015,7 @@ k_conv_3x3_half(float *__restrict__ out, const float *__restrict__ in, const uin
                     if (y >= s.oh || x >= s.ow) continue;
                     float *dst = out + ((size_t)y * s.ow + x) * s.cout + n;
                     if (chunks) {
-                        if (n < s.cout) *reinterpret_cast<f32x4 *>(dst) = v;
+                        if (n < s.cout) store_through(dst, v);
                     } else {
 #pragma unroll
                         for (int e = 0; e < 4; e++)

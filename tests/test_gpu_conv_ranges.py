@@ -42,3 +42,22 @@ def test_against_float64(dev, h, w, cin, cout, pb, pa, bias):
     dev.free_all()
     assert (got[0][want.size:] == 7.0).all() and np.array_equal(got[0], got[1])
     np.testing.assert_allclose(got[0][:want.size].reshape(want.shape), want, atol=2e-5 * np.sqrt(9 * cin))
+
+
+@pytest.mark.parametrize("h,w", [(364, 360), (365, 360)])
+def test_results_up_to_64_megabytes_are_written_through_and_larger_ones_are_not(dev, h, w):
+    """Whole and ragged tiles of both: 128 channels of 131040 and of 131400 pixels."""
+    cin, cout = 64, 128
+    assert (h * w * cout * 4 <= 64 << 20) == (h == 364)
+    rng = np.random.default_rng(h)
+    img = rng.standard_normal((h * w, cin), dtype=np.float32)
+    wt = O.f32_to_bf16((rng.standard_normal((cout, 9 * cin)) * 0.1).astype(np.float32))
+    b = rng.standard_normal(cout).astype(np.float32)
+    want = conv_float64(img, wt, b, h, w, 3, 1, 1, 1)
+    out = dev.put(np.full(want.size + 64, 7.0, np.float32))
+    dev.lib.iris_dev_conv2d(out, dev.put(img), dev.put(wt), dev.put(b), h, w, cin, cout, 3, 1, 1, 1)
+    dev.check()
+    got = dev.get(out, (want.size + 64,), np.float32)
+    dev.free_all()
+    assert (got[want.size:] == 7.0).all()
+    np.testing.assert_allclose(got[:want.size].reshape(want.shape), want, atol=2e-5 * np.sqrt(9 * cin))
