@@ -36,8 +36,6 @@
  * 128 x 128, each of which fetches 224 rows instead of 256. Weights from HBM, us, without / with it: 512 x 2560 -> 6144 24.2 / 22.9,
  * 320 rows 25.3 / 22.6, 512 x 3072 -> 3072 22.4 / 20.2 (two ranges of K instead of three), 700 rows 26.0 / 23.2, 1000 x 4096 -> 2560
  * 32.2 / 30.2, 100 x 2560 -> 19456 33.0 / 30.7; no slower at any of the 60 sizes from 100 to 1000 rows where it is chosen.
- * Results and partial sums are written through (write_through.h): a text-encoder layer of 200 rows 128.0 us / 126.6, of 512 162.8 / 162.4, a
- * double-stream block of 2627 rows 786.8 / 783.1; of 128 + 700 rows, and a single-stream block of 320, the same.
  */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -82,7 +80,7 @@ struct Tile {
 template <typename OUT, int NB, int WM, int NA, int WN, int KG, int STAGES>
 __global__ void __launch_bounds__(64 * WM * WN * KG, WM * WN * KG / 4)
 k_gemm_tiles(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *__restrict__ W, int M, int N, int K,
-             const float *__restrict__ bias, int tiles_m, int tiles_n, int splits, int total, int per_xcd, int turns) {
+             const float *__restrict__ bias, int tiles_m, int tiles_n, int splits, int total, int per_xcd, int turns, int through) {
     using T = Tile<NB, WM, NA, WN, KG, STAGES>;
     constexpr int TM = T::TM, TN = T::TN, STAGE = T::STAGE, PIECES = T::PIECES;
     static_assert(T::LDS <= 160 * 1024 && NA <= 8 && (KG == 1 || (KG == 2 && NB % 2 == 0)), "");
@@ -259,7 +257,8 @@ k_gemm_tiles(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t
                 f32x4 v = *reinterpret_cast<const f32x4 *>(&buf[row * 64 + 4 * (c ^ (row & 15))]);
                 if (c < 4 * na && m < M && n < N) {
                     if (bias) v += *reinterpret_cast<const f32x4 *>(bias + n);
-                    store_through(dst + (size_t)m * N + n, v);
+                    if (through) store_through(dst + (size_t)m * N + n, v);
+                    else *reinterpret_cast<f32x4 *>(dst + (size_t)m * N + n) = v;
                 }
             }
         } else {
@@ -276,7 +275,7 @@ k_gemm_tiles(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t
             for (int it = 0; it < 2 * NBS; it++) {
                 const int row = 8 * it + (lane >> 3), c = lane & 7, m = mw + row, n = nc + 8 * c;
                 const u32x4 v = *reinterpret_cast<const u32x4 *>(&buf[row * 64 + 8 * (c ^ (row & 7))]);
-                if (c < 2 * na && m < M && n < N) store_through(dst + (size_t)m * N + n, v);
+                if (c < 2 * na && m < M && n < N) *reinterpret_cast<u32x4 *>(dst + (size_t)m * N + n) = v;
             }
         }
     }
@@ -319,6 +318,12 @@ static int turns(int M, int N, int K, int wgs) {
     return (long)((M + 255) / 256) * ((N + 255) / 256) > 512 ? 0 : iris_hip_gemm_turns(wgs, (size_t)N * K * 2);
 }
 
+/* Partial sums of up to 20 MB leave the L2s as they are stored (write_through.h) and not in front of the sum. us, plain / through, a
+ * text-encoder layer of 90 rows (11 MB and less) 107.4 / 105.9, 200 rows (18) 129.6 / 126.9, a single-stream block of 24 heads, 85 rows (17) 82.7 / 82.0,
+ * 200 (20) 102.1 / 101.3; beyond that it goes either way: 32 heads, 86 rows (22) 131.7 / 133.0, 24 heads, 320 rows (31) 115.9 / 114.9, 150 (33) 103.2 /
+ * 106.3. bf16 results too: 900 rows of the encoder 251.1 / 247.6, but 507 rows of a single-stream block of 32 heads 255.5 / 259.9. */
+constexpr size_t THROUGH_MOST = (size_t)20 << 20;
+
 template <typename OUT, int NB, int WM, int NA, int WN, int KG, int STAGES>
 int launch_tiles(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, const float *bias, int splits) {
     using T = Tile<NB, WM, NA, WN, KG, STAGES>;
@@ -331,7 +336,8 @@ int launch_tiles(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, i
     }
     const int tiles_m = (M + T::TM - 1) / T::TM, tiles_n = (N + T::TN - 1) / T::TN, total = tiles_m * tiles_n * splits, per_xcd = (total + 7) / 8;
     hipLaunchKernelGGL((k_gemm_tiles<OUT, NB, WM, NA, WN, KG, STAGES>), dim3((unsigned)per_xcd * 8), dim3(T::THREADS), T::LDS, st, y, x, W, M, N, K,
-                       bias, tiles_m, tiles_n, splits, total, per_xcd, turns(M, N, K, total));
+                       bias, tiles_m, tiles_n, splits, total, per_xcd, turns(M, N, K, total),
+                       splits > 1 && (size_t)splits * M * N * 4 <= THROUGH_MOST);
     return (int)hipGetLastError();
 }
 
