@@ -385,7 +385,8 @@ int launch_1x1(hipStream_t st, float *out, const float *in, const uint16_t *W, c
  *  - Waves 0 - 7 multiply: 4 (rows of four pixels) x 2 (64 channels), a wave owns 64 pixels x 64 channels = 4 x 4
  *    accumulator blocks, and a step is 32 products: 16 of the first half of the step's channels, the barrier, 16 of the
  *    second half. The operands of a half are read from the LDS in the gaps between the products of the half before, one to
- *    a gap, across the barrier too: four of weights, and of a tap's four rows of pixels one where the tap before was the one above
+ *    a gap, behind its first four (a decoder stage 128 x 128, 512 -> 512, from the first gap on 860.5 us, behind four 849.5, behind six 853.5), across
+ *    the barrier too: four of weights, and of a tap's four rows of pixels one where the tap before was the one above
  *    it, which the order of the taps makes two of three (all four read for every tap: 512 x 512, 256 -> 256 249 us / 243, 256 -> 128
  *    135.7 / 131.9, 256 x 256, 512 -> 512 228 / 222). They issue no load and wait for none, so a tile's stores drain under the next tile.
  *  - Waves 8 - 11 bring everything in. The image: 2592 units of 8 channels x pixel per group of 64 channels, 11 a thread,
@@ -632,7 +633,7 @@ k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t
 #pragma unroll
         for (int i = 0; i < 16; i++) {
             asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc[i / 4][i % 4]) : "v"(av[ks][i / 4]), "v"(bv[ks][(i + t % 3) % 4]));
-            if (i < 8) operand(img, next, ks ^ 1, i);
+            if (i >= 4 && i < 12) operand(img, next, ks ^ 1, i - 4);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
