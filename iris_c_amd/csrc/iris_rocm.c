@@ -32,7 +32,7 @@ static const char *g_last_kernel = "none";
 #ifndef IRIS_DEV_PATH_ONLY
 #define CONV_SCRATCH_BYTES ((size_t)256 << 20)
 static uint16_t *g_conv_scratch = NULL;
-/* partial sums of linear layers whose K is cut into ranges; allocated at initialisation, so that a linear layer never
+/* partial sums of linear layers and convolutions whose K is cut into ranges; allocated at initialisation, so that a linear layer never
  * allocates */
 static float *g_linear_part = NULL;
 /* group norm of up to 64 groups, which keeps counters there: allocated and cleared once, by iris_dev_init; and of more */
@@ -485,7 +485,7 @@ static int linear_by_library(void *y, int out_bf16, const uint16_t *x, const uin
     return 1;
 }
 
-/* The workspace of the next linear layer, or NULL: K then stays whole. The stream orders the layers that share it, but a layer
+/* The workspace of the next linear layer or 3 x 3 convolution, or NULL: K then stays whole. The stream orders the layers that share it, but a layer
  * that is captured may be replayed on any stream, beside others: it gets none. */
 static float *linear_part(void) {
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
