@@ -77,10 +77,10 @@ struct Tile {
 
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"                          /* M0 in a clobber list */
-template <typename OUT, int NB, int WM, int NA, int WN, int KG, int STAGES>
+template <typename OUT, int NB, int WM, int NA, int WN, int KG, int STAGES, bool THROUGH>
 __global__ void __launch_bounds__(64 * WM * WN * KG, WM * WN * KG / 4)
 k_gemm_tiles(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *__restrict__ W, int M, int N, int K,
-             const float *__restrict__ bias, int tiles_m, int tiles_n, int splits, int total, int per_xcd, int turns, int through) {
+             const float *__restrict__ bias, int tiles_m, int tiles_n, int splits, int total, int per_xcd, int turns) {
     using T = Tile<NB, WM, NA, WN, KG, STAGES>;
     constexpr int TM = T::TM, TN = T::TN, STAGE = T::STAGE, PIECES = T::PIECES;
     static_assert(T::LDS <= 160 * 1024 && NA <= 8 && (KG == 1 || (KG == 2 && NB % 2 == 0)), "");
@@ -257,7 +257,7 @@ k_gemm_tiles(OUT *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t
                 f32x4 v = *reinterpret_cast<const f32x4 *>(&buf[row * 64 + 4 * (c ^ (row & 15))]);
                 if (c < 4 * na && m < M && n < N) {
                     if (bias) v += *reinterpret_cast<const f32x4 *>(bias + n);
-                    if (through) store_through(dst + (size_t)m * N + n, v);
+                    if constexpr (THROUGH) store_through(dst + (size_t)m * N + n, v);
                     else *reinterpret_cast<f32x4 *>(dst + (size_t)m * N + n) = v;
                 }
             }
@@ -321,23 +321,28 @@ static int turns(int M, int N, int K, int wgs) {
 /* Partial sums of up to 20 MB leave the L2s as they are stored (write_through.h) and not in front of the sum. us, plain / through, a
  * text-encoder layer of 90 rows (11 MB and less) 107.4 / 105.9, 200 rows (18) 129.6 / 126.9, a single-stream block of 24 heads, 85 rows (17) 82.7 / 82.0,
  * 200 (20) 102.1 / 101.3; beyond that it goes either way: 32 heads, 86 rows (22) 131.7 / 133.0, 24 heads, 320 rows (31) 115.9 / 114.9, 150 (33) 103.2 /
- * 106.3. bf16 results too: 900 rows of the encoder 251.1 / 247.6, but 507 rows of a single-stream block of 32 heads 255.5 / 259.9. */
+ * 106.3. bf16 results too: 900 rows of the encoder 251.1 / 247.6, but 507 rows of a single-stream block of 32 heads 255.5 / 259.9.
+ * Two kernels: with a test in front of every store of one, plain ones took 0.5 - 2 % longer. us, one kernel / two / one that only stores plainly:
+ * 96 x 2560 -> 6144 16.12 / 15.74 / 15.79, 150 x 12288 -> 3072 29.27 / 29.04 / 28.99, 900 x 12288 -> 3072 77.6 / 76.6 / 76.7; written through
+ * 85 x 12288 -> 3072 24.48 / 24.36. */
 constexpr size_t THROUGH_MOST = (size_t)20 << 20;
 
-template <typename OUT, int NB, int WM, int NA, int WN, int KG, int STAGES>
+template <typename OUT, int NB, int WM, int NA, int WN, int KG, int STAGES, bool THROUGH = false>
 int launch_tiles(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, const float *bias, int splits) {
+    if constexpr (sizeof(OUT) == 4 && !THROUGH)
+        if (splits > 1 && (size_t)splits * M * N * 4 <= THROUGH_MOST)
+            return launch_tiles<OUT, NB, WM, NA, WN, KG, STAGES, true>(st, y, x, W, M, N, K, bias, splits);
     using T = Tile<NB, WM, NA, WN, KG, STAGES>;
     static bool configured = false;
     if (!configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_gemm_tiles<OUT, NB, WM, NA, WN, KG, STAGES>),
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_gemm_tiles<OUT, NB, WM, NA, WN, KG, STAGES, THROUGH>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS);
         if (e != hipSuccess) return (int)e;
         configured = true;
     }
     const int tiles_m = (M + T::TM - 1) / T::TM, tiles_n = (N + T::TN - 1) / T::TN, total = tiles_m * tiles_n * splits, per_xcd = (total + 7) / 8;
-    hipLaunchKernelGGL((k_gemm_tiles<OUT, NB, WM, NA, WN, KG, STAGES>), dim3((unsigned)per_xcd * 8), dim3(T::THREADS), T::LDS, st, y, x, W, M, N, K,
-                       bias, tiles_m, tiles_n, splits, total, per_xcd, turns(M, N, K, total),
-                       splits > 1 && (size_t)splits * M * N * 4 <= THROUGH_MOST);
+    hipLaunchKernelGGL((k_gemm_tiles<OUT, NB, WM, NA, WN, KG, STAGES, THROUGH>), dim3((unsigned)per_xcd * 8), dim3(T::THREADS), T::LDS, st, y, x, W, M, N, K,
+                       bias, tiles_m, tiles_n, splits, total, per_xcd, turns(M, N, K, total));
     return (int)hipGetLastError();
 }
 
