@@ -318,20 +318,12 @@ static int turns(int M, int N, int K, int wgs) {
     return (long)((M + 255) / 256) * ((N + 255) / 256) > 512 ? 0 : iris_hip_gemm_turns(wgs, (size_t)N * K * 2);
 }
 
-/* Partial sums of up to 20 MB leave the L2s as they are stored (write_through.h) and not in front of the sum. us, plain / through, a
- * text-encoder layer of 90 rows (11 MB and less) 107.4 / 105.9, 200 rows (18) 129.6 / 126.9, a single-stream block of 24 heads, 85 rows (17) 82.7 / 82.0,
- * 200 (20) 102.1 / 101.3; beyond that it goes either way: 32 heads, 86 rows (22) 131.7 / 133.0, 24 heads, 320 rows (31) 115.9 / 114.9, 150 (33) 103.2 /
- * 106.3. bf16 results too: 900 rows of the encoder 251.1 / 247.6, but 507 rows of a single-stream block of 32 heads 255.5 / 259.9.
- * Two kernels: with a test in front of every store of one, plain ones took 0.5 - 2 % longer. us, one kernel / two / one that only stores plainly:
- * 96 x 2560 -> 6144 16.12 / 15.74 / 15.79, 150 x 12288 -> 3072 29.27 / 29.04 / 28.99, 900 x 12288 -> 3072 77.6 / 76.6 / 76.7; written through
- * 85 x 12288 -> 3072 24.48 / 24.36. */
-constexpr size_t THROUGH_MOST = (size_t)20 << 20;
-
+/* THROUGH is a template's choice: with a test in front of every store of one kernel, plain ones took 0.5 - 2 % longer. us, one kernel / two / one that
+ * only stores plainly: 96 x 2560 -> 6144 16.12 / 15.74 / 15.79, 150 x 12288 -> 3072 29.27 / 29.04 / 28.99, 900 x 12288 -> 3072 77.6 / 76.6 / 76.7. */
 template <typename OUT, int NB, int WM, int NA, int WN, int KG, int STAGES, bool THROUGH = false>
-int launch_tiles(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, const float *bias, int splits) {
+int launch_tiles(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, const float *bias, int splits, bool through) {
     if constexpr (sizeof(OUT) == 4 && !THROUGH)
-        if (splits > 1 && (size_t)splits * M * N * 4 <= THROUGH_MOST)
-            return launch_tiles<OUT, NB, WM, NA, WN, KG, STAGES, true>(st, y, x, W, M, N, K, bias, splits);
+        if (through) return launch_tiles<OUT, NB, WM, NA, WN, KG, STAGES, true>(st, y, x, W, M, N, K, bias, splits, true);
     using T = Tile<NB, WM, NA, WN, KG, STAGES>;
     static bool configured = false;
     if (!configured) {
@@ -351,24 +343,26 @@ int launch_tiles(hipStream_t st, OUT *y, const uint16_t *x, const uint16_t *W, i
  * between these tiles and k_gemm_wide, which is the faster one there unless its tiles fit badly; with the figures of two rounds
  * these tiles were taken for 12800 x 12288 -> 3072 (752 us on k_gemm_wide, 819 here), 9280 x 12288 -> 4096 (749 / 808),
  * 7176 x 16384 -> 4096 (734 / 804), 3680 x 4096 -> 36864 (862 / 900). A workgroup's first tiles and its epilogue take 3.5 us more.
- * Three digits where sizes are decided by them: 528 - 640 x 4096 -> 2560 24.4 us in four ranges of 160 x 192, 26.2 in five of 128 x 256. */
-struct Shape { int tm, tn; float step, step_two, step_more; };
-constexpr Shape SHAPES[] = {{128, 128, 0.44f, 0.50f, 0.55f}, {128, 192, 0.58f, 0.62f, 0.65f}, {128, 256, 0.736f, 0.80f, 0.82f},
-                            {64, 256, 0.60f, 0.61f, 0.62f},  {160, 192, 0.665f, 0.72f, 0.74f}, {160, 256, 0.90f, 0.93f, 0.94f},
-                            {160, 224, 0.836f, 0.87f, 0.89f}, {128, 96, 0.39f, 0.45f, 0.50f}};
+ * Three digits where sizes are decided by them: 528 - 640 x 4096 -> 2560 24.4 us in four ranges of 160 x 192, 26.2 in five of 128 x 256.
+ * `through`: see iris_hip_gemm_tiles_through. */
+struct Shape { int tm, tn; float step, step_two, step_more; int through; };
+constexpr Shape SHAPES[] = {{128, 128, 0.44f, 0.50f, 0.55f, 100}, {128, 192, 0.58f, 0.62f, 0.65f, 100}, {128, 256, 0.736f, 0.80f, 0.82f, 100},
+                            {64, 256, 0.60f, 0.61f, 0.62f, 80},   {160, 192, 0.665f, 0.72f, 0.74f, 64}, {160, 256, 0.90f, 0.93f, 0.94f, 64},
+                            {160, 224, 0.836f, 0.87f, 0.89f, 64}, {128, 96, 0.39f, 0.45f, 0.50f, 64}};
 constexpr int NSHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
 
 template <typename OUT>
-int launch_shape(hipStream_t st, int shape, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, const float *bias, int splits) {
+int launch_shape(hipStream_t st, int shape, OUT *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, const float *bias, int splits,
+                 bool through = false) {
     switch (shape) {
-    case 0: return launch_tiles<OUT, 4, 2, 4, 2, 2, 4>(st, y, x, W, M, N, K, bias, splits);
-    case 1: return launch_tiles<OUT, 4, 2, 3, 4, 1, 4>(st, y, x, W, M, N, K, bias, splits);
-    case 2: return launch_tiles<OUT, 4, 2, 4, 4, 1, 3>(st, y, x, W, M, N, K, bias, splits);
-    case 3: return launch_tiles<OUT, 4, 1, 4, 4, 2, 4>(st, y, x, W, M, N, K, bias, splits);
-    case 4: return launch_tiles<OUT, 5, 2, 3, 4, 1, 3>(st, y, x, W, M, N, K, bias, splits);
-    case 5: return launch_tiles<OUT, 5, 2, 4, 4, 1, 3>(st, y, x, W, M, N, K, bias, splits);
-    case 6: return launch_tiles<OUT, 5, 2, 7, 2, 1, 3>(st, y, x, W, M, N, K, bias, splits);
-    case 7: return launch_tiles<OUT, 4, 2, 3, 2, 2, 4>(st, y, x, W, M, N, K, bias, splits);
+    case 0: return launch_tiles<OUT, 4, 2, 4, 2, 2, 4>(st, y, x, W, M, N, K, bias, splits, through);
+    case 1: return launch_tiles<OUT, 4, 2, 3, 4, 1, 4>(st, y, x, W, M, N, K, bias, splits, through);
+    case 2: return launch_tiles<OUT, 4, 2, 4, 4, 1, 3>(st, y, x, W, M, N, K, bias, splits, through);
+    case 3: return launch_tiles<OUT, 4, 1, 4, 4, 2, 4>(st, y, x, W, M, N, K, bias, splits, through);
+    case 4: return launch_tiles<OUT, 5, 2, 3, 4, 1, 3>(st, y, x, W, M, N, K, bias, splits, through);
+    case 5: return launch_tiles<OUT, 5, 2, 4, 4, 1, 3>(st, y, x, W, M, N, K, bias, splits, through);
+    case 6: return launch_tiles<OUT, 5, 2, 7, 2, 1, 3>(st, y, x, W, M, N, K, bias, splits, through);
+    case 7: return launch_tiles<OUT, 4, 2, 3, 2, 2, 4>(st, y, x, W, M, N, K, bias, splits, through);
     default: return (int)hipErrorInvalidValue;
     }
 }
@@ -392,6 +386,18 @@ int iris_hip_gemm_tiles_in_order(int shape, int splits, int M, int N, int K) {
     constexpr bool two_groups[NSHAPES] = {true, false, false, true, false, false, false, true};
     const long wgs = (long)((M + SHAPES[shape].tm - 1) / SHAPES[shape].tm) * ((N + SHAPES[shape].tn - 1) / SHAPES[shape].tn);
     return splits == 1 && !two_groups[shape] && turns(M, N, K, (int)(wgs < 1 << 30 ? wgs : 1 << 30)) == 0;
+}
+
+/* 1: the partial sums of a product in ranges of K leave the L2s as they are stored (write_through.h) and not in front of the sum: those of
+ * up to 20 MB, with weights of up to `through` MB. Larger weights, of which a single row of tiles takes a new line with every load, are
+ * slowed down by the stores beside them, from different sizes on with each tile. us, all plain / all through, weights from HBM, up to the bound:
+ * 64 x 9728 -> 2560 (48 MB) 19.5 / 18.1, 128 x 9216 -> 3072 (54) 21.3 / 20.4, 64 x 12288 -> 3072 (72) 23.5 / 22.8, 90 rows 26.6 / 25.7, 72 x 3072 -> 15360
+ * (90) 28.4 / 27.3, 100 x 4096 -> 12288 (96) 33.8 / 32.6, 128 x 12288 -> 4096 30.2 / 28.9; beyond it 123 x 12288 -> 3072 (tiles of 128 x 96) 25.1 / 25.7, 64 x
+ * 3072 -> 15360 (64 x 256) 26.8 / 27.3, 64 x 2560 -> 19456 (95 MB) 28.0 / 28.7, 129 rows (160 x 192) 33.7 / 35.0, 64 x 3072 -> 18432 (108) 29.2 / 30.0, 128 x
+ * 4096 -> 16384 (128) 43.5 / 44.1, 128 x 5120 -> 13824 (135) 39.8 / 41.0, 100 x 13824 -> 5120 37.8 / 38.6. 159 products of 16 to 768 rows up to both bounds
+ * are 0.9 to 8 % faster, half of them by 4 % or more; of 72 up to 20 MB beyond the other, half are slower, by up to 4 %. */
+int iris_hip_gemm_tiles_through(int shape, int splits, int M, int N, int K) {
+    return splits > 1 && (size_t)splits * M * N * 4 <= (size_t)20 << 20 && (size_t)N * K * 2 <= (size_t)SHAPES[shape].through << 20;
 }
 
 /* The cheapest tile and number of K ranges for a product, and its estimated time in us; negative where these kernels do
@@ -428,7 +434,7 @@ int iris_hip_gemm_tiles(void *stream, void *y, int out_size, const uint16_t *x, 
     if (splits == 1)
         return out_size == 2 ? launch_shape<uint16_t>(st, shape, (uint16_t *)y, x, W, M, N, K, nullptr, 1)
                              : launch_shape<float>(st, shape, (float *)y, x, W, M, N, K, bias, 1);
-    int e = launch_shape<float>(st, shape, part, x, W, M, N, K, nullptr, splits);
+    int e = launch_shape<float>(st, shape, part, x, W, M, N, K, nullptr, splits, iris_hip_gemm_tiles_through(shape, splits, M, N, K) != 0);
     if (e) return e;
     const size_t n = (size_t)M * N;
     return out_size == 2 ? launch_sum(st, (uint16_t *)y, part, n, splits) : launch_sum(st, (float *)y, part, n, splits);

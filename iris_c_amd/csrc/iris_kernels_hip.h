@@ -151,6 +151,7 @@ int iris_hip_linear_bf16(void *stream, float *part, uint16_t *y, const uint16_t 
 void iris_hip_linear_plan(int rows, int in, int out, int out_bytes, int *plan);
 int iris_hip_gemm_turns(long wgs, size_t weight_bytes);
 int iris_hip_gemm_tiles_in_order(int shape, int splits, int M, int N, int K);
+int iris_hip_gemm_tiles_through(int shape, int splits, int M, int N, int K);
 float iris_hip_gemm_tiles_plan(int M, int N, int K, int out_size, size_t part_bytes, int *shape, int *splits);
 int iris_hip_gemm_tiles(void *stream, void *y, int out_size, const uint16_t *x, const uint16_t *W, int M, int N, int K,
                         const float *bias, int shape, int splits, float *part);

@@ -185,6 +185,26 @@ def test_orders_of_the_k_tiles_go_by_what_of_the_weights_the_chip_already_holds(
     assert not turned(257, 14) and turned(257, 14.1) and turned(5000, 14.1)                           # several
 
 
+def test_partial_sums_beside_large_weights_are_stored_plainly(linear_plan):
+    lib = C.CDLL(iris_c_amd.LIB_PATH)
+    lib.iris_hip_gemm_tiles_plan.restype = C.c_float
+    lib.iris_hip_gemm_tiles_plan.argtypes = [C.c_int] * 4 + [C.c_size_t] + [C.POINTER(C.c_int)] * 2
+
+    def through(rows, k, out, size):
+        shape, splits = C.c_int(), C.c_int()
+        assert lib.iris_hip_gemm_tiles_plan(rows, out, k, size, 64 << 20, shape, splits) > 0 and splits.value > 1, (rows, k, out)
+        return lib.iris_hip_gemm_tiles_through(shape, splits, rows, out, k)
+
+    for rows, k, out, size in ((64, 9728, 2560, 4), (128, 9216, 3072, 4), (256, 4096, 2560, 4), (640, 3072, 3072, 4), (64, 12288, 3072, 4),
+                               (90, 12288, 3072, 4), (72, 3072, 15360, 2), (100, 4096, 12288, 2), (128, 12288, 4096, 4)):
+        assert through(rows, k, out, size) == 1, (rows, k, out)
+    for rows, k, out, size in ((123, 12288, 3072, 4), (128, 6144, 6144, 4), (64, 3072, 15360, 2), (64, 2560, 19456, 2), (129, 2560, 19456, 2),
+                               (64, 3072, 18432, 2), (64, 3072, 27648, 2), (128, 4096, 16384, 2), (100, 5120, 13824, 2), (100, 13824, 5120, 4),
+                               (320, 12288, 3072, 4), (512, 9728, 2560, 4)):                          # the last two: more than 20 MB
+        assert through(rows, k, out, size) == 0, (rows, k, out)
+    assert lib.iris_hip_gemm_tiles_through(0, 1, 512, 2560, 9728) == 0                                # nothing to add
+
+
 def test_projections_that_normalise_their_tiles_add_as_the_plain_layer_does(linear_plan):
     """Where the epilogue is taken, the plain layer is k_gemm_wide, k_gemm_dma, or tiles that take K whole, in one group and in order."""
     lib = C.CDLL(iris_c_amd.LIB_PATH)
