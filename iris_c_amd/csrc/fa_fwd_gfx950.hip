@@ -1297,8 +1297,12 @@ static FaPlan plan_hd128(int seq_q, int seq_k, int heads, int causal, bool maske
      * x 1355 52.4 / 35.4, 1255 valid keys 50.1 / 34.1; 30 x 1030 43.6 / 29.8, 343 valid 24.4 / 17.9). Not with causal, where a workgroup walks half of the keys on
      * average and those behind the first round are the short ones: there these go on to half as many waves again (us, the next
      * regime's / these, 32 heads x 1100 33.7 / 23.9, x 1280 39.8 / 31.5, 24 x 1400 40.0 / 30.0, x 2040 58.1 / 51.0, 16 x 3000 77.0 / 52.7; below 1024
-     * queries 40 x 900 30.2 / 32.8). Behind a key mask, which may end all walks early, only up to an eighth over a round: 32 x 1100 with 118,
-     * 550, 1100 valid keys 14.6 / 16.0, 25.4 / 22.1, 35.5 / 24.2; 24 x 1400, 350 valid 21.2 / 18.7; but x 1600, 400 valid 23.6 / 24.9.
+     * queries 40 x 900 30.2 / 32.8). Behind a key mask, which may end all walks early, only up to an eighth over a round, and below 2048 queries
+     * with four of these waves a workgroup: eight start late when the walks are short. us, the next regime's / eight / four, 32 x 1100 with 118, 200,
+     * 500, 1100 valid keys 14.2 / 15.6 / 14.7, 16.9 / 17.4 / 16.7, 22.8 / 21.4 / 20.0, 34.6 / 23.4 / 25.1; 24 x 1424, 300 valid 19.6 / 21.6 / 18.7, all 42.1 / 29.0 /
+     * 28.3; x 1536, 500 valid 24.0 / 27.9 / 22.7, all 47.2 / 31.2 / 30.2; but 16 x 2080, 118 valid 15.5 / 15.3 / 13.0, all 58.8 / 38.8 / 42.4; x 2300, 200 valid 18.5 /
+     * 19.6 / 18.4, 800 31.8 / 24.0 / 25.0, all 65.4 / 43.3 / 47.2. Two are slower than both throughout (15 - 20 %). Beyond the eighth 24 x 1600, 400 valid 23.6 /
+     * 24.9 with eight.
      * Measured, clocks settled, rows in the L2, against
      * 32 queries per wave: 32 heads on 8 x 512 tokens causal + mask 11.9 us against 15.5; 24 heads x 320 tokens
      * 7.7 against 10.5, x 576 11.8 against 15.2, x 768 17.4 against 20.2, x 1280 26.0 against 29.8 (x 1536: 56 against
@@ -1321,7 +1325,8 @@ static FaPlan plan_hd128(int seq_q, int seq_k, int heads, int causal, bool maske
     const long wg128 = (long)((seq_q + 127) / 128) * heads;
     const bool longer_causal = causal && seq_q >= 1024 && (masked ? wg128 <= CUS + CUS / 8 : waves16 <= 12 * CUS);
     if (longer_causal || (waves16 <= 8 * CUS && (causal || waves16 <= 4 * CUS || wg128 <= CUS))) {
-        const int w = waves16 <= CUS ? 1 : waves16 <= 640 ? 2 : waves16 <= 4 * CUS ? 4 : 8;
+        const bool short_walks = masked && longer_causal && waves16 > 8 * CUS && seq_q < 2048;
+        const int w = waves16 <= CUS ? 1 : waves16 <= 640 ? 2 : waves16 <= 4 * CUS || short_walks ? 4 : 8;
         const long q_tiles32 = (seq_q + 31) / 32;
         const long keys = causal ? (seq_k < 32 * q_tiles32 ? seq_k : 32 * q_tiles32) : seq_k;
         const long tiles = (keys + BN - 1) / BN;

@@ -33,8 +33,8 @@ def reference(buf, seq, heads, kv, causal, mask):
 
 @pytest.mark.parametrize("heads,kv,seq,causal,valid,kind,waves,blocks", [
     (24, 24, 1281, 0, None, 1, 8, 2), (24, 8, 1360, 0, 1300, 1, 8, 2), (30, 30, 1025, 0, 65, 1, 8, 2), (30, 30, 1088, 0, None, 1, 8, 2),
-    (24, 24, 1361, 1, None, 0, 8, 1), (32, 8, 1025, 1, 118, 0, 8, 1), (32, 8, 1152, 1, 1152, 0, 8, 1), (32, 8, 1536, 1, None, 0, 8, 1),
-    (32, 8, 1153, 1, 700, 0, 8, 2), (32, 8, 1537, 1, None, 0, 8, 2)])
+    (24, 24, 1361, 1, None, 0, 8, 1), (32, 8, 1025, 1, 118, 0, 4, 1), (32, 8, 1152, 1, 1152, 0, 4, 1), (32, 8, 1536, 1, None, 0, 8, 1),
+    (24, 24, 1536, 1, 500, 0, 4, 1), (16, 16, 2049, 1, 200, 0, 8, 1), (32, 8, 1153, 1, 700, 0, 8, 2), (32, 8, 1537, 1, None, 0, 8, 2)])
 def test_against_32_bits(dev, heads, kv, seq, causal, valid, kind, waves, blocks):
     plan = (C.c_int * 6)()
     dev.lib.iris_hip_fa_hd128_route(seq, seq, heads, causal, int(valid is not None), plan)

@@ -122,6 +122,14 @@ def test_two_waves_share_their_queries_only_where_the_number_of_tiles_is_known_a
     assert parts(193, 193, 24, 1) == (2, 2)
 
 
+def test_causal_walks_behind_a_key_mask_get_smaller_workgroups_over_a_round(parts):
+    """the walks may be short: with eight waves of 16 queries a workgroup they start late"""
+    for heads, seq in ((32, 1025), (32, 1100), (32, 1152), (24, 1380), (24, 1536), (20, 1664)):
+        assert parts(seq, seq, heads, 1, 1) == (4, 1) and parts(seq, seq, heads, 1, 0) == (8, 1)
+    for heads, seq in ((32, 1024), (24, 1280), (16, 2048), (16, 2049), (16, 2300), (8, 4128)):   # one round; long walks
+        assert parts(seq, seq, heads, 1, 1) == (8, 1)
+
+
 # ------------------------------------------------------------------ the linear layers' kernel choice
 @pytest.fixture(scope="module")
 def linear_plan():
