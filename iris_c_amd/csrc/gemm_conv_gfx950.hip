@@ -987,7 +987,8 @@ int iris_hip_conv2d_prepare_scratch(void *stream, uint16_t *scratch) {
     return (int)hipGetLastError();
 }
 
-/* scratch: device buffer of scratch_bytes, 16-byte aligned, prepared once by iris_hip_conv2d_prepare_scratch: the
+/* The routes that copy the image first; they take every shape, and the caller asks iris_hip_conv2d_direct before.
+ * scratch: device buffer of scratch_bytes, 16-byte aligned, prepared once by iris_hip_conv2d_prepare_scratch: the
  * page of zeros, then room for the bf16 image rows of a chunk or (gathered shapes) at least one patch row */
 int iris_hip_conv2d(void *stream, uint16_t *scratch, size_t scratch_bytes, float *out, const float *in,
                     const uint16_t *w, const float *bias, int h, int width, int cin, int cout, int k,
@@ -997,8 +998,6 @@ int iris_hip_conv2d(void *stream, uint16_t *scratch, size_t scratch_bytes, float
     const int ow = (width + pad_before + pad_after - k) / stride + 1;
     if (oh <= 0 || ow <= 0) return 0;
     const int ohw = oh * ow, row_len = k * k * cin;
-    const int direct = iris_hip_conv2d_direct(stream, nullptr, out, in, w, bias, h, width, cin, cout, k, stride, pad_before, oh, ow);
-    if (direct != -2) return direct;
 
     if (scratch_bytes <= IRIS_CONV_ZERO_BYTES) return (int)hipErrorInvalidValue;
     const uint16_t *zeros = scratch;

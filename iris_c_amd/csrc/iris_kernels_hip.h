@@ -162,7 +162,7 @@ int iris_hip_linear_qknorm_plan(int rows, int in, int out, int q_cols, int k_col
 int iris_hip_linear_bf16_qknorm(void *stream, float *part, uint16_t *y, const uint16_t *x, const uint16_t *W, int rows, int in,
                                 int out, int q_cols, int k_cols, const float *wq, const float *wk, const float *rope_cos,
                                 const float *rope_sin, float eps, int split_half);
-/* Convolution. `scratch` is a private device buffer, 16-byte aligned, whose first IRIS_CONV_ZERO_BYTES are zeroed
+/* Convolution of any shape, by way of a copy; iris_hip_conv2d_direct below is asked first. `scratch` is a private device buffer, 16-byte aligned, whose first IRIS_CONV_ZERO_BYTES are zeroed
  * once by iris_hip_conv2d_prepare_scratch and never written again (the page that taps outside the image read);
  * the rest holds the image as bf16 (or the bf16 patches of the shapes that are gathered: >= 2 * k * k * cin bytes). */
 #define IRIS_CONV_ZERO_BYTES 256

@@ -196,6 +196,36 @@ def test_routes_that_copy_the_image_in_chunks_of_the_scratch(dev, route, h, w, c
     np.testing.assert_allclose(got[:want.size].reshape(want.shape), want, atol=2e-5 * np.sqrt(k * k * cin))
 
 
+@pytest.mark.parametrize("h,w,cin,cout,k,stride,pb,pa", [
+    (40, 33, 64, 128, 3, 1, 1, 1), (30, 31, 3, 128, 3, 1, 1, 1), (28, 26, 128, 3, 3, 1, 1, 1), (32, 24, 128, 128, 3, 2, 0, 1), (40, 70, 128, 128, 1, 1, 0, 0)])
+def test_routes_that_copy_the_image_take_every_shape(dev, h, w, cin, cout, k, stride, pb, pa):
+    """Also those that iris_dev_conv2d gives to kernels without a copy: asked once, by it, and not again on the way here."""
+    plan = (C.c_int * 2)()
+    dev.lib.iris_hip_conv2d_plan(C.c_void_p(1 << 44), C.c_void_p(1 << 40), C.c_void_p(1 << 46), h, w, cin, cout, k, stride, pb, pa, plan)
+    assert plan[0] != 0
+    rng = np.random.default_rng(h + w + cout)
+    img = rng.standard_normal((h * w, cin)).astype(np.float32)
+    wt = O.f32_to_bf16((rng.standard_normal((cout, k * k * cin)) * 0.1).astype(np.float32))
+    b = rng.standard_normal(cout).astype(np.float32)
+    want = conv_float64(img, wt, b, h, w, k, stride, pb, pa)
+    scratch_bytes = ZERO_BYTES + h * w * k * k * cin * 2
+    room = dev.put(np.full(scratch_bytes, 0x5a, np.uint8))
+    out = dev.put(np.full(want.size, 7.0, np.float32))
+    vp, ci = C.c_void_p, C.c_int
+    stream = vp(dev.lib.iris_dev_stream())
+    conv = dev.lib.iris_hip_conv2d
+    conv.argtypes = [vp, vp, C.c_size_t, vp, vp, vp, vp] + [ci] * 8
+    dev.lib.iris_hip_conv2d_prepare_scratch.argtypes = [vp, vp]
+    assert dev.lib.iris_hip_conv2d_prepare_scratch(stream, room) == 0
+    assert conv(stream, room, scratch_bytes, out, dev.put(img), dev.put(wt), dev.put(b), h, w, cin, cout, k, stride, pb, pa) == 0
+    dev.check()
+    got = dev.get(out, want.shape, np.float32)
+    page = dev.get(room, (scratch_bytes,), np.uint8)
+    dev.free_all()
+    assert not page[:ZERO_BYTES].any() and (page[ZERO_BYTES:ZERO_BYTES + 64] != 0x5a).any()
+    np.testing.assert_allclose(got, want, atol=2e-5 * np.sqrt(k * k * cin))
+
+
 def test_one_by_one_of_large_images(dev):
     """192 MB of pixels and a pixel less: the same bits, and those of the definition."""
     h, cin, cout = (192 << 20) // (384 * 4), 384, 100
