@@ -128,7 +128,10 @@ void iris_dev_fill_rows(float *out, const float *row, int rows, int dim); /* out
  *   oh = (h + pad_before + pad_after - k) / stride + 1 (same for ow),
  * w: bf16 [cout, k * k * cin] in (ky, kx, c) order, bias may be NULL (reference iris_dev.h:111-121).
  * out may share memory with in as long as the image as bf16 (cin a multiple of 64 and cout >= 128), or else its patches, fit
- * the 256 MB of private scratch: such a call copies them there first, and is slower than one into other memory. */
+ * the 256 MB of private scratch: such a call copies them there first, and is slower than one into other memory.
+ * The input channels of some 3 x 3 convolutions of stride 1 are cut into ranges whose f32 sums pass through the private memory of the linear
+ * layers. Under stream capture they are not; the f32 sums are then taken in another order than the same call's outside. A captured
+ * convolution that copies the image, or its patches, does use the private scratch, so it has to be replayed in order with others that do. */
 void iris_dev_conv2d(float *out, const float *in, const uint16_t *w, const float *bias,
                      int h, int width, int cin, int cout, int k, int stride,
                      int pad_before, int pad_after);

@@ -243,3 +243,62 @@ def test_captured_linear_layer_uses_no_shared_memory(bf16):
     g.rt.hipGraphExecDestroy(run)
     g.rt.hipStreamDestroy(other)
     dev.free_all()
+
+
+def test_captured_convolution_uses_no_shared_memory():
+    """64 x 69, 512 -> 256: the last round of tiles is cut into ranges of input channels, whose sums share the workspace of the linear
+    layers in stream order. Captured, the convolution is one kernel on its own operands, so its replays on another stream give their
+    result beside eager convolutions and layers that use the workspace one after the other, and so do those. The replay sums the
+    channels in another order: f32 rounding apart from the eager call."""
+    import oracle as O
+    from test_gpu_conv_direct import conv_float64
+    dev, g = Dev(), Graphs()
+    lib, stream = dev.lib, _vp(dev.lib.iris_dev_stream())
+    h, w, cin, cout = 64, 69, 512, 256
+    rows, k, out = 300, 4096, 640
+    assert lib.iris_hip_conv2d_cut(h, w, cin, cout) == 1
+    plan = (C.c_int * 2)()
+    lib.iris_hip_linear_plan(rows, k, out, 4, plan)
+    assert plan[0] == 4 and plan[1] > 1
+    rng = np.random.default_rng(9)
+    img = rng.standard_normal((h * w, cin), dtype=np.float32)
+    filters = [O.f32_to_bf16((rng.standard_normal((cout, 9 * cin)) * 0.1).astype(np.float32)) for _ in range(2)]
+    bias = rng.standard_normal(cout).astype(np.float32)
+    want = [conv_float64(img, f, bias, h, w, 3, 1, 1, 1) for f in filters]
+    x = O.f32_to_bf16(rng.standard_normal((rows, k)).astype(np.float32))
+    weight = O.f32_to_bf16((rng.standard_normal((out, k)) * 0.05).astype(np.float32))
+    want_layer = O.bf16_to_f32(x).astype(np.float64) @ O.bf16_to_f32(weight).astype(np.float64).T
+    dimg, dbias, dx, dweight = dev.put(img), dev.put(bias), dev.put(x), dev.put(weight)
+    f1, f2 = [dev.put(f) for f in filters]
+    captured, eager, layer = dev.alloc(h * w * cout * 4), dev.alloc(h * w * cout * 4), dev.alloc(rows * out * 4)
+    conv = lambda dst, f: lib.iris_dev_conv2d(dst, dimg, f, dbias, h, w, cin, cout, 3, 1, 1, 1)
+
+    conv(eager, f2)
+    dev.check()
+    lib.iris_dev_sync()
+    first = dev.get(eager, (h * w, cout), np.float32)
+    run = g.capture(stream, lambda: conv(captured, f1))
+    assert g.nodes == 1
+    dev.check()
+    lib.iris_dev_sync()
+    other = _vp()
+    assert g.rt.hipStreamCreate(C.byref(other)) == 0
+    junk = np.full(h * w * cout, np.nan, np.float32)
+    for replay in range(4):
+        for p, n in ((captured, h * w * cout), (eager, h * w * cout), (layer, rows * out)):
+            lib.iris_dev_upload(p, junk.ctypes.data_as(_vp), n * 4)
+        for _ in range(8):
+            assert g.rt.hipGraphLaunch(run, other) == 0
+            conv(eager, f2)
+            lib.iris_dev_linear_f32(layer, dx, dweight, rows, k, out)
+        assert g.rt.hipStreamSynchronize(other) == 0
+        lib.iris_dev_sync()
+        dev.check()
+        got = dev.get(eager, (h * w, cout), np.float32)
+        assert np.array_equal(got, first)
+        for v, e in ((dev.get(captured, (h * w, cout), np.float32), want[0]), (got, want[1])):
+            np.testing.assert_allclose(v.reshape(e.shape), e, atol=2e-5 * np.sqrt(9 * cin))
+        np.testing.assert_allclose(dev.get(layer, (rows, out), np.float32), want_layer, atol=2e-5 * np.sqrt(k) * 0.05)
+    g.rt.hipGraphExecDestroy(run)
+    g.rt.hipStreamDestroy(other)
+    dev.free_all()
