@@ -55,6 +55,20 @@ def test_against_32_bits(dev, seq_q, seq_k, valid):
     assert_parity(O.bf16_to_f32(out), reference(buf, seq_q, seq_k, mask), f"{seq_q} x {seq_k}")
 
 
+@pytest.mark.parametrize("hidden", ["the first tile", "even tiles", "odd tiles", "all but the last key", "the first of each tile"])
+@pytest.mark.parametrize("seq_q,seq_k", [(1089, 1089), (1100, 1153)])
+def test_masks_that_hide_all_that_one_of_two_waves_has_taken_so_far(dev, seq_q, seq_k, hidden):
+    """Two waves take the tiles of 64 keys in turn: one may have met no valid key yet, or none at all, when they merge."""
+    assert route(dev, seq_q, seq_k, True)[0] == 3
+    key = np.arange(seq_k)
+    mask = {"the first tile": key >= 64, "even tiles": key // 64 % 2 == 1, "odd tiles": key // 64 % 2 == 0, "all but the last key": key == seq_k - 1,
+            "the first of each tile": key % 64 != 0}[hidden].astype(np.int32)
+    buf, q = rows(max(seq_q, seq_k)), HEADS * 128
+    out, kernel = dev.attention(buf, q + 2 * KV * 128, 0, q, q + KV * 128, seq_q, seq_k, HEADS, KV, 128, 128 ** -0.5, False, mask)
+    assert kernel == "fa_hd128"
+    assert_parity(O.bf16_to_f32(out), reference(buf, seq_q, seq_k, mask), f"{seq_q} x {seq_k}, {hidden} hidden")
+
+
 def test_no_valid_key_gives_zero_rows(dev):
     assert route(dev, 1089, 1089, True)[0] == 3
     q = HEADS * 128

@@ -40,7 +40,8 @@ def test_short_sequences_split_the_keys_when_workgroups_are_few(plan):
 
 @pytest.mark.parametrize("heads", [8, 16, 20, 24, 30, 32, 40, 48])
 def test_two_size_grids_cover_every_query_and_never_lose_to_one_size(plan, heads):
-    for seq in range(2048 * 16 // heads + 64, 9000, 331):
+    kinds = set()
+    for seq in list(range(2048 * 16 // heads + 64, 9000, 331)) + list(range(2048 * 16 // heads + 40, 9000, 197)):
         p = plan(seq, seq, heads)
         assert p["waves"] in (4, 8) and p["nb"] == 2, (seq, p)
         if p["kind"] == 1:
@@ -51,7 +52,15 @@ def test_two_size_grids_cover_every_query_and_never_lose_to_one_size(plan, heads
             rounds_one_size = -(-(-(-seq // 256) * heads) // 256)
             per_engine = -(-(full_x + tail_x) // 4)
             assert per_engine <= 8 * (rounds_one_size + 1), (seq, p)
+        if p["kind"] == 3:
+            assert p["full"] >= 0 and 256 * p["full"] <= seq, (seq, p)
+            assert 64 * (p["tails"] - 1) < seq - 256 * p["full"] <= 64 * p["tails"], (seq, p)
+            # a 64-query workgroup at 0.33 and two key tiles of a 256-query one: dealt evenly they take 5 % less than whole rounds of one size
+            tail = 33 + 200 // -(-seq // 64)
+            assert heads * (100 * p["full"] + tail * p["tails"]) <= 256 * 95 * -(-(-(-seq // 256) * heads) // 256), (seq, p)
+        kinds.add(p["kind"])
         assert plan(seq, seq, heads, 1)["kind"] == 0                                      # causal calls keep one size
+    assert {1, 3} <= kinds
 
 
 def test_a_few_workgroups_over_a_round_become_small_ones(plan):
