@@ -387,8 +387,8 @@ int launch_1x1(hipStream_t st, float *out, const float *in, const uint16_t *W, c
  *    second half. The operands of a half are read from the LDS in the gaps between the products of the half before, one to
  *    a gap, behind its first four (a decoder stage 128 x 128, 512 -> 512, from the first gap on 860.5 us, behind four 849.5, behind six 853.5), across
  *    the barrier too: four of weights, and of a tap's four rows of pixels one where the tap before was the one above
- *    it, which the order of the taps makes two of three (all four read for every tap: 512 x 512, 256 -> 256 249 us / 243, 256 -> 128
- *    135.7 / 131.9, 256 x 256, 512 -> 512 228 / 222). They issue no load and wait for none, so a tile's stores drain under the next tile.
+ *    it, which the order of the taps makes two of three (all four read for every tap: 2 - 3 % more on the sizes below).
+ *    They issue no load and wait for none, so a tile's stores drain under the next tile.
  *  - Waves 8 - 11 bring everything in. The image: 2592 units of 8 channels x pixel per group of 64 channels, 11 a thread,
  *    all of them in registers on their way while the group before is multiplied. One or two a step are rounded and written
  *    to the image buffer that the last group has left (the epilogue borrows it until the barrier of step 0), and
@@ -407,7 +407,9 @@ int launch_1x1(hipStream_t st, float *out, const float *in, const uint16_t *W, c
  * Measured against a bf16 copy of the image + implicit product that fetches every tap from the L2 (copy + product), against
  * eight waves that did everything (and stood still while a tile's stores landed), and these roles: 512 x 512 pixels, 128 -> 128
  * 30 + 118, 79, 73 us (the image and the result alone take 50 us to move), 256 -> 128 76 + 214, 129, 123, 256 -> 256 88 + 290,
- * 253, 235 us (1320 TFLOP/s). The first is bound by memory (matrix cores busy 43 - 45 % of its cycles), the last by the products
+ * 253, 235 us. Then the taps down the columns and the reads behind four products, on a slower chip: these roles / now, the image in the Infinity Cache,
+ * 75.9 / 74.3, 137.3 / 133.3, 257.9 / 250.3 (1240 TFLOP/s, 0.87 us a step), 256 x 256, 512 -> 512 228.5 / 218.9; the image from memory 80.8 / 79.7, 140.0 / 135.6, 257.9 /
+ * 251.0, 235.7 / 226.5. The first is bound by memory (matrix cores busy 43 - 45 % of its cycles), the last by the products
  * at the clock that the chip's power leaves (62 - 64 % at 1.9 - 2.0 GHz of 2.4; counters, under the profiler). Pixels and
  * weights on waves of their own (three and one) 1 % slower. */
 constexpr int C3_T = 16, C3_H = C3_T + 2, C3_PIXELS = C3_H * C3_H, C3_ROW = 80, C3_IMG = C3_PIXELS * C3_ROW;   /* elements */
@@ -424,8 +426,10 @@ static_assert(c3_first(9) == C3_UNITS && c3_units(0) == 0, "");
 __device__ constexpr int c3_tap(int t) { return t % 3 * 3 + t / 3; }
 
 /* Results of up to 64 MB are written through (write_through.h), larger ones stay for the operator that reads them next: us, plain /
- * through, a decoder stage 64 x 70, 512 -> 512 298.7 / 293.1, the first encoder stage 150 x 200 106.7 / 105.0, 256 x 256 143.0 / 141.7, 320 x 330 (54 MB)
- * 204.5 / 203.3, 512 x 512 (134 MB) 399.3 / 408.0. */
+ * through, a decoder stage 64 x 70, 512 -> 512 308.0 / 301.8, the first encoder stage 150 x 200 107.1 / 104.3, 256 x 256 144.0 / 141.9, 320 x 330 (54 MB)
+ * 205.3 / 203.8, 512 x 512 (134 MB) 399.3 / 408.0; alone 256 x 256, 128 -> 128 (34 MB) 24.3 / 23.2, 128 x 250, 512 -> 512 (66 MB) 117.5 / 117.2, 256 x 256, 256 -> 256 (67
+ * MB) 67.0 / 66.7, 181 x 181, 512 -> 512 137.4 / 138.5, 362 x 362, 128 -> 128 (67 MB) 53.9 / 54.2, 400 x 400 (82 MB) 58.6 / 61.5, 450 x 450 77.4 / 82.0,
+ * 362 x 362, 256 -> 256 (134 MB) 143.6 / 146.7; but 1024 x 1024, 128 -> 128 (537 MB) 310.4 / 308.4. */
 constexpr size_t C3_THROUGH_MOST = (size_t)64 << 20;
 constexpr int C3_SLOTS = 32, C3_PART = 4096;                   /* CUs of an XCD; floats of a wave's sums */
 static_assert((size_t)16 * C3_SLOTS * C3_MUL * C3_PART * 4 <= IRIS_LINEAR_PART_BYTES, "two places a workgroup");
@@ -681,7 +685,9 @@ k_conv_3x3(float *__restrict__ out, const float *__restrict__ in, const uint16_t
         }
     };
 
-    /* the sums of a range of channel groups, as the registers hold them: 128 KB, two places a workgroup */
+    /* the sums of a range of channel groups, as the registers hold them: 128 KB, two places a workgroup. Written through, as the next
+     * kernel reads them: us, plain / through, decoder stages 32 x 32, 512 -> 512 128.0 / 125.7, 64 x 70 305.7 / 301.9, 33 x 40, 512 -> 256 148.9 / 143.7, 64 x 64,
+     * 256 -> 128 129.6 / 130.0; alone 32 x 32, 512 -> 512 19.2 / 18.3, 64 x 64 31.3 / 30.3, 16 x 16 15.5 / 16.4, 64 x 64, 256 -> 256 17.5 / 18.1. */
     auto store_part = [&](int w) {
         float *dst = part + ((size_t)(2 * blockIdx.x + (w != p_w)) * C3_MUL + wave) * C3_PART;
 #pragma unroll
@@ -817,7 +823,10 @@ int launch_3x3(hipStream_t st, float *part, float *out, const float *in, const u
  * the products otherwise. Against a bf16 copy of the image + implicit product: 512 x 512, 128 -> 128 63 -> 42 us, 1024 x 1024
  * 304 -> 164, 128 x 128 30 -> 12, 256 x 256, 256 -> 256 77 -> 28, 128 x 128, 512 -> 512 119 -> 42, 256 x 256 143 -> 113. Pixels
  * straight into registers under every tap instead of a shared tile (nine reads of 2.25 outputs' pixels each): 55 us for the
- * first, 92 for 256 -> 256: a CU takes in 50 - 65 KB/us of what is not in its XCD's L2. */
+ * first, 92 for 256 -> 256: a CU takes in 50 - 65 KB/us of what is not in its XCD's L2.
+ * Results are written through (write_through.h) at every size: us, plain / through, image from memory, 512 x 512, 128 -> 128 (34 MB) 45.7 / 44.6, 640 x 640 75.5 /
+ * 75.8, 724 x 724 (67 MB) 93.6 / 94.1, 800 x 800 102.3 / 103.6, 900 x 900 (104 MB) 136.4 / 136.1, 1024 x 1024 (134 MB) 163.3 / 163.0, 256 -> 256 362 x 362 (34 MB) 87.5 / 86.6,
+ * 512 x 512 (67 MB) 128.2 / 128.0, 724 x 724 (134 MB) 282.6 / 279.7, 512 -> 512 256 x 256 (34 MB) 110.4 / 109.1, 400 x 400 (82 MB) 325.6 / 322.1, 512 x 512 440.4 / 437.6. */
 constexpr int H3_TY = 8, H3_TX = 16, H3_HY = 2 * H3_TY + 1, H3_HX = 2 * H3_TX + 1, H3_PIXELS = H3_HY * H3_HX, H3_C = 32, H3_ROW = 40;
 constexpr int H3_IMG = H3_PIXELS * H3_ROW, H3_TAP = C3_N * H3_C, H3_STAGE = 3 * H3_TAP;      /* elements */
 constexpr int H3_BRING = 3, H3_THREADS = 64 * (C3_MUL + H3_BRING + 1), H3_PIECES = H3_STAGE / 512;

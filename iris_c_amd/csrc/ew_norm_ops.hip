@@ -44,11 +44,13 @@ __device__ __forceinline__ float bf_lo(uint32_t u) { return __uint_as_float(u <<
 __device__ __forceinline__ float bf_hi(uint32_t u) { return __uint_as_float(u & 0xffff0000u); }
 __device__ __forceinline__ float silu(float v) { return v / (1.0f + __expf(-v)); }
 
-/* Written through, while others are still read: us, plain / written through, operands from memory: LayerNorm 1000 x 2560 6.3 / 5.7, 2115 x 3072 11.1 /
- * 10.7, residual 1000 x 2560 8.0 / 7.5, 4608 x 3072 31.2 / 29.3; operands in the Infinity Cache: LayerNorm
- * 2115 x 3072 8.1 / 6.8, residual 12.3 / 8.8, SwiGLU 512 x 9728 5.6 / 4.3. A text-encoder layer of 512 rows 166.5 / 165.1, a single-stream
- * block of 320 rows 118.6 / 117.6, a double-stream block of 2627 803 / 800. Only where the result is what another operator reads:
- * rms_norm_residual and add_bias, called again on the same rows, find them in the L2 (12800 x 3072 76 / 86, 16384 x 512 7.7 / 10.4). */
+/* Add, residual, SwiGLU and row norms store their results through the L2s (write_through.h), while other rows are still read. What counts is the
+ * operator and the one that reads its result behind it: us, plain / written through, residual + LayerNorm 16 - 400 rows of 2560 and 3072
+ * the same (8.1 - 8.5), 1000 x 3072 11.9 / 10.2, 2115 20.8 / 19.9, 4608 39.4 / 38.3, 12800 (157 MB) 117.7 / 117.4, 12000 x 4096 155.6 / 151.7; LayerNorm + a product of
+ * it 16 and 64 rows the same, 100 x 3072 17.3 / 17.1, 400 23.1 / 22.8, 1000 30.4 / 29.5, 4608 85.7 / 84.8, 12800 234.6 / 234.9; SwiGLU + a product 16 x 9728 the same,
+ * 64 rows 19.5 / 19.3, 512 39.6 / 39.2, 4608 x 9216 201.3 / 200.4, 12800 544 / 538; add + group norm of 8 MB 17.3 / 17.2, 134 MB 106.7 / 105.8, 537 MB 518 / 513.
+ * None of 40 such pairs from 0.1 to 537 MB was slower by more than 0.4 %, so there is no bound on either side. rms_norm_residual and add_bias, called again and
+ * again on the same rows, were slower for it (12800 x 3072 76 / 86, 16384 x 512 7.7 / 10.4) and store plainly; with a reader behind them they were not timed. */
 inline unsigned blocks_for(size_t n, int per_block) { return (unsigned)((n + per_block - 1) / per_block); }
 
 /* ---------------------------------------------------------------- elementwise */
