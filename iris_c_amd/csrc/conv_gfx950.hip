@@ -47,15 +47,23 @@ struct ConvShape {
  * registers and walks groups of 16 consecutive pixels: a lane gathers its eight patch values (cached: neighbouring
  * pixels share them), eight products, and the 16 x 128 results leave through the LDS as whole 512-byte rows.
  * What bounds it is the output stream, as long as little else is done: a workgroup puts its weights and the places of the
- * patch's values together once in the LDS (a thread of the form before read 64 weights one by one and divided eight times), and
- * a group that lies inside the image adds eight offsets to one address and tests nothing. 3 -> 128 on 512 x 512 (134 MB out): 902 us
- * as patches + scalar product + bias, 32 - 39 us with every value tested and divided for (image cached / from memory), 25 - 30 now (5.4 TB/s);
- * 256 x 256 20 -> 10 - 12, 301 x 290 24 -> 14, 1024 x 1024 123 -> 108, 400 x 400, 3 -> 256 50 -> 37, 512 x 512, 3 -> 64 with stride 2 14 -> 9. */
+ * patch's values together once in the LDS (a thread of the form before read 64 weights one by one and divided eight times), the
+ * weights are on their way beside the first pixels, and a group that lies inside the image adds eight offsets to one address and tests
+ * nothing. 3 -> 128 on 512 x 512 (134 MB out): 902 us as patches + scalar product + bias, 38.5 with every value tested and divided for, 28.4 without, 26.2
+ * with the weights beside the pixels; likewise 64 x 64 7.1, 6.7, 5.2, 256 x 256 20.0, 10.1, 8.9, 300 x 300 23.4, 12.8, 11.3, 1024 x 1024 123, 108, 103,
+ * 400 x 400, 3 -> 256 48.8, 36.7, 32.7, and, where the tests were few, 64 x 64, 4 -> 128 with 1 x 1 5.8, 6.5, 5.2, 128 x 128 6.7, 7.2, 6.0. */
 constexpr int FI_WAVES = 4, FI_COLS = 128, FI_BEYOND = 1 << 28;
-/* Whole 512-byte pieces of a row are written through as they are stored, as long as the result is neither too small to gain by it nor
- * larger than the Infinity Cache: us, plain / through, 64 x 64, 3 -> 128 (2 MB) 6.2 / 7.4, 128 x 128 7.1 / 7.6, 180 x 180 (17 MB) 9.3 / 8.5,
- * 512 x 512 35 / 30, 1024 x 1024 (537 MB) 108 / 115; rows that are not made of such pieces 512 x 512, 3 -> 64 24.9 / 26.4, 7 -> 260 34 / 40. */
-constexpr size_t FI_THROUGH_LEAST = (size_t)12 << 20, FI_THROUGH_MOST = (size_t)256 << 20;
+/* Whole 512-byte pieces of a row are written through as they are stored, as long as the result is not larger than the Infinity Cache: us,
+ * plain / through, 64 x 64, 3 -> 128 (2 MB) 4.4 / 4.3, 128 x 128 5.3 / 4.7, 180 x 180 7.1 / 5.9, 362 x 362 14.9 / 13.7, 512 x 512 30.6 / 26.2, 724 x 724 (268 MB) 55.1 /
+ * 54.3, 1024 x 1024 (537 MB) 103 / 120; 3 -> 512 32 x 32 4.9 / 4.9, 100 x 100 7.8 / 6.8, 362 x 362 (268 MB) 53.0 / 48.9, 512 x 512 104 / 96. Rows that are not made of
+ * such pieces lose by it (512 x 512, 3 -> 64 24.9 / 26.4, 7 -> 260 34 / 40). */
+constexpr size_t FI_THROUGH_MOST = (size_t)256 << 20;
+/* A wave has up to eight pieces on their way at once. Large results in wide rows, and the largest, are faster with one (PACED). us, eight / one,
+ * 3 -> 1024 160 x 160 (105 MB) 23.0 / 24.4, 181 x 181 31.8 / 29.0, 256 x 256 61.8 / 50.3, 362 x 362 127 / 106; 768 181 x 181 (100 MB) 19.9 / 22.1, 256 x 256 42.0 /
+ * 40.5, 300 x 300 58.0 / 55.8; 512 200 x 200 (82 MB) 16.6 / 18.3, 256 x 256 (134 MB) 27.8 / 27.7, 362 x 362 50.7 / 49.3; 256 362 x 362 (134 MB) 27.2 / 31.7, 600 x 600 73.7 /
+ * 80.3; 128 420 x 420 19.3 / 22.9, 724 x 724 54.6 / 60.4, 900 x 900 (415 MB) 84.3 / 85.1, 1024 x 1024 110.6 / 103.3. */
+constexpr size_t FI_EIGHT_MOST = (size_t)480 << 20, FI_EIGHT_MOST_WIDE = (size_t)120 << 20;
+constexpr int FI_WIDE = 4;                                     /* tiles of 128 channels */
 
 /* p / ow for p < 2^30: umulhi(p, magic) >> shift, magic = ceil(2^(32 + shift) / ow) with 2^shift < ow <= 2^(shift + 1); 0: ow is 1 */
 struct RowOf { unsigned magic, shift; };
@@ -66,7 +74,7 @@ inline RowOf row_of(unsigned ow) {
     return {(unsigned)(((1ull << (32 + shift)) + ow - 1) / ow), shift};
 }
 
-template <bool ALIGNED, bool THROUGH>
+template <bool ALIGNED, bool THROUGH, bool PACED>
 __global__ void __launch_bounds__(64 * FI_WAVES, 4)
 k_conv_few_in(float *__restrict__ out, const float *__restrict__ in, const uint16_t *__restrict__ W, const float *__restrict__ bias,
               ConvShape s, RowOf row_of, int small, int groups) {
@@ -76,34 +84,36 @@ k_conv_few_in(float *__restrict__ out, const float *__restrict__ in, const uint1
     const int row_len = s.k * s.k * s.cin, pixels = s.oh * s.ow;
     float *buf = lds + wave * 16 * FI_COLS;
 
-    /* rows of 32 weights, zeros behind the patch; and for patch value r its tap's row and column (row FI_BEYOND: beyond the patch,
-     * never inside the image) and its offset from the patch's first value */
+    /* rows of 32 weights, zeros behind the patch, on their way beside the first group's pixels; and for patch value r its tap's row and
+     * column (row FI_BEYOND: beyond the patch, never inside the image) and its offset from the patch's first value */
     uint16_t *w_lds = reinterpret_cast<uint16_t *>(lds);
     int *tap_y = reinterpret_cast<int *>(lds + FI_COLS * 16), *tap_x = tap_y + 32, *tap_off = tap_y + 64;
-#pragma unroll
-    for (int i = 0; i < FI_COLS * 32 / (64 * FI_WAVES); i++) {
-        const int e = threadIdx.x + 64 * FI_WAVES * i, n = n0 + (e >> 5), j = e & 31;
-        w_lds[e] = n < s.cout && j < row_len ? W[(size_t)n * row_len + j] : (uint16_t)0;
-    }
     if (threadIdx.x < 32) {
         const int r = threadIdx.x, tap = r / s.cin, c = r - tap * s.cin, y = tap / s.k, x = tap - y * s.k;
         tap_y[r] = r < row_len ? y : FI_BEYOND;
         tap_x[r] = x;
         tap_off[r] = r < row_len ? (y * s.w + x) * s.cin + c : 0;
     }
-    __syncthreads();
-    u32x4 av[8];
+    uint16_t wv[FI_COLS * 32 / (64 * FI_WAVES)];
 #pragma unroll
-    for (int a = 0; a < 8; a++) av[a] = *reinterpret_cast<const u32x4 *>(&w_lds[(16 * a + li) * 32 + 8 * lg]);
+    for (int i = 0; i < FI_COLS * 32 / (64 * FI_WAVES); i++) {
+        const int e = threadIdx.x + 64 * FI_WAVES * i, n = n0 + (e >> 5), j = e & 31;
+        const bool there = n < s.cout && j < row_len;
+        const uint16_t t = W[there ? (size_t)n * row_len + j : 0];
+        wv[i] = there ? t : (uint16_t)0;
+    }
+    const int c = lane & 31, n = n0 + 4 * c;
+    f32x4 bv;                                                  /* of the four channels this lane stores */
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const bool there = bias && n + r < s.cout;
+        const float t = *(there ? bias + n + r : in);
+        bv[r] = there ? t : 0.0f;
+    }
+    __syncthreads();
     int dy[8], dx[8], off[8];                                  /* of patch values 8 lg + j */
 #pragma unroll
     for (int j = 0; j < 8; j++) { dy[j] = tap_y[8 * lg + j]; dx[j] = tap_x[8 * lg + j]; off[j] = tap_off[8 * lg + j]; }
-    const int c = lane & 31, n = n0 + 4 * c;
-    f32x4 bv = {0, 0, 0, 0};                                   /* of the four channels this lane stores */
-#pragma unroll
-    for (int r = 0; r < 4; r++)
-        if (bias && n + r < s.cout) bv[r] = bias[n + r];
-    __syncthreads();                                           /* the LDS is the waves' from here on */
 
     float v[8];
     auto fetch = [&](int g) {
@@ -131,6 +141,13 @@ k_conv_few_in(float *__restrict__ out, const float *__restrict__ in, const uint1
     };
     int g = column * FI_WAVES + wave;
     if (g < groups) fetch(g);
+#pragma unroll
+    for (int i = 0; i < FI_COLS * 32 / (64 * FI_WAVES); i++) w_lds[threadIdx.x + 64 * FI_WAVES * i] = wv[i];
+    __syncthreads();
+    u32x4 av[8];
+#pragma unroll
+    for (int a = 0; a < 8; a++) av[a] = *reinterpret_cast<const u32x4 *>(&w_lds[(16 * a + li) * 32 + 8 * lg]);
+    __syncthreads();                                           /* the LDS is the waves' from here on */
     for (; g < groups; g += columns * FI_WAVES) {
         const u32x4 b = {pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7])};
         /* lane: channels 16 a + 4 lg .. + 3 of pixel li. 16-byte chunk c of pixel r in slot (c & 16) | ((c ^ r) & 15): the
@@ -148,6 +165,7 @@ k_conv_few_in(float *__restrict__ out, const float *__restrict__ in, const uint1
             const int row = 2 * it + (lane >> 5);
             const f32x4 r = *reinterpret_cast<const f32x4 *>(&buf[row * FI_COLS + 4 * ((c & 16) | ((c ^ row) & 15))]) + bv;
             float *dst = first + (unsigned)(row * s.cout + 4 * c);
+            if (PACED) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             if (16 * g + row >= pixels) continue;
             if (ALIGNED && THROUGH) {
                 if (n < s.cout) store_through(dst, r);
@@ -1102,8 +1120,9 @@ inline bool overlap(const void *a, size_t a_bytes, const void *b, size_t b_bytes
 }
 
 /* Workgroups of k_conv_few_in per tile of channels. Four run on a CU at once, and one fetches its weights once for all its groups, so
- * 1024 in all: with 1280 512 x 512 pixels, 3 -> 128 take 38 us in place of 30, with 1024 for each of four tiles (1 x 1, 4 -> 512 over
- * 200 x 200) 26 in place of 21. Of two or three tiles twice as many, within a tenth of the time (400 x 400, 3 -> 256 38 us / 34). */
+ * 1024 in all: with 1280 512 x 512 pixels, 3 -> 64 take 18.7 us in place of 16.4, 1024 x 1024, 3 -> 128 123 in place of 103, with 1280 for each of eight tiles
+ * (256 x 256, 3 -> 1024) 77 in place of 50. Of two or three tiles twice as many, within a tenth of the time either way (us, 1024 in all / twice as many, 400 x 400,
+ * 3 -> 256 34.8 / 32.8, 512 x 512 52.9 / 53.2, 256 x 256 13.7 / 15.2). */
 inline unsigned few_in_columns(int groups, int cout) {
     const int tiles_n = (cout + FI_COLS - 1) / FI_COLS, most = tiles_n == 1 ? 1024 : tiles_n < 4 ? 2048 / tiles_n : tiles_n < 1024 ? 1024 / tiles_n : 1;
     return groups < most * FI_WAVES ? (unsigned)(groups + FI_WAVES - 1) / FI_WAVES : (unsigned)most;
@@ -1238,11 +1257,12 @@ int iris_hip_conv2d_direct(void *stream, float *part, float *out, const float *i
         const RowOf rows = row_of((unsigned)ow);
         const int small = (size_t)h * width * cin * 4 < (size_t)1 << 31;          /* 32-bit byte offsets */
         const size_t out_bytes = (size_t)oh * ow * cout * 4;
-        const bool through = cout % FI_COLS == 0 && out_bytes >= FI_THROUGH_LEAST && out_bytes <= FI_THROUGH_MOST;
+        const bool through = cout % FI_COLS == 0 && out_bytes <= FI_THROUGH_MOST;
         auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(64 * FI_WAVES), 0, st, out, in, w, bias, s, rows, small, groups); };
-        if (cout % 4 || !al16(out)) go(k_conv_few_in<false, false>);
-        else if (through) go(k_conv_few_in<true, true>);
-        else go(k_conv_few_in<true, false>);
+        const bool paced = out_bytes > (tiles_n >= FI_WIDE ? FI_EIGHT_MOST_WIDE : FI_EIGHT_MOST);
+        if (cout % 4 || !al16(out)) go(k_conv_few_in<false, false, false>);
+        else if (paced) go(through ? k_conv_few_in<true, true, true> : k_conv_few_in<true, false, true>);
+        else go(through ? k_conv_few_in<true, true, false> : k_conv_few_in<true, false, false>);
         return (int)hipGetLastError();
     }
     case FEW_OUT:

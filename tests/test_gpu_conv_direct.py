@@ -40,6 +40,23 @@ def test_few_input_channels(dev, orc, h, w, cin, cout, k, stride, pb, pa, bias):
     conv_case(dev, orc, h, w, cin, cout, k, stride, pb, pa, bias)
 
 
+@pytest.mark.parametrize("h,w,cout", [(247, 248, 512), (250, 250, 512), (245, 250, 516), (170, 181, 1024), (333, 65, 1500)])
+def test_few_input_channels_wide_results_around_120_megabytes(dev, h, w, cout):
+    """One store of a wave on its way from there on, written through in whole pieces of 128 channels or not"""
+    rng = np.random.default_rng(cout)
+    img = rng.standard_normal((h * w, 3)).astype(np.float32)
+    wt = O.f32_to_bf16((rng.standard_normal((cout, 27)) * 0.1).astype(np.float32))
+    b = rng.standard_normal(cout).astype(np.float32)
+    want = conv_float64(img, wt, b, h, w, 3, 1, 1, 1)
+    out = dev.put(np.full(want.size + 64, 7.0, np.float32))
+    dev.lib.iris_dev_conv2d(out, dev.put(img), dev.put(wt), dev.put(b), h, w, 3, cout, 3, 1, 1, 1)
+    dev.check()
+    got = dev.get(out, (want.size + 64,), np.float32)
+    dev.free_all()
+    assert (got[want.size:] == 7.0).all()
+    np.testing.assert_allclose(got[:want.size].reshape(want.shape), want, atol=2e-5 * np.sqrt(27))
+
+
 @pytest.mark.parametrize("h,w,cin,cout,k,stride,pb,pa,bias", [
     (1, 1, 128, 3, 3, 1, 1, 1, True), (16, 32, 128, 3, 3, 1, 1, 1, True), (17, 33, 128, 3, 3, 1, 1, 1, False),
     (40, 70, 32, 3, 3, 1, 1, 1, True), (15, 31, 64, 2, 3, 1, 0, 0, True), (33, 20, 64, 28, 1, 1, 0, 0, True),
