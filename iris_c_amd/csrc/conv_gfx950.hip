@@ -50,8 +50,10 @@ struct ConvShape {
  * patch's values together once in the LDS (a thread of the form before read 64 weights one by one and divided eight times), the
  * weights are on their way beside the first pixels, and a group that lies inside the image adds eight offsets to one address and tests
  * nothing. 3 -> 128 on 512 x 512 (134 MB out): 902 us as patches + scalar product + bias, 38.5 with every value tested and divided for, 28.4 without, 26.2
- * with the weights beside the pixels; likewise 64 x 64 7.1, 6.7, 5.2, 256 x 256 20.0, 10.1, 8.9, 300 x 300 23.4, 12.8, 11.3, 1024 x 1024 123, 108, 103,
- * 400 x 400, 3 -> 256 48.8, 36.7, 32.7, and, where the tests were few, 64 x 64, 4 -> 128 with 1 x 1 5.8, 6.5, 5.2, 128 x 128 6.7, 7.2, 6.0. */
+ * with the weights beside the pixels; likewise 64 x 64 7.1, 6.7, 5.2, 256 x 256 20.0, 10.1, 8.9, 300 x 300 23.4, 12.8, 11.3, 1024 x 1024 123, 108, 106,
+ * 400 x 400, 3 -> 256 48.8, 36.7, 32.7, and, where the tests were few, 64 x 64, 4 -> 128 with 1 x 1 5.8, 6.5, 5.2, 128 x 128 6.7, 7.2, 6.0.
+ * A lane without a patch value to read reads the image's first: beside the pixel's own values (more cache lines, read for nothing) 1 x 1, 4 -> 128 on
+ * 1024 x 1024 119.0 / 115.5, 900 x 900 93.4 / 83.5, 4 -> 256 on 700 x 700 111.3 / 104.3, 16 -> 200 on 128 x 128 7.3 / 6.8; 3 x 3, 3 -> 128 the same. */
 constexpr int FI_WAVES = 4, FI_COLS = 128, FI_BEYOND = 1 << 28;
 /* Whole 512-byte pieces of a row are written through as they are stored, as long as the result is not larger than the Infinity Cache: us,
  * plain / through, 64 x 64, 3 -> 128 (2 MB) 4.4 / 4.3, 128 x 128 5.3 / 4.7, 180 x 180 7.1 / 5.9, 362 x 362 14.9 / 13.7, 512 x 512 30.6 / 26.2, 724 x 724 (268 MB) 55.1 /
@@ -124,7 +126,10 @@ k_conv_few_in(float *__restrict__ out, const float *__restrict__ in, const uint1
         if (small && __all(whole)) {
             const unsigned base = (unsigned)(y0 * s.w + x0) * (unsigned)s.cin;
 #pragma unroll
-            for (int j = 0; j < 8; j++) v[j] = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(in) + 4u * (base + (unsigned)off[j]));
+            for (int j = 0; j < 8; j++) {                      /* what is beyond the patch reads one place, whichever the pixel */
+                const unsigned at = dy[j] == FI_BEYOND ? 0 : base + (unsigned)off[j];
+                v[j] = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(in) + 4u * at);
+            }
 #pragma unroll
             for (int j = 0; j < 8; j++)
                 if (dy[j] == FI_BEYOND) v[j] = 0.0f;
